@@ -143,7 +143,8 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
         for (int64_t k = lo; k < hi; ++k) {
             const int64_t o = offsets[k], n = offsets[k + 1] - offsets[k];
             mono[k] = (uint8_t)((forest_monotone(r_comov + o, n) ? 1 : 0) |
-                                (forest_monotone(dist_m + o, n) ? 2 : 0));
+                                (forest_monotone(dist_m + o, n) ? 2 : 0) |
+                                (forest_monotone(z + o, n) ? 4 : 0));
         }
     });
     double max_r = 0, max_d = 0;
@@ -339,6 +340,10 @@ int picca_xi_set_pairs(picca_ctx *ctx, int64_t num_pairs, const int32_t *pair_a,
 
 namespace {
 
+// Windows of r_par rows up to which the cross-correlation takes the specialised kernel: 16
+// windows of 50 rows hold 800 x 50 bins.
+constexpr int XI_MAX_ROW_WINDOWS = 16;
+
 // picca_xi_execute's work with the output rows, the work-queue head and the counters in the
 // given device buffers (out: num_rows * np*nt records; queue: 1 word; stats: XI_NSTATS
 // words), all cleared here by kernels.  Allocates nothing.
@@ -346,8 +351,11 @@ int xi_execute_into(picca_ctx *ctx, const picca::XiConst &C0, int mode,
                     const picca_cf_params *params, picca::XiBin *out, unsigned long long *queue,
                     unsigned long long *stats_dev, bool allow_graph, picca_xi_report *report) {
     picca::XiConst C = C0;
-    // the specialised kernel: standard binning, auto-correlation, r_par_min == 0, no cuts
-    const bool general = !picca::xi_specialised(params, mode);
+    // the specialised kernel: standard binning, auto-correlation with r_par_min == 0 or
+    // cross-correlation
+    bool general = !picca::xi_fast_path(params, mode);
+    const bool cuts = picca::xi_has_cuts(params);
+    const bool xcorr = params->x_correlation != 0;
     // the automatic schedule keeps the pair loop's kernel (no walk) when the store's pixels
     // are too dense for runs of XI_WALK_MIN_DENSITY pixels per r_par bin
     const bool dense = ctx->median_step_r > 0 &&
@@ -366,13 +374,34 @@ int xi_execute_into(picca_ctx *ctx, const picca::XiConst &C0, int mode,
     };
     bool lds_hist = false;
     size_t lds = 0;
-    if (!general) {
+    int share = C.np;   // r_par rows of one launch
+    const int64_t row_bytes = (int64_t)C.ntp * (int64_t)picca::XI_HIST_BIN_BYTES;
+    const int64_t fit_bytes = ctx->lds_limit - (int64_t)(static_lds + lds_bytes(false, 0));
+    if (!general && xcorr) {
+        // the cross-correlation: windows of r_par rows, a launch each.  Every window reads the
+        // pair list again, so that beyond a few of them the general kernel takes over.
+        const int64_t fit = std::min<int64_t>(std::max<int64_t>(fit_bytes, 0) / row_bytes,
+                                              INT32_MAX / 2);
+        share = picca::xi_row_share(C.np, (int)fit);
+        if (share > 0 && (C.np + share - 1) / share <= XI_MAX_ROW_WINDOWS) {
+            lds_hist = true;
+            C.tile_len = 0;
+            const int rows = std::min(C.np + 1, share + 2);
+            lds = (size_t)(rows * row_bytes) + lds_bytes(false, 0);
+        } else {
+            general = true;
+            share = C.np;
+        }
+    } else if (!general) {
         if ((int64_t)(lds_bytes(true, 0) + static_lds) <= ctx->lds_limit) {
             lds_hist = true;
             C.tile_len = 0;
             lds = lds_bytes(true, 0);
+        } else if (cuts) {
+            general = true;
         }
-    } else {
+    }
+    if (general && !(xcorr && mode == picca::MODE_STANDARD)) {
         for (int tile = 64; tile >= 16 && !lds_hist; tile /= 2) {
             if ((int64_t)(lds_bytes(true, tile) + static_lds) <= ctx->lds_limit) {
                 lds_hist = true;
@@ -397,18 +426,24 @@ int xi_execute_into(picca_ctx *ctx, const picca::XiConst &C0, int mode,
     picca::GroupView G{ctx->gbegin.ptr, ctx->grow.ptr, ngroups};
     picca::XiOut O{out, queue, stats_dev};
     const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(ctx->num_cus, ngroups));
-    const bool xcorr = params->x_correlation != 0;
+    const bool signed_rows = xcorr && !general;
     // the launch sequence: output, queue head and counters cleared by kernels (no memset
-    // nodes in a graph), the chunk ranges of the pairs, then the pair kernel
+    // nodes in a graph), the chunk ranges of the pairs, then the pair kernel; the last three
+    // per window of r_par rows
     auto enqueue = [&](hipStream_t st) -> hipError_t {
         hipError_t e = picca::launch_zero_u64(reinterpret_cast<unsigned long long *>(out),
                                               nout * (int64_t)(sizeof(picca::XiBin) / 8), st);
-        if (e == hipSuccess) e = picca::launch_zero_u64(queue, 1, st);
         if (e == hipSuccess) e = picca::launch_zero_u64(stats_dev, picca::XI_NSTATS, st);
-        if (e == hipSuccess && ngroups > 0)
-            e = picca::launch_xi_chunks(mode, C, F, P, ctx->num_pairs, st);
-        if (e == hipSuccess && ngroups > 0)
-            e = picca::launch_xi(mode, xcorr, general, lds_hist, C, F, P, G, O, grid, lds, st);
+        for (int row0 = 0; e == hipSuccess && row0 < C.np; row0 += share) {
+            picca::XiConst K = C;
+            picca::set_xi_rows(K, row0, std::min(share, C.np - row0));
+            e = picca::launch_zero_u64(queue, 1, st);
+            if (e == hipSuccess && ngroups > 0)
+                e = picca::launch_xi_chunks(mode, K, F, P, ctx->num_pairs, signed_rows, st);
+            if (e == hipSuccess && ngroups > 0)
+                e = picca::launch_xi(mode, xcorr, general, cuts, lds_hist, K, F, P, G, O, grid,
+                                     lds, st);
+        }
         return e;
     };
     PICCA_HIP_CHECK(hipEventRecord(ctx->ev_start, ctx->stream));
@@ -419,7 +454,8 @@ int xi_execute_into(picca_ctx *ctx, const picca::XiConst &C0, int mode,
             const unsigned char *b = (const unsigned char *)v;
             key.insert(key.end(), b, b + n);
         };
-        const int32_t flags[4] = {mode, xcorr ? 1 : 0, general ? 1 : 0, lds_hist ? 1 : 0};
+        const int32_t flags[6] = {mode, xcorr ? 1 : 0, general ? 1 : 0, lds_hist ? 1 : 0,
+                                  cuts ? 1 : 0, share};
         put(&C, sizeof(C));
         put(&F, sizeof(F));
         put(&P, sizeof(P));
@@ -471,7 +507,7 @@ int xi_execute_into(picca_ctx *ctx, const picca::XiConst &C0, int mode,
         report->probes = (int64_t)stats[picca::XI_STAT_PROBES];
         report->walk_tasks = (int64_t)stats[picca::XI_STAT_WALK_TASKS];
         report->kernel_ms = (double)ms;
-        report->launches = ngroups > 0 ? 1 : 0;
+        report->launches = ngroups > 0 ? (C.np + share - 1) / share : 0;
     }
     return PICCA_OK;
 }

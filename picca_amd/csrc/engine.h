@@ -67,6 +67,10 @@ struct XiConst {
     // r_trans row window of the cross-correlation kernel's LDS histogram: rows
     // [win_t0, win_t0 + win_rows) of the output, padded to (np + 2) x (win_rows + 2) bins
     int32_t win_t0, win_rows, win_last, win_pad_;
+    // r_par rows [row0, row0 + rows) of one launch of the cross-correlation of two delta
+    // fields (all of them otherwise) and the r_par limits its pixel windows are pruned to
+    int32_t row0, rows;
+    double prune_lo, prune_hi;
 };
 
 // One pixel as the pair kernel streams it through the scalar cache.
@@ -91,7 +95,8 @@ struct ForestView {
     const int64_t *__restrict__ off; // [n + 1]
     const double *__restrict__ zq;
     const int32_t *__restrict__ order;
-    const uint8_t *__restrict__ mono; // bit0 r_comov non-decreasing, bit1 dist_m non-decreasing
+    const uint8_t *__restrict__ mono; // bit0 r_comov non-decreasing, bit1 dist_m
+                                      // non-decreasing, bit2 z non-decreasing
     const double2 *__restrict__ rd;   // (r_comov, dist_m) per pixel
     const PrefixRecord *__restrict__ pre;       // run-walk prefix sums, forest b at off[b] + b
     const double2 *__restrict__ spc;  // per forest: smallest step of r_comov and of dist_m
@@ -511,13 +516,15 @@ hipError_t launch_xcf(int mode, bool lds_hist, bool fast, const XiConst &C,
                       const ForestView &F, const XcfView &X, const XiOut &O, int grid,
                       size_t lds, hipStream_t stream);
 
-hipError_t launch_xi(int mode, bool xcorr, bool general, bool lds_hist, const XiConst &C,
-                     const ForestView &F, const PairView &P, const GroupView &G,
-                     const XiOut &O, int grid, size_t lds, hipStream_t stream);
+hipError_t launch_xi(int mode, bool xcorr, bool general, bool cuts, bool lds_hist,
+                     const XiConst &C, const ForestView &F, const PairView &P,
+                     const GroupView &G, const XiOut &O, int grid, size_t lds,
+                     hipStream_t stream);
 hipError_t launch_zero_u64(unsigned long long *ptr, int64_t n, hipStream_t stream);
-// per pair, the chunks of delta1 whose pixels can pair with delta2 (P.chunks)
+// per pair, the chunks of delta1 whose pixels can pair with delta2 (P.chunks); signed_rows:
+// inside the r_par limits of the launch's window of rows
 hipError_t launch_xi_chunks(int mode, const XiConst &C, const ForestView &F, const PairView &P,
-                            int64_t num_pairs, hipStream_t stream);
+                            int64_t num_pairs, bool signed_rows, hipStream_t stream);
 // device address of the current GPU's scratch array (XI_SCRATCH_WORDS words)
 hipError_t xi_scratch_address(unsigned long long **ptr);
 hipError_t launch_copy16(const void *src, void *dst, int64_t n16, hipStream_t stream);

@@ -27,6 +27,8 @@ inline const char *fill_xi_const(const picca_cf_params *p, XiConst &C, int &mode
     C.nt = p->num_bins_r_trans;
     C.nb = C.np * C.nt;
     C.ntp = C.nt + 1;
+    C.row0 = 0;
+    C.rows = C.np;
     C.rpmin = p->r_par_min;
     C.rpmax = p->r_par_max;
     C.rtmax = p->r_trans_max;
@@ -39,6 +41,8 @@ inline const char *fill_xi_const(const picca_cf_params *p, XiConst &C, int &mode
     C.inv_t = C.nt_d / C.rtmax;
     C.width_p = C.span_p / C.np;
     C.width_t = C.rtmax / C.nt;
+    C.prune_lo = C.rpmin;
+    C.prune_hi = C.rpmax;
     C.edge_tol = p->edge_tol;
     // |t_fast - t_exact| <= 4 ulp(t) << 1e-12 for t < 2^20; the margin also absorbs the
     // rounding of frac * width in the edge test.
@@ -71,7 +75,8 @@ inline const char *fill_xi_const(const picca_cf_params *p, XiConst &C, int &mode
 // max_abs_d bound |r_comov| and |dist_m| over the store.
 inline const char *widen_xi_margins(XiConst &C, double max_abs_r, double max_abs_d) {
     const double u = std::ldexp(1.0, -53);
-    const double err_p = 16.0 * u * max_abs_r * C.inv_p + 8.0 * u * (C.np_d + 1.0);
+    const double err_p = 16.0 * u * max_abs_r * C.inv_p +
+                         8.0 * u * (C.np_d + std::fabs(C.rpmin) * C.inv_p + 1.0);
     const double err_t = 16.0 * u * max_abs_d * C.inv_t + 8.0 * u * (C.nt_d + 1.0);
     C.fast_p += err_p;
     C.fast_t += err_t;
@@ -91,8 +96,37 @@ inline void apply_xi_schedule(XiConst &C, int schedule) {
     else if (schedule == PICCA_XI_SCHEDULE_AUTO) C.flags |= XI_WALK | XI_WALK_AUTO;
 }
 
-// The specialised kernel (and its run walk) covers standard binning, auto-correlation,
-// r_par_min == 0 and no z / zerr / same-half-plate cuts.
+// Windows of r_par rows of the cross-correlation's specialised launches: the fewest equal
+// shares whose padded histogram (hist_rows of the kernel) fits `fit_rows` rows.
+inline int xi_row_share(int np, int fit_rows) {
+    if (np + 1 <= fit_rows) return np;
+    if (fit_rows < 3) return 0;
+    const int windows = (np + fit_rows - 3) / (fit_rows - 2);
+    return (np + windows - 1) / windows;
+}
+
+// The r_par rows [row0, row0 + rows) of one launch and the limits its windows are pruned to.
+inline void set_xi_rows(XiConst &C, int row0, int rows) {
+    C.row0 = row0;
+    C.rows = rows;
+    C.prune_lo = row0 == 0 ? C.rpmin : C.rpmin + row0 * C.width_p;
+    C.prune_hi = row0 + rows == C.np ? C.rpmax : C.rpmin + (row0 + rows) * C.width_p;
+}
+
+// z / zerr / same-half-plate cuts
+inline bool xi_has_cuts(const picca_cf_params *p) {
+    return p->has_z_min_pairs || p->has_z_max_pairs || p->has_zerr_cut ||
+           p->remove_same_half_plate_close_pairs;
+}
+
+// The specialised kernel covers standard binning with either the auto-correlation from
+// r_par_min == 0 or the cross-correlation; the plain case is the auto-correlation without
+// cuts.
+inline bool xi_fast_path(const picca_cf_params *p, int mode) {
+    return mode == MODE_STANDARD && (p->x_correlation || p->r_par_min == 0.0);
+}
+
+// Standard binning, auto-correlation, r_par_min == 0 and no z / zerr / same-half-plate cuts.
 inline bool xi_specialised(const picca_cf_params *p, int mode) {
     return mode == MODE_STANDARD && !p->x_correlation && p->r_par_min == 0.0 &&
            !p->has_z_min_pairs && !p->has_z_max_pairs && !p->has_zerr_cut &&

@@ -15,8 +15,8 @@
 //   * inside a group, waves pull tasks = (pair, chunk of 64 pixels of delta1) from an
 //     LDS counter.  Lane l owns pixel i = 64*chunk + l of delta1 in registers; the wave
 //     walks the pixels j of delta2 in lockstep;
-//   * specialised kernel (standard binning, auto-correlation, no cuts): pixel j is a
-//     wave-uniform record read through the scalar cache;
+//   * specialised kernel (standard binning; auto-correlation with r_par_min == 0, or
+//     cross-correlation): pixel j is a wave-uniform record read through the scalar cache;
 //     general kernel: pixels j are staged per wave through LDS (lane l loads pixel j0 + l,
 //     pixels the reference skips before any arithmetic are dropped, the rest compacted,
 //     the next tile already loading) and read back with broadcast LDS reads;
@@ -31,7 +31,17 @@
 //     increase strictly and a bin holds at least a few of them: each lane walks its own
 //     runs of delta2 pixels with one bin, finds a run's end with about two probes and adds
 //     the run from per-forest prefix sums -- one flush per run instead of one evaluation
-//     per pair.
+//     per pair;
+//   * the cross-correlation's (signed r_par) histogram, 100 x 50 bins in the usual run, does
+//     not fit in LDS: the host runs one launch per window of r_par rows, each pruned to the
+//     window's r_par limits, so that a pair's runs are split over the launches and not
+//     walked twice.  400 x 400 forests of the 0.8 A grid (6.2e10 evaluated pixel pairs): 34 ms,
+//     against 1103 ms for the general loop with its runs added straight to the HBM rows;
+//   * cuts: a lane walks the window of delta2 inside the pair-redshift cut, the runs of r_par
+//     row 0 of a pair of one half plate are dropped, and the tasks the walk cannot take (a
+//     zerr cut, z not rising along delta2) take the pair loop.  500 forests of that grid with
+//     the half-plate cut: 25.9 ms, against 61.2 ms for the general loop, which evaluates every
+//     pair with the reference's arithmetic.
 //
 // Arithmetic: r_par, r_trans and the bin index follow the reference's FP64 operations
 // (built with -ffp-contract=off).  The bin index is first taken with a reciprocal
@@ -151,6 +161,55 @@ __device__ __forceinline__ int exact_fast(const XiConst &K, double r1, double d1
     // f_par, f_trans are small non-negative integers unless the pair is rejected
     const double pbin_f = f_trans + ntp_d * f_par + (f_trans >= nt_d ? 1.0 : 0.0);
     return (out | over) ? trash : (int)fmin(pbin_f, (double)trash);
+}
+
+// exact_fast for the cross-correlation and for the cuts: signed r_par from r_par_min, the
+// launch's r_par rows [row0, row0 + rows) (whose launch counts the pair's edge and overflow),
+// and the close pairs of one half plate (shp) rejected before the overflow test, as
+// exact_pair does.  Returns the padded bin of the launch's histogram, or `trash`.
+template <bool XCORR>
+__device__ __forceinline__ int exact_cut(const XiConst &K, double r1, double d1, double r2,
+                                         double d2, double cos_half, double sin_half, bool shp,
+                                         int trash, __attribute__((address_space(3)))
+                                         unsigned long long *lds_stats) {
+    const double rpmin = K.rpmin, rpmax = K.rpmax, rtmax = K.rtmax, tol = K.edge_tol;
+    const double span = K.span_p, np_d = K.np_d, nt_d = K.nt_d, nb_d = K.nb_d;
+    const double ntp_d = K.ntp_d, width_p = K.width_p, width_t = K.width_t;
+    const double row0 = (double)K.row0, rows = (double)K.rows;
+    const double rps = (r1 - r2) * cos_half;
+    const double r_par = XCORR ? rps : fabs(rps);
+    const double r_trans = (d1 + d2) * sin_half;
+    const bool out = (r_par >= rpmax) | (r_trans >= rtmax) | (r_par < rpmin);
+    const bool edge_out = (r_par - rpmax < tol) & (rpmin - r_par < tol) & (r_trans - rtmax < tol);
+    const double t_par = (r_par - rpmin) / span * np_d;
+    const double t_trans = r_trans / rtmax * nt_d;
+    const double f_par = floor(t_par);
+    const double f_trans = floor(t_trans);
+    const bool edge_in = ((r_par != 0) & (edge_distance(t_par, width_p) < tol)) |
+                         ((r_trans != 0) & (edge_distance(t_trans, width_t) < tol));
+    const double bin_f = f_trans + nt_d * f_par;
+    const bool over = !((bin_f >= 0.0) & (bin_f < nb_d));
+    const bool cut = shp & (fabs(r_par) < width_p);
+    const double own = fmin(fmax(f_par, 0.0), np_d - 1.0);
+    const bool mine = (own >= row0) & (own < row0 + rows);
+    const bool edge = out ? edge_out : edge_in;
+    if (edge & mine)
+        __hip_atomic_fetch_add(&lds_stats[XI_STAT_EDGE], 1ull, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (!out & !cut & over & mine)
+        __hip_atomic_fetch_add(&lds_stats[XI_STAT_OVERFLOW], 1ull, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    // a pair whose r_trans bin rounds to nt is added to column 0 of the next row, which the
+    // histogram of its own row's launch holds
+    const double pbin_f = f_trans + ntp_d * (f_par - row0) + (f_trans >= nt_d ? 1.0 : 0.0);
+    return (out | over | cut | !mine) ? trash : (int)fmin(fmax(pbin_f, 0.0), (double)trash);
+}
+
+// Rows of the padded LDS histogram: the launch's r_par rows, the row that collects rejected
+// pairs and, between them where the launch is not the last, the row after its own (only its
+// column 0, for the pairs whose r_trans bin rounds to nt).
+__device__ __host__ __forceinline__ int hist_rows(const XiConst &C) {
+    return C.rows + 1 + (C.row0 + C.rows < C.np ? 1 : 0);
 }
 
 // Run of the fast loop: consecutive pairs of one lane in one padded bin.  r_par and r_trans
@@ -295,11 +354,12 @@ struct DeviceWalkMem {
 };
 
 // One task: pixels [64*chunk, 64*chunk + 64) of delta1 against the pruned window of delta2.
-//   GENERAL = false: standard binning, auto-correlation, r_par_min == 0, no z / zerr /
-//   same-half-plate cuts (the cuts of the reference that cannot trigger are compiled out).
+//   GENERAL = false: standard binning, auto-correlation with r_par_min == 0 or (XCORR) the
+//   cross-correlation; CUTS: with pair-redshift, zerr or same-half-plate cuts (the cuts of the
+//   reference that cannot trigger are compiled out).
 //   LDS_HIST: the histogram is the padded LDS layout (row stride nt + 1), otherwise the
 //   output row in HBM.
-template <int MODE, bool XCORR, bool GENERAL, bool LDS_HIST, bool WALK, typename Bin>
+template <int MODE, bool XCORR, bool GENERAL, bool CUTS, bool LDS_HIST, bool WALK, typename Bin>
 __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView &F,
                         const PairView &P, int64_t p, int chunk, int lane, Bin *hist,
                         TilePixel *tile, TileExact *tile_x, LaneCounters &cnt,
@@ -316,7 +376,7 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
     bool same_half_plate = false;
     bool zerr_on = false;
     double z_qso_1 = 0, z_qso_2 = 0;
-    if (GENERAL) {
+    if (GENERAL || CUTS) {
         same_half_plate = (uniform_int(P.flags[p]) & PAIR_SAME_HALF_PLATE) != 0;
         zerr_on = (C.flags & XI_HAS_ZERR) && (ang < C.zerr_ang);
         z_qso_1 = uniform_f64(F.zq[a]);
@@ -334,7 +394,7 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
         dw1 = F.dw[oa + i];
         active = w1 != 0;
     }
-    if (GENERAL && zerr_on && active) {
+    if ((GENERAL || CUTS) && zerr_on && active) {
         const double z1 = zh1 * 2.0;
         double z_qf = 0.5 * (z1 + z_qso_2);
         double dv_kms = fabs(z1 - z_qso_2) / (1 + z_qf);
@@ -363,8 +423,11 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
         const double d_min = wave_min(active ? d1 : INFINITY);
         // r_par = (r1 - r2) cos_half must reach [r_par_min - tol, r_par_max + tol)
         const double slack = 4.0 * C.edge_tol / cos_half + 1e-6;
-        double lo_r = r_min - C.rpmax / cos_half;
-        double hi_r = XCORR ? r_max - C.rpmin / cos_half : r_max + C.rpmax / cos_half;
+        // (the cross-correlation's specialised launches: of their window of r_par rows)
+        const double p_lo = !GENERAL && XCORR ? C.prune_lo : C.rpmin;
+        const double p_hi = !GENERAL && XCORR ? C.prune_hi : C.rpmax;
+        double lo_r = r_min - p_hi / cos_half;
+        double hi_r = XCORR ? r_max - p_lo / cos_half : r_max + C.rpmax / cos_half;
         lo_r -= slack + 1e-12 * fabs(lo_r);
         hi_r += slack + 1e-12 * fabs(hi_r);
         j_lo = wave_search<true>(Br, lb, lo_r, lane);
@@ -382,7 +445,18 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
     if (j_lo >= j_hi) return;
 
     if constexpr (!GENERAL && LDS_HIST) {
-        if (WALK && (C.flags & XI_WALK) && pruned) {
+        // Cuts that the walk does not take: zerr (single pixels of delta2 drop out), close
+        // pairs of one half plate in the cross-correlation (r_par_min need not put a bin edge
+        // at r_par = 0), a pair-redshift cut where z does not rise along delta2.
+        bool walk_cuts = true;
+        const bool shp = CUTS && (C.flags & XI_REMOVE_SHP) && same_half_plate;
+        const bool z_cut = CUTS && (C.flags & (XI_HAS_ZMIN | XI_HAS_ZMAX)) != 0;
+        const double z_lo = CUTS && (C.flags & XI_HAS_ZMIN) ? C.zmin : -INFINITY;
+        const double z_hi = CUTS && (C.flags & XI_HAS_ZMAX) ? C.zmax : INFINITY;
+        if (CUTS)
+            walk_cuts = !zerr_on && !(XCORR && shp) &&
+                        (!z_cut || (uniform_int(F.mono[b]) & 4) != 0);
+        if (WALK && (C.flags & XI_WALK) && pruned && walk_cuts) {
             // Run walk (xi_walk.h) for the tasks walk_task admits; otherwise the pair loop
             // below.
             const double spc_r = uniform_f64(F.spc[b].x);
@@ -408,8 +482,34 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
                 T.q0 = q0;
                 DeviceWalkMem mem{F.rd + ob, F.pre + (ob + b), F.w + ob, F.z + ob, F.dw + ob,
                                   hist, lds_stats, 0u, 0u, 0u};
-                const WalkLane L{r1, d1, zh1, w1, dw1};
-                walk_lane(C, T, L, mem, active);
+                WalkLane L{r1, d1, zh1, w1, dw1};
+                if constexpr (CUTS) {
+                    T.shp = shp;
+                    L.j_lo = j_lo;
+                    L.j_hi = j_hi;
+                    if (z_cut && active) {
+                        // (z1 + z2) / 2 rises with j: the lane's pixels inside the cut
+                        int lo = j_lo, hi = j_hi;
+                        for (int n = j_hi - j_lo; n > 0;) {
+                            const int h = n >> 1;
+                            if (zh1 + Bz[lo + h] * 0.5 < z_lo) { lo += h + 1; n -= h + 1; }
+                            else n = h;
+                        }
+                        hi = lo;
+                        for (int n = j_hi - lo; n > 0;) {
+                            const int h = n >> 1;
+                            if (!(zh1 + Bz[hi + h] * 0.5 > z_hi)) { hi += h + 1; n -= h + 1; }
+                            else n = h;
+                        }
+                        if (lo < hi) {
+                            L.j_lo = lo;
+                            L.j_hi = hi;
+                        } else {
+                            active = false;
+                        }
+                    }
+                }
+                walk_lane<XCORR, CUTS>(C, T, L, mem, active);
                 cnt.visit += mem.cover;
                 cnt.runs += mem.runs;
                 cnt.probes += mem.probes;
@@ -433,9 +533,15 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
         const double st = sin_half * C.inv_t;  // bins per Mpc/h of d1 + d2
         const double cap_p = C.np_d;  // clamps of the bin coordinates: row np, column nt
         const double cap_t = C.nt_d;
-        const int trash = (C.np + 1) * C.ntp - 1;
+        const int trash = hist_rows(C) * C.ntp - 1;
         const double r1f = active ? r1 : 1e300;
         uint32_t steps = 0;
+        uint32_t cut_steps = 0;   // CUTS: the lane's pairs inside the pair-redshift cut
+        // cross-correlation: the coordinate counts rows from row0
+        const double off_p = XCORR ? C.rpmin * C.inv_p + (double)C.row0 : 0.0;
+        const double rows_d = (double)C.rows;
+        // |r1 - r2| below which a pair of one half plate is redone exactly (and cut there)
+        const double close = shp ? C.width_p / cos_half * (1.0 + 1e-9) : -1.0;
         FastRun run;
         run.bin = trash;
         run.count = 0.0;
@@ -448,6 +554,12 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
         auto step = [&](const PixelRecord &q) {
             // the reference skips w2 == 0 (either sign) before any arithmetic
             if (uniform_zero_weight(q.w)) return;
+            if (CUTS && zerr_on) {
+                const double z_qf = 0.5 * (q.z + z_qso_1);
+                double dv_kms = fabs(q.z - z_qso_1) / (1 + z_qf);
+                dv_kms *= SPEED_LIGHT_KMS;
+                if (dv_kms < C.zerr_kms) return;
+            }
             ++steps;
             const double diff = r1f - q.r;
             const double sum = d1 + q.d;
@@ -455,21 +567,34 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
             // part; within the rounding margin of an edge (or of the range limits, which
             // are edges) the pair is redone with the reference's arithmetic.  r_par == 0
             // exactly (equal r_comov) is bin 0 and never an edge pair.
-            const double tp = fabs(diff) * cp;
+            const double tp = XCORR ? fma(diff, cp, -off_p) : fabs(diff) * cp;
             const double tt = sum * st;
             const double fp = __builtin_amdgcn_fract(tp);
             const double ft = __builtin_amdgcn_fract(tt);
-            const bool near = ((fabs(fp - 0.5) > C.half_p) & (diff != 0)) |
-                              (fabs(ft - 0.5) > C.half_t);
+            bool near = ((fabs(fp - 0.5) > C.half_p) & (XCORR | (diff != 0))) |
+                        (fabs(ft - 0.5) > C.half_t);
             int bin = (int)__umul24((unsigned)C.ntp, (unsigned)(int)min_f64(tp, cap_p)) +
                       (int)min_f64(tt, cap_t);
+            if (XCORR) bin = ((tp >= 0.0) & (tp < rows_d)) ? bin : trash;
+            const double z = fma(q.z, 0.5, zh1);
+            if (CUTS) {
+                near = near | (fabs(diff) < close);
+                const bool z_in = (z >= z_lo) & (z <= z_hi);
+                near = near & z_in;
+                bin = z_in ? bin : trash;
+                cut_steps += z_in ? 1u : 0u;
+            }
             if (active & near) {
                 // exact re-evaluation (py/picca/cf.py:355-376), constants from the LDS copy
-                bin = exact_fast(C_lds, r1, d1, q.r, q.d, cos_half, sin_half, trash, lds_stats);
+                if (XCORR || CUTS)
+                    bin = exact_cut<XCORR>(C_lds, r1, d1, q.r, q.d, cos_half, sin_half, shp,
+                                           trash, lds_stats);
+                else
+                    bin = exact_fast(C_lds, r1, d1, q.r, q.d, cos_half, sin_half, trash,
+                                     lds_stats);
             }
             const double w12 = w1 * q.w;
             const double dw12 = dw1 * q.dw;
-            const double z = fma(q.z, 0.5, zh1);
             // a new bin adds the lane's run to the histogram and restarts it: the restart is
             // a multiply by 0 (every input is finite), which costs no branch of its own
             const bool change = bin != run.bin;
@@ -479,7 +604,7 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
             run.count = fma(run.count, keep, 1.0);
             run.we = fma(run.we, keep, w12);
             run.xi = fma(run.xi, keep, dw12);
-            run.rp = fma(fabs(diff), w12, run.rp * keep);
+            run.rp = fma(XCORR ? diff : fabs(diff), w12, run.rp * keep);
             run.rt = fma(sum, w12, run.rt * keep);
             run.z = fma(z, w12, run.z * keep);
         };
@@ -492,7 +617,7 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
         }
         flush_fast(run, hist, cos_half, sin_half);
         n_steps += steps;
-        if (active) cnt.visit += steps;
+        if (active) cnt.visit += CUTS ? cut_steps : steps;
         return;
     } else {
         LaneRun run;
@@ -582,12 +707,15 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
     }
 }
 
-// Adds the real bins of the padded LDS histogram to output row `row` in HBM and clears
-// them; returns the pairs this thread moved (the accepted-pair statistic).
+// Adds the real bins of the padded LDS histogram (the launch's r_par rows, and column 0 of the
+// next one where the launch is not the last) to output row `row` in HBM and clears them;
+// returns the pairs this thread moved (the accepted-pair statistic).
 __device__ __forceinline__ uint64_t flush_row(const XiConst &C, LocalBin *hist, XiBin *out,
                                               int tid) {
     uint64_t moved = 0;
-    for (int k = tid; k < C.nb; k += XI_BLOCK) {
+    out += C.row0 * C.nt;
+    const int bins = C.rows * C.nt + (C.row0 + C.rows < C.np ? 1 : 0);
+    for (int k = tid; k < bins; k += XI_BLOCK) {
         const int kp = k + k / C.nt;  // padded index: row k / nt, column k % nt
         const uint32_t n = hist[kp].nb;
         if (n) {
@@ -605,11 +733,11 @@ __device__ __forceinline__ uint64_t flush_row(const XiConst &C, LocalBin *hist, 
     return moved;
 }
 
-template <int MODE, bool XCORR, bool GENERAL, bool LDS_HIST, bool WALK>
+template <int MODE, bool XCORR, bool GENERAL, bool CUTS, bool LDS_HIST, bool WALK>
 __global__ void __launch_bounds__(XI_BLOCK)
 xi_kernel(XiConst C, ForestView F, PairView P, GroupView G, XiOut O) {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int nbp = (C.np + 1) * C.ntp;  // padded LDS histogram
+    const int nbp = hist_rows(C) * C.ntp;  // padded LDS histogram
     LocalBin *hist = (LocalBin *)reinterpret_cast<LdsBin *>(smem);
     const size_t hist_bytes = LDS_HIST ? (size_t)nbp * sizeof(LdsBin) : 0;
     // per wave: (tile_len + 1) staged pixels, then (tile_len + 1) exact coordinates
@@ -696,10 +824,10 @@ xi_kernel(XiConst C, ForestView F, PairView P, GroupView G, XiOut O) {
             const int chunk = uniform_int(s_first[q] + t - s_prefix[q]);
             const uint64_t steps_before = n_steps;
             if (LDS_HIST) {
-                xi_task<MODE, XCORR, GENERAL, true, WALK>(C, s_const, F, P, p0 + q, chunk, lane, hist,
+                xi_task<MODE, XCORR, GENERAL, CUTS, true, WALK>(C, s_const, F, P, p0 + q, chunk, lane, hist,
                                                     tile, tile_x, cnt, lds_stats, n_steps, n_walk);
             } else {
-                xi_task<MODE, XCORR, GENERAL, false, false>(C, s_const, F, P, p0 + q, chunk, lane,
+                xi_task<MODE, XCORR, GENERAL, false, false, false>(C, s_const, F, P, p0 + q, chunk, lane,
                                                      O.bins + (int64_t)row * C.nb, tile, tile_x,
                                                      cnt, lds_stats, n_steps, n_walk);
             }
@@ -752,7 +880,7 @@ hipError_t xi_scratch_address(unsigned long long **ptr) {
 // pixel, each bound widened by twice the pair kernel's window slack, so every skipped chunk
 // is one whose pruned window the pair kernel would find empty.  Other pairs keep every chunk.
 __global__ void xi_chunk_kernel(XiConst C, ForestView F, PairView P, int64_t num_pairs,
-                                bool standard) {
+                                bool standard, bool signed_rows) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= num_pairs) return;
     const int a = P.a[p], b = P.b[p];
@@ -765,9 +893,11 @@ __global__ void xi_chunk_kernel(XiConst C, ForestView F, PairView P, int64_t num
         la > 0 && lb > 0) {
         const double *__restrict__ R1 = F.r + oa;
         const double *__restrict__ D1 = F.d + oa;
+        // signed_rows: r_par = (r1 - r2) cos inside the launch's window of r_par rows
         const double reach = fmax(C.rpmax, fabs(C.rpmin)) / cos_half;
         const double slack = 8.0 * C.edge_tol / cos_half + 2e-6;
-        double lo = F.r[ob] - reach, hi = F.r[ob + lb - 1] + reach;
+        double lo = F.r[ob] + (signed_rows ? C.prune_lo / cos_half : -reach);
+        double hi = F.r[ob + lb - 1] + (signed_rows ? C.prune_hi / cos_half : reach);
         lo -= slack + 2e-12 * fabs(lo);
         hi += slack + 2e-12 * fabs(hi);
         // first pixel with r1 >= lo, first with r1 > hi
@@ -804,11 +934,11 @@ __global__ void xi_chunk_kernel(XiConst C, ForestView F, PairView P, int64_t num
 }
 
 hipError_t launch_xi_chunks(int mode, const XiConst &C, const ForestView &F, const PairView &P,
-                            int64_t num_pairs, hipStream_t stream) {
+                            int64_t num_pairs, bool signed_rows, hipStream_t stream) {
     if (num_pairs <= 0) return hipSuccess;
     const int64_t blocks = (num_pairs + 255) / 256;
-    xi_chunk_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(C, F, P, num_pairs,
-                                                                       mode == MODE_STANDARD);
+    xi_chunk_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(
+        C, F, P, num_pairs, mode == MODE_STANDARD, signed_rows);
     return hipGetLastError();
 }
 
@@ -842,11 +972,11 @@ hipError_t launch_zero_u64(unsigned long long *ptr, int64_t n, hipStream_t strea
     return hipGetLastError();
 }
 
-template <int MODE, bool XCORR, bool GENERAL, bool LDS_HIST, bool WALK>
+template <int MODE, bool XCORR, bool GENERAL, bool CUTS, bool LDS_HIST, bool WALK>
 static hipError_t launch_xi_t(const XiConst &C, const ForestView &F, const PairView &P,
                               const GroupView &G, const XiOut &O, int grid, size_t lds,
                               hipStream_t stream) {
-    auto kern = xi_kernel<MODE, XCORR, GENERAL, LDS_HIST, WALK>;
+    auto kern = xi_kernel<MODE, XCORR, GENERAL, CUTS, LDS_HIST, WALK>;
     hipError_t err = hipFuncSetAttribute((const void *)kern,
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) return err;
@@ -858,26 +988,47 @@ template <int MODE, bool XCORR, bool GENERAL>
 static hipError_t launch_xi_h(bool lds_hist, const XiConst &C, const ForestView &F,
                               const PairView &P, const GroupView &G, const XiOut &O, int grid,
                               size_t lds, hipStream_t stream) {
-    return lds_hist
-               ? launch_xi_t<MODE, XCORR, GENERAL, true, false>(C, F, P, G, O, grid, lds, stream)
-               : launch_xi_t<MODE, XCORR, GENERAL, false, false>(C, F, P, G, O, grid, lds, stream);
+    return lds_hist ? launch_xi_t<MODE, XCORR, GENERAL, false, true, false>(C, F, P, G, O, grid,
+                                                                            lds, stream)
+                    : launch_xi_t<MODE, XCORR, GENERAL, false, false, false>(C, F, P, G, O, grid,
+                                                                             lds, stream);
 }
 
-// general == false is only valid for MODE_STANDARD, auto-correlation, r_par_min == 0 and
-// no z / zerr / same-half-plate cuts (the host decides).  The run walk (XI_WALK) has a
-// kernel of its own, so that its registers do not weigh on the pair loop's.
-hipError_t launch_xi(int mode, bool xcorr, bool general, bool lds_hist, const XiConst &C,
-                     const ForestView &F, const PairView &P, const GroupView &G,
-                     const XiOut &O, int grid, size_t lds, hipStream_t stream) {
+// the specialised kernel with its histogram in LDS; the run walk (XI_WALK) has a kernel of
+// its own, so that its registers do not weigh on the pair loop's
+template <bool XCORR, bool CUTS>
+static hipError_t launch_xi_fast(const XiConst &C, const ForestView &F, const PairView &P,
+                                 const GroupView &G, const XiOut &O, int grid, size_t lds,
+                                 hipStream_t stream) {
+    if (C.flags & XI_WALK)
+        return launch_xi_t<MODE_STANDARD, XCORR, false, CUTS, true, true>(C, F, P, G, O, grid,
+                                                                          lds, stream);
+    return launch_xi_t<MODE_STANDARD, XCORR, false, CUTS, true, false>(C, F, P, G, O, grid, lds,
+                                                                       stream);
+}
+
+// general == false is only valid for MODE_STANDARD and either the auto-correlation with
+// r_par_min == 0 or, with lds_hist, the cross-correlation; z / zerr / same-half-plate cuts
+// (`cuts`) need lds_hist there (the host decides).
+hipError_t launch_xi(int mode, bool xcorr, bool general, bool cuts, bool lds_hist,
+                     const XiConst &C, const ForestView &F, const PairView &P,
+                     const GroupView &G, const XiOut &O, int grid, size_t lds,
+                     hipStream_t stream) {
     if (mode == MODE_STANDARD) {
-        if (!general && !xcorr) {
-            if (lds_hist && (C.flags & XI_WALK))
-                return launch_xi_t<MODE_STANDARD, false, false, true, true>(C, F, P, G, O, grid,
-                                                                            lds, stream);
-            return launch_xi_h<MODE_STANDARD, false, false>(lds_hist, C, F, P, G, O, grid, lds, stream);
+        if (!general && lds_hist) {
+            if (xcorr)
+                return cuts ? launch_xi_fast<true, true>(C, F, P, G, O, grid, lds, stream)
+                            : launch_xi_fast<true, false>(C, F, P, G, O, grid, lds, stream);
+            return cuts ? launch_xi_fast<false, true>(C, F, P, G, O, grid, lds, stream)
+                        : launch_xi_fast<false, false>(C, F, P, G, O, grid, lds, stream);
         }
-        return xcorr ? launch_xi_h<MODE_STANDARD, true, true>(lds_hist, C, F, P, G, O, grid, lds, stream)
-                     : launch_xi_h<MODE_STANDARD, false, true>(lds_hist, C, F, P, G, O, grid, lds, stream);
+        if (!general)
+            return launch_xi_t<MODE_STANDARD, false, false, false, false, false>(C, F, P, G, O,
+                                                                                 grid, lds, stream);
+        if (xcorr)   // only where no window of rows fits in LDS
+            return launch_xi_t<MODE_STANDARD, true, true, false, false, false>(C, F, P, G, O,
+                                                                               grid, lds, stream);
+        return launch_xi_h<MODE_STANDARD, false, true>(lds_hist, C, F, P, G, O, grid, lds, stream);
     }
     if (mode == MODE_RMU)
         return xcorr ? launch_xi_h<MODE_RMU, true, true>(lds_hist, C, F, P, G, O, grid, lds, stream)

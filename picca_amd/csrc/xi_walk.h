@@ -18,6 +18,11 @@
 // are more than four margins apart in both coordinates (the kernel walks only such pairs),
 // and those pixels get the reference's edge, overflow and wrap-around treatment one by one.
 //
+// The cross-correlation (signed r_par, r_par_min any) walks the same way with the run index
+// m = -row - 1, which rises with j; the cuts of the auto-correlation that leave whole runs
+// (pair redshift, close pairs of one half plate) are a pixel window per lane and a dropped
+// run.  Both are template parameters, so that the plain auto-correlation's code is its own.
+//
 // The header is compiled into the kernel and into a CPU harness of the tests, which runs
 // the same lane program under bounds checks; `Mem` supplies the memory accesses.
 #pragma once
@@ -85,18 +90,21 @@ struct WalkTask {
     double rc, dc;       // r_c and d_c of delta2's prefix sums
     double q0;           // mean delta2 pixels per unit of the r_par coordinate in the window
     int32_t j_lo, j_hi;  // pruned pixel window of delta2
+    bool shp = false;    // CUTS: close pairs of one half plate are removed
 };
 
 // Pixel i of delta1 (weight != 0).
 struct WalkLane {
     double r1, d1, zh1, w1, dw1;  // zh1 = z1 / 2, dw1 = delta1 * w1
+    int32_t j_lo = 0, j_hi = 0;   // CUTS: the lane's window, inside [T.j_lo, T.j_hi)
 };
 
 // Everything the reference does with one pixel pair (standard binning, auto-correlation,
 // r_par_min == 0, no cuts), py/picca/cf.py:355-376, with its key: m is the signed r_par run
 // index, m = bin for r_comov2 >= r_comov1 and -bin - 1 below it, clamped to [-np - 1, np]
 // (|m| beyond np - 1 is rejected); c is the r_trans bin clamped to nt (nt is rejected, or a
-// wrap-around pair).
+// wrap-around pair).  The cross-correlation (XC): m = -bin - 1 for every pair, clamped to
+// [-np - 1, 0] (0: r_par < r_par_min, rejected).
 struct WalkExact {
     int32_t m, c;
     bool edge;      // within edge_tol of a bin edge, or outside the range but within
@@ -105,6 +113,9 @@ struct WalkExact {
     bool wrap;      // accepted with its r_trans bin rounded to nt: the flat index is
                     // column 0 of the next r_par row, where the pair is added
     int32_t pbin;   // padded histogram bin of a wrap pair
+    bool mine;      // XC: the pair's r_par row lies in the launch's rows [row0, row0 + rows),
+                    // which count its edge and overflow pairs (rows beyond the range belong
+                    // to the first and last launch)
     double r_par, r_trans;
 };
 
@@ -115,31 +126,41 @@ PICCA_HD inline double walk_edge_distance(double t, double width) {
     return lo < hi ? lo : hi;
 }
 
+template <bool XC = false>
 PICCA_HD inline WalkExact walk_exact(const XiConst &C, double r1, double d1, double r2,
                                      double d2, double cos_half, double sin_half) {
     WalkExact e;
     const double rps = (r1 - r2) * cos_half;
-    const double r_par = fabs(rps);
+    const double r_par = XC ? rps : fabs(rps);
     const double r_trans = (d1 + d2) * sin_half;
-    const double t_par = r_par / C.span_p * C.np_d;
+    const double t_par = (XC ? r_par - C.rpmin : r_par) / C.span_p * C.np_d;
     const double t_trans = r_trans / C.rtmax * C.nt_d;
     const double f_par = floor(t_par);
     const double f_trans = floor(t_trans);
     const double row = fmin(f_par, C.np_d);
-    e.m = (int32_t)(rps > 0 ? -row - 1.0 : row);
+    if (XC) {
+        e.m = (int32_t)(-fmax(row, -1.0) - 1.0);
+        const double own = fmin(fmax(row, 0.0), C.np_d - 1.0);
+        e.mine = own >= (double)C.row0 && own < (double)(C.row0 + C.rows);
+    } else {
+        e.m = (int32_t)(rps > 0 ? -row - 1.0 : row);
+        e.mine = true;
+    }
     e.c = (int32_t)fmin(f_trans, C.nt_d);
-    const bool out_p = r_par >= C.rpmax;
+    const bool out_p = XC ? (r_par >= C.rpmax) | (r_par < C.rpmin) : r_par >= C.rpmax;
     const bool out_t = r_trans >= C.rtmax;
     const bool out = out_p | out_t;
     // outside the range, but within edge_tol of it in both coordinates
-    const bool edge_out = (r_par - C.rpmax < C.edge_tol) & (r_trans - C.rtmax < C.edge_tol);
+    bool edge_out = (r_par - C.rpmax < C.edge_tol) & (r_trans - C.rtmax < C.edge_tol);
+    if (XC) edge_out = edge_out & (C.rpmin - r_par < C.edge_tol);
     const bool edge_in = (r_par != 0 && walk_edge_distance(t_par, C.width_p) < C.edge_tol) ||
                          (r_trans != 0 && walk_edge_distance(t_trans, C.width_t) < C.edge_tol);
     e.edge = out ? edge_out : edge_in;
     const double bin_f = f_trans + C.nt_d * f_par;
     e.over = !out & !(bin_f < C.nb_d);
     e.wrap = !out & !e.over & (f_trans >= C.nt_d);
-    e.pbin = e.wrap ? (int32_t)(C.ntp_d * (f_par + 1.0)) : 0;
+    // (the cross-correlation's histogram holds the rows from row0 on)
+    e.pbin = e.wrap ? (int32_t)(C.ntp_d * (f_par + 1.0)) - (XC ? C.row0 * C.ntp : 0) : 0;
     e.r_par = r_par;
     e.r_trans = r_trans;
     return e;
@@ -147,21 +168,38 @@ PICCA_HD inline WalkExact walk_exact(const XiConst &C, double r1, double d1, dou
 
 // The reference's treatment of a pixel within the margin of an edge: edge and overflow
 // counts, and the wrap-around pair, which no run holds.  Pixels with w == 0 (either sign)
-// are skipped before any arithmetic, as in the reference.
-template <class Mem>
+// are skipped before any arithmetic, as in the reference.  With T.shp the walk drops the runs
+// of r_par row 0; the reference drops the pairs with r_par < the row's width, which can
+// differ from the row by rounding: such a pair is added here, or taken back from its run.
+template <bool XC, bool CUTS, class Mem>
 PICCA_HD inline void walk_special(const XiConst &C, const WalkTask &T, const WalkLane &L,
                                   Mem &mem, int p) {
     const double w2 = mem.w(p);
     if (w2 == 0) return;
     double r2, d2;
     mem.rd(p, r2, d2);
-    const WalkExact e = walk_exact(C, L.r1, L.d1, r2, d2, T.cos_half, T.sin_half);
+    const WalkExact e = walk_exact<XC>(C, L.r1, L.d1, r2, d2, T.cos_half, T.sin_half);
+    if (XC && !e.mine) return;
     if (e.edge) mem.count_edge();
-    if (e.over) mem.count_overflow();
-    if (e.wrap) {
-        const double w12 = L.w1 * w2;
+    bool cut = false;
+    double sign = e.wrap ? 1.0 : 0.0;
+    int bin = e.pbin;
+    if constexpr (CUTS && !XC) {
+        cut = T.shp & (fabs(e.r_par) < C.width_p);
+        const bool in = !e.over & !e.wrap & (e.r_par < C.rpmax) & (e.r_trans < C.rtmax);
+        const int row = e.m >= 0 ? e.m : -e.m - 1;
+        if (T.shp & in) {
+            sign = row == 0 ? (cut ? 0.0 : 1.0) : (cut ? -1.0 : 0.0);
+            bin = row * C.ntp + e.c;
+        }
+        if (e.wrap & cut) sign = 0.0;
+    }
+    if (e.over & !cut) mem.count_overflow();
+    if (sign != 0.0) {
+        const double w12 = L.w1 * w2 * sign;
         const double z = L.zh1 + mem.z(p) * 0.5;
-        mem.add(e.pbin, w12, L.dw1 * mem.dw(p), e.r_par * w12, e.r_trans * w12, z * w12, 1u);
+        mem.add(bin, w12, L.dw1 * mem.dw(p) * sign, e.r_par * w12, e.r_trans * w12, z * w12,
+                sign > 0 ? 1u : ~0u);   // ~0u: -1 modulo 2^32
     }
 }
 
@@ -173,6 +211,7 @@ struct RunSums {
     uint32_t n;
 };
 
+template <bool XC>
 PICCA_HD inline bool walk_run_sums(const XiConst &C, const WalkTask &T, const WalkLane &L, int m,
                                    int c, const PrefixRecord &ps, const PrefixRecord &pe,
                                    RunSums &o) {
@@ -185,10 +224,11 @@ PICCA_HD inline bool walk_run_sums(const XiConst &C, const WalkTask &T, const Wa
     // sum over the run of w2 (r2 - r1) and w2 (d1 + d2), from the centred sums
     const double s_r = dr - (L.r1 - T.rc) * dw;
     const double s_d = (L.d1 + T.dc) * dw + dd;
-    o.bin = (m >= 0 ? m : -m - 1) * C.ntp + c;
+    const bool up = !XC && m >= 0;   // r_par counted as r2 - r1
+    o.bin = (up ? m : XC ? -m - 1 - C.row0 : -m - 1) * C.ntp + c;
     o.we = L.w1 * dw;
     o.xi = L.dw1 * dx;
-    o.rp = T.cos_half * (L.w1 * (m >= 0 ? s_r : -s_r));
+    o.rp = T.cos_half * (L.w1 * (up ? s_r : -s_r));
     o.rt = T.sin_half * (L.w1 * s_d);
     o.z = L.w1 * (L.zh1 * dw + 0.5 * dz);
     o.n = (uint32_t)fmax(n, 0.0);
@@ -209,12 +249,14 @@ PICCA_HD inline double walk_rcp_guess(double x) {
 // Key of pixel p from its coordinates relative to the upper edges of the run key (m, c):
 // a = (r2 - r1) cp - (m + 1) and b = (d1 + d2) st - (c + 1), so the pixel's r_par run index
 // is m + 1 + floor(a) and its r_trans bin c + 1 + floor(b), clamped as in walk_exact.
+template <bool XC>
 PICCA_HD inline void walk_key_from(const XiConst &C, int m, int c, double a, double b,
                                    int &mp, int &cp) {
     // |a| and |b| stay within a few times the bin counts inside the pruned window
     const int fm = (int)floor(a) + (m + 1);
     const int fc = (int)floor(b) + (c + 1);
-    mp = fm < -C.np - 1 ? -C.np - 1 : (fm > C.np ? C.np : fm);
+    const int top = XC ? 0 : C.np;
+    mp = fm < -C.np - 1 ? -C.np - 1 : (fm > top ? top : fm);
     cp = fc > C.nt ? C.nt : fc;
 }
 
@@ -229,10 +271,11 @@ PICCA_HD inline bool walk_task(const XiConst &C, double spc_r, double spc_d, dou
            (!(C.flags & XI_WALK_AUTO) || q0 >= XI_WALK_MIN_DENSITY);
 }
 
-// r_comov2 beyond r_par_max on the far side, or r_trans beyond r_trans_max: every later
-// pixel is rejected too
+// r_comov2 beyond r_par_max on the far side (XC: r_par below the launch's rows), or r_trans
+// beyond r_trans_max: every later pixel is rejected too
+template <bool XC>
 PICCA_HD inline bool walk_terminal(const XiConst &C, int m, int c) {
-    return m >= C.np || c >= C.nt;
+    return m >= (XC ? -C.row0 : C.np) || c >= C.nt;
 }
 
 // All pairs of lane pixel L with delta2's window [T.j_lo, T.j_hi).
@@ -262,19 +305,22 @@ PICCA_HD inline bool walk_terminal(const XiConst &C, int m, int c) {
 // A coordinate within the rounding margin of an integer is redone with the reference's
 // arithmetic (walk_exact); such a pixel is the first or last pixel of its run and gets the
 // reference's edge, overflow and wrap-around treatment (walk_special).
-template <class Mem>
+// XC: cross-correlation (signed r_par; the launch's rows [C.row0, C.row0 + C.rows)).  CUTS:
+// the lane's own window [L.j_lo, L.j_hi) (pair-redshift cuts; empty: `alive` false) and T.shp.
+template <bool XC = false, bool CUTS = false, class Mem = void>
 PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLane &L, Mem &mem,
                                bool alive) {
-    const int j_hi = T.j_hi;
-    if (T.j_lo >= j_hi) return;  // wave-uniform
-    const int last = j_hi - 1;  // pixel reads stay inside the window
-    const double r1cp = L.r1 * T.cp;
+    const int j_hi = CUTS ? L.j_hi : T.j_hi;
+    if (T.j_lo >= T.j_hi) return;  // wave-uniform
+    const int last = T.j_hi - 1;  // pixel reads stay inside the window
+    // the run coordinate is (r2 - r1) cp, from r_par_min for the cross-correlation
+    const double r1cp = XC ? L.r1 * T.cp - C.rpmin * C.inv_p : L.r1 * T.cp;
     const double d1st = L.d1 * T.st;
     // Before the first run opens the key is (-1, -1), which no pixel has (r_trans >= 0
     // here), so the thresholds give each pixel's own coordinates.
     int m = -1, c = -1;
     double Ka = r1cp, Kb = -d1st;
-    int j = T.j_lo;
+    int j = CUTS ? L.j_lo : T.j_lo;
     bool starting = true;
     PrefixRecord ps = {0, 0, 0, 0, 0, 0};
     int lo = j, hi = j_hi, g = j, misses = 0, step = 1;
@@ -291,7 +337,7 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
         // of the wave if the run closes in this pass (`on`); computed by every lane, so that
         // the values the flush moves between lanes are finite
         RunSums run;
-        const bool nonempty = walk_run_sums(C, T, L, m, c, ps, pg, run);
+        const bool nonempty = walk_run_sums<XC>(C, T, L, m, c, ps, pg, run);
         mem.pin(run);
         bool on = false;
         if (alive) {
@@ -303,15 +349,15 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
                 (fabs(aB - rint(aB)) < C.fast_p) || (fabs(bB - rint(bB)) < C.fast_t);
             const bool nearA = (fabs(aA) < C.fast_p) || (fabs(bA) < C.fast_t);
             int mB, cB;
-            walk_key_from(C, m, c, aB, bB, mB, cB);
+            walk_key_from<XC>(C, m, c, aB, bB, mB, cB);
             if (nearB) {
-                const WalkExact e = walk_exact(C, L.r1, L.d1, rb, db, T.cos_half, T.sin_half);
+                const WalkExact e = walk_exact<XC>(C, L.r1, L.d1, rb, db, T.cos_half, T.sin_half);
                 mB = e.m;
                 cB = e.c;
             }
             bool inA = (aA < 0) && (bA < 0);
             if (nearA && !starting) {
-                const WalkExact e = walk_exact(C, L.r1, L.d1, ra, da, T.cos_half, T.sin_half);
+                const WalkExact e = walk_exact<XC>(C, L.r1, L.d1, ra, da, T.cos_half, T.sin_half);
                 inA = (e.m == m) && (e.c == c);
             }
             // outcome of the pass
@@ -323,7 +369,7 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
             const bool gallop = !starting && same1 && same2; // the run goes on past g
             const bool close = !starting && same1 && !same2; // the run is [j, g)
             const bool open = starting || (close && has2);   // a run starts at pb
-            const bool terminal = open && walk_terminal(C, mB, cB);
+            const bool terminal = open && walk_terminal<XC>(C, mB, cB);
             const bool done = (close && !has2) || terminal;
             const bool special_last = close && (has1 ? nearA : near_lo) && g - 1 > j;
             const int p_last = g - 1;
@@ -332,7 +378,8 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
             // the closing run [j, g): prefix entries ps and pg (the entry at g)
             if (close) {
                 mem.count_run(run.n);
-                on = nonempty && m >= -C.np;
+                on = nonempty && m >= (XC ? -(C.row0 + C.rows) : -C.np);
+                if constexpr (CUTS && !XC) on = on && !(T.shp && (m == 0 || m == -1));
             }
             // next state
             const int g_miss = misses == 0 ? g - 1 : lo + 1 + ((g - 1 - lo) >> 1);
@@ -372,8 +419,8 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
                 pa = g - 1;
                 pb = g;
             }
-            if (special_last) walk_special(C, T, L, mem, p_last);
-            if (special_first) walk_special(C, T, L, mem, p_first);
+            if (special_last) walk_special<XC, CUTS>(C, T, L, mem, p_last);
+            if (special_first) walk_special<XC, CUTS>(C, T, L, mem, p_first);
             if (done) alive = false;
         }
         // the next pass's probes, issued before the histogram additions (a lane that is done

@@ -6,6 +6,7 @@
 // against the forest's bounds.  Tasks the kernel would not walk are evaluated pair by pair
 // with the reference's arithmetic.  The tests compare the result with the oracle, so the
 // walk's keys, probes, prefix sums and edge pixels are checked on the CPU.
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -104,21 +105,25 @@ int lower(const double *arr, int n, double x, bool strict) {
 }
 
 // One pixel pair with the reference's arithmetic (py/picca/cf.py:355-387), specialised
-// case; same edge / overflow conventions as the kernel.
+// case (XC: cross-correlation, the rows [C.row0, C.row0 + C.rows); shp: close pairs of one
+// half plate removed); same edge / overflow conventions as the kernel.
+template <bool XC>
 void exact_pair(const XiConst &C, double r1, double d1, double zh1, double w1, double dw1,
                 double r2, double d2, double z2, double w2, double dw2, double cos_half,
-                double sin_half, Hist &h, int64_t *stats) {
-    const picca::WalkExact e = picca::walk_exact(C, r1, d1, r2, d2, cos_half, sin_half);
+                double sin_half, bool shp, Hist &h, int64_t *stats) {
+    const picca::WalkExact e = picca::walk_exact<XC>(C, r1, d1, r2, d2, cos_half, sin_half);
+    if (!e.mine) return;
+    const bool cut = shp && std::fabs(e.r_par) < C.width_p;
     if (e.edge) ++stats[ST_EDGE];
-    if (e.over) ++stats[ST_OVER];
-    const bool out = (e.r_par >= C.rpmax) | (e.r_trans >= C.rtmax);
-    if (out || e.over) return;
+    if (e.over && !cut) ++stats[ST_OVER];
+    const bool out = (e.r_par >= C.rpmax) | (e.r_trans >= C.rtmax) | (XC && e.r_par < C.rpmin);
+    if (out || e.over || cut) return;
     int pbin;
     if (e.wrap) {
         pbin = e.pbin;
     } else {
-        const int row = e.m >= 0 ? e.m : -e.m - 1;
-        pbin = row * C.ntp + e.c;
+        const int row = !XC && e.m >= 0 ? e.m : -e.m - 1;
+        pbin = (row - C.row0) * C.ntp + e.c;
     }
     const double w12 = w1 * w2;
     h.we[pbin] += w12;
@@ -129,27 +134,22 @@ void exact_pair(const XiConst &C, double r1, double d1, double zh1, double w1, d
     h.nb[pbin] += 1;
 }
 
-}  // namespace
-
-extern "C" {
-
-// The walk's guess reciprocal (walk_rcp_guess), for its unit test.
-double xi_walk_rcp_guess(double x) { return picca::walk_rcp_guess(x); }
-
-// Correlation of the listed forest pairs (specialised case of the pair kernel only).
-// Outputs are [num_rows * np * nt] each; stats = edge, overflow, walked tasks, pair-by-pair
-// tasks, runs, probes, out-of-bounds accesses, pixel pairs covered by runs.  Returns 0, or
-// -1 when the parameters are not the specialised case.
-int xi_walk_host(const picca_cf_params *params, int64_t num_forests, const int64_t *off,
+// The launch of the kernel over the rows [row0, row0 + rows) of r_par; pflags: the pairs'
+// same-half-plate flags (CUTS).
+template <bool XC, bool CUTS>
+int walk_launch(const picca_cf_params *params, int64_t num_forests, const int64_t *off,
                  const double *z, const double *r, const double *d, const double *w,
                  const double *delta, int64_t num_pairs, const int32_t *pa, const int32_t *pb,
-                 const double *pang, const int32_t *prow, int32_t num_rows, int32_t schedule,
+                 const double *pang, const uint8_t *pflags, const int32_t *prow,
+                 int32_t num_rows, int32_t schedule, int32_t row0, int32_t rows_n,
                  double *o_we, double *o_xi, double *o_rp, double *o_rt, double *o_z,
                  int64_t *o_nb, int64_t *stats) {
     XiConst C;
     int mode = 0;
-    if (picca::fill_xi_const(params, C, mode) || !picca::xi_specialised(params, mode))
+    if (picca::fill_xi_const(params, C, mode) || !picca::xi_fast_path(params, mode) ||
+        (!XC && !CUTS && !picca::xi_specialised(params, mode)))
         return -1;
+    if (rows_n > 0) picca::set_xi_rows(C, row0, std::min(rows_n, C.np - row0));
     const int64_t npix = off[num_forests];
     double max_r = 0, max_d = 0;
     for (int64_t k = 0; k < npix; ++k) {
@@ -168,10 +168,13 @@ int xi_walk_host(const picca_cf_params *params, int64_t num_forests, const int64
         const int64_t o = off[b], n = off[b + 1] - off[b];
         picca::build_walk_forest(r + o, d + o, z + o, w + o, dw.data() + o, n,
                                  pre.data() + o + b, spc_r[b], spc_d[b]);
-        mono[b] = (uint8_t)((monotone(r + o, n) ? 1 : 0) | (monotone(d + o, n) ? 2 : 0));
+        mono[b] = (uint8_t)((monotone(r + o, n) ? 1 : 0) | (monotone(d + o, n) ? 2 : 0) |
+                            (monotone(z + o, n) ? 4 : 0));
     }
-    std::memset(stats, 0, sizeof(int64_t) * ST_N);
-    const size_t nbp = (size_t)(C.np + 1) * C.ntp;
+    const bool z_cut = (C.flags & (picca::XI_HAS_ZMIN | picca::XI_HAS_ZMAX)) != 0;
+    const double z_lo = (C.flags & picca::XI_HAS_ZMIN) ? C.zmin : -INFINITY;
+    const double z_hi = (C.flags & picca::XI_HAS_ZMAX) ? C.zmax : INFINITY;
+    const size_t nbp = (size_t)(C.rows + 1 + (C.row0 + C.rows < C.np ? 1 : 0)) * C.ntp;
     std::vector<Hist> rows;
     rows.reserve((size_t)num_rows);
     for (int32_t k = 0; k < num_rows; ++k) rows.emplace_back(nbp);
@@ -188,7 +191,8 @@ int xi_walk_host(const picca_cf_params *params, int64_t num_forests, const int64
         if (cos_half > 0 && (mono[b] & 3) == 3 && (mono[a] & 1) && la > 0 && lb > 0) {
             const double reach = std::fmax(C.rpmax, std::fabs(C.rpmin)) / cos_half;
             const double slack = 8.0 * C.edge_tol / cos_half + 2e-6;
-            double lo = r[ob] - reach, hi = r[ob + lb - 1] + reach;
+            double lo = r[ob] + (XC ? C.prune_lo / cos_half : -reach);
+            double hi = r[ob + lb - 1] + (XC ? C.prune_hi / cos_half : reach);
             lo -= slack + 2e-12 * std::fabs(lo);
             hi += slack + 2e-12 * std::fabs(hi);
             const int i_lo = lower(r + oa, la, lo, true);
@@ -218,8 +222,8 @@ int xi_walk_host(const picca_cf_params *params, int64_t num_forests, const int64
             if (cos_half > 0 && (mono[b] & 3) == 3) {
                 pruned = true;
                 const double slack = 4.0 * C.edge_tol / cos_half + 1e-6;
-                double lo_r = r_min - C.rpmax / cos_half;
-                double hi_r = r_max + C.rpmax / cos_half;
+                double lo_r = r_min - (XC ? C.prune_hi : C.rpmax) / cos_half;
+                double hi_r = XC ? r_max - C.prune_lo / cos_half : r_max + C.rpmax / cos_half;
                 lo_r -= slack + 1e-12 * std::fabs(lo_r);
                 hi_r += slack + 1e-12 * std::fabs(hi_r);
                 j_lo = lower(r + ob, lb, lo_r, true);
@@ -239,7 +243,10 @@ int xi_walk_host(const picca_cf_params *params, int64_t num_forests, const int64
                 const double span = (r[ob + j_hi - 1] - r[ob + j_lo]) * cp;
                 if (span > 0) q0 = (double)(j_hi - 1 - j_lo) / span;
             }
-            const bool walk = pruned && picca::walk_task(C, spc_r[b], spc_d[b], cp, st, q0);
+            const bool shp = CUTS && (C.flags & picca::XI_REMOVE_SHP) &&
+                             (pflags[p] & picca::PAIR_SAME_HALF_PLATE);
+            const bool cuts_ok = !(XC && shp) && (!z_cut || (mono[b] & 4));
+            const bool walk = pruned && cuts_ok && picca::walk_task(C, spc_r[b], spc_d[b], cp, st, q0);
             if (walk) {
                 ++stats[ST_WALK_TASKS];
                 picca::WalkTask T;
@@ -264,9 +271,18 @@ int xi_walk_host(const picca_cf_params *params, int64_t num_forests, const int64
                 mem.stats = stats;
                 for (int i = i0; i < i1; ++i) {
                     if (w[oa + i] == 0) continue;
-                    const picca::WalkLane L{r[oa + i], d[oa + i], z[oa + i] * 0.5, w[oa + i],
-                                            dw[oa + i]};
-                    picca::walk_lane(C, T, L, mem, true);
+                    picca::WalkLane L{r[oa + i], d[oa + i], z[oa + i] * 0.5, w[oa + i],
+                                      dw[oa + i]};
+                    T.shp = shp;
+                    if (CUTS) {
+                        // the kernel's binary searches of the pair-redshift cut
+                        L.j_lo = j_lo;
+                        while (L.j_lo < j_hi && L.zh1 + z[ob + L.j_lo] * 0.5 < z_lo) ++L.j_lo;
+                        L.j_hi = L.j_lo;
+                        while (L.j_hi < j_hi && !(L.zh1 + z[ob + L.j_hi] * 0.5 > z_hi)) ++L.j_hi;
+                        if (L.j_lo >= L.j_hi) continue;
+                    }
+                    picca::walk_lane<XC, CUTS>(C, T, L, mem, true);
                 }
             } else {
                 ++stats[ST_PAIR_TASKS];
@@ -274,9 +290,11 @@ int xi_walk_host(const picca_cf_params *params, int64_t num_forests, const int64
                     if (w[oa + i] == 0) continue;
                     for (int j = j_lo; j < j_hi; ++j) {
                         if (w[ob + j] == 0) continue;
-                        exact_pair(C, r[oa + i], d[oa + i], z[oa + i] * 0.5, w[oa + i],
+                        const double zp = z[oa + i] * 0.5 + z[ob + j] * 0.5;
+                        if (CUTS && (zp < z_lo || zp > z_hi)) continue;
+                        exact_pair<XC>(C, r[oa + i], d[oa + i], z[oa + i] * 0.5, w[oa + i],
                                    dw[oa + i], r[ob + j], d[ob + j], z[ob + j], w[ob + j],
-                                   dw[ob + j], cos_half, sin_half, h, stats);
+                                   dw[ob + j], cos_half, sin_half, shp, h, stats);
                     }
                 }
             }
@@ -285,16 +303,65 @@ int xi_walk_host(const picca_cf_params *params, int64_t num_forests, const int64
     // padded layout -> flat rows
     for (int32_t row = 0; row < num_rows; ++row) {
         const Hist &h = rows[(size_t)row];
-        for (int k = 0; k < C.nb; ++k) {
+        // (column 0 of the row after the launch's: pairs whose r_trans bin rounds to nt)
+        const int bins = C.rows * C.nt + (C.row0 + C.rows < C.np ? 1 : 0);
+        for (int k = 0; k < bins; ++k) {
             const int kp = k + k / C.nt;
-            const size_t o = (size_t)row * C.nb + k;
-            o_we[o] = h.we[kp];
-            o_xi[o] = h.xi[kp];
-            o_rp[o] = h.rp[kp];
-            o_rt[o] = h.rt[kp];
-            o_z[o] = h.z[kp];
-            o_nb[o] = h.nb[kp];
+            const size_t o = (size_t)row * C.nb + C.row0 * C.nt + k;
+            o_we[o] += h.we[kp];
+            o_xi[o] += h.xi[kp];
+            o_rp[o] += h.rp[kp];
+            o_rt[o] += h.rt[kp];
+            o_z[o] += h.z[kp];
+            o_nb[o] += h.nb[kp];
         }
+    }
+    return 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+// The walk's guess reciprocal (walk_rcp_guess), for its unit test.
+double xi_walk_rcp_guess(double x) { return picca::walk_rcp_guess(x); }
+
+// Correlation of the listed forest pairs (specialised case of the pair kernel only).
+// Outputs are [num_rows * np * nt] each, added to; stats = edge, overflow, walked tasks,
+// pair-by-pair tasks, runs, probes, out-of-bounds accesses, pixel pairs covered by runs.
+// Returns 0, or -1 when the parameters are not the specialised case.
+int xi_walk_host(const picca_cf_params *params, int64_t num_forests, const int64_t *off,
+                 const double *z, const double *r, const double *d, const double *w,
+                 const double *delta, int64_t num_pairs, const int32_t *pa, const int32_t *pb,
+                 const double *pang, const int32_t *prow, int32_t num_rows, int32_t schedule,
+                 double *o_we, double *o_xi, double *o_rp, double *o_rt, double *o_z,
+                 int64_t *o_nb, int64_t *stats) {
+    std::memset(stats, 0, sizeof(int64_t) * ST_N);
+    return walk_launch<false, false>(params, num_forests, off, z, r, d, w, delta, num_pairs, pa,
+                                     pb, pang, nullptr, prow, num_rows, schedule, 0, 0, o_we,
+                                     o_xi, o_rp, o_rt, o_z, o_nb, stats);
+}
+
+// The same for the cross-correlation and the cuts (no zerr cut), in launches of `share` rows
+// of r_par (the cross-correlation) or one launch.
+int xi_walk_host_cuts(const picca_cf_params *params, int64_t num_forests, const int64_t *off,
+                      const double *z, const double *r, const double *d, const double *w,
+                      const double *delta, int64_t num_pairs, const int32_t *pa,
+                      const int32_t *pb, const double *pang, const uint8_t *pflags,
+                      const int32_t *prow, int32_t num_rows, int32_t share, double *o_we,
+                      double *o_xi, double *o_rp, double *o_rt, double *o_z, int64_t *o_nb,
+                      int64_t *stats) {
+    std::memset(stats, 0, sizeof(int64_t) * ST_N);
+    const bool xc = params->x_correlation != 0;
+    const int np = params->num_bins_r_par;
+    if (params->has_zerr_cut) return -1;
+    const int step = xc ? share : np;
+    for (int row0 = 0; row0 < np; row0 += step) {
+        auto launch = xc ? walk_launch<true, true> : walk_launch<false, true>;
+        const int rc = launch(params, num_forests, off, z, r, d, w, delta, num_pairs, pa, pb,
+                              pang, pflags, prow, num_rows, PICCA_XI_SCHEDULE_RUNS, row0, step,
+                              o_we, o_xi, o_rp, o_rt, o_z, o_nb, stats);
+        if (rc) return rc;
     }
     return 0;
 }

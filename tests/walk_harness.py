@@ -57,6 +57,29 @@ def _p(a):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
+def xi_walk_cuts(params, store, pair_a, pair_b, pair_ang, pair_flags, pair_row, num_rows, share):
+    """xi_walk for the cross-correlation (in launches of `share` rows of r_par) and the
+    pair-redshift and same-half-plate cuts."""
+    arr = lambda x, t: np.ascontiguousarray(x, dtype=t)
+    off = arr(store.offsets, np.int64)
+    cols = [arr(getattr(store, k), np.float64)
+            for k in ("z", "r_comov", "dist_m", "weights", "delta")]
+    a, b, row = (arr(x, np.int32) for x in (pair_a, pair_b, pair_row))
+    ang, flags = arr(pair_ang, np.float64), arr(pair_flags, np.uint8)
+    nb = params.num_bins_r_par * params.num_bins_r_trans
+    out = [np.zeros((num_rows, nb)) for _ in range(5)]
+    nbs = np.zeros((num_rows, nb), dtype=np.int64)
+    stats = np.zeros(len(STATS), dtype=np.int64)
+    status = lib().xi_walk_host_cuts(
+        ctypes.byref(params), ctypes.c_int64(len(off) - 1), _p(off), *[_p(c) for c in cols],
+        ctypes.c_int64(len(a)), _p(a), _p(b), _p(ang), _p(flags), _p(row),
+        ctypes.c_int32(num_rows), ctypes.c_int32(share), *[_p(o) for o in out], _p(nbs),
+        _p(stats))
+    if status != 0:
+        raise ValueError("xi_walk_host_cuts: parameters outside the specialised kernel")
+    return out + [nbs], dict(zip(STATS, (int(s) for s in stats)))
+
+
 def xi_walk(params, store, pair_a, pair_b, pair_ang, pair_row, num_rows,
             schedule=SCHEDULE_RUNS):
     """Un-normalised (we, xi, rp, rt, z, nb) rows [num_rows, nb] and a stats dict."""
