@@ -12,6 +12,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBRARY = os.path.join(HERE, "libpicca_hip.so")
 SOURCES = ["api.hip", "cont_api.hip", "mlp_api.hip", "metal_api.hip", "cov_api.hip",
            "wick_api.hip", "xi_kernel.hip", "xcf_kernel.hip", "dmat_kernel.hip",
+           "dmat_band_kernel.hip",
            "metal_kernel.hip", "cov_kernel.hip", "wick_kernel.hip",
            "cont_kernel.hip", "mlp_kernel.hip",
            "neighbours.cpp"]

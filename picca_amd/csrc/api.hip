@@ -216,6 +216,7 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
                                                ctx->stream));
         PICCA_HIP_CHECK(ctx->spc.upload(spc.data(), (size_t)num_forests, ctx->stream));
         PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+        ctx->h_spc = std::move(spc);
         // typical pixel spacing of the store, for the automatic schedule of the xi kernel
         std::vector<double> steps;
         steps.reserve((size_t)num_forests);
@@ -231,6 +232,7 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
     }
     PICCA_HIP_CHECK(ctx->zq.upload(z_qso, (size_t)num_forests, ctx->stream));
     PICCA_HIP_CHECK(ctx->mono.upload(mono.data(), (size_t)num_forests, ctx->stream));
+    ctx->h_mono = mono;
     ctx->has_log_lambda = log_lambda != nullptr;
     if (log_lambda) {
         PICCA_HIP_CHECK(ctx->ll.upload(log_lambda, (size_t)npix, ctx->stream));
@@ -239,6 +241,7 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
         std::vector<double> dll((size_t)std::max<int64_t>(npix, 1));
         std::vector<double> sum_w((size_t)std::max<int64_t>(num_forests, 1));
         std::vector<double> sw_dll((size_t)std::max<int64_t>(num_forests, 1));
+        ctx->h_fit.assign((size_t)num_forests, 0);
         parallel_for(num_forests, [&](int64_t lo, int64_t hi) {
             for (int64_t k = lo; k < hi; ++k) {
                 const int64_t o = offsets[k], e = offsets[k + 1];
@@ -253,6 +256,7 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
                 }
                 sum_w[k] = sw;
                 sw_dll[k] = s2;
+                ctx->h_fit[(size_t)k] = std::isfinite(sw) && sw > 0 && std::isfinite(s2) && s2 > 0;
             }
         });
         PICCA_HIP_CHECK(ctx->dll.upload_padded(dll.data(), (size_t)npix, pad, ctx->stream));
@@ -925,6 +929,302 @@ int picca_diag_copy(picca_ctx *ctx, int64_t bytes, double *kernel_ms) {
     return PICCA_OK;
 }
 
+namespace {
+
+// One picca_dmat_run: its launch constants and device views, and the batches so far.
+struct DmatRun {
+    picca_ctx *ctx;
+    const picca_cf_params *params;
+    picca::DmatConst C;
+    picca::DmatForests F;
+    picca::DmatOut O;
+    size_t pass_lds;        // of dmat_pass_kernel
+    int64_t batches;
+    // uploads of the general kernels, kept until the stream is done
+    std::vector<double> cs;
+    std::vector<std::vector<int64_t>> pix_off;
+    // the downloads; host_buffers() makes them while the kernels run
+    std::vector<double> h_wdm, h_dmat, h_eff;
+    void host_buffers() {
+        h_wdm.resize((size_t)C.nb);
+        h_dmat.resize((size_t)C.nb * (size_t)C.nm);
+        h_eff.resize(4 * (size_t)C.nm);
+    }
+};
+
+struct DmatPairList {
+    std::vector<int32_t> a, b;
+    std::vector<double> ang;
+    std::vector<uint8_t> flags;
+    void push(int32_t pa, int32_t pb, double t, uint8_t f) {
+        a.push_back(pa);
+        b.push_back(pb);
+        ang.push_back(t);
+        flags.push_back(f);
+    }
+    int64_t size() const { return (int64_t)a.size(); }
+};
+
+// The three events of the next batch (before the pass, between, after the fill).
+hipError_t dmat_next_events(DmatRun &R, hipEvent_t **ev) {
+    const size_t first = 3 * (size_t)R.batches++;
+    while (R.ctx->dmat_events.size() < first + 3) {
+        hipEvent_t e = nullptr;
+        const hipError_t err = hipEventCreate(&e);
+        if (err != hipSuccess) return err;
+        R.ctx->dmat_events.push_back(e);
+    }
+    *ev = R.ctx->dmat_events.data() + first;
+    return hipSuccess;
+}
+
+// The general kernels (dmat_kernel.hip) over a pair list, which the caller keeps until the
+// stream is done.
+int dmat_run_general(DmatRun &R, const DmatPairList &L) {
+    picca_ctx *ctx = R.ctx;
+    const picca::DmatConst &C = R.C;
+    const int64_t num_pairs = L.size();
+    if (num_pairs == 0) return PICCA_OK;
+    std::vector<double> &cs = R.cs;
+    cs.resize((size_t)(2 * num_pairs));
+    for (int64_t k = 0; k < num_pairs; ++k) {
+        cs[2 * k] = std::cos(L.ang[k] / 2);
+        cs[2 * k + 1] = std::sin(L.ang[k] / 2);
+    }
+    PICCA_HIP_CHECK(ctx->dpa.upload(L.a.data(), (size_t)num_pairs, ctx->stream));
+    PICCA_HIP_CHECK(ctx->dpb.upload(L.b.data(), (size_t)num_pairs, ctx->stream));
+    PICCA_HIP_CHECK(ctx->dang.upload(L.ang.data(), (size_t)num_pairs, ctx->stream));
+    PICCA_HIP_CHECK(ctx->dcs.upload(cs.data(), (size_t)(2 * num_pairs), ctx->stream));
+    PICCA_HIP_CHECK(ctx->dflags.upload(L.flags.data(), (size_t)num_pairs, ctx->stream));
+
+    // workspace per slot
+    const size_t slot_bytes = 8 * (4 * (size_t)C.nt * C.np + 4 * (size_t)C.ntm * C.npm) +
+                              4 * (size_t)C.words_u + 16 + 16 * (size_t)(C.nt + C.ntm);
+    const size_t ws_budget = (size_t)1536 << 20;
+    const int64_t cap = std::max<int64_t>(
+        1, std::min<int64_t>({num_pairs, (int64_t)(ws_budget / slot_bytes), (int64_t)1 << 20}));
+    const int64_t touched_words = ((int64_t)C.nt * C.ntm + 63) / 64;
+    PICCA_HIP_CHECK(ctx->ws_S.reserve((size_t)cap * 4 * C.nt * C.np));
+    PICCA_HIP_CHECK(ctx->ws_eta.reserve((size_t)cap * 4 * C.ntm * C.npm));
+    PICCA_HIP_CHECK(ctx->ws_U.reserve((size_t)cap * C.words_u));
+    PICCA_HIP_CHECK(ctx->ws_band.reserve((size_t)cap * 4));
+    PICCA_HIP_CHECK(ctx->ws_rng.reserve((size_t)cap * 4 * (C.nt + C.ntm)));
+    PICCA_HIP_CHECK(ctx->ws_pix.reserve((size_t)cap));
+    PICCA_HIP_CHECK(ctx->ws_touched.reserve((size_t)touched_words));
+
+    for (int64_t p0 = 0; p0 < num_pairs; p0 += cap) {
+        const int64_t count = std::min(cap, num_pairs - p0);
+        R.pix_off.emplace_back((size_t)count, 0);
+        std::vector<int64_t> &pix_off = R.pix_off.back();
+        int64_t total = 0;
+        for (int64_t k = 0; k < count; ++k) {
+            pix_off[k] = total;
+            const int32_t a = L.a[(size_t)(p0 + k)];
+            total += ctx->h_offsets[a + 1] - ctx->h_offsets[a];
+        }
+        PICCA_HIP_CHECK(ctx->ws_pix.upload(pix_off.data(), (size_t)count, ctx->stream));
+        PICCA_HIP_CHECK(ctx->ws_cnt.reserve((size_t)std::max<int64_t>(total, 1)));
+        PICCA_HIP_CHECK(picca::launch_zero_u64(ctx->ws_touched.ptr, touched_words, ctx->stream));
+        picca::DmatPairs P{ctx->dpa.ptr + p0, ctx->dpb.ptr + p0, ctx->dang.ptr + p0,
+                           ctx->dcs.ptr + 2 * p0, ctx->dflags.ptr + p0, (int32_t)count};
+        int32_t *rng = ctx->ws_rng.ptr;
+        picca::DmatWork W{ctx->ws_S.ptr,
+                          ctx->ws_eta.ptr,
+                          ctx->ws_U.ptr,
+                          ctx->ws_band.ptr,
+                          rng,
+                          rng + (size_t)count * 2 * C.nt,
+                          rng + (size_t)count * (2 * C.nt + 2 * C.ntm),
+                          rng + (size_t)count * (4 * C.nt + 2 * C.ntm),
+                          ctx->ws_cnt.ptr,
+                          ctx->ws_pix.ptr,
+                          (uint32_t *)ctx->ws_touched.ptr,
+                          ctx->dstats.ptr};
+        hipEvent_t *ev = nullptr;
+        PICCA_HIP_CHECK(dmat_next_events(R, &ev));
+        PICCA_HIP_CHECK(hipEventRecord(ev[0], ctx->stream));
+        PICCA_HIP_CHECK(picca::launch_dmat_pass(C, R.F, P, W, R.O, R.pass_lds, ctx->stream));
+        PICCA_HIP_CHECK(hipEventRecord(ev[1], ctx->stream));
+        const int groups = (int)std::max<int64_t>(1, std::min<int64_t>(32, count / 16));
+        bool quasar = true;   // every delta2 of the batch unprojected
+        for (int64_t k = 0; k < count && quasar; ++k)
+            quasar = ctx->h_order[(size_t)L.b[(size_t)(p0 + k)]] < 0;
+        PICCA_HIP_CHECK(picca::launch_dmat_fill(C, R.F, P, W, R.O, groups, quasar, ctx->stream));
+        PICCA_HIP_CHECK(hipEventRecord(ev[2], ctx->stream));
+    }
+    return PICCA_OK;
+}
+
+bool power_of_two_times(int n, int base) {
+    if (base <= 0 || n % base != 0) return false;
+    const int k = n / base;
+    return (k & (k - 1)) == 0;
+}
+
+// The kernels for pairs without cuts (dmat_band_kernel.hip): takes the pairs they cover from
+// the list into `rest` what is left, and the pairs that they hand back.  Rule, per call: the
+// standard auto-correlation binning without a pair-redshift cut, model bins that split the data
+// bins in 2^k parts, LDS for a row of model bins; per pair: no zerr or same-half-plate cut, a
+// projected delta2, both forests with a proper fit normalisation and strictly rising r_comov and dist_m whose steps lie above
+// the rounding margins in both coordinates (the run walk's condition; 1e4 margins, so that the
+// index tables' 1e-3 of a step covers the rounding too).
+int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
+    picca_ctx *ctx = R.ctx;
+    const picca::DmatConst &C = R.C;
+    const int64_t num_pairs = L.size();
+    picca_cf_params model = *R.params;
+    model.num_bins_r_par = C.npm;
+    model.num_bins_r_trans = C.ntm;
+    model.edge_tol = 0.0;
+    picca::XiConst M;
+    int mode = 0;
+    const int kt = C.ntm / C.nt;
+    int band_rows = 0;
+    bool covered = !(C.flags & (picca::XI_HAS_ZMIN | picca::XI_HAS_ZMAX | picca::DMAT_XCORR |
+                                picca::DMAT_RMU)) &&
+                   C.rpmin == 0.0 && power_of_two_times(C.npm, C.np) &&
+                   power_of_two_times(C.ntm, C.nt) && !picca::fill_xi_const(&model, M, mode) &&
+                   !picca::widen_xi_margins(M, ctx->max_abs_r, ctx->max_abs_d);
+    if (covered) {
+        picca::apply_xi_schedule(M, PICCA_XI_SCHEDULE_RUNS);
+        const size_t row = picca::dmat_band_pass_lds(C, 1) - picca::dmat_band_pass_lds(C, 0);
+        const size_t fixed = picca::dmat_band_pass_lds(C, 0);
+        const size_t aim = std::min<size_t>(picca::DMAT_BAND_LDS, (size_t)ctx->lds_limit);
+        band_rows = fixed + row * kt <= aim ? (int)((aim - fixed) / (row * kt)) * kt : kt;
+        band_rows = std::min(band_rows, C.ntm);
+        covered = (int64_t)(picca::dmat_band_pass_lds(C, band_rows) + 1024) <= ctx->lds_limit;
+    }
+    if (!covered) {
+        rest = L;
+        return PICCA_OK;
+    }
+    std::vector<picca::DmatBandSlot> slots;
+    std::vector<double> cs;
+    std::vector<int64_t> origin;
+    for (int64_t k = 0; k < num_pairs; ++k) {
+        const int32_t a = L.a[(size_t)k], b = L.b[(size_t)k];
+        const double ang = L.ang[(size_t)k];
+        const uint8_t flags = L.flags[(size_t)k];
+        const double cos_half = std::cos(ang / 2), sin_half = std::sin(ang / 2);
+        const double cp = cos_half * M.inv_p, st = sin_half * M.inv_t;
+        auto steps = [&](int32_t f) {
+            const double2 spc = ctx->h_spc[(size_t)f];
+            return picca::walk_task(M, spc.x, spc.y, cp, st, 1.0) &&
+                   cp * spc.x > 1e4 * M.fast_p && st * spc.y > 1e4 * M.fast_t &&
+                   (ctx->h_mono[(size_t)f] & 3) == 3 && ctx->h_fit[(size_t)f] != 0;
+        };
+        const bool cut = ((C.flags & picca::XI_HAS_ZERR) && ang < C.zerr_ang) ||
+                         ((C.flags & picca::XI_REMOVE_SHP) &&
+                          (flags & picca::PAIR_SAME_HALF_PLATE)) ||
+                         (flags & picca::PAIR_XCF_COUNT);
+        if (cut || !(cos_half > 0) || ctx->h_order[(size_t)b] < 0 || !steps(a) || !steps(b)) {
+            rest.push(a, b, ang, flags);
+            continue;
+        }
+        // r_trans and its bin arithmetic do not fall with either dist_m, so the rows of the
+        // first and the last pixels' sums bound every pair's rows
+        const double y_lo = (ctx->h_dmin[(size_t)a] + ctx->h_dmin[(size_t)b]) * sin_half / C.rtmax;
+        const double y_hi = (ctx->h_dmax[(size_t)a] + ctx->h_dmax[(size_t)b]) * sin_half / C.rtmax;
+        const double t0 = std::fmax(std::floor(y_lo * C.nt_d), 0.0);
+        const double t1 = std::fmin(std::floor(y_hi * C.nt_d), C.nt_d - 1);
+        if (!(t0 <= t1)) continue;   // out of range: the pair adds nothing
+        picca::DmatBandSlot s;
+        s.a = a;
+        s.b = b;
+        s.t0 = (int)t0;
+        s.nt = (int)(t1 - t0) + 1;
+        s.u0 = s.t0 * kt;
+        s.nu = s.nt * kt;
+        s.t_row = s.u_row = 0;
+        slots.push_back(s);
+        cs.push_back(cos_half);
+        cs.push_back(sin_half);
+        origin.push_back(k);
+    }
+    const int64_t total = (int64_t)slots.size();
+    if (total == 0) return PICCA_OK;
+    hipStream_t st = ctx->stream;
+    const size_t entries = (size_t)(ctx->num_pixels + ctx->num_forests);
+    const bool differ = R.params->redshift_evolution && R.params->alpha != R.params->alpha2;
+    PICCA_HIP_CHECK(ctx->db_pre_b.reserve(entries));
+    if (differ) PICCA_HIP_CHECK(ctx->db_pre_a.reserve(entries));
+    picca::DmatPrefix *pre_b = ctx->db_pre_b.ptr, *pre_a = differ ? ctx->db_pre_a.ptr : pre_b;
+    PICCA_HIP_CHECK(ctx->db_table_r.reserve((size_t)ctx->num_pixels));
+    PICCA_HIP_CHECK(ctx->db_table_d.reserve((size_t)ctx->num_pixels));
+    PICCA_HIP_CHECK(picca::launch_dmat_prefix(R.F, ctx->num_forests, differ, pre_a, pre_b,
+                                              ctx->db_table_r.ptr, ctx->db_table_d.ptr, st));
+    const int tiles = C.nt * C.ntm;
+    PICCA_HIP_CHECK(ctx->db_cs.upload(cs.data(), cs.size(), st));
+    PICCA_HIP_CHECK(ctx->db_tile.reserve((size_t)tiles + 1));
+    PICCA_HIP_CHECK(ctx->db_redo.reserve((size_t)total));
+    // two 32-bit counters a word: items and queue, redo count
+    PICCA_HIP_CHECK(ctx->db_num.reserve(4));
+    PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->db_num.ptr, 2, st));
+    // batches: about 1.5 GiB of workspace rows
+    const double budget = 1536.0 * 1048576.0;
+    const double t_bytes = 8.0 * 4 * C.np + 16, u_bytes = 8.0 * 9 * C.npm + 16;
+    for (int64_t p0 = 0; p0 < total;) {
+        int64_t p1 = p0, t_rows = 0, u_rows = 0, list = 0;
+        while (p1 < total && p1 - p0 < (1 << 22)) {
+            picca::DmatBandSlot &s = slots[(size_t)p1];
+            if (p1 > p0 && (t_rows + s.nt) * t_bytes + (u_rows + s.nu) * u_bytes > budget) break;
+            if (p1 > p0 && list + (int64_t)s.nt * s.nu > (1 << 30)) break;
+            s.t_row = t_rows;
+            s.u_row = u_rows;
+            t_rows += s.nt;
+            u_rows += s.nu;
+            list += (int64_t)s.nt * s.nu;
+            ++p1;
+        }
+        const int64_t count = p1 - p0;
+        PICCA_HIP_CHECK(ctx->db_slot.upload(slots.data() + p0, (size_t)count, st));
+        PICCA_HIP_CHECK(ctx->db_S.reserve((size_t)t_rows * 4 * C.np));
+        PICCA_HIP_CHECK(ctx->db_eta.reserve((size_t)u_rows * 4 * C.npm));
+        PICCA_HIP_CHECK(ctx->db_eff.reserve((size_t)u_rows * 5 * C.npm));
+        PICCA_HIP_CHECK(ctx->db_rng_t.reserve((size_t)t_rows));
+        PICCA_HIP_CHECK(ctx->db_rng_u.reserve((size_t)u_rows));
+        PICCA_HIP_CHECK(ctx->db_list.reserve((size_t)list));
+        PICCA_HIP_CHECK(ctx->db_items.reserve((size_t)(list / picca::DMAT_BAND_ITEM + tiles)));
+        picca::DmatBandSlots P{ctx->db_slot.ptr, ctx->db_cs.ptr + 2 * p0, (int32_t)count,
+                               (int32_t)p0};
+        int32_t *num = ctx->db_num.ptr;
+        picca::DmatBandWork W{pre_a, pre_b, ctx->db_table_r.ptr, ctx->db_table_d.ptr,
+                              ctx->db_S.ptr, ctx->db_eta.ptr, ctx->db_eff.ptr,
+                              ctx->db_rng_t.ptr, ctx->db_rng_u.ptr, ctx->db_tile.ptr,
+                              ctx->db_list.ptr, ctx->db_items.ptr, num, num + 1,
+                              ctx->db_redo.ptr, num + 2, ctx->dstats.ptr};
+        PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->db_tile.ptr,
+                                               (tiles + 1) / 2, st));
+        hipEvent_t *ev = nullptr;
+        PICCA_HIP_CHECK(dmat_next_events(R, &ev));
+        PICCA_HIP_CHECK(hipEventRecord(ev[0], st));
+        PICCA_HIP_CHECK(picca::launch_dmat_band_pass(M, C, R.F, P, W, R.O, band_rows, st));
+        PICCA_HIP_CHECK(hipEventRecord(ev[1], st));
+        PICCA_HIP_CHECK(picca::launch_dmat_band_fill(M, C, R.F, P, W, R.O, ctx->num_cus, st));
+        PICCA_HIP_CHECK(hipEventRecord(ev[2], st));
+        p0 = p1;
+    }
+    R.host_buffers();
+    int32_t num_redo = 0;
+    PICCA_HIP_CHECK(hipMemcpyAsync(&num_redo, ctx->db_num.ptr + 2, sizeof(num_redo),
+                                   hipMemcpyDeviceToHost, st));
+    PICCA_HIP_CHECK(hipStreamSynchronize(st));
+    if (num_redo > 0) {
+        std::vector<int32_t> redo((size_t)num_redo);
+        PICCA_HIP_CHECK(hipMemcpyAsync(redo.data(), ctx->db_redo.ptr,
+                                       sizeof(int32_t) * redo.size(), hipMemcpyDeviceToHost, st));
+        PICCA_HIP_CHECK(hipStreamSynchronize(st));
+        std::sort(redo.begin(), redo.end());
+        for (int32_t r : redo) {
+            const size_t k = (size_t)origin[(size_t)r];
+            rest.push(L.a[k], L.b[k], L.ang[k], L.flags[k]);
+        }
+    }
+    return PICCA_OK;
+}
+
+}  // namespace
+
 int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pairs,
                    const int32_t *pair_a, const int32_t *pair_b, const double *pair_ang,
                    const uint8_t *pair_flags, double *weights_dmat, double *dmat,
@@ -1024,17 +1324,6 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
         PICCA_HIP_CHECK(ctx->zfa.upload_padded(fa.data(), (size_t)npix, pad, ctx->stream));
         PICCA_HIP_CHECK(ctx->zfb.upload_padded(fb.data(), (size_t)npix, pad, ctx->stream));
     }
-    std::vector<double> cs((size_t)std::max<int64_t>(2 * num_pairs, 1));
-    for (int64_t k = 0; k < num_pairs; ++k) {
-        cs[2 * k] = std::cos(pair_ang[k] / 2);
-        cs[2 * k + 1] = std::sin(pair_ang[k] / 2);
-    }
-    PICCA_HIP_CHECK(ctx->dpa.upload(pair_a, (size_t)num_pairs, ctx->stream));
-    PICCA_HIP_CHECK(ctx->dpb.upload(pair_b, (size_t)num_pairs, ctx->stream));
-    PICCA_HIP_CHECK(ctx->dang.upload(pair_ang, (size_t)num_pairs, ctx->stream));
-    PICCA_HIP_CHECK(ctx->dcs.upload(cs.data(), (size_t)(2 * num_pairs), ctx->stream));
-    PICCA_HIP_CHECK(ctx->dflags.upload(pair_flags, (size_t)num_pairs, ctx->stream));
-
     // outputs, accumulated over all batches on the device
     const int64_t nb = C.nb, nm = C.nm;
     PICCA_HIP_CHECK(ctx->o_wdm.reserve((size_t)nb));
@@ -1048,73 +1337,24 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
                                            ctx->stream));
     PICCA_HIP_CHECK(picca::launch_zero_u64(ctx->dstats.ptr, picca::DMAT_NSTATS, ctx->stream));
 
-    // workspace per slot
-    const size_t slot_bytes = 8 * (4 * (size_t)C.nt * C.np + 4 * (size_t)C.ntm * C.npm) +
-                              4 * (size_t)C.words_u + 16 + 16 * (size_t)(C.nt + C.ntm);
-    const size_t ws_budget = (size_t)1536 << 20;
-    const int64_t cap = std::max<int64_t>(
-        1, std::min<int64_t>({num_pairs, (int64_t)(ws_budget / slot_bytes), (int64_t)1 << 20}));
-    const int64_t touched_words = ((int64_t)C.nt * C.ntm + 63) / 64;
-    PICCA_HIP_CHECK(ctx->ws_S.reserve((size_t)cap * 4 * C.nt * C.np));
-    PICCA_HIP_CHECK(ctx->ws_eta.reserve((size_t)cap * 4 * C.ntm * C.npm));
-    PICCA_HIP_CHECK(ctx->ws_U.reserve((size_t)cap * C.words_u));
-    PICCA_HIP_CHECK(ctx->ws_band.reserve((size_t)cap * 4));
-    PICCA_HIP_CHECK(ctx->ws_rng.reserve((size_t)cap * 4 * (C.nt + C.ntm)));
-    PICCA_HIP_CHECK(ctx->ws_pix.reserve((size_t)cap));
-    PICCA_HIP_CHECK(ctx->ws_touched.reserve((size_t)touched_words));
-
     picca::DmatForests F{ctx->r.ptr,   ctx->d.ptr,     ctx->z.ptr,     ctx->w.ptr,   ctx->dll.ptr,
                          ctx->zfa.ptr, ctx->zfb.ptr,   ctx->off.ptr,   ctx->zq.ptr,  ctx->sum_w.ptr,
                          ctx->sw_dll.ptr, ctx->order.ptr, ctx->mono.ptr};
     picca::DmatOut O{ctx->o_wdm.ptr, ctx->o_dmat.ptr, ctx->o_eff.ptr, ctx->o_eff.ptr + nm,
                      ctx->o_eff.ptr + 2 * nm, ctx->o_eff.ptr + 3 * nm};
-    std::vector<int64_t> pix_off;
-    int64_t batches = 0;
-    for (int64_t p0 = 0; p0 < num_pairs; p0 += cap) {
-        const int64_t count = std::min(cap, num_pairs - p0);
-        pix_off.assign((size_t)count, 0);
-        int64_t total = 0;
-        for (int64_t k = 0; k < count; ++k) {
-            pix_off[k] = total;
-            const int32_t a = pair_a[p0 + k];
-            total += ctx->h_offsets[a + 1] - ctx->h_offsets[a];
-        }
-        PICCA_HIP_CHECK(ctx->ws_pix.upload(pix_off.data(), (size_t)count, ctx->stream));
-        PICCA_HIP_CHECK(ctx->ws_cnt.reserve((size_t)std::max<int64_t>(total, 1)));
-        PICCA_HIP_CHECK(picca::launch_zero_u64(ctx->ws_touched.ptr, touched_words, ctx->stream));
-        picca::DmatPairs P{ctx->dpa.ptr + p0, ctx->dpb.ptr + p0, ctx->dang.ptr + p0,
-                           ctx->dcs.ptr + 2 * p0, ctx->dflags.ptr + p0, (int32_t)count};
-        int32_t *rng = ctx->ws_rng.ptr;
-        picca::DmatWork W{ctx->ws_S.ptr,
-                          ctx->ws_eta.ptr,
-                          ctx->ws_U.ptr,
-                          ctx->ws_band.ptr,
-                          rng,
-                          rng + (size_t)count * 2 * C.nt,
-                          rng + (size_t)count * (2 * C.nt + 2 * C.ntm),
-                          rng + (size_t)count * (4 * C.nt + 2 * C.ntm),
-                          ctx->ws_cnt.ptr,
-                          ctx->ws_pix.ptr,
-                          (uint32_t *)ctx->ws_touched.ptr,
-                          ctx->dstats.ptr};
-        const size_t ev = 3 * (size_t)batches++;
-        while (ctx->dmat_events.size() < ev + 3) {
-            hipEvent_t e = nullptr;
-            PICCA_HIP_CHECK(hipEventCreate(&e));
-            ctx->dmat_events.push_back(e);
-        }
-        PICCA_HIP_CHECK(hipEventRecord(ctx->dmat_events[ev], ctx->stream));
-        PICCA_HIP_CHECK(picca::launch_dmat_pass(C, F, P, W, O, pass_lds, ctx->stream));
-        PICCA_HIP_CHECK(hipEventRecord(ctx->dmat_events[ev + 1], ctx->stream));
-        const int groups = (int)std::max<int64_t>(1, std::min<int64_t>(32, count / 16));
-        bool quasar = true;   // every delta2 of the batch unprojected
-        for (int64_t k = 0; k < count && quasar; ++k)
-            quasar = ctx->h_order[(size_t)pair_b[p0 + k]] < 0;
-        PICCA_HIP_CHECK(picca::launch_dmat_fill(C, F, P, W, O, groups, quasar, ctx->stream));
-        PICCA_HIP_CHECK(hipEventRecord(ctx->dmat_events[ev + 2], ctx->stream));
-    }
+    DmatRun R{ctx, params, C, F, O, pass_lds, 0, {}, {}, {}, {}, {}};
+    DmatPairList pairs, rest;
+    pairs.a.assign(pair_a, pair_a + num_pairs);
+    pairs.b.assign(pair_b, pair_b + num_pairs);
+    pairs.ang.assign(pair_ang, pair_ang + num_pairs);
+    pairs.flags.assign(pair_flags, pair_flags + num_pairs);
+    status = dmat_run_band(R, pairs, rest);
+    if (status == PICCA_OK) status = dmat_run_general(R, rest);
+    if (status != PICCA_OK) return status;
+    const int64_t batches = R.batches;
 
-    std::vector<double> h_wdm((size_t)nb), h_dmat((size_t)(nb * nm)), h_eff((size_t)(4 * nm));
+    R.host_buffers();
+    std::vector<double> &h_wdm = R.h_wdm, &h_dmat = R.h_dmat, &h_eff = R.h_eff;
     unsigned long long h_stats[picca::DMAT_NSTATS];
     PICCA_HIP_CHECK(hipMemcpyAsync(h_wdm.data(), ctx->o_wdm.ptr, sizeof(double) * nb,
                                    hipMemcpyDeviceToHost, ctx->stream));

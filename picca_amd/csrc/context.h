@@ -12,6 +12,7 @@
 
 #include "../../include/picca_hip.h"
 #include "engine.h"
+#include "dmat_band.h"
 #include "xi_walk.h"
 
 namespace picca_host {
@@ -120,6 +121,9 @@ struct picca_ctx {
     std::vector<int32_t> h_order;   // host copy of the fit orders (< 0: unprojected)
     std::vector<int64_t> h_offsets;
     std::vector<double> h_dmin, h_dmax;   // per forest: smallest / largest dist_m
+    std::vector<double2> h_spc;           // per forest: smallest steps (ForestView::spc)
+    std::vector<uint8_t> h_mono;          // per forest: ForestView::mono
+    std::vector<uint8_t> h_fit;           // per forest: sum w and sum w dll^2 are positive
     DeviceBuffer<double> z, r, d, w, dw, ll, zq;
     DeviceBuffer<picca::PixelRecord> pix;
     DeviceBuffer<int64_t> off;
@@ -163,6 +167,12 @@ struct picca_ctx {
     DeviceBuffer<int64_t> ws_pix;
     DeviceBuffer<unsigned long long> ws_touched, dstats;
     DeviceBuffer<double> o_wdm, o_dmat, o_eff;
+    // forest pairs without cuts: prefix sums of both roles and the workspace of a batch
+    DeviceBuffer<picca::DmatPrefix> db_pre_a, db_pre_b;
+    DeviceBuffer<picca::DmatBandSlot> db_slot;
+    DeviceBuffer<double> db_cs, db_S, db_eta, db_eff;
+    DeviceBuffer<int4> db_rng_t, db_rng_u, db_items;
+    DeviceBuffer<int32_t> db_tile, db_list, db_redo, db_num, db_table_r, db_table_d;
 
     // metal distortion matrix: absorber tables per slot (store order) and per-pass tasks
     struct MetalSlot {

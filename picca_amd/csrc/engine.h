@@ -233,6 +233,59 @@ struct DmatOut {
     double *r_par_eff, *r_trans_eff, *z_eff, *weight_eff;  // [nm]
 };
 
+// Forest pairs without cuts (dmat_band_kernel.hip)
+constexpr int DMAT_BAND_PASS_BLOCK = 256;   // threads of the pair pass (lane per pixel i)
+constexpr int DMAT_BAND_FILL_BLOCK = 256;   // threads of the fill (4 waves)
+constexpr int DMAT_BAND_SUMS = 11;          // LDS sums per model bin of the pair pass
+constexpr size_t DMAT_BAND_LDS = 53 * 1024; // LDS aim of the pair pass: three workgroups a CU
+constexpr int DMAT_BAND_ITEM = 8;           // forest pairs of one tile per work item
+
+// One forest pair of a batch: its r_trans rows [t0, t0 + nt) of the data bins and
+// [u0, u0 + nu) of the model bins (bounds from the forests' dist_m) and its first rows in the
+// workspace.
+struct DmatBandSlot {
+    int32_t a, b, t0, nt, u0, nu;
+    int64_t t_row, u_row;
+};
+
+struct DmatBandSlots {
+    const DmatBandSlot *__restrict__ slot;
+    const double *__restrict__ cs;   // cos(ang/2), sin(ang/2)
+    int32_t count;
+    int32_t first;                   // index of slot 0 among the call's pairs of this kind
+};
+
+struct DmatPrefix;   // dmat_band.h
+
+struct DmatBandWork {
+    const DmatPrefix *__restrict__ pre_a;   // prefix sums with delta1's evolution factors
+    const DmatPrefix *__restrict__ pre_b;   // and with delta2's
+    const int32_t *__restrict__ table_r;    // index tables of r_comov and dist_m, forest f at
+    const int32_t *__restrict__ table_d;    // off[f]
+    double *S;            // [t row][4][np]   S0, Sj, Si, Sij
+    double *eta;          // [u row][4][npm]  eta5..eta8
+    double *eff;          // [u row][5][npm]  effective-coordinate sums, pair-bin term
+    int4 *rng_t, *rng_u;  // [row] first and last pixel of delta1, of delta2 (empty: first > last)
+    int32_t *tile_count;  // [nt * ntm]
+    int32_t *list;        // forest pairs of each tile
+    int4 *items;          // tile, first list entry, entries
+    int32_t *num_items, *queue;
+    int32_t *redo, *num_redo;   // pairs left to the general kernels
+    unsigned long long *stats;  // [DMAT_NSTATS]
+};
+
+// prefix sums and index tables (dmat_band.h) of every forest
+hipError_t launch_dmat_prefix(const DmatForests &F, int64_t num_forests, bool roles_differ,
+                              DmatPrefix *pa, DmatPrefix *pb, int32_t *table_r,
+                              int32_t *table_d, hipStream_t stream);
+hipError_t launch_dmat_band_pass(const XiConst &M, const DmatConst &C, const DmatForests &F,
+                                 const DmatBandSlots &P, const DmatBandWork &W,
+                                 const DmatOut &O, int band_rows, hipStream_t stream);
+hipError_t launch_dmat_band_fill(const XiConst &M, const DmatConst &C, const DmatForests &F,
+                                 const DmatBandSlots &P, const DmatBandWork &W,
+                                 const DmatOut &O, int num_cus, hipStream_t stream);
+size_t dmat_band_pass_lds(const DmatConst &C, int rows);
+
 hipError_t launch_dmat_pass(const DmatConst &C, const DmatForests &F, const DmatPairs &P,
                             const DmatWork &W, const DmatOut &O, size_t lds,
                             hipStream_t stream);

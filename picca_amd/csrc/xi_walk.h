@@ -235,6 +235,19 @@ PICCA_HD inline bool walk_run_sums(const XiConst &C, const WalkTask &T, const Wa
     return n > 0;
 }
 
+// What a walk sums over its runs: the prefix records it reads, the sums of a run, and whether
+// its memory wants each closed run (mem.closed).  XiAcc: compute_xi's sums.
+template <bool XC>
+struct XiAcc {
+    using Prefix = PrefixRecord;
+    using Sums = RunSums;
+    static constexpr bool RUNS = false;
+    PICCA_HD static bool sums(const XiConst &C, const WalkTask &T, const WalkLane &L, int m, int c,
+                              const Prefix &ps, const Prefix &pe, Sums &o) {
+        return walk_run_sums<XC>(C, T, L, m, c, ps, pe, o);
+    }
+};
+
 // Reciprocal of x > 0 within 2.5e-4 relative, the same on the host and the device: the
 // seed is the bit pattern of 2.0^1023 (0x7FE0...) minus that of x, within 12.5 % of 1 / x
 // for a normal x, then two Newton steps y (2 - x y).  For the guess of a run's end only.
@@ -307,7 +320,7 @@ PICCA_HD inline bool walk_terminal(const XiConst &C, int m, int c) {
 // reference's edge, overflow and wrap-around treatment (walk_special).
 // XC: cross-correlation (signed r_par; the launch's rows [C.row0, C.row0 + C.rows)).  CUTS:
 // the lane's own window [L.j_lo, L.j_hi) (pair-redshift cuts; empty: `alive` false) and T.shp.
-template <bool XC = false, bool CUTS = false, class Mem = void>
+template <bool XC = false, bool CUTS = false, class Acc = XiAcc<XC>, class Mem = void>
 PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLane &L, Mem &mem,
                                bool alive) {
     const int j_hi = CUTS ? L.j_hi : T.j_hi;
@@ -322,7 +335,7 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
     double Ka = r1cp, Kb = -d1st;
     int j = CUTS ? L.j_lo : T.j_lo;
     bool starting = true;
-    PrefixRecord ps = {0, 0, 0, 0, 0, 0};
+    typename Acc::Prefix ps = {};
     int lo = j, hi = j_hi, g = j, misses = 0, step = 1;
     bool near_lo = false;
     // the pass's probes: pixels pa and pb and the prefix entry at pb, loaded at the end of
@@ -331,13 +344,13 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
     double ra, da, rb, db;
     mem.rd(pa, ra, da);
     mem.rd(pb, rb, db);
-    PrefixRecord pg = mem.prefix(pb);
+    typename Acc::Prefix pg = mem.prefix(pb);
     for (;;) {
         // the sums of the run [j, g) of the current key, added by mem.flush with every lane
         // of the wave if the run closes in this pass (`on`); computed by every lane, so that
         // the values the flush moves between lanes are finite
-        RunSums run;
-        const bool nonempty = walk_run_sums<XC>(C, T, L, m, c, ps, pg, run);
+        typename Acc::Sums run;
+        const bool nonempty = Acc::sums(C, T, L, m, c, ps, pg, run);
         mem.pin(run);
         bool on = false;
         if (alive) {
@@ -380,6 +393,7 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
                 mem.count_run(run.n);
                 on = nonempty && m >= (XC ? -(C.row0 + C.rows) : -C.np);
                 if constexpr (CUTS && !XC) on = on && !(T.shp && (m == 0 || m == -1));
+                if constexpr (Acc::RUNS) mem.closed(on, j, g, c);
             }
             // next state
             const int g_miss = misses == 0 ? g - 1 : lo + 1 + ((g - 1 - lo) >> 1);

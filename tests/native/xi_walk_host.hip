@@ -12,6 +12,7 @@
 #include <cstring>
 #include <vector>
 
+#include "../../picca_amd/csrc/dmat_band.h"
 #include "../../picca_amd/csrc/xi_const.h"
 #include "../../picca_amd/csrc/xi_walk.h"
 
@@ -325,6 +326,23 @@ extern "C" {
 
 // The walk's guess reciprocal (walk_rcp_guess), for its unit test.
 double xi_walk_rcp_guess(double x) { return picca::walk_rcp_guess(x); }
+
+// The banded distortion matrix's keys and edges (dmat_band.h) of one pixel along a partner of n
+// rising values v, par: along r_par, else r_trans.  keys[k]: of pixel k; edges[k]: first pixel
+// whose key is at least k_lo + k.  The index table is made as the table kernel makes it.
+void dmat_band_host(int par, int n, const double *v, double self, double scale, double range,
+                    int bins, double margin, int *keys, int k_lo, int num, int *edges) {
+    const double mul = scale * bins / range;
+    const picca::BandAxis A = par ? picca::band_par_axis(self, mul, scale, range, bins, margin)
+                                  : picca::band_trans_axis(self, mul, scale, range, bins, margin);
+    const double h = picca::band_mean_step(v[0], v[n - 1], n);
+    std::vector<int32_t> first((size_t)n);
+    for (int k = 0; k < n; ++k) first[(size_t)k] = lower(v, n, v[0] + k * h, true);
+    const picca::BandTable T{first.data(), v[0], 1.0 / h, n};
+    for (int k = 0; k < n; ++k) keys[k] = picca::band_key(A, v[k]);
+    for (int k = 0; k < num; ++k)
+        edges[k] = picca::band_edge(A, T, [&](int p) { return v[p]; }, k_lo + k);
+}
 
 // Correlation of the listed forest pairs (specialised case of the pair kernel only).
 // Outputs are [num_rows * np * nt] each, added to; stats = edge, overflow, walked tasks,

@@ -1,0 +1,90 @@
+"""The distortion matrix of forest pairs without cuts (prefix sums over runs) on the GPU against
+the FP64 oracle: exact bin edges, zero weights, short and non-monotone forests, random
+geometries, model bins that split the data bins in 1, 2, 4 (taken) or 3 (general kernels) parts,
+more r_par bins than one chunk of the fill and more r_trans rows than one band of the pass.
+Counts equal; sums within 1e-9 relative or 1e-12 of the largest entry, as in test_gpu_dmat."""
+import numpy as np
+import pytest
+
+import walk_cases as W
+from oracle import cf_oracle as O
+from picca_amd import _native
+from picca_amd.engine import get_engine, params_from_globals
+from picca_amd.store import ForestStore
+from test_gpu_dmat import assert_outputs_close
+
+pytestmark = pytest.mark.gpu
+
+
+def dmat_store(store, seed, orders):
+    rng = np.random.default_rng(seed)
+    n = len(store.offsets) - 1
+    return ForestStore(store.offsets, store.z, store.r_comov, store.dist_m, store.weights,
+                       store.delta, store.z_qso, store.ra, store.dec, store.thingid,
+                       log_lambda=np.log10(1215.67 * (1 + store.z)),
+                       order=rng.choice(orders, n).astype(np.int32))
+
+
+def check(case, orders=(1,), flags=None, seed=0):
+    g, p = case.g, case.pairs
+    store = dmat_store(case.store, seed, orders)
+    # a forest without two weighted pixels has no projection
+    used = np.array([(store.weights[o:e] != 0).sum() for o, e in zip(store.offsets[:-1],
+                                                                    store.offsets[1:])])
+    keep = (used[p.pair_a] > 1) & (used[p.pair_b] > 1)
+    a, b, ang = p.pair_a[keep], p.pair_b[keep], p.pair_ang[keep]
+    flags = np.zeros(len(a), np.uint8) if flags is None else flags(len(a))
+    eng = get_engine(0)
+    eng.set_forests(store)
+    mine = eng.dmat(params_from_globals(g), a, b, ang, flags)
+    ref, stats = O.dmat_rows(O.params_from_module(g), store, a, b, ang, flags)
+    assert list(mine[6]) == list(stats) and stats[0] > 0
+    assert_outputs_close(mine[:6], ref)
+
+
+def with_model(case, kp, kt):
+    case.g.num_model_bins_r_par = kp * case.g.num_bins_r_par
+    case.g.num_model_bins_r_trans = kt * case.g.num_bins_r_trans
+    return case
+
+
+@pytest.mark.parametrize("kp,kt", [(1, 1), (2, 1), (2, 2), (4, 1), (3, 1)])
+def test_exact_bin_edges(kp, kt):
+    case = W.lattice_case()
+    case.g.num_bins_r_par = case.g.num_bins_r_trans = 20
+    check(with_model(case, kp, kt))
+
+
+@pytest.mark.parametrize("orders", [(1,), (0, 1)])
+def test_irregular_forests(orders):
+    case = W.irregular_case()
+    case.g.num_bins_r_par = case.g.num_bins_r_trans = 25
+    check(with_model(case, 2, 1), orders)
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2, 3, 4, 5, 6, 7, 9])   # (8: no pair in range)
+def test_random_geometries(seed):
+    case = W.random_case(seed)
+    case.g.num_bins_r_par = 1 + case.g.num_bins_r_par % 30
+    case.g.num_bins_r_trans = 1 + case.g.num_bins_r_trans % 30
+    check(with_model(case, (1, 2)[seed % 2], 1), (0, 1), seed=seed)
+
+
+@pytest.mark.parametrize("n_par,n_trans", [(64, 12), (65, 12), (16, 40), (1, 1)])
+def test_chunks_and_bands(n_par, n_trans):
+    """64 data and 112 model r_par bins make a chunk of the fill; a wide pair reaches more
+    r_trans rows than a band of the pass holds."""
+    case = W.random_case(3)
+    case.g.num_bins_r_par, case.g.num_bins_r_trans = n_par, n_trans
+    case.g.r_par_max, case.g.r_trans_max = 120.0, 400.0
+    case.pairs.pair_ang[:] = np.linspace(0.001, 0.09, case.pairs.num_pairs)
+    check(with_model(case, 2, 1))
+
+
+def test_cut_pairs_take_the_general_kernels():
+    case = with_model(W.irregular_case(), 1, 1)
+    case.g.num_bins_r_par = case.g.num_bins_r_trans = 15
+    with_model(case, 1, 1)
+    case.g.remove_same_half_plate_close_pairs = True
+    check(case, flags=lambda n: (np.arange(n) % 3 == 0).astype(np.uint8)
+          * _native.PICCA_PAIR_SAME_HALF_PLATE)

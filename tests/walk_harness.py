@@ -12,7 +12,8 @@ import numpy as np
 HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCE = os.path.join(HERE, "native", "xi_walk_host.hip")
 CSRC = os.path.join(os.path.dirname(HERE), "picca_amd", "csrc")
-DEPENDS = [SOURCE] + [os.path.join(CSRC, h) for h in ("xi_walk.h", "xi_const.h", "engine.h")]
+DEPENDS = [SOURCE] + [os.path.join(CSRC, h) for h in ("xi_walk.h", "xi_const.h", "engine.h",
+                                                        "dmat_band.h")]
 LIBRARY = os.path.join(HERE, "native", "libxi_walk_host.so")
 STATS = ("edge", "overflow", "walk_tasks", "pair_tasks", "runs", "probes", "oob", "cover")
 
@@ -55,6 +56,17 @@ def rcp_guess(x):
 
 def _p(a):
     return a.ctypes.data_as(ctypes.c_void_p)
+
+
+def dmat_band(par, values, own, scale, span, bins, margin, k_lo, num):
+    """Keys of the pixels and the first pixel of each key from k_lo on (dmat_band.h)."""
+    v = np.ascontiguousarray(values, dtype=np.float64)
+    keys, edges = np.zeros(len(v), dtype=np.int32), np.zeros(num, dtype=np.int32)
+    lib().dmat_band_host(ctypes.c_int(par), ctypes.c_int(len(v)), _p(v), ctypes.c_double(own),
+                         ctypes.c_double(scale), ctypes.c_double(span), ctypes.c_int(bins),
+                         ctypes.c_double(margin), _p(keys), ctypes.c_int(k_lo),
+                         ctypes.c_int(num), _p(edges))
+    return keys, edges
 
 
 def xi_walk_cuts(params, store, pair_a, pair_b, pair_ang, pair_flags, pair_row, num_rows, share):
