@@ -42,6 +42,22 @@ int picca_cont_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *o
     PICCA_HIP_CHECK(ctx->c_lss.upload(var_lss, n, st));
     PICCA_HIP_CHECK(ctx->c_fudge.upload(fudge, n, st));
     PICCA_HIP_CHECK(ctx->c_order.upload(order, (size_t)num_forests, st));
+    // forests by the waves that hold their pixels
+    std::vector<int32_t> by_class[picca::CONT_CLASSES];
+    for (int64_t k = 0; k < num_forests; ++k) {
+        const int64_t len = offsets[k + 1] - offsets[k];
+        int c = 0;
+        while (c < picca::CONT_CLASSES - 1 && len > ((int64_t)64 * picca::CONT_PIXELS_PER_LANE) << c)
+            ++c;
+        by_class[c].push_back((int32_t)k);
+    }
+    std::vector<int32_t> ordered;
+    for (int c = 0; c < picca::CONT_CLASSES; ++c) {
+        ctx->cont_class_begin[c] = (int64_t)ordered.size();
+        ordered.insert(ordered.end(), by_class[c].begin(), by_class[c].end());
+    }
+    ctx->cont_class_begin[picca::CONT_CLASSES] = (int64_t)ordered.size();
+    PICCA_HIP_CHECK(ctx->c_class.upload(ordered.data(), ordered.size(), st));
     const size_t nf = (size_t)std::max<int64_t>(num_forests, 1);
     PICCA_HIP_CHECK(ctx->c_a0.reserve(nf));
     PICCA_HIP_CHECK(ctx->c_b0.reserve(nf));
@@ -84,7 +100,8 @@ int picca_cont_fit(picca_ctx *ctx, const picca_cont_params *params, const double
     picca::ContOut O{ctx->c_a.ptr, ctx->c_b.ptr, ctx->c_chi2.ptr, ctx->c_ndata.ptr,
                      ctx->c_status.ptr, ctx->c_evals.ptr};
     PICCA_HIP_CHECK(hipEventRecord(ctx->ev_start, st));
-    PICCA_HIP_CHECK(picca::launch_cont_fit(K, I, O, nf, st));
+    PICCA_HIP_CHECK(picca::launch_cont_fit(K, I, O, ctx->c_class.ptr, ctx->cont_class_begin,
+                                           st));
     PICCA_HIP_CHECK(hipEventRecord(ctx->ev_stop, st));
     if (nf > 0) {
         PICCA_HIP_CHECK(hipMemcpyAsync(a, ctx->c_a.ptr, sizeof(double) * nf, hipMemcpyDeviceToHost, st));

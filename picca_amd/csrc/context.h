@@ -200,6 +200,8 @@ struct picca_ctx {
     int64_t cont_forests = 0;
     int64_t cont_pixels = 0;
     DeviceBuffer<int64_t> c_off;
+    DeviceBuffer<int32_t> c_class;   // forests ordered by the waves their fit takes
+    int64_t cont_class_begin[picca::CONT_CLASSES + 1] = {0, 0, 0, 0, 0, 0};
     DeviceBuffer<double> c_flux, c_ivar, c_mean, c_x, c_eta, c_lss, c_fudge;
     DeviceBuffer<int32_t> c_order;
     DeviceBuffer<double> c_a0, c_b0, c_a, c_b, c_chi2;

@@ -493,8 +493,16 @@ struct ContOut {
     int32_t *ndata, *status, *evals;
 };
 
+// Pixels of a forest that one lane of the fit holds in registers: a forest takes 1, 2, 4 or 8
+// waves, or the kernel that reads its pixels at every evaluation.
+constexpr int CONT_PIXELS_PER_LANE = 10;
+constexpr int CONT_CLASSES = 5;
+
+// forests: indices ordered by class (1, 2, 4, 8 waves, longer); class c is
+// [class_begin[c], class_begin[c + 1])
 hipError_t launch_cont_fit(const ContConst &K, const ContIn &I, const ContOut &O,
-                           int64_t n_forests, hipStream_t stream);
+                           const int32_t *forests, const int64_t *class_begin,
+                           hipStream_t stream);
 // DR16 iteration: weighted F / C stack in rest-frame bins over the forests whose last fit
 // is valid (status 0); interpolation of the new mean continuum to every pixel
 hipError_t launch_cont_stack(const ContIn &I, const double *a, const double *b,
