@@ -189,12 +189,13 @@ struct picca_ctx {
     // subsampling covariance: rows, weights, per-bin means and weight sums, matrix
     DeviceBuffer<double> cv_xi, cv_w, cv_y, cv_s, cv_cov;
 
-    // Wick terms: evolution factors, weighted 1-D correlations, per-batch lists and tasks
-    DeviceBuffer<double> wk_zev1, wk_zev2, wk_wx, wk_c1;
-    DeviceBuffer<int64_t> wk_wxoff, wk_base, wk_list, wk_c1off;
-    DeviceBuffer<int32_t> wk_count, wk_task, wk_segcount, wk_forests;
-    DeviceBuffer<int4> wk_seg;
-    DeviceBuffer<unsigned long long> wk_nb, wk_stats, wk_ntasks;
+    // Wick terms: evolution factors, weighted 1-D correlations, per-batch segments and tasks
+    DeviceBuffer<double> wk_zev1, wk_zev2, wk_wx, wk_rsum, wk_diag, wk_wz;
+    DeviceBuffer<int64_t> wk_wxoff;
+    DeviceBuffer<int32_t> wk_segcount, wk_segpos, wk_forests;
+    DeviceBuffer<int4> wk_seg, wk_seg_raw;
+    DeviceBuffer<picca::WickTask> wk_task;
+    DeviceBuffer<unsigned long long> wk_nb, wk_stats;
 
     // continuum fit: resident spectra (forest pixels) and per-forest results
     int64_t cont_forests = 0;

@@ -398,6 +398,7 @@ hipError_t launch_cov_syrk(const double *xi, const double *w, const double *S,
 // ---------------------------------------------------------------------------------------
 
 constexpr int WICK_BLOCK = 256;
+constexpr int WICK_SORT = 4096;   // segments of one (pair, bin) that are sorted in LDS
 
 enum : int {
     WICK_STAT_IN_RANGE = 0,    // listed pixel pairs
@@ -420,8 +421,6 @@ struct WickInputs {
     const double *__restrict__ zev2;     // ((1+z)/(1+z_ref))^(alpha2-1)
     const double *__restrict__ wx;       // weighted 1-D correlations, n x n per forest
     const int64_t *__restrict__ wx_off;  // [forest] offset of its matrix in wx
-    const double *__restrict__ c1;       // row prefix sums of wx, n x (n + 1) per forest
-    const int64_t *__restrict__ c1_off;  // [forest] offset of its prefix sums in c1
 };
 
 struct WickPairs {
@@ -431,17 +430,23 @@ struct WickPairs {
     int32_t count;
 };
 
+// One (pair, bin P): the pair's segments in the bin, all of the pair's segments, and the first
+// entry of its rows in rsum.
+struct WickTask {
+    int32_t pair, bin, start, count, pair_start, pair_count;
+    int64_t rows;
+};
+
 struct WickWork {
-    int64_t *list;             // per pair, its in-range pixel pairs sorted by bin
-    const int64_t *base;       // [pair] offset of its list (capacity n1 n2)
-    int32_t *count;            // [pair] listed pixel pairs
-    int4 *seg;                 // per pair (same offsets as list), its segments sorted by bin:
-                               // (bin, j, i_lo, i_hi), pixels i_lo..i_hi of delta1 that
-                               // pixel j of delta2 pairs with in that bin
-    int32_t *seg_count;        // [pair] segments
-    int32_t *task_pair, *task_bin, *task_start, *task_count;
-    unsigned long long *num_tasks;
-    int64_t max_tasks;
+    int32_t *seg_count;        // [pair][nb] segments per bin
+    int32_t *seg_pos;          // [pair][nb] fill positions (their prefix sums)
+    int4 *seg_raw, *seg;       // per pair, its segments by bin: (bin, j, i_lo, i_hi), pixels
+                               // i_lo..i_hi of delta1 that pixel j of delta2 pairs with in that
+                               // bin; as they came, and by rising j in each bin
+    const WickTask *task;
+    double *rsum;              // [segment of a task][n1 + 1]
+    const double *diag, *wz;   // prefix sums of the diagonal of wx and of w zev1 of each forest,
+                               // forest f at off[f] + f
 };
 
 struct WickOut {
@@ -451,17 +456,18 @@ struct WickOut {
     unsigned long long *stats;             // [WICK_NSTATS]
 };
 
-hipError_t launch_wick_list(const WickConst &C, const WickInputs &I, const WickPairs &P,
-                            const WickWork &W, const WickOut &O, hipStream_t stream);
+hipError_t launch_wick_diag(const WickInputs &I, const int32_t *forests, int32_t num_forests,
+                            double *diag, double *wz, hipStream_t stream);
+// longest: pixels of the longest delta2 of the pairs
+hipError_t launch_wick_segments(bool place, const WickConst &C, const WickInputs &I,
+                                const WickPairs &P, const WickWork &W, const WickOut &O,
+                                int64_t longest, hipStream_t stream);
+hipError_t launch_wick_sort(const WickWork &W, int64_t tasks, hipStream_t stream);
 hipError_t launch_wick_rows(const WickConst &C, const WickInputs &I, const WickPairs &P,
                             const WickWork &W, const WickOut &O, int64_t tasks,
                             hipStream_t stream);
 size_t wick_list_lds(const WickConst &C);
 size_t wick_row_lds(const WickConst &C);
-// row prefix sums c1 of the weighted 1-D correlation of each listed forest
-hipError_t launch_wick_prefix(const double *wx, const int64_t *wx_off, const int64_t *off,
-                              const int32_t *forests, int32_t num_forests, double *c1,
-                              const int64_t *c1_off, hipStream_t stream);
 
 // ---------------------------------------------------------------------------------------
 // continuum fit

@@ -74,56 +74,55 @@ int picca_wick_t123(picca_ctx *ctx, const picca_cf_params *params, int64_t num_p
     PICCA_HIP_CHECK(ctx->wk_nb.reserve((size_t)nb));
     PICCA_HIP_CHECK(ctx->o_dmat.reserve((size_t)(3 * nb * nb)));
     PICCA_HIP_CHECK(ctx->wk_stats.reserve(picca::WICK_NSTATS));
-    PICCA_HIP_CHECK(ctx->wk_ntasks.reserve(1));
     PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->o_wdm.ptr, nb, ctx->stream));
     PICCA_HIP_CHECK(picca::launch_zero_u64(ctx->wk_nb.ptr, nb, ctx->stream));
     PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->o_dmat.ptr, 3 * nb * nb,
                                            ctx->stream));
     PICCA_HIP_CHECK(picca::launch_zero_u64(ctx->wk_stats.ptr, picca::WICK_NSTATS, ctx->stream));
-    // row prefix sums of the weighted 1-D correlation of every forest of the pairs
-    std::vector<int64_t> c1off((size_t)nf, 0);
+    // prefix sums of the diagonal and of w zev1 for every forest of the pairs
     std::vector<int32_t> forests;
     {
         std::vector<char> used((size_t)nf, 0);
         for (int64_t k = 0; k < num_pairs; ++k) used[(size_t)pair_a[k]] = used[(size_t)pair_b[k]] = 1;
-        int64_t total = 0;
-        for (int64_t f = 0; f < nf; ++f) {
-            if (!used[(size_t)f]) continue;
-            const int64_t n = off[f + 1] - off[f];
-            c1off[(size_t)f] = total;
-            total += n * (n + 1);
-            forests.push_back((int32_t)f);
-        }
-        PICCA_HIP_CHECK(ctx->wk_c1.reserve((size_t)std::max<int64_t>(total, 1)));
+        for (int64_t f = 0; f < nf; ++f)
+            if (used[(size_t)f]) forests.push_back((int32_t)f);
     }
-    PICCA_HIP_CHECK(ctx->wk_c1off.upload(c1off.data(), c1off.size(), ctx->stream));
     PICCA_HIP_CHECK(ctx->wk_forests.upload(forests.data(), forests.size(), ctx->stream));
-    PICCA_HIP_CHECK(picca::launch_wick_prefix(ctx->wk_wx.ptr, ctx->wk_wxoff.ptr, ctx->off.ptr,
-                                              ctx->wk_forests.ptr, (int32_t)forests.size(),
-                                              ctx->wk_c1.ptr, ctx->wk_c1off.ptr, ctx->stream));
-    picca::WickInputs I{ctx->off.ptr,      ctx->r.ptr,        ctx->w.ptr,
-                        ctx->wk_zev1.ptr,  ctx->wk_zev2.ptr,  ctx->wk_wx.ptr,
-                        ctx->wk_wxoff.ptr, ctx->wk_c1.ptr,    ctx->wk_c1off.ptr};
+    PICCA_HIP_CHECK(ctx->wk_diag.reserve((size_t)(npix + nf)));
+    PICCA_HIP_CHECK(ctx->wk_wz.reserve((size_t)(npix + nf)));
+    picca::WickInputs I{ctx->off.ptr,     ctx->r.ptr,       ctx->w.ptr,       ctx->wk_zev1.ptr,
+                        ctx->wk_zev2.ptr, ctx->wk_wx.ptr,   ctx->wk_wxoff.ptr};
+    PICCA_HIP_CHECK(picca::launch_wick_diag(I, ctx->wk_forests.ptr, (int32_t)forests.size(),
+                                            ctx->wk_diag.ptr, ctx->wk_wz.ptr, ctx->stream));
     picca::WickOut O{ctx->o_wdm.ptr, ctx->wk_nb.ptr, ctx->o_dmat.ptr, ctx->o_dmat.ptr + nb * nb,
                      ctx->o_dmat.ptr + 2 * nb * nb, ctx->wk_stats.ptr};
 
-    // batches of pairs whose lists (n1 n2 entries each, an upper bound) fit 1 GiB (and their
-    // segment lists, 16 bytes per entry at most, 2 GiB)
-    const int64_t list_budget = (int64_t)1 << 27;
+    // batches of pairs: at most 2^20 (pair, bin) counts and 2^27 pixel pairs (the segments are
+    // fewer); inside a batch, runs of tasks whose segment sums fit 1 GiB
+    const int64_t pixel_budget = (int64_t)1 << 27, count_budget = (int64_t)1 << 20;
+    const int64_t rsum_budget = (int64_t)1 << 27;
     double total_ms = 0.0;
     int64_t batches = 0;
     std::vector<double> cs;
-    std::vector<int64_t> base;
+    std::vector<int32_t> seg_count, seg_pos;
+    std::vector<picca::WickTask> tasks;
+    auto add_time = [&]() -> int {
+        PICCA_HIP_CHECK(hipEventRecord(ctx->ev_stop, ctx->stream));
+        PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+        float ms = 0.f;
+        PICCA_HIP_CHECK(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
+        total_ms += ms;
+        return PICCA_OK;
+    };
     for (int64_t p0 = 0; p0 < num_pairs;) {
-        int64_t p1 = p0, entries = 0, max_tasks = 0;
-        base.clear();
-        while (p1 < num_pairs && p1 - p0 < INT32_MAX) {
+        int64_t p1 = p0, entries = 0, longest = 0;
+        while (p1 < num_pairs && (p1 == p0 || (p1 - p0 + 1) * nb <= count_budget) &&
+               p1 - p0 < 65535) {
             const int64_t n1 = off[pair_a[p1] + 1] - off[pair_a[p1]];
             const int64_t n2 = off[pair_b[p1] + 1] - off[pair_b[p1]];
-            if (p1 > p0 && entries + n1 * n2 > list_budget) break;
-            base.push_back(entries);
+            if (p1 > p0 && entries + n1 * n2 > pixel_budget) break;
             entries += n1 * n2;
-            max_tasks += std::min<int64_t>(nb, n1 * n2);
+            longest = std::max(longest, n2);
             ++p1;
         }
         const int64_t count = p1 - p0;
@@ -135,35 +134,81 @@ int picca_wick_t123(picca_ctx *ctx, const picca_cf_params *params, int64_t num_p
         PICCA_HIP_CHECK(ctx->dpa.upload(pair_a + p0, (size_t)count, ctx->stream));
         PICCA_HIP_CHECK(ctx->dpb.upload(pair_b + p0, (size_t)count, ctx->stream));
         PICCA_HIP_CHECK(ctx->dcs.upload(cs.data(), cs.size(), ctx->stream));
-        PICCA_HIP_CHECK(ctx->wk_base.upload(base.data(), base.size(), ctx->stream));
-        PICCA_HIP_CHECK(ctx->wk_list.reserve((size_t)std::max<int64_t>(entries, 1)));
-        PICCA_HIP_CHECK(ctx->wk_seg.reserve((size_t)std::max<int64_t>(entries, 1)));
-        PICCA_HIP_CHECK(ctx->wk_count.reserve((size_t)count));
-        PICCA_HIP_CHECK(ctx->wk_segcount.reserve((size_t)count));
-        PICCA_HIP_CHECK(ctx->wk_task.reserve((size_t)(4 * std::max<int64_t>(max_tasks, 1))));
-        PICCA_HIP_CHECK(picca::launch_zero_u64(ctx->wk_ntasks.ptr, 1, ctx->stream));
-        int32_t *tk = ctx->wk_task.ptr;
-        const int64_t mt = std::max<int64_t>(max_tasks, 1);
+        // (zeroed in 64-bit words)
+        const int64_t cells = count * nb;
+        PICCA_HIP_CHECK(ctx->wk_segcount.reserve((size_t)cells + 1));
+        PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->wk_segcount.ptr,
+                                               (cells + 1) / 2, ctx->stream));
         picca::WickPairs P{ctx->dpa.ptr, ctx->dpb.ptr, ctx->dcs.ptr, (int32_t)count};
-        picca::WickWork W{ctx->wk_list.ptr,  ctx->wk_base.ptr,     ctx->wk_count.ptr,
-                          ctx->wk_seg.ptr,   ctx->wk_segcount.ptr, tk,
-                          tk + mt,           tk + 2 * mt,          tk + 3 * mt,
-                          ctx->wk_ntasks.ptr, max_tasks};
+        picca::WickWork W{ctx->wk_segcount.ptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+                          ctx->wk_diag.ptr, ctx->wk_wz.ptr};
         PICCA_HIP_CHECK(hipEventRecord(ctx->ev_start, ctx->stream));
-        PICCA_HIP_CHECK(picca::launch_wick_list(C, I, P, W, O, ctx->stream));
-        unsigned long long tasks = 0;
-        PICCA_HIP_CHECK(hipMemcpyAsync(&tasks, ctx->wk_ntasks.ptr, sizeof(tasks),
-                                       hipMemcpyDeviceToHost, ctx->stream));
+        PICCA_HIP_CHECK(picca::launch_wick_segments(false, C, I, P, W, O, longest, ctx->stream));
+        int status = add_time();
+        if (status != PICCA_OK) return status;
+        seg_count.resize((size_t)cells);
+        PICCA_HIP_CHECK(hipMemcpyAsync(seg_count.data(), ctx->wk_segcount.ptr,
+                                       sizeof(int32_t) * (size_t)cells, hipMemcpyDeviceToHost,
+                                       ctx->stream));
         PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-        if ((int64_t)tasks > max_tasks)
-            return fail(PICCA_E_RUNTIME, "Wick task list overflow");
-        PICCA_HIP_CHECK(picca::launch_wick_rows(C, I, P, W, O, (int64_t)tasks, ctx->stream));
-        PICCA_HIP_CHECK(hipEventRecord(ctx->ev_stop, ctx->stream));
-        PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-        float ms = 0.f;
-        PICCA_HIP_CHECK(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
-        total_ms += ms;
+        // tasks in (pair, bin) order and the segments' positions
+        seg_pos.resize((size_t)cells);
+        tasks.clear();
+        int64_t segs = 0;
+        for (int64_t k = 0; k < count; ++k) {
+            const int64_t start = segs;
+            const size_t first_task = tasks.size();
+            for (int64_t p = 0; p < nb; ++p) {
+                const int32_t n = seg_count[(size_t)(k * nb + p)];
+                seg_pos[(size_t)(k * nb + p)] = (int32_t)segs;
+                if (n > 0)
+                    tasks.push_back(picca::WickTask{(int32_t)k, (int32_t)p, (int32_t)segs, n,
+                                                    (int32_t)start, 0, 0});
+                segs += n;
+            }
+            for (size_t t = first_task; t < tasks.size(); ++t)
+                tasks[t].pair_count = (int32_t)(segs - start);
+        }
         ++batches;
+        if (!tasks.empty()) {
+            // runs of tasks: rsum rows from 0 in each
+            std::vector<int64_t> run_begin{0};
+            int64_t rows = 0, most = 0;
+            for (size_t t = 0; t < tasks.size(); ++t) {
+                const int32_t f = pair_a[p0 + tasks[t].pair];
+                const int64_t need = (int64_t)tasks[t].count * (off[f + 1] - off[f] + 1);
+                if (rows > 0 && rows + need > rsum_budget) {
+                    run_begin.push_back((int64_t)t);
+                    rows = 0;
+                }
+                tasks[t].rows = rows;
+                rows += need;
+                most = std::max(most, rows);
+            }
+            run_begin.push_back((int64_t)tasks.size());
+            PICCA_HIP_CHECK(ctx->wk_segpos.upload(seg_pos.data(), (size_t)cells, ctx->stream));
+            PICCA_HIP_CHECK(ctx->wk_task.upload(tasks.data(), tasks.size(), ctx->stream));
+            PICCA_HIP_CHECK(ctx->wk_seg_raw.reserve((size_t)segs));
+            PICCA_HIP_CHECK(ctx->wk_seg.reserve((size_t)segs));
+            PICCA_HIP_CHECK(ctx->wk_rsum.reserve((size_t)most));
+            W.seg_pos = ctx->wk_segpos.ptr;
+            W.seg_raw = ctx->wk_seg_raw.ptr;
+            W.seg = ctx->wk_seg.ptr;
+            W.rsum = ctx->wk_rsum.ptr;
+            PICCA_HIP_CHECK(hipEventRecord(ctx->ev_start, ctx->stream));
+            PICCA_HIP_CHECK(picca::launch_wick_segments(true, C, I, P, W, O, longest,
+                                                        ctx->stream));
+            W.task = ctx->wk_task.ptr;
+            PICCA_HIP_CHECK(picca::launch_wick_sort(W, (int64_t)tasks.size(), ctx->stream));
+            for (size_t r = 0; r + 1 < run_begin.size(); ++r) {
+                W.task = ctx->wk_task.ptr + run_begin[r];
+                PICCA_HIP_CHECK(picca::launch_wick_rows(C, I, P, W, O,
+                                                        run_begin[r + 1] - run_begin[r],
+                                                        ctx->stream));
+            }
+            status = add_time();
+            if (status != PICCA_OK) return status;
+        }
         p0 = p1;
     }
 
