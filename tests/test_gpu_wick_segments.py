@@ -28,7 +28,7 @@ def forests(rng, lengths, shuffled):
 @pytest.mark.parametrize("shuffled", [False, True])
 @pytest.mark.parametrize("lengths,bins,r_max", [((130, 140), 1, 300.0), ((1, 2, 100), 1, 300.0),
                                                 ((1, 2, 300), 7, 20.0),
-                                                ((255, 256, 257, 65), 7, 8.0)])
+                                                ((255, 256, 257, 65), 7, 20.0)])
 def test_segments(lengths, shuffled, bins, r_max):
     rng = np.random.default_rng(len(lengths) + 10 * bins)
     store = forests(rng, lengths, shuffled)
