@@ -1068,16 +1068,20 @@ bool power_of_two_times(int n, int base) {
 }
 
 // The kernels for pairs without cuts (dmat_band_kernel.hip): takes the pairs they cover from
-// the list into `rest` what is left, and the pairs that they hand back.  Rule, per call: the
-// standard auto-correlation binning without a pair-redshift cut, model bins that split the data
-// bins in 2^k parts, LDS for a row of model bins; per pair: no zerr or same-half-plate cut, a
-// projected delta2, both forests with a proper fit normalisation and strictly rising r_comov and dist_m whose steps lie above
-// the rounding margins in both coordinates (the run walk's condition; 1e4 margins, so that the
-// index tables' 1e-3 of a step covers the rounding too).
+// the list into `rest` what is left, and the pairs that they hand back.  Rule, per call: standard
+// binning without a pair-redshift cut, model bins that split the data bins in 2^k parts, and
+// either the auto-correlation from r_par_min == 0 (with LDS for a row of model bins) or the
+// signed r_par of forest x quasar pairs; per pair: no zerr or same-half-plate cut, the forests
+// (of a quasar's pair: the first) with a proper fit normalisation and strictly rising r_comov and
+// dist_m whose steps lie above the rounding margins in both coordinates (the run walk's
+// condition; 1e4 margins, so that the index tables' 1e-3 of a step covers the rounding too), and
+// a projected delta2, or with signed r_par a one-pixel delta2 that is not projected and xcf's
+// count pass.
 int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
     picca_ctx *ctx = R.ctx;
     const picca::DmatConst &C = R.C;
     const int64_t num_pairs = L.size();
+    const bool quasar = (C.flags & picca::DMAT_XCORR) != 0;
     picca_cf_params model = *R.params;
     model.num_bins_r_par = C.npm;
     model.num_bins_r_trans = C.ntm;
@@ -1086,13 +1090,12 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
     int mode = 0;
     const int kt = C.ntm / C.nt;
     int band_rows = 0;
-    bool covered = !(C.flags & (picca::XI_HAS_ZMIN | picca::XI_HAS_ZMAX | picca::DMAT_XCORR |
-                                picca::DMAT_RMU)) &&
-                   C.rpmin == 0.0 && power_of_two_times(C.npm, C.np) &&
+    bool covered = !(C.flags & (picca::XI_HAS_ZMIN | picca::XI_HAS_ZMAX | picca::DMAT_RMU)) &&
+                   (quasar || C.rpmin == 0.0) && power_of_two_times(C.npm, C.np) &&
                    power_of_two_times(C.ntm, C.nt) && !picca::fill_xi_const(&model, M, mode) &&
                    !picca::widen_xi_margins(M, ctx->max_abs_r, ctx->max_abs_d);
-    if (covered) {
-        picca::apply_xi_schedule(M, PICCA_XI_SCHEDULE_RUNS);
+    if (covered) picca::apply_xi_schedule(M, PICCA_XI_SCHEDULE_RUNS);
+    if (covered && !quasar) {
         const size_t row = picca::dmat_band_pass_lds(C, 1) - picca::dmat_band_pass_lds(C, 0);
         const size_t fixed = picca::dmat_band_pass_lds(C, 0);
         const size_t aim = std::min<size_t>(picca::DMAT_BAND_LDS, (size_t)ctx->lds_limit);
@@ -1104,47 +1107,64 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
         rest = L;
         return PICCA_OK;
     }
+    // the pairs: 0 covered, 1 left to the general kernels, 2 out of range
+    std::vector<picca::DmatBandSlot> all((size_t)num_pairs);
+    std::vector<uint8_t> kind((size_t)num_pairs);
+    std::vector<double> half((size_t)(2 * num_pairs));
+    parallel_for(num_pairs, [&](int64_t lo, int64_t hi) {
+        for (int64_t k = lo; k < hi; ++k) {
+            const int32_t a = L.a[(size_t)k], b = L.b[(size_t)k];
+            const double ang = L.ang[(size_t)k];
+            const uint8_t flags = L.flags[(size_t)k];
+            const double cos_half = std::cos(ang / 2), sin_half = std::sin(ang / 2);
+            half[(size_t)(2 * k)] = cos_half;
+            half[(size_t)(2 * k + 1)] = sin_half;
+            const double cp = cos_half * M.inv_p, st = sin_half * M.inv_t;
+            auto steps = [&](int32_t f) {
+                const double2 spc = ctx->h_spc[(size_t)f];
+                return picca::walk_task(M, spc.x, spc.y, cp, st, 1.0) &&
+                       cp * spc.x > 1e4 * M.fast_p && st * spc.y > 1e4 * M.fast_t &&
+                       (ctx->h_mono[(size_t)f] & 3) == 3 && ctx->h_fit[(size_t)f] != 0;
+            };
+            const bool cut = ((C.flags & picca::XI_HAS_ZERR) && ang < C.zerr_ang) ||
+                             ((C.flags & picca::XI_REMOVE_SHP) &&
+                              (flags & picca::PAIR_SAME_HALF_PLATE));
+            const int64_t lb = ctx->h_offsets[(size_t)b + 1] - ctx->h_offsets[(size_t)b];
+            const bool second = quasar ? ctx->h_order[(size_t)b] < 0 && lb == 1 &&
+                                             (flags & picca::PAIR_XCF_COUNT)
+                                       : ctx->h_order[(size_t)b] >= 0 && steps(b) &&
+                                             !(flags & picca::PAIR_XCF_COUNT);
+            kind[(size_t)k] = 1;
+            if (cut || !(cos_half > 0) || !second || !steps(a)) continue;
+            // r_trans and its bin arithmetic do not fall with either dist_m, so the rows of the
+            // first and the last pixels' sums bound every pair's rows
+            const double y_lo = (ctx->h_dmin[(size_t)a] + ctx->h_dmin[(size_t)b]) * sin_half /
+                                C.rtmax;
+            const double y_hi = (ctx->h_dmax[(size_t)a] + ctx->h_dmax[(size_t)b]) * sin_half /
+                                C.rtmax;
+            const double t0 = std::fmax(std::floor(y_lo * C.nt_d), 0.0);
+            const double t1 = std::fmin(std::floor(y_hi * C.nt_d), C.nt_d - 1);
+            kind[(size_t)k] = t0 <= t1 ? 0 : 2;
+            if (!(t0 <= t1)) continue;
+            picca::DmatBandSlot &s = all[(size_t)k];
+            s.a = a;
+            s.b = b;
+            s.t0 = (int)t0;
+            s.nt = (int)(t1 - t0) + 1;
+            s.u0 = s.t0 * kt;
+            s.nu = s.nt * kt;
+        }
+    });
     std::vector<picca::DmatBandSlot> slots;
     std::vector<double> cs;
     std::vector<int64_t> origin;
     for (int64_t k = 0; k < num_pairs; ++k) {
-        const int32_t a = L.a[(size_t)k], b = L.b[(size_t)k];
-        const double ang = L.ang[(size_t)k];
-        const uint8_t flags = L.flags[(size_t)k];
-        const double cos_half = std::cos(ang / 2), sin_half = std::sin(ang / 2);
-        const double cp = cos_half * M.inv_p, st = sin_half * M.inv_t;
-        auto steps = [&](int32_t f) {
-            const double2 spc = ctx->h_spc[(size_t)f];
-            return picca::walk_task(M, spc.x, spc.y, cp, st, 1.0) &&
-                   cp * spc.x > 1e4 * M.fast_p && st * spc.y > 1e4 * M.fast_t &&
-                   (ctx->h_mono[(size_t)f] & 3) == 3 && ctx->h_fit[(size_t)f] != 0;
-        };
-        const bool cut = ((C.flags & picca::XI_HAS_ZERR) && ang < C.zerr_ang) ||
-                         ((C.flags & picca::XI_REMOVE_SHP) &&
-                          (flags & picca::PAIR_SAME_HALF_PLATE)) ||
-                         (flags & picca::PAIR_XCF_COUNT);
-        if (cut || !(cos_half > 0) || ctx->h_order[(size_t)b] < 0 || !steps(a) || !steps(b)) {
-            rest.push(a, b, ang, flags);
-            continue;
-        }
-        // r_trans and its bin arithmetic do not fall with either dist_m, so the rows of the
-        // first and the last pixels' sums bound every pair's rows
-        const double y_lo = (ctx->h_dmin[(size_t)a] + ctx->h_dmin[(size_t)b]) * sin_half / C.rtmax;
-        const double y_hi = (ctx->h_dmax[(size_t)a] + ctx->h_dmax[(size_t)b]) * sin_half / C.rtmax;
-        const double t0 = std::fmax(std::floor(y_lo * C.nt_d), 0.0);
-        const double t1 = std::fmin(std::floor(y_hi * C.nt_d), C.nt_d - 1);
-        if (!(t0 <= t1)) continue;   // out of range: the pair adds nothing
-        picca::DmatBandSlot s;
-        s.a = a;
-        s.b = b;
-        s.t0 = (int)t0;
-        s.nt = (int)(t1 - t0) + 1;
-        s.u0 = s.t0 * kt;
-        s.nu = s.nt * kt;
-        s.t_row = s.u_row = 0;
-        slots.push_back(s);
-        cs.push_back(cos_half);
-        cs.push_back(sin_half);
+        if (kind[(size_t)k] == 1)
+            rest.push(L.a[(size_t)k], L.b[(size_t)k], L.ang[(size_t)k], L.flags[(size_t)k]);
+        if (kind[(size_t)k] != 0) continue;
+        slots.push_back(all[(size_t)k]);
+        cs.push_back(half[(size_t)(2 * k)]);
+        cs.push_back(half[(size_t)(2 * k + 1)]);
         origin.push_back(k);
     }
     const int64_t total = (int64_t)slots.size();
@@ -1168,7 +1188,8 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
     PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->db_num.ptr, 2, st));
     // batches: about 1.5 GiB of workspace rows
     const double budget = 1536.0 * 1048576.0;
-    const double t_bytes = 8.0 * 4 * C.np + 16, u_bytes = 8.0 * 9 * C.npm + 16;
+    const double t_bytes = 16 + (quasar ? 0 : 8.0 * 4 * C.np);
+    const double u_bytes = 16 + (quasar ? 0 : 8.0 * 9 * C.npm);
     for (int64_t p0 = 0; p0 < total;) {
         int64_t p1 = p0, t_rows = 0, u_rows = 0, list = 0;
         while (p1 < total && p1 - p0 < (1 << 22)) {
@@ -1184,9 +1205,11 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
         }
         const int64_t count = p1 - p0;
         PICCA_HIP_CHECK(ctx->db_slot.upload(slots.data() + p0, (size_t)count, st));
-        PICCA_HIP_CHECK(ctx->db_S.reserve((size_t)t_rows * 4 * C.np));
-        PICCA_HIP_CHECK(ctx->db_eta.reserve((size_t)u_rows * 4 * C.npm));
-        PICCA_HIP_CHECK(ctx->db_eff.reserve((size_t)u_rows * 5 * C.npm));
+        if (!quasar) {
+            PICCA_HIP_CHECK(ctx->db_S.reserve((size_t)t_rows * 4 * C.np));
+            PICCA_HIP_CHECK(ctx->db_eta.reserve((size_t)u_rows * 4 * C.npm));
+            PICCA_HIP_CHECK(ctx->db_eff.reserve((size_t)u_rows * 5 * C.npm));
+        }
         PICCA_HIP_CHECK(ctx->db_rng_t.reserve((size_t)t_rows));
         PICCA_HIP_CHECK(ctx->db_rng_u.reserve((size_t)u_rows));
         PICCA_HIP_CHECK(ctx->db_list.reserve((size_t)list));
@@ -1204,9 +1227,12 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
         hipEvent_t *ev = nullptr;
         PICCA_HIP_CHECK(dmat_next_events(R, &ev));
         PICCA_HIP_CHECK(hipEventRecord(ev[0], st));
-        PICCA_HIP_CHECK(picca::launch_dmat_band_pass(M, C, R.F, P, W, R.O, band_rows, st));
+        PICCA_HIP_CHECK(quasar ? picca::launch_dmat_quasar_rows(M, C, R.F, P, W, st)
+                               : picca::launch_dmat_band_pass(M, C, R.F, P, W, R.O, band_rows,
+                                                              st));
         PICCA_HIP_CHECK(hipEventRecord(ev[1], st));
-        PICCA_HIP_CHECK(picca::launch_dmat_band_fill(M, C, R.F, P, W, R.O, ctx->num_cus, st));
+        PICCA_HIP_CHECK(picca::launch_dmat_band_fill(M, C, R.F, P, W, R.O, quasar, ctx->num_cus,
+                                                     st));
         PICCA_HIP_CHECK(hipEventRecord(ev[2], st));
         p0 = p1;
     }

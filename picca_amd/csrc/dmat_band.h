@@ -67,22 +67,37 @@ struct BandAxis {
     double scale;      // cos(ang/2) or sin(ang/2)
     double range;      // r_par_max - r_par_min or r_trans_max
     double n;          // bins of the range
-    bool par;
+    int kind;          // BAND_*
+    double from;       // BAND_SIGNED: r_par_min
 };
+
+// r_trans; |r_par| of the auto-correlation; r_par = (partner - self) cos(ang/2) of a forest
+// (the partner) with a quasar, whose bins count from r_par_min
+enum : int { BAND_TRANS = 0, BAND_PAR = 1, BAND_SIGNED = 2 };
 
 PICCA_HD inline BandAxis band_par_axis(double r, double mul, double cos_half, double span, int n,
                                        double margin) {
-    return BandAxis{mul, -r * mul, margin, r, cos_half, span, (double)n, true};
+    return BandAxis{mul, -r * mul, margin, r, cos_half, span, (double)n, BAND_PAR, 0.0};
 }
 
 PICCA_HD inline BandAxis band_trans_axis(double d, double mul, double sin_half, double rtmax,
                                          int n, double margin) {
-    return BandAxis{mul, d * mul, margin, d, sin_half, rtmax, (double)n, false};
+    return BandAxis{mul, d * mul, margin, d, sin_half, rtmax, (double)n, BAND_TRANS, 0.0};
+}
+
+PICCA_HD inline BandAxis band_signed_axis(double r, double mul, double cos_half, double from,
+                                          double span, int n, double margin) {
+    return BandAxis{mul, -r * mul - from / span * n, margin, r, cos_half, span, (double)n,
+                    BAND_SIGNED, from};
 }
 
 // The key with the reference's arithmetic, clamped to [-n - 1, n].
 PICCA_HD inline int band_exact_key(const BandAxis &A, double v) {
-    if (A.par) {
+    if (A.kind == BAND_SIGNED) {
+        const double t = ((v - A.self) * A.scale - A.from) / A.range * A.n;
+        return (int)fmin(fmax(floor(t), -1.0), A.n);
+    }
+    if (A.kind == BAND_PAR) {
         const double rps = (A.self - v) * A.scale;
         const double row = fmin(floor(fabs(rps) / A.range * A.n), A.n);
         return (int)(rps > 0 ? -row - 1.0 : row);

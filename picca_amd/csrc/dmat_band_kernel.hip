@@ -2,7 +2,8 @@
 // dmat_kernel.hip (compute_dmat_forest_pairs_fast, py/picca/cf.py:520-887) taken from prefix
 // sums over the forests instead of pixel pair by pixel pair.
 //
-// It covers the standard auto-correlation binning (r_par_min == 0, |r_par|), forests whose
+// It covers the standard auto-correlation binning (r_par_min == 0, |r_par|; forest x quasar
+// pairs below), forests whose
 // r_comov and dist_m rise strictly with steps above the rounding margins, model bins that
 // split the data bins in 2^k parts (so that a model bin lies in one data bin to the last bit)
 // and no pair-redshift, zerr or same-half-plate cut on the pair; the host sends the other pairs
@@ -505,6 +506,39 @@ __global__ __launch_bounds__(256) void dmat_band_list_kernel(DmatConst C, DmatBa
     }
 }
 
+namespace {
+
+// The sums per r_par bin of one pixel per group of 16 lanes over its partner's pixels [j0, j1),
+// whose bins are k0 .. k0 + kn - 1: lane li takes bin edges 15 at a time, and add(k, x, y,
+// first, end) gets a bin, the differences of the two prefix sums over its pixels [first, end).
+// pre: the prefix records' pair of sums (stride 4).  Every lane of the wave takes part.
+template <class Add>
+__device__ __forceinline__ void band_bins(const BandAxis &A, const BandTable &T,
+                                          const double *__restrict__ v,
+                                          const double2 *__restrict__ pre, int j0, int j1, int k0,
+                                          int kn, int li, Add add) {
+    const int groups = wave_max_int((kn + 14) / 15);
+    for (int g = 0; g < groups; ++g) {
+        // lane li: the first pixel of bin k; the sums of bin k lie between its edge and the
+        // next lane's
+        const int at = 15 * g + li;
+        const int k = k0 + at;
+        double2 here = make_double2(0.0, 0.0);
+        int e = 0;
+        if (at <= kn && kn > 0) {
+            e = at == 0 ? j0 : j1;
+            if (at > 0 && at < kn) e = band_edge(A, T, [&](int p) { return v[p]; }, k);
+            here = pre[4 * (int64_t)e];
+        }
+        const double x = dpp_f64<DPP_ROW_SHL1>(here.x) - here.x;
+        const double y = dpp_f64<DPP_ROW_SHL1>(here.y) - here.y;
+        const int end = dpp_int<DPP_ROW_SHL1>(e);
+        if (at < kn && li < 15) add(k, x, y, e, end);
+    }
+}
+
+}  // namespace
+
 __global__ __launch_bounds__(DMAT_BAND_FILL_BLOCK, 3) void dmat_band_fill_kernel(
     XiConst M, DmatConst C, DmatForests F, DmatBandSlots P, DmatBandWork W, DmatOut O) {
     extern __shared__ __align__(16) double panel[];   // [PX][VLEN]
@@ -646,29 +680,14 @@ __global__ __launch_bounds__(DMAT_BAND_FILL_BLOCK, 3) void dmat_band_fill_kernel
                                 const int chunk = h ? mrp0 : rp0, count = h ? nmrp : nrp;
                                 double *dst = px + (h ? VE : VP);
                                 const int second = h ? VE2 - VE : VP2 - VP;
-                                const int groups = wave_max_int((kn[h] + 14) / 15);
-                                for (int g = 0; g < groups; ++g) {
-                                    // lane li: the first pixel of bin k; the sums of bin k lie
-                                    // between its edge and the next lane's
-                                    const int at = 15 * g + li;
-                                    const int k = k0[h] + at;
-                                    const bool on = at <= kn[h] && kn[h] > 0;
-                                    double2 here = make_double2(0.0, 0.0);
-                                    if (on) {
-                                        int e = at == 0 ? j0[h] : j1[h];
-                                        if (at > 0 && at < kn[h])
-                                            e = band_edge(A, Tr, [&](int x) { return Pr[x]; }, k);
-                                        here = pre[4 * (int64_t)e + h];
-                                    }
-                                    const double x = dpp_f64<DPP_ROW_SHL1>(here.x) - here.x;
-                                    const double y = dpp_f64<DPP_ROW_SHL1>(here.y) - here.y;
+                                band_bins(A, Tr, Pr, pre + h, j0[h], j1[h], k0[h], kn[h], li,
+                                          [&](int k, double x, double y, int, int) {
                                     const int b = (k >= 0 ? k : -k - 1) - chunk;
-                                    if (at < kn[h] && li < 15 && b >= 0 && b < count) {
-                                        if (h) cols |= 1u << (b >> 4);
-                                        lds_add(dst + b, f1 * x);
-                                        lds_add(dst + second + b, f2 * y);
-                                    }
-                                }
+                                    if (b < 0 || b >= count) return;
+                                    if (h) cols |= 1u << (b >> 4);
+                                    lds_add(dst + b, f1 * x);
+                                    lds_add(dst + second + b, f2 * y);
+                                });
                             }
                             if (cols) atomicOr(&s_cols, cols);
                             __syncthreads();
@@ -713,6 +732,249 @@ __global__ __launch_bounds__(DMAT_BAND_FILL_BLOCK, 3) void dmat_band_fill_kernel
     if (lane == 0 && n_mfma) atomicAdd(&W.stats[DMAT_STAT_MFMA], (unsigned long long)n_mfma);
 }
 
+// ---------------------------------------------------------------------------------------
+// Forest x quasar pairs: delta2 is one unprojected pixel (py/picca/xcf.py:427-658), whose pairs
+// leave the identity and the Q eta2 + Q' eta4 terms.  No pass: a pair's rows come from its
+// edges, the matrix-core panel holds 16 pairs (K = the pairs), and the tile of a data row and
+// its own model rows adds the pair-bin term, weights_dmat and the effective sums.  With a pair
+// per workgroup and one quasar pixel a tile, the general pass and fill leave 15 of 16 lanes and
+// rows of K idle: 3000 forests, 50k kept pairs, 100 x 50 bins take 2.4 ms here, 36 ms (fill) and
+// 11 ms (pass) there.  Bound by the chain of table, probe and prefix loads of an edge.
+
+// Rows that each pair reaches (as non-empty pixel ranges for the tile lists), and the pairs
+// whose bins do not follow the runs: a pixel at the end of a range whose bin rounds past it, or
+// r_par == r_par_min exactly, which xcf's count pass leaves out.  One thread per pair.
+__global__ __launch_bounds__(256) void dmat_quasar_rows_kernel(XiConst M, DmatConst C,
+                                                               DmatForests F, DmatBandSlots P,
+                                                               DmatBandWork W) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= P.count) return;
+    const DmatBandSlot q = P.slot[s];
+    const int64_t oa = F.off[q.a], ob = F.off[q.b];
+    const int n = (int)(F.off[q.a + 1] - oa);
+    const double *__restrict__ R = F.r + oa;
+    const double *__restrict__ D = F.d + oa;
+    const double cos_half = P.cs[2 * s], sin_half = P.cs[2 * s + 1];
+    const double rq = F.r[ob], dq = F.d[ob];
+    const BandTable Tr{W.table_r + oa, R[0], 1.0 / band_mean_step(R[0], R[n - 1], n), n};
+    const BandTable Td{W.table_d + oa, D[0], 1.0 / band_mean_step(D[0], D[n - 1], n), n};
+    auto r = [&](int p) { return R[p]; };
+    auto d = [&](int p) { return D[p]; };
+    const BandAxis Ap = band_signed_axis(rq, cos_half * C.npm / C.span_p, cos_half, C.rpmin,
+                                         C.span_p, C.npm, M.fast_p);
+    const int lo = band_edge(Ap, Tr, r, 0), hi = band_edge(Ap, Tr, r, C.npm);
+    const BandAxis At = band_trans_axis(dq, sin_half * C.ntm / C.rtmax, sin_half, C.rtmax, C.ntm,
+                                        M.fast_t);
+    const int top = band_edge(At, Td, d, C.ntm);
+    const bool special = (lo < n && !((R[lo] - rq) * cos_half > C.rpmin)) ||
+                         (hi < n && (R[hi] - rq) * cos_half < C.rpmax) ||
+                         (top < n && (D[top] + dq) * sin_half < C.rtmax);
+    if (special) W.redo[atomicAdd(W.num_redo, 1)] = P.first + s;
+    const int4 empty = make_int4(INT_MAX, -1, INT_MAX, -1), full = make_int4(0, 0, 0, 0);
+    int first = band_edge(At, Td, d, q.u0);
+    const int kt = C.ntm / C.nt;
+    bool any = false;
+    for (int u = 0; u < q.nu; ++u) {
+        const int end = band_edge(At, Td, d, q.u0 + u + 1);
+        const bool in = !special && max(first, lo) < min(end, hi);
+        W.rng_u[q.u_row + u] = in ? full : empty;
+        any = any || in;
+        if ((u + 1) % kt == 0) {
+            W.rng_t[q.t_row + u / kt] = any ? full : empty;
+            any = false;
+        }
+        first = end;
+    }
+}
+
+__global__ __launch_bounds__(DMAT_BAND_FILL_BLOCK, 3) void dmat_quasar_fill_kernel(
+    XiConst M, DmatConst C, DmatForests F, DmatBandSlots P, DmatBandWork W, DmatOut O) {
+    extern __shared__ __align__(16) double panel[];   // [PX][VLEN]
+    // effective sums, weight and pair-bin term of the tile's model bins (own rows' tiles only)
+    __shared__ double s_eff[5][DMAT_CHUNK_MRP];
+    __shared__ int s_item;
+    __shared__ unsigned int s_cols;
+    __shared__ unsigned long long s_in;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int li = lane & 15;
+    const int lk = lane >> 4;
+    const int row = 16 * wave + li;
+    const int kp = C.npm / C.np, kt = C.ntm / C.nt;
+    uint32_t n_mfma = 0;
+    for (;;) {
+        __syncthreads();
+        if (tid == 0) {
+            s_item = atomicAdd(W.queue, 1);
+            s_in = 0;
+        }
+        __syncthreads();
+        const int item = s_item;
+        if (item >= *W.num_items) break;
+        const int4 work = W.items[item];
+        const int tile = uniform_int(work.x);
+        const int t = tile / C.ntm, u = tile - t * C.ntm;
+        const bool own = u / kt == t;   // model row u lies in data row t
+        for (int rp0 = 0; rp0 < C.np; rp0 += DMAT_CHUNK_RP) {
+            for (int mrp0 = 0; mrp0 < C.npm; mrp0 += DMAT_CHUNK_MRP) {
+                const int nrp = min(DMAT_CHUNK_RP, C.np - rp0);
+                const int nmrp = min(DMAT_CHUNK_MRP, C.npm - mrp0);
+                const bool eff = own && rp0 == 0;
+                double4_t acc[FILL_CB];
+#pragma unroll
+                for (int b = 0; b < FILL_CB; ++b) acc[b] = (double4_t){0.0, 0.0, 0.0, 0.0};
+                for (int k = tid; k < 5 * DMAT_CHUNK_MRP; k += DMAT_BAND_FILL_BLOCK)
+                    (&s_eff[0][0])[k] = 0.0;
+                for (int base = 0; base < work.z; base += PX) {
+                    __syncthreads();   // the last panel is read
+                    for (int k = tid; k < PX * VLEN / 2; k += DMAT_BAND_FILL_BLOCK)
+                        ((double2 *)panel)[k] = make_double2(0.0, 0.0);
+                    if (tid == 0) s_cols = 0;
+                    // lane group lk: pair base + 4 wave + lk of the item
+                    const int e = base + 4 * wave + lk;
+                    const int s = W.list[work.y + min(e, work.z - 1)];
+                    const DmatBandSlot q = P.slot[s];
+                    const int64_t oa = F.off[q.a], ob = F.off[q.b];
+                    const int n = (int)(F.off[q.a + 1] - oa);
+                    const double *__restrict__ Pr = F.r + oa;
+                    const double *__restrict__ Pd = F.d + oa;
+                    const DmatPrefix *__restrict__ rec = W.pre_a + (oa + q.a);
+                    const double2 *__restrict__ pre = (const double2 *)rec;
+                    const BandTable Tr{W.table_r + oa, Pr[0],
+                                       1.0 / band_mean_step(Pr[0], Pr[n - 1], n), n};
+                    const BandTable Td{W.table_d + oa, Pd[0],
+                                       1.0 / band_mean_step(Pd[0], Pd[n - 1], n), n};
+                    const double cos_half = P.cs[2 * s], sin_half = P.cs[2 * s + 1];
+                    const double rq = F.r[ob], dq = F.d[ob], zq = F.z[ob];
+                    const double wq = e < work.z ? F.w[ob] : 0.0;
+                    const double fq = F.zfb[ob];
+                    auto par = [&](bool model) {
+                        const int bins = model ? C.npm : C.np;
+                        return band_signed_axis(rq, cos_half * bins / C.span_p, cos_half,
+                                                C.rpmin, C.span_p, bins, M.fast_p);
+                    };
+                    int edge = 0;
+                    if (li < 6 && wq != 0) {
+                        const bool p = li >= 4, model = li >= 2;
+                        const int bins = model ? C.ntm : C.nt;
+                        const BandAxis A =
+                            p ? par(true)
+                              : band_trans_axis(dq, sin_half * bins / C.rtmax, sin_half, C.rtmax,
+                                                bins, M.fast_t);
+                        const int K = p ? (li == 4 ? 0 : C.npm) : (model ? u : t) + (li & 1);
+                        const double *__restrict__ V = p ? Pr : Pd;
+                        edge = band_edge(A, p ? Tr : Td, [&](int x) { return V[x]; }, K);
+                    }
+                    const int first = lane & 48;
+                    const int r_lo = __shfl(edge, first + 4, 64);
+                    const int r_hi = __shfl(edge, first + 5, 64);
+                    int j0[2], j1[2], k0[2], kn[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        j0[h] = max(__shfl(edge, first + 2 * h, 64), r_lo);
+                        j1[h] = min(__shfl(edge, first + 2 * h + 1, 64), r_hi);
+                        k0[h] = kn[h] = 0;
+                        if (j0[h] < j1[h]) {
+                            const BandAxis A = par(h != 0);
+                            k0[h] = band_key(A, Pr[j0[h]]);
+                            kn[h] = band_key(A, Pr[j1[h] - 1]) - k0[h] + 1;
+                        }
+                    }
+                    const double inv_w = 1.0 / F.sum_w[q.a];
+                    const double inv_s = F.order[q.a] == 1 ? 1.0 / F.sw_dll[q.a] : 0.0;
+                    __syncthreads();
+                    double *px = panel + (4 * wave + lk) * VLEN;
+                    uint32_t cols = 0;
+                    if (eff && mrp0 == 0 && li == 0 && kn[1] > 0)
+                        atomicAdd(&s_in, (unsigned long long)(rec[j1[1]].c - rec[j0[1]].c));
+                    band_bins(par(false), Tr, Pr, pre, j0[0], j1[0], k0[0], kn[0], li,
+                              [&](int k, double x, double y, int, int) {
+                        const int b = k - rp0;
+                        if (b < 0 || b >= nrp) return;
+                        lds_add(px + VP + b, wq * x);
+                        lds_add(px + VP2 + b, wq * y);
+                    });
+                    band_bins(par(true), Tr, Pr, pre + 1, j0[1], j1[1], k0[1], kn[1], li,
+                              [&](int k, double x, double y, int j, int end) {
+                        const int b = k - mrp0;
+                        if (b < 0 || b >= nmrp) return;
+                        cols |= 1u << (b >> 4);
+                        lds_add(px + VE + b, fq * inv_w * x);
+                        lds_add(px + VE2 + b, fq * inv_s * y);
+                        if (!eff) return;
+                        // over the bin's pixels: w2 sum w1 (r1 - r2) cos and so on
+                        const DmatPrefix a = rec[j], z = rec[end];
+                        const double w = wq * (z.w - a.w);
+                        const double rc = Pr[n / 2], dc = Pd[n / 2];
+                        lds_add(&s_eff[0][b], cos_half * (wq * (z.r - a.r) + (rc - rq) * w));
+                        lds_add(&s_eff[1][b], sin_half * (wq * (z.d - a.d) + (dc + dq) * w));
+                        lds_add(&s_eff[2][b], 0.5 * (wq * (z.z - a.z) + zq * w));
+                        lds_add(&s_eff[3][b], w);
+                        lds_add(&s_eff[4][b], wq * fq * x);
+                    });
+                    if (cols) atomicOr(&s_cols, cols);
+                    __syncthreads();
+                    // acc -= Q x eta2 + Q' x eta4, K = the pairs, four at a time
+                    const uint32_t blocks = (uint32_t)uniform_int((int)s_cols);
+#pragma unroll
+                    for (int k4 = 0; k4 < PX / 4; ++k4) {
+                        const double *v = panel + (4 * k4 + lk) * VLEN;
+                        const double a1 = -v[VP + row], a2 = -v[VP2 + row];
+                        if (__ballot(a1 != 0.0 || a2 != 0.0) == 0) continue;
+#pragma unroll
+                        for (int b = 0; b < FILL_CB; ++b) {
+                            if (!((blocks >> b) & 1u)) continue;
+                            n_mfma += 2;
+                            acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                                a1, v[VE + 16 * b + li], acc[b], 0, 0, 0);
+                            acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                                a2, v[VE2 + 16 * b + li], acc[b], 0, 0, 0);
+                        }
+                    }
+                }
+                __syncthreads();
+                // block -> dmat
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    const int r = 16 * wave + 4 * a + lk;
+#pragma unroll
+                    for (int b = 0; b < FILL_CB; ++b) {
+                        const int m = 16 * b + li;
+                        if (r < nrp && m < nmrp && acc[b][a] != 0) {
+                            const int64_t A = (int64_t)(rp0 + r) * C.nt + t;
+                            const int64_t k = (int64_t)(mrp0 + m) * C.ntm + u;
+                            unsafeAtomicAdd(&O.dmat[A * C.nm + k], acc[b][a]);
+                        }
+                    }
+                }
+                if (eff) {
+                    for (int m = tid; m < nmrp; m += DMAT_BAND_FILL_BLOCK) {
+                        const int kb = (mrp0 + m) * C.ntm + u;
+                        const int64_t A = (int64_t)((mrp0 + m) / kp) * C.nt + t;
+                        if (s_eff[3][m] != 0)
+                            unsafeAtomicAdd(&O.weights_dmat[A], s_eff[3][m]);
+                        if (s_eff[3][m] != 0 || s_eff[0][m] != 0 || s_eff[1][m] != 0 ||
+                            s_eff[2][m] != 0) {
+                            unsafeAtomicAdd(&O.r_par_eff[kb], s_eff[0][m]);
+                            unsafeAtomicAdd(&O.r_trans_eff[kb], s_eff[1][m]);
+                            unsafeAtomicAdd(&O.z_eff[kb], s_eff[2][m]);
+                            unsafeAtomicAdd(&O.weight_eff[kb], s_eff[3][m]);
+                        }
+                        if (s_eff[4][m] != 0) unsafeAtomicAdd(&O.dmat[A * C.nm + kb], s_eff[4][m]);
+                    }
+                }
+                __syncthreads();
+            }
+        }
+        if (tid == 0 && s_in) {
+            atomicAdd(&W.stats[DMAT_STAT_IN_RANGE], s_in);
+            atomicAdd(&W.stats[DMAT_STAT_SELECTED], s_in);
+        }
+    }
+    if (lane == 0 && n_mfma) atomicAdd(&W.stats[DMAT_STAT_MFMA], (unsigned long long)n_mfma);
+}
+
 size_t dmat_band_pass_lds(const DmatConst &C, int rows) {
     return ((16 * (size_t)C.ntm + 15) & ~(size_t)15) +
            sizeof(double) * DMAT_BAND_SUMS * (size_t)C.npm * rows;
@@ -743,21 +1005,40 @@ hipError_t launch_dmat_band_pass(const XiConst &M, const DmatConst &C, const Dma
     return hipGetLastError();
 }
 
-hipError_t launch_dmat_band_fill(const XiConst &M, const DmatConst &C, const DmatForests &F,
-                                 const DmatBandSlots &P, const DmatBandWork &W,
-                                 const DmatOut &O, int num_cus, hipStream_t stream) {
-    if (P.count <= 0) return hipSuccess;
+// the work items of the tiles, whose rows the pass or the rows kernel has set
+static hipError_t launch_tile_lists(const DmatConst &C, const DmatBandSlots &P,
+                                    const DmatBandWork &W, int item_pairs, hipStream_t stream) {
     const dim3 pairs((unsigned)((P.count + 255) / 256));
     hipLaunchKernelGGL(dmat_band_count_kernel, pairs, dim3(256), 0, stream, C, P, W);
     hipLaunchKernelGGL(dmat_band_scan_kernel, dim3(1), dim3(1024), 0, stream, C.nt * C.ntm,
-                       DMAT_BAND_ITEM, W);
+                       item_pairs, W);
     hipLaunchKernelGGL(dmat_band_list_kernel, pairs, dim3(256), 0, stream, C, P, W);
-    const size_t lds = sizeof(double) * PX * VLEN;
-    hipError_t err = hipFuncSetAttribute((const void *)dmat_band_fill_kernel,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    return hipGetLastError();
+}
+
+hipError_t launch_dmat_band_fill(const XiConst &M, const DmatConst &C, const DmatForests &F,
+                                 const DmatBandSlots &P, const DmatBandWork &W,
+                                 const DmatOut &O, bool quasar, int num_cus,
+                                 hipStream_t stream) {
+    if (P.count <= 0) return hipSuccess;
+    hipError_t err = launch_tile_lists(C, P, W, quasar ? DMAT_QUASAR_ITEM : DMAT_BAND_ITEM, stream);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(dmat_band_fill_kernel, dim3(3 * num_cus), dim3(DMAT_BAND_FILL_BLOCK), lds,
-                       stream, M, C, F, P, W, O);
+    const size_t lds = sizeof(double) * PX * VLEN;
+    auto kern = quasar ? dmat_quasar_fill_kernel : dmat_band_fill_kernel;
+    err = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)lds);
+    if (err != hipSuccess) return err;
+    hipLaunchKernelGGL(kern, dim3(3 * num_cus), dim3(DMAT_BAND_FILL_BLOCK), lds, stream, M, C, F,
+                       P, W, O);
+    return hipGetLastError();
+}
+
+hipError_t launch_dmat_quasar_rows(const XiConst &M, const DmatConst &C, const DmatForests &F,
+                                   const DmatBandSlots &P, const DmatBandWork &W,
+                                   hipStream_t stream) {
+    if (P.count <= 0) return hipSuccess;
+    hipLaunchKernelGGL(dmat_quasar_rows_kernel, dim3((unsigned)((P.count + 255) / 256)),
+                       dim3(256), 0, stream, M, C, F, P, W);
     return hipGetLastError();
 }
 

@@ -239,6 +239,7 @@ constexpr int DMAT_BAND_FILL_BLOCK = 256;   // threads of the fill (4 waves)
 constexpr int DMAT_BAND_SUMS = 11;          // LDS sums per model bin of the pair pass
 constexpr size_t DMAT_BAND_LDS = 53 * 1024; // LDS aim of the pair pass: three workgroups a CU
 constexpr int DMAT_BAND_ITEM = 8;           // forest pairs of one tile per work item
+constexpr int DMAT_QUASAR_ITEM = 64;        // forest x quasar pairs (16 to a panel)
 
 // One forest pair of a batch: its r_trans rows [t0, t0 + nt) of the data bins and
 // [u0, u0 + nu) of the model bins (bounds from the forests' dist_m) and its first rows in the
@@ -283,7 +284,12 @@ hipError_t launch_dmat_band_pass(const XiConst &M, const DmatConst &C, const Dma
                                  const DmatOut &O, int band_rows, hipStream_t stream);
 hipError_t launch_dmat_band_fill(const XiConst &M, const DmatConst &C, const DmatForests &F,
                                  const DmatBandSlots &P, const DmatBandWork &W,
-                                 const DmatOut &O, int num_cus, hipStream_t stream);
+                                 const DmatOut &O, bool quasar, int num_cus,
+                                 hipStream_t stream);
+// forest x quasar pairs: the rows each pair reaches (in place of the pass)
+hipError_t launch_dmat_quasar_rows(const XiConst &M, const DmatConst &C, const DmatForests &F,
+                                   const DmatBandSlots &P, const DmatBandWork &W,
+                                   hipStream_t stream);
 size_t dmat_band_pass_lds(const DmatConst &C, int rows);
 
 hipError_t launch_dmat_pass(const DmatConst &C, const DmatForests &F, const DmatPairs &P,

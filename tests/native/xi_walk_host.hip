@@ -328,12 +328,15 @@ extern "C" {
 double xi_walk_rcp_guess(double x) { return picca::walk_rcp_guess(x); }
 
 // The banded distortion matrix's keys and edges (dmat_band.h) of one pixel along a partner of n
-// rising values v, par: along r_par, else r_trans.  keys[k]: of pixel k; edges[k]: first pixel
+// rising values v (kind: BAND_*; from: r_par_min of BAND_SIGNED).  keys[k]: of pixel k; edges[k]: first pixel
 // whose key is at least k_lo + k.  The index table is made as the table kernel makes it.
-void dmat_band_host(int par, int n, const double *v, double self, double scale, double range,
+void dmat_band_host(int kind, double from, int n, const double *v, double self, double scale, double range,
                     int bins, double margin, int *keys, int k_lo, int num, int *edges) {
     const double mul = scale * bins / range;
-    const picca::BandAxis A = par ? picca::band_par_axis(self, mul, scale, range, bins, margin)
+    const picca::BandAxis A =
+        kind == picca::BAND_SIGNED
+            ? picca::band_signed_axis(self, mul, scale, from, range, bins, margin)
+        : kind == picca::BAND_PAR ? picca::band_par_axis(self, mul, scale, range, bins, margin)
                                   : picca::band_trans_axis(self, mul, scale, range, bins, margin);
     const double h = picca::band_mean_step(v[0], v[n - 1], n);
     std::vector<int32_t> first((size_t)n);

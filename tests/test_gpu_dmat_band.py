@@ -88,3 +88,87 @@ def test_cut_pairs_take_the_general_kernels():
     case.g.remove_same_half_plate_close_pairs = True
     check(case, flags=lambda n: (np.arange(n) % 3 == 0).astype(np.uint8)
           * _native.PICCA_PAIR_SAME_HALF_PLATE)
+
+
+def check_quasars(case, kp, kt, seed=0, orders=(0, 1)):
+    """Every pair's second forest replaced by a quasar at one of its pixels, or between them."""
+    g, p, store = case.g, case.pairs, case.store
+    rng = np.random.default_rng(seed)
+    used = np.array([(store.weights[o:e] != 0).sum() for o, e in zip(store.offsets[:-1],
+                                                                    store.offsets[1:])])
+    keep = used[p.pair_a] > 1
+    a, b, ang = p.pair_a[keep], p.pair_b[keep], p.pair_ang[keep]
+    m = len(a)
+    first, length = store.offsets[b], store.offsets[b + 1] - store.offsets[b]
+    pixel = first + rng.integers(0, 1 << 30, m) % length
+    away = rng.choice([0.0, 0.37, -21.0], m)
+    both = dict(offsets=np.concatenate([store.offsets, store.offsets[-1] + np.arange(1, m + 1)]),
+                r_comov=np.concatenate([store.r_comov, store.r_comov[pixel] + away]),
+                dist_m=np.concatenate([store.dist_m, store.dist_m[pixel] + away]),
+                z=np.concatenate([store.z, store.z[pixel]]),
+                weights=np.concatenate([store.weights,
+                                        rng.uniform(0.5, 2, m) * (rng.random(m) < 0.9)]),
+                delta=np.concatenate([store.delta, np.zeros(m)]),
+                log_lambda=np.concatenate([np.log10(1215.67 * (1 + store.z)), np.zeros(m)]),
+                order=np.concatenate([rng.choice(orders, store.num_forests),
+                                      np.full(m, -1)]).astype(np.int32))
+    for name in ("z_qso", "ra", "dec"):
+        both[name] = np.concatenate([getattr(store, name), getattr(store, name)[b]])
+    both["thingid"] = np.arange(store.num_forests + m)
+    new = ForestStore(**both)
+    g.x_correlation = True
+    g.r_par_min = -g.r_par_max if seed % 2 == 0 else -0.6 * g.r_par_max
+    with_model(case, kp, kt)
+    flags = np.full(m, _native.PICCA_PAIR_XCF_COUNT, np.uint8)
+    eng = get_engine(0)
+    eng.set_forests(new)
+    args = a, store.num_forests + np.arange(m), ang, flags
+    mine = eng.dmat(params_from_globals(g), *args)
+    params = O.params_from_module(g)
+    nm = g.num_model_bins_r_par * g.num_model_bins_r_trans
+    nb = g.num_bins_r_par * g.num_bins_r_trans
+    ref = [np.zeros(nb), np.zeros(nb * nm)] + [np.zeros(nm) for _ in range(4)]
+    stats = np.zeros(4, dtype=np.int64)
+    for x, y, angle in zip(*args[:3]):
+        i, j = (slice(new.offsets[k], new.offsets[k + 1]) for k in (x, y))
+        O.xdmat_forest(params, new.log_lambda[i], new.r_comov[i], new.dist_m[i], new.z[i],
+                       new.weights[i], new.r_comov[j], new.dist_m[j], new.z[j], new.weights[j],
+                       [angle], ref, new.order[x], stats)
+    ref[1] = ref[1].reshape(nb, nm)
+    assert list(mine[6]) == list(stats) and stats[0] > 0
+    assert_outputs_close(mine[:6], ref)
+
+
+@pytest.mark.parametrize("kp,kt", [(1, 1), (2, 1), (2, 2), (3, 1)])
+def test_quasars_on_exact_bin_edges(kp, kt):
+    case = W.lattice_case()
+    case.g.num_bins_r_par = case.g.num_bins_r_trans = 20
+    check_quasars(case, kp, kt)
+
+
+@pytest.mark.parametrize("angle", [0.004, 0.03])
+def test_quasars_with_irregular_forests(angle):
+    case = W.irregular_case()
+    case.pairs.pair_ang[:] = angle
+    case.g.num_bins_r_par = case.g.num_bins_r_trans = 25
+    check_quasars(case, 2, 1)
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2, 3, 5, 6, 7])   # (4: no pair in range)
+def test_quasars_in_random_geometries(seed):
+    case = W.random_case(seed)
+    case.g.num_bins_r_par = 1 + case.g.num_bins_r_par % 30
+    case.g.num_bins_r_trans = 1 + case.g.num_bins_r_trans % 30
+    case.g.r_par_max = max(case.g.r_par_max, 120.0)
+    case.g.r_trans_max = max(case.g.r_trans_max, 120.0)
+    case.pairs.pair_ang[:] *= 0.3
+    check_quasars(case, (1, 2)[seed % 2], (1, 1, 4)[seed % 3], seed=seed)
+
+
+@pytest.mark.parametrize("n_par,n_trans", [(64, 12), (65, 12), (130, 40), (1, 1)])
+def test_quasar_chunks(n_par, n_trans):
+    case = W.random_case(3)
+    case.g.num_bins_r_par, case.g.num_bins_r_trans = n_par, n_trans
+    case.g.r_par_max, case.g.r_trans_max = 120.0, 400.0
+    case.pairs.pair_ang[:] = np.linspace(0.001, 0.09, case.pairs.num_pairs)
+    check_quasars(case, 2, 1)

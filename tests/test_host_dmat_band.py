@@ -27,7 +27,7 @@ def test_r_par(grid, bins, span):
             rps = (own - v) * scale
             row = np.minimum(np.floor(np.abs(rps) / span * bins), bins)
             ref = np.where(rps > 0, -row - 1, row).astype(int)
-            keys, edges = H.dmat_band(1, v, own, scale, span, bins, margin, -bins, 2 * bins + 1)
+            keys, edges = H.dmat_band(H.BAND_PAR, v, own, scale, span, bins, margin, -bins, 2 * bins + 1)
             assert np.array_equal(keys, ref)
             assert np.array_equal(edges, np.searchsorted(ref, np.arange(-bins, bins + 1)))
 
@@ -40,6 +40,21 @@ def test_r_trans(grid, bins, span):
         for scale in (0.001, 0.004, 0.02):
             margin = 1e-12 + 20 * 2.0 ** -53 * (9000.0 * scale * bins / span + bins)
             ref = np.minimum(np.floor((own + v) * scale / span * bins), bins).astype(int)
-            keys, edges = H.dmat_band(0, v, own, scale, span, bins, margin, 0, bins + 1)
+            keys, edges = H.dmat_band(H.BAND_TRANS, v, own, scale, span, bins, margin, 0, bins + 1)
             assert np.array_equal(keys, ref)
+            assert np.array_equal(edges, np.searchsorted(ref, np.arange(bins + 1)))
+
+
+@pytest.mark.parametrize("bins,lo,hi", [(100, -200.0, 200.0), (30, -60.0, 60.0), (7, -11.0, 3.0)])
+@pytest.mark.parametrize("grid", sorted(GRIDS))
+def test_signed_r_par(grid, bins, lo, hi):
+    v, span = GRIDS[grid], hi - lo
+    for own in (v[0], v[len(v) // 2] + 0.25, v[-1], v[0] - 300.0, v[-1] + 150.0, 3850.0):
+        for scale in (1.0, 0.9998):
+            margin = 1e-12 + 20 * 2.0 ** -53 * (5000.0 * bins / span + 2 * bins)
+            t = np.floor(((v - own) * scale - lo) / span * bins)
+            ref = np.minimum(np.maximum(t, -1), bins).astype(int)
+            keys, edges = H.dmat_band(H.BAND_SIGNED, v, own, scale, span, bins, margin, 0,
+                                      bins + 1, lo)
+            assert np.array_equal(np.maximum(keys, -1), ref)
             assert np.array_equal(edges, np.searchsorted(ref, np.arange(bins + 1)))

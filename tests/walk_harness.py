@@ -58,11 +58,14 @@ def _p(a):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
-def dmat_band(par, values, own, scale, span, bins, margin, k_lo, num):
+BAND_TRANS, BAND_PAR, BAND_SIGNED = 0, 1, 2
+
+
+def dmat_band(kind, values, own, scale, span, bins, margin, k_lo, num, r_par_min=0.0):
     """Keys of the pixels and the first pixel of each key from k_lo on (dmat_band.h)."""
     v = np.ascontiguousarray(values, dtype=np.float64)
     keys, edges = np.zeros(len(v), dtype=np.int32), np.zeros(num, dtype=np.int32)
-    lib().dmat_band_host(ctypes.c_int(par), ctypes.c_int(len(v)), _p(v), ctypes.c_double(own),
+    lib().dmat_band_host(ctypes.c_int(kind), ctypes.c_double(r_par_min), ctypes.c_int(len(v)), _p(v), ctypes.c_double(own),
                          ctypes.c_double(scale), ctypes.c_double(span), ctypes.c_int(bins),
                          ctypes.c_double(margin), _p(keys), ctypes.c_int(k_lo),
                          ctypes.c_int(num), _p(edges))
