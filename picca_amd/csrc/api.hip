@@ -949,14 +949,12 @@ struct DmatRun {
     // uploads of the general kernels, kept until the stream is done
     std::vector<double> cs;
     std::vector<std::vector<int64_t>> pix_off;
-    // the downloads; host_buffers() makes them while the kernels run
-    std::vector<double> h_wdm, h_dmat, h_eff;
-    void host_buffers() {
-        h_wdm.resize((size_t)C.nb);
-        h_dmat.resize((size_t)C.nb * (size_t)C.nm);
-        h_eff.resize(4 * (size_t)C.nm);
-    }
 };
+
+// the redshift-evolution factors of delta1 and delta2 differ
+bool roles_differ(const picca_cf_params &p) {
+    return p.redshift_evolution && p.alpha != p.alpha2;
+}
 
 struct DmatPairList {
     std::vector<int32_t> a, b;
@@ -1171,7 +1169,7 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
     if (total == 0) return PICCA_OK;
     hipStream_t st = ctx->stream;
     const size_t entries = (size_t)(ctx->num_pixels + ctx->num_forests);
-    const bool differ = R.params->redshift_evolution && R.params->alpha != R.params->alpha2;
+    const bool differ = roles_differ(*R.params);
     PICCA_HIP_CHECK(ctx->db_pre_b.reserve(entries));
     if (differ) PICCA_HIP_CHECK(ctx->db_pre_a.reserve(entries));
     picca::DmatPrefix *pre_b = ctx->db_pre_b.ptr, *pre_a = differ ? ctx->db_pre_a.ptr : pre_b;
@@ -1236,7 +1234,6 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
         PICCA_HIP_CHECK(hipEventRecord(ev[2], st));
         p0 = p1;
     }
-    R.host_buffers();
     int32_t num_redo = 0;
     PICCA_HIP_CHECK(hipMemcpyAsync(&num_redo, ctx->db_num.ptr + 2, sizeof(num_redo),
                                    hipMemcpyDeviceToHost, st));
@@ -1341,21 +1338,23 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
     const int64_t npix = ctx->num_pixels;
     const size_t pad = picca::PIXEL_PAD;
     {   // redshift-evolution factors of each pixel (py/picca/cf.py:680-685)
-        std::vector<double> fa((size_t)std::max<int64_t>(npix, 1), 1.0);
-        std::vector<double> fb((size_t)std::max<int64_t>(npix, 1), 1.0);
-        if (params->redshift_evolution) {
-            const double zr = 1 + params->z_ref;
-            const double ea = params->alpha - 1, eb = params->alpha2 - 1;
+        std::vector<double> f((size_t)std::max<int64_t>(npix, 1), 1.0);
+        auto factors = [&](double alpha) {
+            const double zr = 1 + params->z_ref, e = alpha - 1;
             parallel_for(npix, [&](int64_t lo, int64_t hi) {
-                for (int64_t k = lo; k < hi; ++k) {
-                    fa[k] = std::pow((1 + ctx->h_z[k]) / zr, ea);
-                    fb[k] = std::pow((1 + ctx->h_z[k]) / zr, eb);
-                }
+                for (int64_t k = lo; k < hi; ++k) f[k] = std::pow((1 + ctx->h_z[k]) / zr, e);
             });
+        };
+        if (params->redshift_evolution) factors(params->alpha);
+        PICCA_HIP_CHECK(ctx->zfa.upload_padded(f.data(), (size_t)npix, pad, ctx->stream));
+        PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+        if (roles_differ(*params)) {
+            factors(params->alpha2);
+            PICCA_HIP_CHECK(ctx->zfb.upload_padded(f.data(), (size_t)npix, pad, ctx->stream));
+            PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
         }
-        PICCA_HIP_CHECK(ctx->zfa.upload_padded(fa.data(), (size_t)npix, pad, ctx->stream));
-        PICCA_HIP_CHECK(ctx->zfb.upload_padded(fb.data(), (size_t)npix, pad, ctx->stream));
     }
+    const double *zfb = roles_differ(*params) ? ctx->zfb.ptr : ctx->zfa.ptr;
     // outputs, accumulated over all batches on the device
     const int64_t nb = C.nb, nm = C.nm;
     PICCA_HIP_CHECK(ctx->o_wdm.reserve((size_t)nb));
@@ -1370,11 +1369,11 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
     PICCA_HIP_CHECK(picca::launch_zero_u64(ctx->dstats.ptr, picca::DMAT_NSTATS, ctx->stream));
 
     picca::DmatForests F{ctx->r.ptr,   ctx->d.ptr,     ctx->z.ptr,     ctx->w.ptr,   ctx->dll.ptr,
-                         ctx->zfa.ptr, ctx->zfb.ptr,   ctx->off.ptr,   ctx->zq.ptr,  ctx->sum_w.ptr,
+                         ctx->zfa.ptr, zfb,            ctx->off.ptr,   ctx->zq.ptr,  ctx->sum_w.ptr,
                          ctx->sw_dll.ptr, ctx->order.ptr, ctx->mono.ptr};
     picca::DmatOut O{ctx->o_wdm.ptr, ctx->o_dmat.ptr, ctx->o_eff.ptr, ctx->o_eff.ptr + nm,
                      ctx->o_eff.ptr + 2 * nm, ctx->o_eff.ptr + 3 * nm};
-    DmatRun R{ctx, params, C, F, O, pass_lds, 0, {}, {}, {}, {}, {}};
+    DmatRun R{ctx, params, C, F, O, pass_lds, 0, {}, {}};
     DmatPairList pairs, rest;
     pairs.a.assign(pair_a, pair_a + num_pairs);
     pairs.b.assign(pair_b, pair_b + num_pairs);
@@ -1385,15 +1384,7 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
     if (status != PICCA_OK) return status;
     const int64_t batches = R.batches;
 
-    R.host_buffers();
-    std::vector<double> &h_wdm = R.h_wdm, &h_dmat = R.h_dmat, &h_eff = R.h_eff;
     unsigned long long h_stats[picca::DMAT_NSTATS];
-    PICCA_HIP_CHECK(hipMemcpyAsync(h_wdm.data(), ctx->o_wdm.ptr, sizeof(double) * nb,
-                                   hipMemcpyDeviceToHost, ctx->stream));
-    PICCA_HIP_CHECK(hipMemcpyAsync(h_dmat.data(), ctx->o_dmat.ptr, sizeof(double) * nb * nm,
-                                   hipMemcpyDeviceToHost, ctx->stream));
-    PICCA_HIP_CHECK(hipMemcpyAsync(h_eff.data(), ctx->o_eff.ptr, sizeof(double) * 4 * nm,
-                                   hipMemcpyDeviceToHost, ctx->stream));
     PICCA_HIP_CHECK(hipMemcpyAsync(h_stats, ctx->dstats.ptr, sizeof(h_stats),
                                    hipMemcpyDeviceToHost, ctx->stream));
     PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
@@ -1410,16 +1401,8 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
     }
     if (h_stats[picca::DMAT_STAT_NEGATIVE] > 0)
         return fail(PICCA_E_INDEX, "a selected pair has a negative data bin index");
-    for (int64_t k = 0; k < nb; ++k) weights_dmat[k] += h_wdm[k];
-    parallel_for(nb * nm, [&](int64_t lo, int64_t hi) {
-        for (int64_t k = lo; k < hi; ++k) dmat[k] += h_dmat[k];
-    });
-    for (int64_t k = 0; k < nm; ++k) {
-        r_par_eff[k] += h_eff[k];
-        r_trans_eff[k] += h_eff[nm + k];
-        z_eff[k] += h_eff[2 * nm + k];
-        weight_eff[k] += h_eff[3 * nm + k];
-    }
+    PICCA_HIP_CHECK(add_dmat_outputs(ctx, nb, nm, weights_dmat, dmat, r_par_eff, r_trans_eff,
+                                     z_eff, weight_eff));
     if (stats) {
         stats[0] = (int64_t)h_stats[picca::DMAT_STAT_IN_RANGE];
         stats[1] = (int64_t)h_stats[picca::DMAT_STAT_SELECTED];

@@ -61,12 +61,7 @@ int picca_cont_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *o
     const size_t nf = (size_t)std::max<int64_t>(num_forests, 1);
     PICCA_HIP_CHECK(ctx->c_a0.reserve(nf));
     PICCA_HIP_CHECK(ctx->c_b0.reserve(nf));
-    PICCA_HIP_CHECK(ctx->c_a.reserve(nf));
-    PICCA_HIP_CHECK(ctx->c_b.reserve(nf));
-    PICCA_HIP_CHECK(ctx->c_chi2.reserve(nf));
-    PICCA_HIP_CHECK(ctx->c_ndata.reserve(nf));
-    PICCA_HIP_CHECK(ctx->c_status.reserve(nf));
-    PICCA_HIP_CHECK(ctx->c_evals.reserve(nf));
+    PICCA_HIP_CHECK(ctx->c_fit.reserve(5 * nf));
     PICCA_HIP_CHECK(hipStreamSynchronize(st));
     ctx->cont_forests = num_forests;
     ctx->cont_pixels = npix;
@@ -97,20 +92,27 @@ int picca_cont_fit(picca_ctx *ctx, const picca_cont_params *params, const double
     picca::ContIn I{ctx->c_off.ptr,  ctx->c_flux.ptr, ctx->c_ivar.ptr,  ctx->c_mean.ptr,
                     ctx->c_x.ptr,    ctx->c_eta.ptr,  ctx->c_lss.ptr,   ctx->c_fudge.ptr,
                     ctx->c_order.ptr, ctx->c_a0.ptr,  ctx->c_b0.ptr};
-    picca::ContOut O{ctx->c_a.ptr, ctx->c_b.ptr, ctx->c_chi2.ptr, ctx->c_ndata.ptr,
-                     ctx->c_status.ptr, ctx->c_evals.ptr};
+    const picca::ContOut O = ctx->cont_out();
     PICCA_HIP_CHECK(hipEventRecord(ctx->ev_start, st));
     PICCA_HIP_CHECK(picca::launch_cont_fit(K, I, O, ctx->c_class.ptr, ctx->cont_class_begin,
                                            st));
     PICCA_HIP_CHECK(hipEventRecord(ctx->ev_stop, st));
-    if (nf > 0) {
-        PICCA_HIP_CHECK(hipMemcpyAsync(a, ctx->c_a.ptr, sizeof(double) * nf, hipMemcpyDeviceToHost, st));
-        PICCA_HIP_CHECK(hipMemcpyAsync(b, ctx->c_b.ptr, sizeof(double) * nf, hipMemcpyDeviceToHost, st));
-        PICCA_HIP_CHECK(hipMemcpyAsync(chi2, ctx->c_chi2.ptr, sizeof(double) * nf, hipMemcpyDeviceToHost, st));
-        PICCA_HIP_CHECK(hipMemcpyAsync(ndata, ctx->c_ndata.ptr, sizeof(int32_t) * nf, hipMemcpyDeviceToHost, st));
-        PICCA_HIP_CHECK(hipMemcpyAsync(status, ctx->c_status.ptr, sizeof(int32_t) * nf, hipMemcpyDeviceToHost, st));
-        PICCA_HIP_CHECK(hipMemcpyAsync(evaluations, ctx->c_evals.ptr, sizeof(int32_t) * nf, hipMemcpyDeviceToHost, st));
-    }
+    // bytes of the six results, in the order of the device's block
+    struct Field {
+        void *to;
+        int64_t size;
+    };
+    const Field fields[6] = {{a, 8 * nf},     {b, 8 * nf},      {chi2, 8 * nf},
+                             {ndata, 4 * nf}, {status, 4 * nf}, {evaluations, 4 * nf}};
+    PICCA_HIP_CHECK(picca_host::download(
+        ctx->ring, ctx->c_fit.ptr, 36 * nf, st, [&](const char *src, int64_t lo, int64_t hi) {
+            int64_t first = 0;
+            for (const Field &f : fields) {
+                const int64_t p = std::max(lo, first), q = std::min(hi, first + f.size);
+                if (p < q) std::memcpy((char *)f.to + (p - first), src + (p - lo), (size_t)(q - p));
+                first += f.size;
+            }
+        }));
     PICCA_HIP_CHECK(hipStreamSynchronize(st));
     float ms = 0.f;
     PICCA_HIP_CHECK(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
@@ -165,7 +167,8 @@ int picca_cont_stack(picca_ctx *ctx, double *sum_ratio, double *sum_weight,
                     ctx->c_x.ptr,    ctx->c_eta.ptr,  ctx->c_lss.ptr,   ctx->c_fudge.ptr,
                     ctx->c_order.ptr, ctx->c_a0.ptr,  ctx->c_b0.ptr};
     PICCA_HIP_CHECK(hipEventRecord(ctx->ev_start, st));
-    PICCA_HIP_CHECK(picca::launch_cont_stack(I, ctx->c_a.ptr, ctx->c_b.ptr, ctx->c_status.ptr,
+    const picca::ContOut fit = ctx->cont_out();
+    PICCA_HIP_CHECK(picca::launch_cont_stack(I, fit.a, fit.b, fit.status,
                                              ctx->c_bin.ptr, nbins, d_ratio, d_weight,
                                              ctx->cont_forests, ctx->num_cus, st));
     PICCA_HIP_CHECK(hipEventRecord(ctx->ev_stop, st));

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <string>
 #include <thread>
@@ -12,6 +13,7 @@
 
 #include "../../include/picca_hip.h"
 #include "engine.h"
+#include "download.h"
 #include "dmat_band.h"
 #include "xi_walk.h"
 
@@ -93,16 +95,31 @@ inline void parallel_for(int64_t n, F body) {
     for (auto &th : pool) th.join();
 }
 
+// All of [0, n) pass ok(k).
+template <typename F>
+inline bool parallel_all(int64_t n, F ok) {
+    std::atomic<bool> all{true};
+    parallel_for(n, [&](int64_t lo, int64_t hi) {
+        bool good = true;
+        for (int64_t k = lo; k < hi; ++k) good = good && ok(k);
+        if (!good) all.store(false, std::memory_order_relaxed);
+    });
+    return all.load();
+}
+
 }  // namespace picca_host
 
 using picca_host::DeviceBuffer;
+using picca_host::download_values;
 using picca_host::fail;
+using picca_host::parallel_all;
 using picca_host::parallel_for;
 
 struct picca_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev_start = nullptr, ev_stop = nullptr, ev_mid = nullptr;
+    picca_host::DownloadRing ring;
     // distortion matrix: events around each batch's pass and fill kernels (a pool that
     // grows with the batches of a run) and the last run's report
     std::vector<hipEvent_t> dmat_events;
@@ -205,8 +222,14 @@ struct picca_ctx {
     int64_t cont_class_begin[picca::CONT_CLASSES + 1] = {0, 0, 0, 0, 0, 0};
     DeviceBuffer<double> c_flux, c_ivar, c_mean, c_x, c_eta, c_lss, c_fudge;
     DeviceBuffer<int32_t> c_order;
-    DeviceBuffer<double> c_a0, c_b0, c_a, c_b, c_chi2;
-    DeviceBuffer<int32_t> c_ndata, c_status, c_evals;
+    DeviceBuffer<double> c_a0, c_b0;
+    // the fit's a, b, chi2, then ndata, status, evaluations, one array after the other
+    DeviceBuffer<double> c_fit;
+    picca::ContOut cont_out() const {
+        const size_t n = (size_t)cont_forests;
+        int32_t *whole = (int32_t *)(c_fit.ptr + 3 * n);
+        return {c_fit.ptr, c_fit.ptr + n, c_fit.ptr + 2 * n, whole, whole + n, whole + 2 * n};
+    }
     // DR16 iteration: per pixel rest-frame log lambda, transmission correction, rest-frame
     // bin; the stacked sums; the mean continuum's interpolation nodes
     DeviceBuffer<double> c_llr, c_trans, c_stack, c_xs, c_ys;
@@ -258,4 +281,17 @@ struct picca_ctx {
     DeviceBuffer<picca::XiBin> o_bins;
     DeviceBuffer<unsigned long long> queue, stats;
 };
+
+// Adds a distortion matrix's device outputs (o_wdm, o_dmat, o_eff) to the caller's.
+inline hipError_t add_dmat_outputs(picca_ctx *ctx, int64_t nb, int64_t nm, double *weights_dmat,
+                                   double *dmat, double *r_par_eff, double *r_trans_eff,
+                                   double *z_eff, double *weight_eff) {
+    hipError_t err = download_values<true>(ctx->ring, ctx->o_wdm.ptr, nb, ctx->stream,
+                                           weights_dmat);
+    double *const eff[4] = {r_par_eff, r_trans_eff, z_eff, weight_eff};
+    for (int k = 0; k < 4 && err == hipSuccess; ++k)
+        err = download_values<true>(ctx->ring, ctx->o_eff.ptr + k * nm, nm, ctx->stream, eff[k]);
+    if (err != hipSuccess) return err;
+    return download_values<true>(ctx->ring, ctx->o_dmat.ptr, nb * nm, ctx->stream, dmat);
+}
 

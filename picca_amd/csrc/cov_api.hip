@@ -17,9 +17,10 @@ int picca_cov_subsample(picca_ctx *ctx, int64_t num_samples, int64_t num_bins,
     if (num_bins > 0 && (!cov || (num_samples > 0 && (!xi || !weights))))
         return fail(PICCA_E_VALUE, "arrays must not be NULL");
     const int64_t n = num_samples * num_bins;
-    for (int64_t k = 0; k < n; ++k)
-        if (!std::isfinite(xi[k]) || !std::isfinite(weights[k]))
-            return fail(PICCA_E_VALUE, "xi and weights must be finite");
+    if (!parallel_all(n, [&](int64_t k) {
+            return std::isfinite(xi[k]) && std::isfinite(weights[k]);
+        }))
+        return fail(PICCA_E_VALUE, "xi and weights must be finite");
     if (num_bins == 0) return PICCA_OK;
     PICCA_HIP_CHECK(hipSetDevice(ctx->device));
     PICCA_HIP_CHECK(ctx->cv_xi.upload(xi, (size_t)n, ctx->stream));
@@ -36,10 +37,8 @@ int picca_cov_subsample(picca_ctx *ctx, int64_t num_samples, int64_t num_bins,
                                            ctx->cv_y.ptr, num_samples, (int)num_bins,
                                            ctx->cv_cov.ptr, ctx->stream));
     PICCA_HIP_CHECK(hipEventRecord(ctx->ev_stop, ctx->stream));
-    PICCA_HIP_CHECK(hipMemcpyAsync(cov, ctx->cv_cov.ptr,
-                                   sizeof(double) * (size_t)(num_bins * num_bins),
-                                   hipMemcpyDeviceToHost, ctx->stream));
-    PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+    PICCA_HIP_CHECK(download_values<false>(ctx->ring, ctx->cv_cov.ptr, num_bins * num_bins,
+                                           ctx->stream, cov));
     float ms = 0.f, ms_syrk = 0.f;
     PICCA_HIP_CHECK(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
     PICCA_HIP_CHECK(hipEventElapsedTime(&ms_syrk, ctx->ev_mid, ctx->ev_stop));

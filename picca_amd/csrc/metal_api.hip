@@ -167,29 +167,14 @@ int picca_metal_pass(picca_ctx *ctx, const picca_cf_params *params, int32_t mode
                                         ctx->stream));
     PICCA_HIP_CHECK(hipEventRecord(ctx->ev_stop, ctx->stream));
 
-    std::vector<double> h_wdm((size_t)nb), h_dmat((size_t)(nb * nm)), h_eff((size_t)(4 * nm));
     unsigned long long h_stats[picca::METAL_NSTATS];
-    PICCA_HIP_CHECK(hipMemcpyAsync(h_wdm.data(), ctx->o_wdm.ptr, sizeof(double) * nb,
-                                   hipMemcpyDeviceToHost, ctx->stream));
-    PICCA_HIP_CHECK(hipMemcpyAsync(h_dmat.data(), ctx->o_dmat.ptr, sizeof(double) * nb * nm,
-                                   hipMemcpyDeviceToHost, ctx->stream));
-    PICCA_HIP_CHECK(hipMemcpyAsync(h_eff.data(), ctx->o_eff.ptr, sizeof(double) * 4 * nm,
-                                   hipMemcpyDeviceToHost, ctx->stream));
     PICCA_HIP_CHECK(hipMemcpyAsync(h_stats, ctx->m_stats.ptr, sizeof(h_stats),
                                    hipMemcpyDeviceToHost, ctx->stream));
     PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     float ms = 0.f;
     PICCA_HIP_CHECK(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
-    for (int64_t k = 0; k < nb; ++k) weights_dmat[k] += h_wdm[k];
-    parallel_for(nb * nm, [&](int64_t lo, int64_t hi) {
-        for (int64_t k = lo; k < hi; ++k) dmat[k] += h_dmat[k];
-    });
-    for (int64_t k = 0; k < nm; ++k) {
-        r_par_eff[k] += h_eff[k];
-        r_trans_eff[k] += h_eff[nm + k];
-        z_eff[k] += h_eff[2 * nm + k];
-        weight_eff[k] += h_eff[3 * nm + k];
-    }
+    PICCA_HIP_CHECK(add_dmat_outputs(ctx, nb, nm, weights_dmat, dmat, r_par_eff, r_trans_eff,
+                                     z_eff, weight_eff));
     if (report) {
         report->data_pairs = (int64_t)h_stats[picca::METAL_STAT_DATA];
         report->model_pairs = (int64_t)h_stats[picca::METAL_STAT_MODEL];
