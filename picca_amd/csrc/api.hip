@@ -197,7 +197,7 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
         // run walk of the xi kernel: (r, d) pairs, prefix sums (L + 1 entries per forest)
         // and the smallest pixel steps per forest
         std::vector<double2> rd((size_t)std::max<int64_t>(npix, 1));
-        std::vector<picca::PrefixRecord> pre((size_t)(npix + num_forests));
+        std::vector<picca::PrefixPair> pre(picca::PREFIX_PLANES * (size_t)(npix + num_forests));
         std::vector<double2> spc((size_t)std::max<int64_t>(num_forests, 1));
         parallel_for(npix, [&](int64_t lo, int64_t hi) {
             for (int64_t k = lo; k < hi; ++k) rd[k] = make_double2(r_comov[k], dist_m[k]);
@@ -207,13 +207,13 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
                 const int64_t o = offsets[k], n = offsets[k + 1] - offsets[k];
                 double sr, sd;
                 picca::build_walk_forest(r_comov + o, dist_m + o, z + o, weights + o,
-                                         dw.data() + o, n, pre.data() + o + k, sr, sd);
+                                         dw.data() + o, n,
+                                         pre.data() + picca::PREFIX_PLANES * (o + k), sr, sd);
                 spc[k] = make_double2(sr, sd);
             }
         });
         PICCA_HIP_CHECK(ctx->rd.upload_padded(rd.data(), (size_t)npix, pad, ctx->stream));
-        PICCA_HIP_CHECK(ctx->pre.upload_padded(pre.data(), (size_t)(npix + num_forests), pad,
-                                               ctx->stream));
+        PICCA_HIP_CHECK(ctx->pre.upload_padded(pre.data(), pre.size(), pad, ctx->stream));
         PICCA_HIP_CHECK(ctx->spc.upload(spc.data(), (size_t)num_forests, ctx->stream));
         PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
         ctx->h_spc = std::move(spc);

@@ -148,7 +148,7 @@ struct picca_ctx {
     DeviceBuffer<uint8_t> mono;
     // run walk of the xi kernel (xi_walk.h)
     DeviceBuffer<double2> rd, spc;
-    DeviceBuffer<picca::PrefixRecord> pre;
+    DeviceBuffer<picca::PrefixPair> pre;
     int32_t xi_schedule = 0;   // PICCA_XI_SCHEDULE_*
     double median_step_r = 0;  // median over forests of the mean r_comov step between pixels
     // the xi launch sequence (zero kernels + pair kernel) as a HIP graph, replayed while

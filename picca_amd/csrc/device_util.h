@@ -95,4 +95,18 @@ __device__ __forceinline__ double dpp_f64(double v) {
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
+// Sum over the wave of a value that is mostly below 2^26.
+__device__ __forceinline__ uint64_t wave_sum_small(uint64_t v) {
+    if (__builtin_amdgcn_ballot_w64((v >> 26) != 0)) return wave_sum_u64(v);
+    int x = (int)(uint32_t)v;
+    x += dpp_int<DPP_ROW_SHR1>(x);
+    x += dpp_int<DPP_ROW_SHR2>(x);
+    x += dpp_int<DPP_ROW_SHR4>(x);
+    x += dpp_int<DPP_ROW_SHR8>(x);
+    uint64_t sum = 0;
+    for (int row = 0; row < 4; ++row)
+        sum += (uint32_t)__builtin_amdgcn_readlane(x, 16 * row + 15);
+    return sum;
+}
+
 }  // namespace picca

@@ -44,7 +44,7 @@ struct DmatAcc {
         const double dw = pe.w - ps.w;
         const double s_r = (pe.r - ps.r) - (L.r1 - T.rc) * dw;
         const double s_d = (L.d1 + T.dc) * dw + (pe.d - ps.d);
-        o.bin = c * C.np + (m >= 0 ? m : -m - 1);
+        o.bin = walk_bin(c, C.np, m >= 0 ? m : -m - 1);
         o.s0 = L.w1 * dw;
         o.sj = L.w1 * (pe.wl - ps.wl);
         o.z0 = L.dw1 * (pe.zw - ps.zw);

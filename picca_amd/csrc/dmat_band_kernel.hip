@@ -115,6 +115,7 @@ struct BandPassMem {
     int u0;               // first model row of the pair
     int i;                // the lane's pixel of delta1
     double l1;            // its dll
+    const XiConst *exact;   // LDS copy
     uint64_t n_in;
     int row, r_first, r_last;   // run of runs in one model row
 
@@ -123,6 +124,7 @@ struct BandPassMem {
         d = dp[p];
     }
     __device__ DmatPrefix prefix(int p) const { return pre[p]; }
+    __device__ const XiConst &consts(const XiConst &) const { return *exact; }
     __device__ double w(int p) const { return wp[p]; }
     __device__ double z(int p) const { return zp[p]; }
     __device__ double dw(int) const { return 0.0; }
@@ -169,12 +171,12 @@ struct BandPassMem {
         }
         r_last = g - 1;
     }
-    __device__ bool any(bool v) const { return __ballot(v) != 0; }
+    __device__ bool any(bool v) const { return __builtin_amdgcn_ballot_w64(v) != 0; }
     __device__ static void pin(DmatSums &) {}
     __device__ void count_edge() {}
     __device__ void count_overflow() { *special = 1; }
     __device__ void count_probe() {}
-    __device__ void count_run(uint32_t) {}
+    __device__ void count_run(bool, uint32_t) {}
 };
 
 }  // namespace
@@ -263,6 +265,7 @@ __global__ __launch_bounds__(DMAT_BAND_PASS_BLOCK) void dmat_band_pass_kernel(
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ unsigned long long s_in;
     __shared__ int s_special;
+    __shared__ XiConst s_const;
     const int s = blockIdx.x;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -281,6 +284,7 @@ __global__ __launch_bounds__(DMAT_BAND_PASS_BLOCK) void dmat_band_pass_kernel(
     if (tid == 0) {
         s_in = 0;
         s_special = 0;
+        s_const = M;   // published by the first __syncthreads below
     }
     const double *__restrict__ Br = F.r + q.ob;
     const double *__restrict__ Bd = F.d + q.ob;
@@ -320,8 +324,8 @@ __global__ __launch_bounds__(DMAT_BAND_PASS_BLOCK) void dmat_band_pass_kernel(
             if (T.j_lo >= T.j_hi) continue;
             T.cos_half = q.cos_half;
             T.sin_half = q.sin_half;
-            T.cp = q.cos_half * M.inv_p;
-            T.st = mul_t;
+            T.cp = uniform_f64(q.cos_half * M.inv_p);
+            T.st = uniform_f64(mul_t);
             T.rc = uniform_f64(Br[q.lb >> 1]);
             T.dc = uniform_f64(Bd[q.lb >> 1]);
             T.q0 = 1.0;
@@ -346,7 +350,7 @@ __global__ __launch_bounds__(DMAT_BAND_PASS_BLOCK) void dmat_band_pass_kernel(
                 }
             }
             BandPassMem mem{Br, Bd, F.w + q.ob, F.z + q.ob, W.pre_b + (q.ob + q.b), acc, rng,
-                            &s_special, stride, nu, uc0 * C.npm, u0, i, l1, 0, -1, 0, 0};
+                            &s_special, stride, nu, uc0 * C.npm, u0, i, l1, &s_const, 0, -1, 0, 0};
             walk_lane<false, true, DmatAcc>(M, T, L, mem, active);
             mem.note();
             n_in += mem.n_in;

@@ -82,7 +82,7 @@ struct PixelRecord {
     double dw;  // delta * weight
 };
 
-struct PrefixRecord;  // xi_walk.h
+struct PrefixPair;  // xi_walk.h
 
 struct ForestView {
     const PixelRecord *__restrict__ pix;  // the same pixels, one 40-byte record each
@@ -98,7 +98,7 @@ struct ForestView {
     const uint8_t *__restrict__ mono; // bit0 r_comov non-decreasing, bit1 dist_m
                                       // non-decreasing, bit2 z non-decreasing
     const double2 *__restrict__ rd;   // (r_comov, dist_m) per pixel
-    const PrefixRecord *__restrict__ pre;       // run-walk prefix sums, forest b at off[b] + b
+    const PrefixPair *__restrict__ pre;   // run-walk prefix sums, forest b at 3 (off[b] + b)
     const double2 *__restrict__ spc;  // per forest: smallest step of r_comov and of dist_m
                                       // between consecutive pixels, -1 unless both increase
                                       // strictly

@@ -255,29 +255,46 @@ __device__ __forceinline__ double min_f64(double a, double b) {
 
 typedef __attribute__((address_space(3))) unsigned long long LocalU64;
 
-// Lanes whose closed runs the walk merges before its LDS atomics (a power of two, <= 16).
-// On the 100k-forest survey: no merging 28.7 s, groups of 16 / 8 / 4 / 2 lanes 26.5 / 25.5 /
-// 24.7 / 24.8 s; each step of the segmented sum costs ~20 VALU instructions per pass.
-constexpr int WALK_FLUSH_GROUP = 4;
+// Lanes whose closed runs the walk merges before its LDS atomics.  Each step of the segmented
+// sum costs ~20 vector instructions per pass, and the six FP64 atomics of a pass ~20 LDS cycles
+// each, so the pass is bound by both.  2.7M pairs of a linear grid, of which a pass takes 178
+// vector instructions with groups of 4 and 198 with 8: 341 ms (LDS) and 337 ms.  Fewer
+// instructions alone did not show there (345 ms with 199); with the half-plate cut on 500 forests
+// the call takes 21.7 ms against 23.9 ms, signed r_par 30.8 ms against 33.0 ms.
+constexpr int WALK_FLUSH_GROUP = 8;
+// pixels of a forest that the walk's 24-bit indexes reach
+constexpr int WALK_MAX_PIXELS = 1 << 24;
 
 // Memory of the run walk on the device: delta2's pixels and prefix sums in HBM (read
 // per lane), the LDS histogram of the output row, the LDS statistics.
 struct DeviceWalkMem {
     const double2 *__restrict__ rdp;
-    const PrefixRecord *__restrict__ pre;
+    const PrefixPair *__restrict__ pre[PREFIX_PLANES];
     const double *__restrict__ wp;
     const double *__restrict__ zp;
     const double *__restrict__ dwp;
     LocalBin *hist;
     LocalU64 *stats;
-    uint32_t probes, runs, cover;
+    const XiConst *exact;     // LDS copy of the constants
+    uint32_t probes, cover;   // of the lane
+    uint32_t runs;            // of the wave
 
     __device__ void rd(int p, double &r, double &d) const {
-        const double2 v = rdp[p];
+        // 32-bit byte offsets from the forest's uniform address: the task holds less than
+        // WALK_MAX_PIXELS pixels
+        const double2 v = *(const double2 *)((const char *)rdp + (uint32_t)p * 16u);
         r = v.x;
         d = v.y;
     }
-    __device__ PrefixRecord prefix(int p) const { return pre[p]; }
+    __device__ PrefixRecord prefix(int p) const {
+        auto pair = [&](int plane) {
+            return *(const PrefixPair *)((const char *)pre[plane] + (uint32_t)p * 16u);
+        };
+        return prefix_entry(pair(0), pair(1), pair(2));
+    }
+    // the exact arithmetic is rare: its constants come from LDS and not from scalar registers,
+    // of which the loop has too few
+    __device__ const XiConst &consts(const XiConst &) const { return *exact; }
     __device__ double w(int p) const { return wp[p]; }
     __device__ double z(int p) const { return zp[p]; }
     __device__ double dw(int p) const { return dwp[p]; }
@@ -299,38 +316,46 @@ struct DeviceWalkMem {
     // of each segment makes the six LDS atomics, so that a bin takes one atomic per group
     // instead of one per lane.
     __device__ void flush(bool on, const RunSums &run) {
-        static_assert(WALK_FLUSH_GROUP >= 1 && WALK_FLUSH_GROUP <= 16 &&
-                      (WALK_FLUSH_GROUP & (WALK_FLUSH_GROUP - 1)) == 0, "group of 1..16 lanes");
+        static_assert(WALK_FLUSH_GROUP == 8, "three steps of the segmented sum");
         // segment key: bin + 1 for a lane with a run, 0 without (and outside the row)
         const int key = on ? run.bin + 1 : 0;
         const int gl = __lane_id() & (WALK_FLUSH_GROUP - 1);
         int head = (key != dpp_int<DPP_ROW_SHR1>(key)) || gl == 0;
-        double we = run.we, xi = run.xi, rp = run.rp, rt = run.rt, z = run.z;
-        uint32_t n = run.n;
-        if constexpr (WALK_FLUSH_GROUP > 1) segment_step<DPP_ROW_SHR1>(head, we, xi, rp, rt, z, n);
-        if constexpr (WALK_FLUSH_GROUP > 2) segment_step<DPP_ROW_SHR2>(head, we, xi, rp, rt, z, n);
-        if constexpr (WALK_FLUSH_GROUP > 4) segment_step<DPP_ROW_SHR4>(head, we, xi, rp, rt, z, n);
-        if constexpr (WALK_FLUSH_GROUP > 8) segment_step<DPP_ROW_SHR8>(head, we, xi, rp, rt, z, n);
         const bool tail = (key != dpp_int<DPP_ROW_SHL1>(key)) || gl == WALK_FLUSH_GROUP - 1;
-        if (on && tail) add(run.bin, we, xi, rp, rt, z, n);
+        const bool write = on && tail;
+        // a lane takes nothing from the lane (two, four lanes) before it if a segment starts at
+        // it or between them
+        const int head2 = head | dpp_int<DPP_ROW_SHR1>(head);
+        const int head4 = head2 | dpp_int<DPP_ROW_SHR2>(head2);
+        const double take1 = head ? 0.0 : 1.0, take2 = head2 ? 0.0 : 1.0;
+        const double take4 = head4 ? 0.0 : 1.0;
+        LocalBin *b = (LocalBin *)((LocalByte *)hist +
+                                   __umul24((uint32_t)run.bin, (uint32_t)sizeof(LdsBin)));
+        // One sum after the other, each with its atomic: six atomics in a row wait for the LDS
+        // queue (SQ_WAIT_INST_LDS), between the sums' arithmetic they do not.
+        auto add_sum = [&](auto *to, double v) {
+            v = fma(dpp_f64<DPP_ROW_SHR1>(v), take1, v);
+            v = fma(dpp_f64<DPP_ROW_SHR2>(v), take2, v);
+            v = fma(dpp_f64<DPP_ROW_SHR4>(v), take4, v);
+            if (write)
+                __hip_atomic_fetch_add(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        add_sum(&b->we, run.we);
+        add_sum(&b->xi, run.xi);
+        add_sum(&b->rp, run.rp);
+        add_sum(&b->rt, run.rt);
+        add_sum(&b->z, run.z);
+        uint32_t n = run.n;
+        const uint32_t n1 = (uint32_t)dpp_int<DPP_ROW_SHR1>((int)n);
+        n += head ? 0u : n1;
+        const uint32_t n2 = (uint32_t)dpp_int<DPP_ROW_SHR2>((int)n);
+        n += head2 ? 0u : n2;
+        const uint32_t n4 = (uint32_t)dpp_int<DPP_ROW_SHR4>((int)n);
+        n += head4 ? 0u : n4;
+        if (write)
+            __hip_atomic_fetch_add(&b->nb, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    // One step of the inclusive segmented sum: a lane whose segment head lies within the
-    // last CTRL lanes keeps its value, the others add the value of lane l - CTRL.
-    template <int CTRL>
-    __device__ static void segment_step(int &head, double &we, double &xi, double &rp,
-                                        double &rt, double &z, uint32_t &n) {
-        const double g = head ? 0.0 : 1.0;
-        const int h = dpp_int<CTRL>(head);
-        we = fma(dpp_f64<CTRL>(we), g, we);
-        xi = fma(dpp_f64<CTRL>(xi), g, xi);
-        rp = fma(dpp_f64<CTRL>(rp), g, rp);
-        rt = fma(dpp_f64<CTRL>(rt), g, rt);
-        z = fma(dpp_f64<CTRL>(z), g, z);
-        const uint32_t m = (uint32_t)dpp_int<CTRL>((int)n);
-        n += head ? 0u : m;
-        head |= h;
-    }
-    __device__ bool any(bool v) const { return __ballot(v) != 0; }
+    __device__ bool any(bool v) const { return __builtin_amdgcn_ballot_w64(v) != 0; }
     // Keeps the run's sums where the walk computes them, at the top of the pass: left to
     // itself the compiler moves them to the flush, after the prefix record of the run's
     // start has been replaced, and keeps two copies of that record around the pass.
@@ -347,9 +372,9 @@ struct DeviceWalkMem {
                                __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     __device__ void count_probe() { ++probes; }
-    __device__ void count_run(uint32_t n) {
-        ++runs;
-        cover += n;
+    __device__ void count_run(bool closed, uint32_t n) {
+        runs += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(closed));
+        cover += closed ? n : 0u;
     }
 };
 
@@ -461,15 +486,15 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
             // below.
             const double spc_r = uniform_f64(F.spc[b].x);
             const double spc_d = uniform_f64(F.spc[b].y);
-            const double cp = cos_half * C.inv_p;
-            const double st = sin_half * C.inv_t;
+            const double cp = uniform_f64(cos_half * C.inv_p);
+            const double st = uniform_f64(sin_half * C.inv_t);
             double q0 = 1.0;
             if (j_hi - j_lo >= 2) {
                 const double span = (uniform_f64(F.rd[ob + j_hi - 1].x) -
                                      uniform_f64(F.rd[ob + j_lo].x)) * cp;
                 if (span > 0) q0 = (double)(j_hi - 1 - j_lo) / span;
             }
-            if (walk_task(C, spc_r, spc_d, cp, st, q0)) {
+            if (j_hi < WALK_MAX_PIXELS && walk_task(C, spc_r, spc_d, cp, st, q0)) {
                 WalkTask T;
                 T.cos_half = cos_half;
                 T.sin_half = sin_half;
@@ -479,9 +504,11 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
                 T.dc = uniform_f64(F.rd[ob + (lb >> 1)].y);
                 T.j_lo = j_lo;
                 T.j_hi = j_hi;
-                T.q0 = q0;
-                DeviceWalkMem mem{F.rd + ob, F.pre + (ob + b), F.w + ob, F.z + ob, F.dw + ob,
-                                  hist, lds_stats, 0u, 0u, 0u};
+                T.q0 = uniform_f64(q0);
+                const PrefixPair *pre = F.pre + PREFIX_PLANES * (ob + b);
+                DeviceWalkMem mem{F.rd + ob, {pre, pre + (lb + 1), pre + 2 * ((int64_t)lb + 1)},
+                                  F.w + ob, F.z + ob, F.dw + ob,
+                                  hist, lds_stats, &C_lds, 0u, 0u, 0u};
                 WalkLane L{r1, d1, zh1, w1, dw1};
                 if constexpr (CUTS) {
                     T.shp = shp;
@@ -509,9 +536,13 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
                         }
                     }
                 }
-                walk_lane<XCORR, CUTS>(C, T, L, mem, active);
+                // what the loop reads of C, held in scalar registers (left to itself the
+                // compiler loads them again in every pass)
+                XiConst K = C;
+                asm volatile("" : "+s"(K.np), "+s"(K.nt), "+s"(K.fast_p), "+s"(K.fast_t));
+                walk_lane<XCORR, CUTS>(K, T, L, mem, active);
                 cnt.visit += mem.cover;
-                cnt.runs += mem.runs;
+                cnt.runs += lane == 0 ? mem.runs : 0u;
                 cnt.probes += mem.probes;
                 ++n_walk;
                 // wave passes of the walk: the lanes' loops run until the longest is done
@@ -733,9 +764,53 @@ __device__ __forceinline__ uint64_t flush_row(const XiConst &C, LocalBin *hist, 
     return moved;
 }
 
+// Counters of a wave into the workgroup's.
+__device__ __forceinline__ void add_counters(unsigned long long *stats, uint64_t visit,
+                                             uint64_t edge, uint64_t overflow, uint64_t runs,
+                                             uint64_t probes, uint64_t steps, uint64_t tasks,
+                                             uint64_t empty, uint64_t walk, int lane) {
+    // one addition, by the lane of the counter's number
+    uint64_t v = 0;
+    v = lane == XI_STAT_VISITED ? visit : v;
+    v = lane == XI_STAT_EDGE ? edge : v;
+    v = lane == XI_STAT_OVERFLOW ? overflow : v;
+    v = lane == XI_STAT_STEPS ? steps : v;
+    v = lane == XI_STAT_TASKS ? tasks : v;
+    v = lane == XI_STAT_EMPTY_TASKS ? empty : v;
+    v = lane == XI_STAT_RUNS ? runs : v;
+    v = lane == XI_STAT_PROBES ? probes : v;
+    v = lane == XI_STAT_WALK_TASKS ? walk : v;
+    if (v) atomicAdd(&stats[lane], (unsigned long long)v);
+}
+
+// The pair kernel's arguments as they lie in its argument segment.
+struct XiArgs {
+    XiConst C;
+    ForestView F;
+    PairView P;
+    GroupView G;
+    XiOut O;
+};
+
+// The arguments through the segment's address, as loads that the compiler does not move to the
+// kernel's start: the run walk needs the scalar registers that the pointers of the whole kernel
+// would hold through its loop (101 spilled without this, 28 with it).  The pair loop has enough
+// and is 1.5 % faster with the arguments by value.
+__device__ __forceinline__ const XiArgs &kernel_args() {
+    typedef const __attribute__((address_space(4))) XiArgs *Segment;
+    Segment s = (Segment)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(s));
+    return *(const XiArgs *)s;
+}
+
 template <int MODE, bool XCORR, bool GENERAL, bool CUTS, bool LDS_HIST, bool WALK>
 __global__ void __launch_bounds__(XI_BLOCK)
-xi_kernel(XiConst C, ForestView F, PairView P, GroupView G, XiOut O) {
+xi_kernel(XiArgs by_value) {
+    auto args = [&]() -> const XiArgs & {
+        if constexpr (WALK) return kernel_args();
+        return by_value;
+    };
+    const XiConst &C = args().C;
     extern __shared__ __align__(16) unsigned char smem[];
     const int nbp = hist_rows(C) * C.ntp;  // padded LDS histogram
     LocalBin *hist = (LocalBin *)reinterpret_cast<LdsBin *>(smem);
@@ -766,22 +841,25 @@ xi_kernel(XiConst C, ForestView F, PairView P, GroupView G, XiOut O) {
         }
     }
     if (tid < XI_NSTATS) s_stats[tid] = 0;
-    if (tid == 0) s_const = C;  // published by the first __syncthreads of the group loop
+    if (tid == 0) s_const = args().C;  // published by the first __syncthreads of the group loop
 
-    LaneCounters cnt = {0, 0, 0, 0, 0, 0};
+    LaneCounters cnt = {0, 0, 0, 0, 0, 0};   // (the run walk's kernel: of one task)
     uint64_t accepted = 0;  // LDS_HIST: pairs moved from the histogram to HBM
     uint64_t n_steps = 0, n_tasks = 0, n_empty_tasks = 0, n_walk = 0;  // wave-uniform
     int current_row = -1;
 
     for (;;) {
         __syncthreads();
-        if (tid == 0) s_group = (int64_t)atomicAdd(O.queue, 1ull);
+        const XiArgs &A = args();
+        const GroupView &G = A.G;
+        const PairView &P = A.P;
+        if (tid == 0) s_group = (int64_t)atomicAdd(A.O.queue, 1ull);
         __syncthreads();
         const int64_t g = s_group;
         if (g >= G.count) break;
         const int row = G.row[g];
         if (LDS_HIST && row != current_row && current_row >= 0)
-            accepted += flush_row(C, hist, O.bins + (int64_t)current_row * C.nb, tid);
+            accepted += flush_row(A.C, hist, A.O.bins + (int64_t)current_row * A.C.nb, tid);
         current_row = row;
         const int64_t p0 = G.begin[g];
         const int npairs = (int)(G.begin[g + 1] - p0);
@@ -824,42 +902,43 @@ xi_kernel(XiConst C, ForestView F, PairView P, GroupView G, XiOut O) {
             const int chunk = uniform_int(s_first[q] + t - s_prefix[q]);
             const uint64_t steps_before = n_steps;
             if (LDS_HIST) {
-                xi_task<MODE, XCORR, GENERAL, CUTS, true, WALK>(C, s_const, F, P, p0 + q, chunk, lane, hist,
-                                                    tile, tile_x, cnt, lds_stats, n_steps, n_walk);
+                const XiArgs &T = args();
+                xi_task<MODE, XCORR, GENERAL, CUTS, true, WALK>(T.C, s_const, T.F, T.P, p0 + q,
+                                                    chunk, lane, hist, tile, tile_x, cnt,
+                                                    lds_stats, n_steps, n_walk);
             } else {
-                xi_task<MODE, XCORR, GENERAL, false, false, false>(C, s_const, F, P, p0 + q, chunk, lane,
-                                                     O.bins + (int64_t)row * C.nb, tile, tile_x,
-                                                     cnt, lds_stats, n_steps, n_walk);
+                xi_task<MODE, XCORR, GENERAL, false, false, false>(A.C, s_const, A.F, P, p0 + q,
+                                                     chunk, lane, A.O.bins + (int64_t)row * A.C.nb,
+                                                     tile, tile_x, cnt, lds_stats, n_steps,
+                                                     n_walk);
             }
             ++n_tasks;
             if (n_steps == steps_before) ++n_empty_tasks;
+            if (WALK) {
+                // the task's counters to LDS, so that no register holds them through the walk
+                add_counters(s_stats, wave_sum_small(cnt.visit), wave_sum_small(cnt.edge),
+                             wave_sum_small(cnt.overflow), wave_sum_small(cnt.runs),
+                             wave_sum_small(cnt.probes), n_steps, n_tasks, n_empty_tasks, n_walk,
+                             lane);
+                cnt = LaneCounters{0, 0, 0, 0, 0, 0};
+                n_steps = n_tasks = n_empty_tasks = n_walk = 0;
+            }
         }
     }
     // final flush (all waves are past the last __syncthreads of the loop)
+    const XiArgs &A = args();
     if (LDS_HIST && current_row >= 0)
-        accepted += flush_row(C, hist, O.bins + (int64_t)current_row * C.nb, tid);
+        accepted += flush_row(A.C, hist, A.O.bins + (int64_t)current_row * A.C.nb, tid);
     if (!LDS_HIST) accepted = cnt.accept;
     // statistics: lane values -> wave sums -> workgroup -> HBM
-    const uint64_t v_visit = wave_sum_u64(cnt.visit);
-    const uint64_t v_edge = wave_sum_u64(cnt.edge);
-    const uint64_t v_over = wave_sum_u64(cnt.overflow);
     const uint64_t v_accept = wave_sum_u64(accepted);
-    const uint64_t v_runs = wave_sum_u64(cnt.runs);
-    const uint64_t v_probes = wave_sum_u64(cnt.probes);
-    if (lane == 0) {
-        atomicAdd(&s_stats[XI_STAT_VISITED], (unsigned long long)v_visit);
-        atomicAdd(&s_stats[XI_STAT_EDGE], (unsigned long long)v_edge);
-        atomicAdd(&s_stats[XI_STAT_OVERFLOW], (unsigned long long)v_over);
-        atomicAdd(&s_stats[XI_STAT_STEPS], (unsigned long long)n_steps);
-        atomicAdd(&s_stats[XI_STAT_ACCEPTED], (unsigned long long)v_accept);
-        atomicAdd(&s_stats[XI_STAT_TASKS], (unsigned long long)n_tasks);
-        atomicAdd(&s_stats[XI_STAT_EMPTY_TASKS], (unsigned long long)n_empty_tasks);
-        atomicAdd(&s_stats[XI_STAT_RUNS], (unsigned long long)v_runs);
-        atomicAdd(&s_stats[XI_STAT_PROBES], (unsigned long long)v_probes);
-        atomicAdd(&s_stats[XI_STAT_WALK_TASKS], (unsigned long long)n_walk);
-    }
+    if (lane == 0) atomicAdd(&s_stats[XI_STAT_ACCEPTED], (unsigned long long)v_accept);
+    if (!WALK)
+        add_counters(s_stats, wave_sum_u64(cnt.visit), wave_sum_u64(cnt.edge),
+                     wave_sum_u64(cnt.overflow), wave_sum_u64(cnt.runs),
+                     wave_sum_u64(cnt.probes), n_steps, n_tasks, n_empty_tasks, n_walk, lane);
     __syncthreads();
-    if (tid < XI_NSTATS) atomicAdd(O.stats + tid, s_stats[tid]);
+    if (tid < XI_NSTATS) atomicAdd(A.O.stats + tid, s_stats[tid]);
 }
 
 // Work-queue head and counters of picca_xi_execute_noalloc: one copy per GPU, held until
@@ -980,7 +1059,7 @@ static hipError_t launch_xi_t(const XiConst &C, const ForestView &F, const PairV
     hipError_t err = hipFuncSetAttribute((const void *)kern,
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) return err;
-    kern<<<dim3(grid), dim3(XI_BLOCK), lds, stream>>>(C, F, P, G, O);
+    kern<<<dim3(grid), dim3(XI_BLOCK), lds, stream>>>(XiArgs{C, F, P, G, O});
     return hipGetLastError();
 }
 

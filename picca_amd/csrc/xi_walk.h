@@ -43,11 +43,24 @@ namespace picca {
 // Entry k of a forest's prefix sums covers its pixels [0, k): pixels with w != 0, and the
 // sums of w, w * delta, w * (r_comov - r_c), w * (dist_m - d_c) and w * z, where r_c and
 // d_c are r_comov and dist_m of the forest's pixel L / 2.  A forest of L pixels has L + 1
-// entries, starting at entry offsets[b] + b.
-struct alignas(16) PrefixRecord {
+// entries.
+struct PrefixRecord {
     double c, w, x, r, d, z;
 };
-static_assert(sizeof(PrefixRecord) == 48, "PrefixRecord layout");
+
+// The entries in memory: per forest three planes of L + 1 pairs, (c, w), (x, r) and (d, z); the
+// forests' blocks follow each other, so forest b's starts at pair 3 (offsets[b] + b).  The
+// lanes of a wave read entries a pixel or a few apart: in planes 16 of them lie in two or three
+// cache lines, as records of 48 bytes in six, and the walk reads at the L1 cache's line rate.
+struct alignas(16) PrefixPair {
+    double a, b;
+};
+constexpr int PREFIX_PLANES = 3;
+
+PICCA_HD inline PrefixRecord prefix_entry(const PrefixPair &cw, const PrefixPair &xr,
+                                          const PrefixPair &dz) {
+    return PrefixRecord{cw.a, cw.b, xr.a, xr.b, dz.a, dz.b};
+}
 
 // Host side: the prefix entries of one forest of n pixels (n + 1 entries) and the smallest
 // step of r_comov and of dist_m between consecutive pixels (-1 unless both increase
@@ -55,11 +68,16 @@ static_assert(sizeof(PrefixRecord) == 48, "PrefixRecord layout");
 // the same products the pair loops use.
 inline void build_walk_forest(const double *r, const double *d, const double *z,
                               const double *w, const double *dw, int64_t n,
-                              PrefixRecord *pre, double &spc_r, double &spc_d) {
+                              PrefixPair *pre, double &spc_r, double &spc_d) {
     const double rc = n > 0 ? r[n / 2] : 0.0;
     const double dc = n > 0 ? d[n / 2] : 0.0;
     PrefixRecord acc = {0, 0, 0, 0, 0, 0};
-    pre[0] = acc;
+    auto store = [&](int64_t k) {
+        pre[k] = PrefixPair{acc.c, acc.w};
+        pre[n + 1 + k] = PrefixPair{acc.x, acc.r};
+        pre[2 * (n + 1) + k] = PrefixPair{acc.d, acc.z};
+    };
+    store(0);
     spc_r = 1e300;
     spc_d = 1e300;
     for (int64_t k = 0; k < n; ++k) {
@@ -69,7 +87,7 @@ inline void build_walk_forest(const double *r, const double *d, const double *z,
         acc.r += w[k] * (r[k] - rc);
         acc.d += w[k] * (d[k] - dc);
         acc.z += w[k] * z[k];
-        pre[k + 1] = acc;
+        store(k + 1);
         if (k > 0) {
             const double sr = r[k] - r[k - 1];
             const double sd = d[k] - d[k - 1];
@@ -137,7 +155,8 @@ PICCA_HD inline WalkExact walk_exact(const XiConst &C, double r1, double d1, dou
     const double t_trans = r_trans / C.rtmax * C.nt_d;
     const double f_par = floor(t_par);
     const double f_trans = floor(t_trans);
-    const double row = fmin(f_par, C.np_d);
+    // (no fmin: it would quiet the constants once per call, also in passes without a call)
+    const double row = f_par < C.np_d ? f_par : C.np_d;
     if (XC) {
         e.m = (int32_t)(-fmax(row, -1.0) - 1.0);
         const double own = fmin(fmax(row, 0.0), C.np_d - 1.0);
@@ -146,7 +165,7 @@ PICCA_HD inline WalkExact walk_exact(const XiConst &C, double r1, double d1, dou
         e.m = (int32_t)(rps > 0 ? -row - 1.0 : row);
         e.mine = true;
     }
-    e.c = (int32_t)fmin(f_trans, C.nt_d);
+    e.c = (int32_t)(f_trans < C.nt_d ? f_trans : C.nt_d);
     const bool out_p = XC ? (r_par >= C.rpmax) | (r_par < C.rpmin) : r_par >= C.rpmax;
     const bool out_t = r_trans >= C.rtmax;
     const bool out = out_p | out_t;
@@ -203,6 +222,15 @@ PICCA_HD inline void walk_special(const XiConst &C, const WalkTask &T, const Wal
     }
 }
 
+// row * len + col of a histogram, whose rows and columns are below 2^23
+PICCA_HD inline int walk_bin(int row, int len, int col) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __mul24(row, len) + col;   // the full multiply takes four times as long
+#else
+    return row * len + col;
+#endif
+}
+
 // Histogram addition of the run [j, jn) of key (m, c): prefix differences times the lane's
 // pixel.  False for an empty run.  No branch, and finite for any finite state.
 struct RunSums {
@@ -222,16 +250,16 @@ PICCA_HD inline bool walk_run_sums(const XiConst &C, const WalkTask &T, const Wa
     const double dd = pe.d - ps.d;
     const double dz = pe.z - ps.z;
     // sum over the run of w2 (r2 - r1) and w2 (d1 + d2), from the centred sums
-    const double s_r = dr - (L.r1 - T.rc) * dw;
-    const double s_d = (L.d1 + T.dc) * dw + dd;
+    const double s_r = fma(T.rc - L.r1, dw, dr);
+    const double s_d = fma(L.d1 + T.dc, dw, dd);
     const bool up = !XC && m >= 0;   // r_par counted as r2 - r1
-    o.bin = (up ? m : XC ? -m - 1 - C.row0 : -m - 1) * C.ntp + c;
+    o.bin = walk_bin(up ? m : XC ? -m - 1 - C.row0 : -m - 1, C.ntp, c);
     o.we = L.w1 * dw;
     o.xi = L.dw1 * dx;
     o.rp = T.cos_half * (L.w1 * (up ? s_r : -s_r));
     o.rt = T.sin_half * (L.w1 * s_d);
-    o.z = L.w1 * (L.zh1 * dw + 0.5 * dz);
-    o.n = (uint32_t)fmax(n, 0.0);
+    o.z = L.w1 * fma(L.zh1, dw, 0.5 * dz);
+    o.n = (uint32_t)(int32_t)n;
     return n > 0;
 }
 
@@ -269,8 +297,9 @@ PICCA_HD inline void walk_key_from(const XiConst &C, int m, int c, double a, dou
     const int fm = (int)floor(a) + (m + 1);
     const int fc = (int)floor(b) + (c + 1);
     const int top = XC ? 0 : C.np;
-    mp = fm < -C.np - 1 ? -C.np - 1 : (fm > top ? top : fm);
-    cp = fc > C.nt ? C.nt : fc;
+    const int below = fm < top ? fm : top;
+    mp = below > -C.np - 1 ? below : -C.np - 1;
+    cp = fc < C.nt ? fc : C.nt;
 }
 
 // Whether a task takes the run walk: delta2 increases strictly with consecutive pixels more
@@ -332,12 +361,12 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
     // Before the first run opens the key is (-1, -1), which no pixel has (r_trans >= 0
     // here), so the thresholds give each pixel's own coordinates.
     int m = -1, c = -1;
-    double Ka = r1cp, Kb = -d1st;
+    double nKa = -r1cp, nKb = d1st;   // -Ka, -Kb
     int j = CUTS ? L.j_lo : T.j_lo;
     bool starting = true;
     typename Acc::Prefix ps = {};
-    int lo = j, hi = j_hi, g = j, misses = 0, step = 1;
-    bool near_lo = false;
+    int lo = j, hi = j_hi, g = j, step = 1;
+    bool near_lo = false, missed = false;
     // the pass's probes: pixels pa and pb and the prefix entry at pb, loaded at the end of
     // the previous pass so that the loads overlap that pass's histogram additions
     int pa = j, pb = j;
@@ -352,11 +381,11 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
         typename Acc::Sums run;
         const bool nonempty = Acc::sums(C, T, L, m, c, ps, pg, run);
         mem.pin(run);
-        bool on = false;
+        bool on = false, close = false;
         if (alive) {
             mem.count_probe();
-            const double aA = fma(ra, T.cp, -Ka), bA = fma(da, T.st, -Kb);
-            const double aB = fma(rb, T.cp, -Ka), bB = fma(db, T.st, -Kb);
+            const double aA = fma(ra, T.cp, nKa), bA = fma(da, T.st, nKb);
+            const double aB = fma(rb, T.cp, nKa), bB = fma(db, T.st, nKb);
             // pixel pb: within the margin of any bin edge; pixel pa: of the run's upper edges
             const bool nearB =
                 (fabs(aB - rint(aB)) < C.fast_p) || (fabs(bB - rint(bB)) < C.fast_t);
@@ -364,44 +393,44 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
             int mB, cB;
             walk_key_from<XC>(C, m, c, aB, bB, mB, cB);
             if (nearB) {
-                const WalkExact e = walk_exact<XC>(C, L.r1, L.d1, rb, db, T.cos_half, T.sin_half);
+                const WalkExact e =
+                    walk_exact<XC>(mem.consts(C), L.r1, L.d1, rb, db, T.cos_half, T.sin_half);
                 mB = e.m;
                 cB = e.c;
             }
-            bool inA = (aA < 0) && (bA < 0);
-            if (nearA && !starting) {
-                const WalkExact e = walk_exact<XC>(C, L.r1, L.d1, ra, da, T.cos_half, T.sin_half);
+            bool inA = (aA < 0) & (bA < 0);
+            if (nearA & !starting) {
+                const WalkExact e =
+                    walk_exact<XC>(mem.consts(C), L.r1, L.d1, ra, da, T.cos_half, T.sin_half);
                 inA = (e.m == m) && (e.c == c);
             }
             // outcome of the pass
             const bool has1 = g - 1 > lo;    // pa is not yet known to have the run's key
             const bool has2 = g < j_hi;      // pb lies inside the window
-            const bool same1 = !has1 || inA;
-            const bool same2 = has2 && (mB == m) && (cB == c);
-            const bool miss = !starting && !same1;           // the run ends at g - 1 or before
-            const bool gallop = !starting && same1 && same2; // the run goes on past g
-            const bool close = !starting && same1 && !same2; // the run is [j, g)
-            const bool open = starting || (close && has2);   // a run starts at pb
-            const bool terminal = open && walk_terminal<XC>(C, mB, cB);
-            const bool done = (close && !has2) || terminal;
-            const bool special_last = close && (has1 ? nearA : near_lo) && g - 1 > j;
+            const bool same1 = !has1 | inA;
+            const bool same2 = has2 & (mB == m) & (cB == c);
+            const bool miss = !starting & !same1;            // the run ends at g - 1 or before
+            const bool gallop = !starting & same1 & same2;   // the run goes on past g
+            close = !starting & same1 & !same2;              // the run is [j, g)
+            const bool open = starting | (close & has2);     // a run starts at pb
+            const bool terminal = open & walk_terminal<XC>(C, mB, cB);
+            const bool done = (close & !has2) | terminal;
+            const bool special_last =
+                close & ((has1 & nearA) | (!has1 & near_lo)) & (g - 1 > j);
             const int p_last = g - 1;
-            const bool special_first = open && nearB;
+            const bool special_first = open & nearB;
             const int p_first = pb;
             // the closing run [j, g): prefix entries ps and pg (the entry at g)
-            if (close) {
-                mem.count_run(run.n);
-                on = nonempty && m >= (XC ? -(C.row0 + C.rows) : -C.np);
-                if constexpr (CUTS && !XC) on = on && !(T.shp && (m == 0 || m == -1));
-                if constexpr (Acc::RUNS) mem.closed(on, j, g, c);
-            }
+            on = close & nonempty & (m >= (XC ? -(C.row0 + C.rows) : -C.np));
+            if constexpr (CUTS && !XC) on = on & !(T.shp & ((m == 0) | (m == -1)));
+            if constexpr (Acc::RUNS) mem.closed(on, j, g, c);
             // next state
-            const int g_miss = misses == 0 ? g - 1 : lo + 1 + ((g - 1 - lo) >> 1);
+            const int g_miss = missed ? lo + 1 + ((g - 1 - lo) >> 1) : g - 1;
             const int g_gallop = g + step < hi ? g + step : hi;
             if (miss) {
                 hi = g - 1;
                 g = g_miss;
-                ++misses;
+                missed = true;
             }
             if (gallop) {
                 lo = g;
@@ -418,25 +447,26 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
                 c = cB;
                 ps = pg;
                 starting = false;
-                Ka = r1cp + (double)(m + 1);
-                Kb = (double)(c + 1) - d1st;
+                nKa = -r1cp - (double)(m + 1);
+                nKb = d1st - (double)(c + 1);
                 lo = j;
                 hi = j_hi;
                 near_lo = nearB;
-                misses = 0;
+                missed = false;
                 step = 1;
                 // pixels to the run's upper r_par edge
-                const double ahead = ceil(-fma(rb, T.cp, -Ka) * q);
+                const double ahead = ceil(-fma(rb, T.cp, nKa) * q);
                 g = j + (int)fmin(fmax(ahead, 1.0), (double)(j_hi - j));
             }
             if (!done) {
                 pa = g - 1;
                 pb = g;
             }
-            if (special_last) walk_special<XC, CUTS>(C, T, L, mem, p_last);
-            if (special_first) walk_special<XC, CUTS>(C, T, L, mem, p_first);
+            if (special_last) walk_special<XC, CUTS>(mem.consts(C), T, L, mem, p_last);
+            if (special_first) walk_special<XC, CUTS>(mem.consts(C), T, L, mem, p_first);
             if (done) alive = false;
         }
+        mem.count_run(close, run.n);
         // the next pass's probes, issued before the histogram additions (a lane that is done
         // reloads its last probes, which lie inside the window)
         const bool more = mem.any(alive);

@@ -34,7 +34,7 @@ struct Hist {
 // outside them is counted and answered with a harmless value.
 struct HostMem {
     const double *rp_, *dp_, *wp_, *zp_, *dwp_;
-    const PrefixRecord *pre_;
+    const picca::PrefixPair *pre_;
     int64_t lb;
     Hist *hist;
     int64_t *stats;
@@ -56,7 +56,7 @@ struct HostMem {
     }
     PrefixRecord prefix(int p) {
         if (bad(p, lb + 1)) return PrefixRecord{0, 0, 0, 0, 0, 0};
-        return pre_[p];
+        return picca::prefix_entry(pre_[p], pre_[lb + 1 + p], pre_[2 * (lb + 1) + p]);
     }
     double w(int p) { return bad(p, lb) ? 0.0 : wp_[p]; }
     double z(int p) { return bad(p, lb) ? 0.0 : zp_[p]; }
@@ -77,11 +77,13 @@ struct HostMem {
         if (on) add(r.bin, r.we, r.xi, r.rp, r.rt, r.z, r.n);
     }
     bool any(bool v) { return v; }
+    const picca::XiConst &consts(const picca::XiConst &C) { return C; }
     void pin(picca::RunSums &) {}
     void count_edge() { ++stats[ST_EDGE]; }
     void count_overflow() { ++stats[ST_OVER]; }
     void count_probe() { ++stats[ST_PROBES]; }
-    void count_run(uint32_t n) {
+    void count_run(bool closed, uint32_t n) {
+        if (!closed) return;
         ++stats[ST_RUNS];
         stats[ST_COVER] += (int64_t)n;
     }
@@ -162,13 +164,13 @@ int walk_launch(const picca_cf_params *params, int64_t num_forests, const int64_
 
     std::vector<double> dw((size_t)npix);
     for (int64_t k = 0; k < npix; ++k) dw[k] = delta[k] * w[k];
-    std::vector<PrefixRecord> pre((size_t)(npix + num_forests));
+    std::vector<picca::PrefixPair> pre(picca::PREFIX_PLANES * (size_t)(npix + num_forests));
     std::vector<double> spc_r((size_t)num_forests), spc_d((size_t)num_forests);
     std::vector<uint8_t> mono((size_t)num_forests);
     for (int64_t b = 0; b < num_forests; ++b) {
         const int64_t o = off[b], n = off[b + 1] - off[b];
         picca::build_walk_forest(r + o, d + o, z + o, w + o, dw.data() + o, n,
-                                 pre.data() + o + b, spc_r[b], spc_d[b]);
+                                 pre.data() + picca::PREFIX_PLANES * (o + b), spc_r[b], spc_d[b]);
         mono[b] = (uint8_t)((monotone(r + o, n) ? 1 : 0) | (monotone(d + o, n) ? 2 : 0) |
                             (monotone(z + o, n) ? 4 : 0));
     }
@@ -266,7 +268,7 @@ int walk_launch(const picca_cf_params *params, int64_t num_forests, const int64_
                 mem.wp_ = w + ob;
                 mem.zp_ = z + ob;
                 mem.dwp_ = dw.data() + ob;
-                mem.pre_ = pre.data() + ob + b;
+                mem.pre_ = pre.data() + picca::PREFIX_PLANES * (ob + b);
                 mem.lb = lb;
                 mem.hist = &h;
                 mem.stats = stats;
