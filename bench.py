@@ -295,7 +295,7 @@ def bench_xi(args):
                 "flops_per_launch": flops,
                 "executed_tflops": executed / (kernel_ms / 1e3) / 1e12,
                 # the run-walk instance runs whenever any task took the walk
-                "kernel": "picca::xi_kernel<0,false,false,true,%s>"
+                "kernel": "picca::xi_kernel<0,false,false,false,true,%s>"
                           % ("true" if rep["walk_tasks"] > 0 else "false"),
                 "kernel_ms": kernel_ms,
                 "hbm_gbs_at_traffic": (args.traffic_bytes / (kernel_ms / 1e3) / 1e9
@@ -493,7 +493,7 @@ def bench_dmat(args):
                      "achieved": rep["mfma_flops"] / (rep["fill_ms"] * 1e-3) / 1e12,
                      "frac": rep["mfma_flops"] / (rep["fill_ms"] * 1e-3) / 1e12
                      / FP64_VALU_PEAK_TFLOPS, "traffic": None,
-                     "kernel": "picca::dmat_fill_kernel<false>", "kernel_ms": rep["fill_ms"],
+                     "kernel": "picca::dmat_band_fill_kernel", "kernel_ms": rep["fill_ms"],
                      "pass_kernel_ms": rep["pass_ms"], "batches": rep["batches"],
                      "mfma_flops": rep["mfma_flops"]},
         "cpu_baseline": None,
