@@ -33,7 +33,7 @@
 // each other (stepping from pixel to pixel or from run to run along the partner is a serial
 // chain: 88 ms on 21k pairs of the 0.8 A grid where this takes 61 ms), and the barriers come
 // every 16 pixels.  On those pairs (2500 forests, 50 x 50 data and 100 x 50 model bins) the
-// call takes 114 ms against 350 ms, the fill 61 ms against 264 ms, the pass 18 ms against 83 ms.
+// call takes 88 ms against 350 ms, the fill 61 ms against 264 ms, the pass 15 ms against 83 ms.
 //
 // A pair whose bins do not follow the runs (an r_trans or r_par that rounds up to the range's
 // end, which the reference writes into the next row or past the end) is left to
@@ -129,26 +129,40 @@ struct BandPassMem {
     __device__ double z(int p) const { return zp[p]; }
     __device__ double dw(int) const { return 0.0; }
     __device__ void add(int, double, double, double, double, double, uint32_t) { *special = 1; }
+    // Adds the runs that the wave's lanes closed in one pass (every lane calls it).  As in the xi
+    // kernel the lanes of a group of four that closed runs of one bin are summed first: eleven
+    // FP64 atomics per lane, many of them on one address, bound the pass (21k pairs of the 0.8 A
+    // grid: 15.0 ms, one lane at a time 17.6 ms).
     __device__ void flush(bool on, const DmatSums &o) {
-        if (!on) return;
-        n_in += o.n;
         const int k = o.bin - base;
-        if ((unsigned)k >= (unsigned)stride) {   // outside the rows that the host bounded
+        if (on) n_in += o.n;
+        if (on && (unsigned)k >= (unsigned)stride) {   // outside the rows that the host bounded
             *special = 1;
-            return;
+            on = false;
         }
-        double *b = acc + k;
-        lds_add(b, o.s0);
-        lds_add(b + stride, o.sj);
-        lds_add(b + 2 * stride, l1 * o.s0);
-        lds_add(b + 3 * stride, l1 * o.sj);
-        lds_add(b + 4 * stride, o.z0);
-        lds_add(b + 5 * stride, o.zj);
-        lds_add(b + 6 * stride, l1 * o.z0);
-        lds_add(b + 7 * stride, l1 * o.zj);
-        lds_add(b + 8 * stride, o.rp);
-        lds_add(b + 9 * stride, o.rt);
-        lds_add(b + 10 * stride, o.z);
+        const int key = on ? k + 1 : 0;
+        const int gl = __lane_id() & 3;
+        const int head = (key != dpp_int<DPP_ROW_SHR1>(key)) || gl == 0;
+        const int head2 = head | dpp_int<DPP_ROW_SHR1>(head);
+        const bool write = on && ((key != dpp_int<DPP_ROW_SHL1>(key)) || gl == 3);
+        const double take1 = head ? 0.0 : 1.0, take2 = head2 ? 0.0 : 1.0;
+        double *b = acc + (on ? k : 0);
+        auto add_sum = [&](int c, double v) {
+            v = fma(dpp_f64<DPP_ROW_SHR1>(v), take1, v);
+            v = fma(dpp_f64<DPP_ROW_SHR2>(v), take2, v);
+            if (write) lds_add(b + c * stride, v);
+        };
+        add_sum(0, o.s0);
+        add_sum(1, o.sj);
+        add_sum(2, l1 * o.s0);
+        add_sum(3, l1 * o.sj);
+        add_sum(4, o.z0);
+        add_sum(5, o.zj);
+        add_sum(6, l1 * o.z0);
+        add_sum(7, l1 * o.zj);
+        add_sum(8, o.rp);
+        add_sum(9, o.rt);
+        add_sum(10, o.z);
     }
     __device__ void note() {
         if (row < 0) return;
