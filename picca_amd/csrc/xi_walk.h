@@ -62,22 +62,18 @@ PICCA_HD inline PrefixRecord prefix_entry(const PrefixPair &cw, const PrefixPair
     return PrefixRecord{cw.a, cw.b, xr.a, xr.b, dz.a, dz.b};
 }
 
-// Host side: the prefix entries of one forest of n pixels (n + 1 entries) and the smallest
-// step of r_comov and of dist_m between consecutive pixels (-1 unless both increase
-// strictly; a forest of fewer than two pixels has no step and gets +1e300).  dw = delta * w,
-// the same products the pair loops use.
-inline void build_walk_forest(const double *r, const double *d, const double *z,
-                              const double *w, const double *dw, int64_t n,
-                              PrefixPair *pre, double &spc_r, double &spc_d) {
+// Host side: the prefix entries of one forest of n pixels, store(k, entry) for k = 0 .. n, and
+// the smallest step of r_comov and of dist_m between consecutive pixels (-1 unless both
+// increase strictly; a forest of fewer than two pixels has no step and gets +1e300).  dw =
+// delta * w, the same products the pair loops use.
+template <class Store>
+inline void walk_forest_entries(const double *r, const double *d, const double *z,
+                                const double *w, const double *dw, int64_t n,
+                                const Store &store, double &spc_r, double &spc_d) {
     const double rc = n > 0 ? r[n / 2] : 0.0;
     const double dc = n > 0 ? d[n / 2] : 0.0;
     PrefixRecord acc = {0, 0, 0, 0, 0, 0};
-    auto store = [&](int64_t k) {
-        pre[k] = PrefixPair{acc.c, acc.w};
-        pre[n + 1 + k] = PrefixPair{acc.x, acc.r};
-        pre[2 * (n + 1) + k] = PrefixPair{acc.d, acc.z};
-    };
-    store(0);
+    store(0, acc);
     spc_r = 1e300;
     spc_d = 1e300;
     for (int64_t k = 0; k < n; ++k) {
@@ -87,7 +83,7 @@ inline void build_walk_forest(const double *r, const double *d, const double *z,
         acc.r += w[k] * (r[k] - rc);
         acc.d += w[k] * (d[k] - dc);
         acc.z += w[k] * z[k];
-        store(k + 1);
+        store(k + 1, acc);
         if (k > 0) {
             const double sr = r[k] - r[k - 1];
             const double sd = d[k] - d[k - 1];
@@ -99,6 +95,24 @@ inline void build_walk_forest(const double *r, const double *d, const double *z,
         spc_r = -1.0;
         spc_d = -1.0;
     }
+}
+
+// The n + 1 entries as records, and as the kernel's planes.
+inline void build_walk_forest(const double *r, const double *d, const double *z,
+                              const double *w, const double *dw, int64_t n,
+                              PrefixRecord *pre, double &spc_r, double &spc_d) {
+    walk_forest_entries(r, d, z, w, dw, n, [&](int64_t k, const PrefixRecord &e) { pre[k] = e; },
+                        spc_r, spc_d);
+}
+
+inline void build_walk_forest(const double *r, const double *d, const double *z,
+                              const double *w, const double *dw, int64_t n,
+                              PrefixPair *pre, double &spc_r, double &spc_d) {
+    walk_forest_entries(r, d, z, w, dw, n, [&](int64_t k, const PrefixRecord &e) {
+        pre[k] = PrefixPair{e.c, e.w};
+        pre[n + 1 + k] = PrefixPair{e.x, e.r};
+        pre[2 * (n + 1) + k] = PrefixPair{e.d, e.z};
+    }, spc_r, spc_d);
 }
 
 // Per (forest pair, chunk of delta1): wave-uniform constants of the walk.
@@ -276,6 +290,27 @@ struct XiAcc {
     }
 };
 
+// What a memory type need not have: constants of its own for the exact arithmetic (the walk's
+// are taken), and the count of runs of every lane with each pass (count_run(closed, n)): without
+// it the closed runs alone are counted.
+template <class Mem>
+PICCA_HD inline auto walk_consts(Mem &mem, const XiConst &C, int) -> decltype(mem.consts(C)) {
+    return mem.consts(C);
+}
+template <class Mem>
+PICCA_HD inline const XiConst &walk_consts(Mem &, const XiConst &C, long) {
+    return C;
+}
+template <class Mem>
+PICCA_HD inline auto walk_count_run(Mem &mem, bool closed, uint32_t n, int)
+    -> decltype(mem.count_run(closed, n)) {
+    mem.count_run(closed, n);
+}
+template <class Mem>
+PICCA_HD inline void walk_count_run(Mem &mem, bool closed, uint32_t n, long) {
+    if (closed) mem.count_run(n);
+}
+
 // Reciprocal of x > 0 within 2.5e-4 relative, the same on the host and the device: the
 // seed is the bit pattern of 2.0^1023 (0x7FE0...) minus that of x, within 12.5 % of 1 / x
 // for a normal x, then two Newton steps y (2 - x y).  For the guess of a run's end only.
@@ -354,6 +389,7 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
                                bool alive) {
     const int j_hi = CUTS ? L.j_hi : T.j_hi;
     if (T.j_lo >= T.j_hi) return;  // wave-uniform
+    const XiConst &exact = walk_consts(mem, C, 0);
     const int last = T.j_hi - 1;  // pixel reads stay inside the window
     // the run coordinate is (r2 - r1) cp, from r_par_min for the cross-correlation
     const double r1cp = XC ? L.r1 * T.cp - C.rpmin * C.inv_p : L.r1 * T.cp;
@@ -394,14 +430,14 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
             walk_key_from<XC>(C, m, c, aB, bB, mB, cB);
             if (nearB) {
                 const WalkExact e =
-                    walk_exact<XC>(mem.consts(C), L.r1, L.d1, rb, db, T.cos_half, T.sin_half);
+                    walk_exact<XC>(exact, L.r1, L.d1, rb, db, T.cos_half, T.sin_half);
                 mB = e.m;
                 cB = e.c;
             }
             bool inA = (aA < 0) & (bA < 0);
             if (nearA & !starting) {
                 const WalkExact e =
-                    walk_exact<XC>(mem.consts(C), L.r1, L.d1, ra, da, T.cos_half, T.sin_half);
+                    walk_exact<XC>(exact, L.r1, L.d1, ra, da, T.cos_half, T.sin_half);
                 inA = (e.m == m) && (e.c == c);
             }
             // outcome of the pass
@@ -462,11 +498,11 @@ PICCA_HD inline void walk_lane(const XiConst &C, const WalkTask &T, const WalkLa
                 pa = g - 1;
                 pb = g;
             }
-            if (special_last) walk_special<XC, CUTS>(mem.consts(C), T, L, mem, p_last);
-            if (special_first) walk_special<XC, CUTS>(mem.consts(C), T, L, mem, p_first);
+            if (special_last) walk_special<XC, CUTS>(exact, T, L, mem, p_last);
+            if (special_first) walk_special<XC, CUTS>(exact, T, L, mem, p_first);
             if (done) alive = false;
         }
-        mem.count_run(close, run.n);
+        walk_count_run(mem, close, run.n, 0);
         // the next pass's probes, issued before the histogram additions (a lane that is done
         // reloads its last probes, which lie inside the window)
         const bool more = mem.any(alive);
