@@ -147,11 +147,12 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
                                 (forest_monotone(z + o, n) ? 4 : 0));
         }
     });
-    double max_r = 0, max_d = 0;
+    double max_r = 0, max_d = 0, min_d = 0;
     bool finite = true;
     for (int64_t k = 0; k < npix; ++k) {
         max_r = std::max(max_r, std::fabs(r_comov[k]));
         max_d = std::max(max_d, std::fabs(dist_m[k]));
+        min_d = std::min(min_d, dist_m[k]);
         finite = finite && std::isfinite(z[k]) && std::isfinite(weights[k]) &&
                  std::isfinite(delta[k]) && std::isfinite(dw[k]);
     }
@@ -160,6 +161,7 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
                                    "weights, delta, delta*weights)");
     ctx->max_abs_r = max_r;
     ctx->max_abs_d = max_d;
+    ctx->negative_d = min_d < 0;
     ctx->have_result = false;
     ctx->num_pairs = 0;
     ctx->h_offsets.assign(offsets, offsets + num_forests + 1);
@@ -362,8 +364,9 @@ int xi_execute_into(picca_ctx *ctx, const picca::XiConst &C0, int mode,
                     unsigned long long *stats_dev, bool allow_graph, picca_xi_report *report) {
     picca::XiConst C = C0;
     // the specialised kernel: standard binning, auto-correlation with r_par_min == 0 or
-    // cross-correlation
-    bool general = !picca::xi_fast_path(params, mode);
+    // cross-correlation, no negative dist_m (its r_trans bins count from 0 up: a negative one,
+    // which the general kernel counts as an overflow, would lie before the histogram)
+    bool general = !picca::xi_fast_path(params, mode) || ctx->negative_d;
     const bool cuts = picca::xi_has_cuts(params);
     const bool xcorr = params->x_correlation != 0;
     // the automatic schedule keeps the pair loop's kernel (no walk) when the store's pixels
@@ -1070,7 +1073,7 @@ bool power_of_two_times(int n, int base) {
 // binning without a pair-redshift cut, model bins that split the data bins in 2^k parts, and
 // either the auto-correlation from r_par_min == 0 (with LDS for a row of model bins) or the
 // signed r_par of forest x quasar pairs; per pair: no zerr or same-half-plate cut, the forests
-// (of a quasar's pair: the first) with a proper fit normalisation and strictly rising r_comov and
+// (of a quasar's pair: the first) with no negative r_trans, a proper fit normalisation and strictly rising r_comov and
 // dist_m whose steps lie above the rounding margins in both coordinates (the run walk's
 // condition; 1e4 margins, so that the index tables' 1e-3 of a step covers the rounding too), and
 // a projected delta2, or with signed r_par a one-pixel delta2 that is not projected and xcf's
@@ -1140,7 +1143,8 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
                                 C.rtmax;
             const double y_hi = (ctx->h_dmax[(size_t)a] + ctx->h_dmax[(size_t)b]) * sin_half /
                                 C.rtmax;
-            const double t0 = std::fmax(std::floor(y_lo * C.nt_d), 0.0);
+            if (y_lo < 0) continue;   // negative data bins, which the general kernels refuse
+            const double t0 = std::floor(y_lo * C.nt_d);
             const double t1 = std::fmin(std::floor(y_hi * C.nt_d), C.nt_d - 1);
             kind[(size_t)k] = t0 <= t1 ? 0 : 2;
             if (!(t0 <= t1)) continue;

@@ -133,6 +133,7 @@ struct picca_ctx {
     int64_t num_pixels = 0;
     double max_abs_r = 0;   // largest |r_comov| and |dist_m| of the store: bound the
     double max_abs_d = 0;   // rounding of the pre-scaled coordinates of the fast loop
+    bool negative_d = false;   // some dist_m is negative
     bool has_log_lambda = false;
     bool has_order = false;
     std::vector<int32_t> h_order;   // host copy of the fit orders (< 0: unprojected)
