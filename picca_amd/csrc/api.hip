@@ -140,13 +140,15 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
     });
     std::vector<uint8_t> mono((size_t)std::max<int64_t>(num_forests, 1));
     parallel_for(num_forests, [&](int64_t lo, int64_t hi) {
+        std::vector<double> scratch;
         for (int64_t k = lo; k < hi; ++k) {
             const int64_t o = offsets[k], n = offsets[k + 1] - offsets[k];
-            mono[k] = (uint8_t)((forest_monotone(r_comov + o, n) ? 1 : 0) |
-                                (forest_monotone(dist_m + o, n) ? 2 : 0) |
-                                (forest_monotone(z + o, n) ? 4 : 0));
+            mono[k] = (uint8_t)((forest_monotone(r_comov + o, n) ? picca::FOREST_RISES_R : 0) |
+                                (forest_monotone(dist_m + o, n) ? picca::FOREST_RISES_D : 0) |
+                                (forest_monotone(z + o, n) ? picca::FOREST_RISES_Z : 0) |
+                                picca::level_flags(weights + o, dw.data() + o, n, scratch));
         }
-    });
+    }, npix / 2);
     double max_r = 0, max_d = 0, min_d = 0;
     bool finite = true;
     for (int64_t k = 0; k < npix; ++k) {
@@ -177,7 +179,7 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
             ctx->h_dmin[k] = a;
             ctx->h_dmax[k] = b;
         }
-    });
+    }, npix / 2);
     PICCA_HIP_CHECK(ctx->off.upload(offsets, (size_t)num_forests + 1, ctx->stream));
     // the pair kernel reads pixel batches of four, up to three past a forest's end
     const size_t pad = picca::PIXEL_PAD;
@@ -213,7 +215,7 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
                                          pre.data() + picca::PREFIX_PLANES * (o + k), sr, sd);
                 spc[k] = make_double2(sr, sd);
             }
-        });
+        }, npix / 2);
         PICCA_HIP_CHECK(ctx->rd.upload_padded(rd.data(), (size_t)npix, pad, ctx->stream));
         PICCA_HIP_CHECK(ctx->pre.upload_padded(pre.data(), pre.size(), pad, ctx->stream));
         PICCA_HIP_CHECK(ctx->spc.upload(spc.data(), (size_t)num_forests, ctx->stream));
@@ -260,7 +262,7 @@ int picca_set_forests(picca_ctx *ctx, int64_t num_forests, const int64_t *offset
                 sw_dll[k] = s2;
                 ctx->h_fit[(size_t)k] = std::isfinite(sw) && sw > 0 && std::isfinite(s2) && s2 > 0;
             }
-        });
+        }, npix / 2);
         PICCA_HIP_CHECK(ctx->dll.upload_padded(dll.data(), (size_t)npix, pad, ctx->stream));
         PICCA_HIP_CHECK(ctx->sum_w.upload(sum_w.data(), (size_t)num_forests, ctx->stream));
         PICCA_HIP_CHECK(ctx->sw_dll.upload(sw_dll.data(), (size_t)num_forests, ctx->stream));
@@ -1075,7 +1077,8 @@ bool power_of_two_times(int n, int base) {
 // signed r_par of forest x quasar pairs; per pair: no zerr or same-half-plate cut, the forests
 // (of a quasar's pair: the first) with no negative r_trans, a proper fit normalisation and strictly rising r_comov and
 // dist_m whose steps lie above the rounding margins in both coordinates (the run walk's
-// condition; 1e4 margins, so that the index tables' 1e-3 of a step covers the rounding too), and
+// condition; 1e4 margins, so that the index tables' 1e-3 of a step covers the rounding too) and
+// level weights (level_values), and
 // a projected delta2, or with signed r_par a one-pixel delta2 that is not projected and xcf's
 // count pass.
 int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
@@ -1112,6 +1115,8 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
     std::vector<picca::DmatBandSlot> all((size_t)num_pairs);
     std::vector<uint8_t> kind((size_t)num_pairs);
     std::vector<double> half((size_t)(2 * num_pairs));
+    constexpr int rising_level = picca::FOREST_RISES_R | picca::FOREST_RISES_D |
+                                 picca::FOREST_LEVEL_W;
     parallel_for(num_pairs, [&](int64_t lo, int64_t hi) {
         for (int64_t k = lo; k < hi; ++k) {
             const int32_t a = L.a[(size_t)k], b = L.b[(size_t)k];
@@ -1125,7 +1130,8 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
                 const double2 spc = ctx->h_spc[(size_t)f];
                 return picca::walk_task(M, spc.x, spc.y, cp, st, 1.0) &&
                        cp * spc.x > 1e4 * M.fast_p && st * spc.y > 1e4 * M.fast_t &&
-                       (ctx->h_mono[(size_t)f] & 3) == 3 && ctx->h_fit[(size_t)f] != 0;
+                       (ctx->h_mono[(size_t)f] & rising_level) == rising_level &&
+                       ctx->h_fit[(size_t)f] != 0;
             };
             const bool cut = ((C.flags & picca::XI_HAS_ZERR) && ang < C.zerr_ang) ||
                              ((C.flags & picca::XI_REMOVE_SHP) &&

@@ -75,12 +75,14 @@ struct DeviceBuffer {
     }
 };
 
-// Runs body(begin, end) over [0, n) on up to hardware_concurrency threads.
+// Runs body(begin, end) over [0, n) on up to hardware_concurrency threads, on the calling one
+// alone below 65536 elements of work (`work`: of n items that are several each, as forests; a
+// started thread takes as long as a few thousand forest pixels, so those count half).
 template <typename F>
-inline void parallel_for(int64_t n, F body) {
+inline void parallel_for(int64_t n, F body, int64_t work = 0) {
     unsigned hw = std::thread::hardware_concurrency();
     int64_t nthreads = std::max<int64_t>(1, std::min<int64_t>(hw ? hw : 1, 16));
-    if (n < 65536) nthreads = 1;
+    if (std::max(n, work) < 65536) nthreads = 1;
     if (nthreads == 1) {
         body(0, n);
         return;

@@ -95,8 +95,8 @@ struct ForestView {
     const int64_t *__restrict__ off; // [n + 1]
     const double *__restrict__ zq;
     const int32_t *__restrict__ order;
-    const uint8_t *__restrict__ mono; // bit0 r_comov non-decreasing, bit1 dist_m
-                                      // non-decreasing, bit2 z non-decreasing
+    const uint8_t *__restrict__ mono; // FOREST_* of xi_walk.h: bits 0 to 2 r_comov, dist_m, z
+                                      // non-decreasing, bits 3 and 4 level weights and delta w
     const double2 *__restrict__ rd;   // (r_comov, dist_m) per pixel
     const PrefixPair *__restrict__ pre;   // run-walk prefix sums, forest b at 3 (off[b] + b)
     const double2 *__restrict__ spc;  // per forest: smallest step of r_comov and of dist_m

@@ -472,15 +472,18 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
     if constexpr (!GENERAL && LDS_HIST) {
         // Cuts that the walk does not take: zerr (single pixels of delta2 drop out), close
         // pairs of one half plate in the cross-correlation (r_par_min need not put a bin edge
-        // at r_par = 0), a pair-redshift cut where z does not rise along delta2.
+        // at r_par = 0), a pair-redshift cut where z does not rise along delta2, weights that
+        // are not level (level_values).
         bool walk_cuts = true;
         const bool shp = CUTS && (C.flags & XI_REMOVE_SHP) && same_half_plate;
         const bool z_cut = CUTS && (C.flags & (XI_HAS_ZMIN | XI_HAS_ZMAX)) != 0;
         const double z_lo = CUTS && (C.flags & XI_HAS_ZMIN) ? C.zmin : -INFINITY;
         const double z_hi = CUTS && (C.flags & XI_HAS_ZMAX) ? C.zmax : INFINITY;
-        if (CUTS)
+        if (CUTS || XCORR) {
+            const int need = FOREST_LEVEL_W | FOREST_LEVEL_DW | (z_cut ? FOREST_RISES_Z : 0);
             walk_cuts = !zerr_on && !(XCORR && shp) &&
-                        (!z_cut || (uniform_int(F.mono[b]) & 4) != 0);
+                        (uniform_int(F.mono[b]) & need) == need;
+        }
         if (WALK && (C.flags & XI_WALK) && pruned && walk_cuts) {
             // Run walk (xi_walk.h) for the tasks walk_task admits; otherwise the pair loop
             // below.

@@ -22,6 +22,8 @@
 // m = -row - 1, which rises with j; the cuts of the auto-correlation that leave whole runs
 // (pair redshift, close pairs of one half plate) are a pixel window per lane and a dropped
 // run.  Both are template parameters, so that the plain auto-correlation's code is its own.
+// They walk only forests with level weights (level_values); the plain auto-correlation, whose
+// bins collect the pairs of a whole survey, walks the others too.
 //
 // The header is compiled into the kernel and into a CPU harness of the tests, which runs
 // the same lane program under bounds checks; `Mem` supplies the memory accesses.
@@ -29,6 +31,10 @@
 
 #include <math.h>
 #include <stdint.h>
+
+#include <algorithm>
+#include <cstddef>
+#include <vector>
 
 #include "engine.h"
 
@@ -113,6 +119,74 @@ inline void build_walk_forest(const double *r, const double *d, const double *z,
         pre[n + 1 + k] = PrefixPair{e.x, e.r};
         pre[2 * (n + 1) + k] = PrefixPair{e.d, e.z};
     }, spc_r, spc_d);
+}
+
+// Whether sums over pixels of a forest may be differences of its prefix sums v[0] + v[1] + ...:
+// a difference carries the rounding of everything before it, 2^-53 of the prefix, however light
+// its own pixels are.  Level values: without their largest eighth the sum S of |v| is at most
+// `most` mean values (8192 for weights: a typical pixel's share of the error stays below 1e-12;
+// twice that for delta * weight), and no value other than 0 is below S / `least` (2^25 for
+// weights: 4e-9 of the lightest pixel at worst; deltas may vanish).  The synthetic surveys reach
+// 2100 mean weights and 2^13.2 smallest ones, with weights spread log-uniformly over 1e-3..1e2
+// 5900 and 2^24, and 9200 mean delta * weight with heavy-tailed deltas too.  One pixel 1e4 times
+// heavier than the others of a forest (not level): signed r_par 2.2e-13 in the weights, 5.2e-12
+// in the r_par sums near 0 and 5.6e-13 in xi at worst from prefix sums (1e8 times: 1.9e-9,
+// 9.6e-8 and 1.3e-8), 4e-14 to 6e-14 pair by pair (40 forests of the 0.8 A grid against 80-bit
+// sums).  Up to 1e3 times the prefix sums' 2-norms are the smaller ones, 2e-15 to 4e-15 against
+// 1e-14.
+inline bool level_values(const double *v, int64_t n, double most, double least,
+                         std::vector<double> &scratch) {
+    // (eight values at a time, so that the additions do not wait for each other)
+    constexpr int LANES = 8;
+    double s[LANES] = {}, l[LANES], h[LANES] = {}, c[LANES] = {};   // h: of squares
+    for (int q = 0; q < LANES; ++q) l[q] = INFINITY;
+    auto take = [&](int q, double a) {
+        s[q] += a;
+        h[q] += a * a;
+        c[q] += a != 0 ? 1.0 : 0.0;
+        a = a != 0 ? a : INFINITY;
+        l[q] = a < l[q] ? a : l[q];
+    };
+    int64_t k0 = 0;
+    for (; k0 + LANES <= n; k0 += LANES)
+        for (int q = 0; q < LANES; ++q) take(q, fabs(v[k0 + q]));
+    for (; k0 < n; ++k0) take(0, fabs(v[k0]));
+    double sum = 0.0, low = INFINITY, squares = 0.0, number = 0.0;
+    for (int q = 0; q < LANES; ++q) {
+        sum += s[q];
+        low = l[q] < low ? l[q] : low;
+        squares += h[q];
+        number += c[q];
+    }
+    const int64_t count = (int64_t)number;
+    const int64_t top = (count + 7) / 8, rest = count - top;
+    if (rest == 0) return true;   // no value, or one: its prefix sums are exact
+    // (a sum that overflows is not level)
+    if (!(sum < 1e290) || !(sum <= least * low)) return false;
+    // what the largest eighth holds at most (Cauchy-Schwarz): settles most forests in one pass
+    if (sum * (double)rest <= most * (sum - sqrt((double)top * squares))) return true;
+    scratch.clear();
+    for (int64_t k = 0; k < n; ++k)
+        if (v[k] != 0) scratch.push_back(fabs(v[k]));
+    std::nth_element(scratch.begin(), scratch.begin() + (std::ptrdiff_t)(rest - 1), scratch.end());
+    double low_sum = 0.0;
+    for (int64_t k = 0; k < rest; ++k) low_sum += scratch[(size_t)k];
+    return sum * (double)rest <= most * low_sum;
+}
+
+// Flags of a forest for the kernels (ForestView::mono).
+enum : int {
+    FOREST_RISES_R = 1,        // r_comov non-decreasing
+    FOREST_RISES_D = 2,        // dist_m non-decreasing
+    FOREST_RISES_Z = 4,        // z non-decreasing
+    FOREST_LEVEL_W = 8,        // level weights
+    FOREST_LEVEL_DW = 16       // level delta * weights
+};
+
+inline int level_flags(const double *w, const double *dw, int64_t n,
+                       std::vector<double> &scratch) {
+    return (level_values(w, n, 8192.0, 0x1p25, scratch) ? FOREST_LEVEL_W : 0) |
+           (level_values(dw, n, 16384.0, INFINITY, scratch) ? FOREST_LEVEL_DW : 0);
 }
 
 // Per (forest pair, chunk of delta1): wave-uniform constants of the walk.

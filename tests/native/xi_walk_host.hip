@@ -167,12 +167,14 @@ int walk_launch(const picca_cf_params *params, int64_t num_forests, const int64_
     std::vector<picca::PrefixPair> pre(picca::PREFIX_PLANES * (size_t)(npix + num_forests));
     std::vector<double> spc_r((size_t)num_forests), spc_d((size_t)num_forests);
     std::vector<uint8_t> mono((size_t)num_forests);
+    std::vector<double> scratch;
     for (int64_t b = 0; b < num_forests; ++b) {
         const int64_t o = off[b], n = off[b + 1] - off[b];
         picca::build_walk_forest(r + o, d + o, z + o, w + o, dw.data() + o, n,
                                  pre.data() + picca::PREFIX_PLANES * (o + b), spc_r[b], spc_d[b]);
         mono[b] = (uint8_t)((monotone(r + o, n) ? 1 : 0) | (monotone(d + o, n) ? 2 : 0) |
-                            (monotone(z + o, n) ? 4 : 0));
+                            (monotone(z + o, n) ? 4 : 0) |
+                            picca::level_flags(w + o, dw.data() + o, n, scratch));
     }
     const bool z_cut = (C.flags & (picca::XI_HAS_ZMIN | picca::XI_HAS_ZMAX)) != 0;
     const double z_lo = (C.flags & picca::XI_HAS_ZMIN) ? C.zmin : -INFINITY;
@@ -248,7 +250,9 @@ int walk_launch(const picca_cf_params *params, int64_t num_forests, const int64_
             }
             const bool shp = CUTS && (C.flags & picca::XI_REMOVE_SHP) &&
                              (pflags[p] & picca::PAIR_SAME_HALF_PLATE);
-            const bool cuts_ok = !(XC && shp) && (!z_cut || (mono[b] & 4));
+            const int level = picca::FOREST_LEVEL_W | picca::FOREST_LEVEL_DW;
+            const bool cuts_ok = !(XC && shp) && (!z_cut || (mono[b] & 4)) &&
+                                 (!(XC || CUTS) || (mono[b] & level) == level);
             const bool walk = pruned && cuts_ok && picca::walk_task(C, spc_r[b], spc_d[b], cp, st, q0);
             if (walk) {
                 ++stats[ST_WALK_TASKS];
@@ -328,6 +332,12 @@ extern "C" {
 
 // The walk's guess reciprocal (walk_rcp_guess), for its unit test.
 double xi_walk_rcp_guess(double x) { return picca::walk_rcp_guess(x); }
+
+// A forest's level_flags.
+int xi_level_flags(int n, const double *w, const double *dw) {
+    std::vector<double> scratch;
+    return picca::level_flags(w, dw, n, scratch);
+}
 
 // The banded distortion matrix's keys and edges (dmat_band.h) of one pixel along a partner of n
 // rising values v (kind: BAND_*; from: r_par_min of BAND_SIGNED).  keys[k]: of pixel k; edges[k]: first pixel
