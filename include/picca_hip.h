@@ -229,6 +229,29 @@ typedef struct picca_dmat_report {
 } picca_dmat_report;
 int picca_dmat_last_report(picca_ctx *ctx, picca_dmat_report *report);
 
+/*
+ * Which kernels the pairs of the last picca_dmat_run took (no counterpart in picca):
+ * routes[0] pairs evaluated from prefix sums over the forests, [1] those of them handed back
+ * because a bin does not follow the runs, [2] pairs evaluated by the general kernels (among them
+ * the ones handed back), [3] pairs whose r_trans lies outside the range.
+ */
+#define PICCA_DMAT_ROUTES 4
+#define PICCA_DMAT_ROUTE_SUMS 0
+#define PICCA_DMAT_ROUTE_HANDED_BACK 1
+#define PICCA_DMAT_ROUTE_GENERAL 2
+#define PICCA_DMAT_ROUTE_OUTSIDE 3
+int picca_dmat_last_routes(picca_ctx *ctx, int64_t *routes);
+
+/*
+ * Device memory of the following picca_dmat_run calls: batch_bytes of workspace for the pairs
+ * evaluated at a time (PICCA_DMAT_BATCH_BYTES at first; one pair is always taken), prefix_bytes
+ * for the forests' prefix sums (64 bytes a pixel of the forests in the pair list, twice that when
+ * alpha2 differs from alpha; INT64_MAX at first).  Pairs whose prefix sums or workspace do not
+ * fit, there or on the device, take the general kernels.
+ */
+#define PICCA_DMAT_BATCH_BYTES ((int64_t)1536 << 20)
+int picca_dmat_set_workspace(picca_ctx *ctx, int64_t batch_bytes, int64_t prefix_bytes);
+
 int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pairs,
                    const int32_t *pair_a, const int32_t *pair_b, const double *pair_ang,
                    const uint8_t *pair_flags, double *weights_dmat, double *dmat,

@@ -95,6 +95,11 @@ class DmatReport(ctypes.Structure):
         return {name: getattr(self, name) for name, _ in self._fields_}
 
 
+# picca_dmat_last_routes (PICCA_DMAT_ROUTE_*) and picca_dmat_set_workspace's first batch_bytes
+DMAT_ROUTES = ("sums", "handed_back", "general", "outside")
+DMAT_BATCH_BYTES = 1536 << 20
+
+
 class WickReport(ctypes.Structure):
     """``picca_wick_report``."""
     _fields_ = [
@@ -150,6 +155,8 @@ _PROTOTYPES = {
     "picca_xi_execute_noalloc": [_P, _P, _P, _I64, _P],
     "picca_dmat_run": [_P, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P],
     "picca_dmat_last_report": [_P, _P],
+    "picca_dmat_last_routes": [_P, _P],
+    "picca_dmat_set_workspace": [_P, _I64, _I64],
     "picca_diag_copy": [_P, _I64, _P],
     "picca_cov_subsample": [_P, _I64, _I64, _P, _P, _P, _P],
     "picca_wick_t123": [_P, _P, _I64, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _P],

@@ -591,6 +591,20 @@ int picca_dmat_last_report(picca_ctx *ctx, picca_dmat_report *report) {
     return PICCA_OK;
 }
 
+int picca_dmat_last_routes(picca_ctx *ctx, int64_t *routes) {
+    if (!ctx || !routes) return fail(PICCA_E_VALUE, "ctx or routes is NULL");
+    std::copy(ctx->dmat_routes, ctx->dmat_routes + PICCA_DMAT_ROUTES, routes);
+    return PICCA_OK;
+}
+
+int picca_dmat_set_workspace(picca_ctx *ctx, int64_t batch_bytes, int64_t prefix_bytes) {
+    if (!ctx) return fail(PICCA_E_VALUE, "ctx is NULL");
+    if (batch_bytes < 0 || prefix_bytes < 0) return fail(PICCA_E_VALUE, "negative size");
+    ctx->dmat_batch_bytes = batch_bytes;
+    ctx->dmat_prefix_bytes = prefix_bytes;
+    return PICCA_OK;
+}
+
 int picca_xi_set_schedule(picca_ctx *ctx, int32_t schedule) {
     if (!ctx) return fail(PICCA_E_VALUE, "ctx is NULL");
     if (schedule != PICCA_XI_SCHEDULE_AUTO && schedule != PICCA_XI_SCHEDULE_PAIRS &&
@@ -951,6 +965,7 @@ struct DmatRun {
     picca::DmatOut O;
     size_t pass_lds;        // of dmat_pass_kernel
     int64_t batches;
+    int64_t routes[PICCA_DMAT_ROUTES];
     // uploads of the general kernels, kept until the stream is done
     std::vector<double> cs;
     std::vector<std::vector<int64_t>> pix_off;
@@ -1009,7 +1024,7 @@ int dmat_run_general(DmatRun &R, const DmatPairList &L) {
     // workspace per slot
     const size_t slot_bytes = 8 * (4 * (size_t)C.nt * C.np + 4 * (size_t)C.ntm * C.npm) +
                               4 * (size_t)C.words_u + 16 + 16 * (size_t)(C.nt + C.ntm);
-    const size_t ws_budget = (size_t)1536 << 20;
+    const size_t ws_budget = (size_t)ctx->dmat_batch_bytes;
     const int64_t cap = std::max<int64_t>(
         1, std::min<int64_t>({num_pairs, (int64_t)(ws_budget / slot_bytes), (int64_t)1 << 20}));
     const int64_t touched_words = ((int64_t)C.nt * C.ntm + 63) / 64;
@@ -1178,52 +1193,113 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
     const int64_t total = (int64_t)slots.size();
     if (total == 0) return PICCA_OK;
     hipStream_t st = ctx->stream;
-    const size_t entries = (size_t)(ctx->num_pixels + ctx->num_forests);
-    const bool differ = roles_differ(*R.params);
-    PICCA_HIP_CHECK(ctx->db_pre_b.reserve(entries));
-    if (differ) PICCA_HIP_CHECK(ctx->db_pre_a.reserve(entries));
-    picca::DmatPrefix *pre_b = ctx->db_pre_b.ptr, *pre_a = differ ? ctx->db_pre_a.ptr : pre_b;
-    PICCA_HIP_CHECK(ctx->db_table_r.reserve((size_t)ctx->num_pixels));
-    PICCA_HIP_CHECK(ctx->db_table_d.reserve((size_t)ctx->num_pixels));
-    PICCA_HIP_CHECK(picca::launch_dmat_prefix(R.F, ctx->num_forests, differ, pre_a, pre_b,
-                                              ctx->db_table_r.ptr, ctx->db_table_d.ptr, st));
+    // the forests whose prefix sums and tables the pairs read: both of a forest pair, the first
+    // of a quasar's
+    std::vector<int64_t> at((size_t)ctx->num_forests, -1);
+    for (const picca::DmatBandSlot &s : slots) {
+        at[(size_t)s.a] = 0;
+        if (!quasar) at[(size_t)s.b] = 0;
+    }
+    std::vector<int32_t> listed;
+    std::vector<int64_t> listed_at;
+    int64_t entries = 0;
+    for (int64_t f = 0; f < ctx->num_forests; ++f) {
+        if (at[(size_t)f] < 0) continue;
+        at[(size_t)f] = entries;
+        listed.push_back((int32_t)f);
+        listed_at.push_back(entries);
+        entries += ctx->h_offsets[(size_t)f + 1] - ctx->h_offsets[(size_t)f] + 1;
+    }
+    const bool differ = roles_differ(*R.params) && !quasar;
+    // batches: at most dmat_batch_bytes of workspace rows, tile lists and work items
     const int tiles = C.nt * C.ntm;
-    PICCA_HIP_CHECK(ctx->db_cs.upload(cs.data(), cs.size(), st));
-    PICCA_HIP_CHECK(ctx->db_tile.reserve((size_t)tiles + 1));
-    PICCA_HIP_CHECK(ctx->db_redo.reserve((size_t)total));
-    // two 32-bit counters a word: items and queue, redo count
-    PICCA_HIP_CHECK(ctx->db_num.reserve(4));
-    PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->db_num.ptr, 2, st));
-    // batches: about 1.5 GiB of workspace rows
-    const double budget = 1536.0 * 1048576.0;
+    const int item_pairs = quasar ? picca::DMAT_QUASAR_ITEM : picca::DMAT_BAND_ITEM;
     const double t_bytes = 16 + (quasar ? 0 : 8.0 * 4 * C.np);
     const double u_bytes = 16 + (quasar ? 0 : 8.0 * 9 * C.npm);
+    const double list_bytes = 4 + 16.0 / item_pairs;
+    struct Batch {
+        int64_t begin, end, t_rows, u_rows, list;
+    };
+    std::vector<Batch> plan;
+    Batch most{0, 0, 0, 0, 0};
     for (int64_t p0 = 0; p0 < total;) {
-        int64_t p1 = p0, t_rows = 0, u_rows = 0, list = 0;
-        while (p1 < total && p1 - p0 < (1 << 22)) {
-            picca::DmatBandSlot &s = slots[(size_t)p1];
-            if (p1 > p0 && (t_rows + s.nt) * t_bytes + (u_rows + s.nu) * u_bytes > budget) break;
-            if (p1 > p0 && list + (int64_t)s.nt * s.nu > (1 << 30)) break;
-            s.t_row = t_rows;
-            s.u_row = u_rows;
-            t_rows += s.nt;
-            u_rows += s.nu;
-            list += (int64_t)s.nt * s.nu;
-            ++p1;
+        Batch b{p0, p0, 0, 0, 0};
+        while (b.end < total && b.end - p0 < (1 << 22)) {
+            picca::DmatBandSlot &s = slots[(size_t)b.end];
+            const int64_t list = b.list + (int64_t)s.nt * s.nu;
+            if (b.end > p0 && ((b.t_rows + s.nt) * t_bytes + (b.u_rows + s.nu) * u_bytes +
+                                   list * list_bytes > (double)ctx->dmat_batch_bytes ||
+                               list > (1 << 30)))
+                break;
+            s.t_row = b.t_rows;
+            s.u_row = b.u_rows;
+            s.at_a = at[(size_t)s.a];
+            s.at_b = quasar ? 0 : at[(size_t)s.b];
+            b.t_rows += s.nt;
+            b.u_rows += s.nu;
+            b.list = list;
+            ++b.end;
         }
-        const int64_t count = p1 - p0;
-        PICCA_HIP_CHECK(ctx->db_slot.upload(slots.data() + p0, (size_t)count, st));
+        plan.push_back(b);
+        most.end = std::max(most.end, b.end - p0);
+        most.t_rows = std::max(most.t_rows, b.t_rows);
+        most.u_rows = std::max(most.u_rows, b.u_rows);
+        most.list = std::max(most.list, b.list);
+        p0 = b.end;
+    }
+    // everything is allocated before anything is launched: where it does not fit the general
+    // kernels, which need less, take the pairs
+    auto reserve = [&]() -> hipError_t {
+        if ((double)entries * sizeof(picca::DmatPrefix) * (differ ? 2 : 1) >
+            (double)ctx->dmat_prefix_bytes)
+            return hipErrorOutOfMemory;
+        hipError_t e = ctx->db_pre_a.reserve((size_t)entries);
+        auto next = [&](auto &buffer, int64_t n) {
+            if (e == hipSuccess) e = buffer.reserve((size_t)n);
+        };
+        if (differ) next(ctx->db_pre_b, entries);
+        next(ctx->db_table_r, entries);
+        next(ctx->db_table_d, entries);
+        next(ctx->db_forest, (int64_t)listed.size());
+        next(ctx->db_at, (int64_t)listed.size());
+        next(ctx->db_cs, 2 * total);
+        next(ctx->db_tile, (int64_t)tiles + 1);
+        next(ctx->db_redo, total);
+        next(ctx->db_num, 4);
+        next(ctx->db_slot, most.end);
         if (!quasar) {
-            PICCA_HIP_CHECK(ctx->db_S.reserve((size_t)t_rows * 4 * C.np));
-            PICCA_HIP_CHECK(ctx->db_eta.reserve((size_t)u_rows * 4 * C.npm));
-            PICCA_HIP_CHECK(ctx->db_eff.reserve((size_t)u_rows * 5 * C.npm));
+            next(ctx->db_S, most.t_rows * 4 * C.np);
+            next(ctx->db_eta, most.u_rows * 4 * C.npm);
+            next(ctx->db_eff, most.u_rows * 5 * C.npm);
         }
-        PICCA_HIP_CHECK(ctx->db_rng_t.reserve((size_t)t_rows));
-        PICCA_HIP_CHECK(ctx->db_rng_u.reserve((size_t)u_rows));
-        PICCA_HIP_CHECK(ctx->db_list.reserve((size_t)list));
-        PICCA_HIP_CHECK(ctx->db_items.reserve((size_t)(list / picca::DMAT_BAND_ITEM + tiles)));
-        picca::DmatBandSlots P{ctx->db_slot.ptr, ctx->db_cs.ptr + 2 * p0, (int32_t)count,
-                               (int32_t)p0};
+        next(ctx->db_rng_t, most.t_rows);
+        next(ctx->db_rng_u, most.u_rows);
+        next(ctx->db_list, most.list);
+        next(ctx->db_items, most.list / item_pairs + tiles);
+        return e;
+    };
+    const hipError_t fits = reserve();
+    if (fits == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        ctx->release_dmat_band();
+        rest = L;
+        return PICCA_OK;
+    }
+    PICCA_HIP_CHECK(fits);
+    picca::DmatPrefix *pre_a = ctx->db_pre_a.ptr, *pre_b = differ ? ctx->db_pre_b.ptr : pre_a;
+    PICCA_HIP_CHECK(ctx->db_forest.upload(listed.data(), listed.size(), st));
+    PICCA_HIP_CHECK(ctx->db_at.upload(listed_at.data(), listed_at.size(), st));
+    PICCA_HIP_CHECK(ctx->db_cs.upload(cs.data(), cs.size(), st));
+    const picca::DmatListed T{ctx->db_forest.ptr, ctx->db_at.ptr, (int64_t)listed.size()};
+    PICCA_HIP_CHECK(picca::launch_dmat_prefix(R.F, T, pre_a, differ ? pre_b : nullptr,
+                                              ctx->db_table_r.ptr, ctx->db_table_d.ptr, st));
+    // two 32-bit counters a word: items and queue, redo count
+    PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->db_num.ptr, 2, st));
+    for (const Batch &b : plan) {
+        const int64_t count = b.end - b.begin;
+        PICCA_HIP_CHECK(ctx->db_slot.upload(slots.data() + b.begin, (size_t)count, st));
+        picca::DmatBandSlots P{ctx->db_slot.ptr, ctx->db_cs.ptr + 2 * b.begin, (int32_t)count,
+                               (int32_t)b.begin};
         int32_t *num = ctx->db_num.ptr;
         picca::DmatBandWork W{pre_a, pre_b, ctx->db_table_r.ptr, ctx->db_table_d.ptr,
                               ctx->db_S.ptr, ctx->db_eta.ptr, ctx->db_eff.ptr,
@@ -1242,12 +1318,14 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
         PICCA_HIP_CHECK(picca::launch_dmat_band_fill(M, C, R.F, P, W, R.O, quasar, ctx->num_cus,
                                                      st));
         PICCA_HIP_CHECK(hipEventRecord(ev[2], st));
-        p0 = p1;
     }
+    R.routes[PICCA_DMAT_ROUTE_SUMS] = total;
+    R.routes[PICCA_DMAT_ROUTE_OUTSIDE] = num_pairs - total - rest.size();
     int32_t num_redo = 0;
     PICCA_HIP_CHECK(hipMemcpyAsync(&num_redo, ctx->db_num.ptr + 2, sizeof(num_redo),
                                    hipMemcpyDeviceToHost, st));
     PICCA_HIP_CHECK(hipStreamSynchronize(st));
+    R.routes[PICCA_DMAT_ROUTE_HANDED_BACK] = num_redo;
     if (num_redo > 0) {
         std::vector<int32_t> redo((size_t)num_redo);
         PICCA_HIP_CHECK(hipMemcpyAsync(redo.data(), ctx->db_redo.ptr,
@@ -1383,7 +1461,7 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
                          ctx->sw_dll.ptr, ctx->order.ptr, ctx->mono.ptr};
     picca::DmatOut O{ctx->o_wdm.ptr, ctx->o_dmat.ptr, ctx->o_eff.ptr, ctx->o_eff.ptr + nm,
                      ctx->o_eff.ptr + 2 * nm, ctx->o_eff.ptr + 3 * nm};
-    DmatRun R{ctx, params, C, F, O, pass_lds, 0, {}, {}};
+    DmatRun R{ctx, params, C, F, O, pass_lds, 0, {}, {}, {}};
     DmatPairList pairs, rest;
     pairs.a.assign(pair_a, pair_a + num_pairs);
     pairs.b.assign(pair_b, pair_b + num_pairs);
@@ -1392,6 +1470,8 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
     status = dmat_run_band(R, pairs, rest);
     if (status == PICCA_OK) status = dmat_run_general(R, rest);
     if (status != PICCA_OK) return status;
+    R.routes[PICCA_DMAT_ROUTE_GENERAL] = rest.size();
+    std::copy(R.routes, R.routes + PICCA_DMAT_ROUTES, ctx->dmat_routes);
     const int64_t batches = R.batches;
 
     unsigned long long h_stats[picca::DMAT_NSTATS];

@@ -187,12 +187,27 @@ struct picca_ctx {
     DeviceBuffer<int64_t> ws_pix;
     DeviceBuffer<unsigned long long> ws_touched, dstats;
     DeviceBuffer<double> o_wdm, o_dmat, o_eff;
-    // forest pairs without cuts: prefix sums of both roles and the workspace of a batch
+    // forest pairs without cuts: prefix sums of both roles (64 bytes a pixel of the call's
+    // forests and role, 8 of index tables) and the workspace of a batch
+    int64_t dmat_batch_bytes = PICCA_DMAT_BATCH_BYTES, dmat_prefix_bytes = INT64_MAX;
+    int64_t dmat_routes[PICCA_DMAT_ROUTES] = {0, 0, 0, 0};
     DeviceBuffer<picca::DmatPrefix> db_pre_a, db_pre_b;
     DeviceBuffer<picca::DmatBandSlot> db_slot;
     DeviceBuffer<double> db_cs, db_S, db_eta, db_eff;
     DeviceBuffer<int4> db_rng_t, db_rng_u, db_items;
-    DeviceBuffer<int32_t> db_tile, db_list, db_redo, db_num, db_table_r, db_table_d;
+    DeviceBuffer<int32_t> db_tile, db_list, db_redo, db_num, db_table_r, db_table_d, db_forest;
+    DeviceBuffer<int64_t> db_at;
+    void release_dmat_band() {
+        db_pre_a.release();
+        db_pre_b.release();
+        db_table_r.release();
+        db_table_d.release();
+        db_S.release();
+        db_eta.release();
+        db_eff.release();
+        db_list.release();
+        db_items.release();
+    }
 
     // metal distortion matrix: absorber tables per slot (store order) and per-pass tasks
     struct MetalSlot {

@@ -73,7 +73,7 @@ __device__ __forceinline__ void lds_add(double *p, double v) {
 
 struct BandPair {
     int a, b, la, lb;
-    int64_t oa, ob;
+    int64_t oa, ob, at_a, at_b;
     double cos_half, sin_half;
     double inv_w1, inv_w2, inv_s1, inv_s2;
     bool order1, order2;
@@ -87,6 +87,8 @@ __device__ BandPair load_band_pair(const DmatForests &F, const DmatBandSlots &P,
     q.la = (int)(uniform_i64(F.off[q.a + 1]) - q.oa);
     q.ob = uniform_i64(F.off[q.b]);
     q.lb = (int)(uniform_i64(F.off[q.b + 1]) - q.ob);
+    q.at_a = uniform_i64(P.slot[s].at_a);
+    q.at_b = uniform_i64(P.slot[s].at_b);
     q.cos_half = uniform_f64(P.cs[2 * s]);
     q.sin_half = uniform_f64(P.cs[2 * s + 1]);
     q.inv_w1 = 1.0 / uniform_f64(F.sum_w[q.a]);
@@ -195,31 +197,29 @@ struct BandPassMem {
 
 }  // namespace
 
-// Prefix sums of every forest for both roles: one thread per forest and field, in pixel order
-// (so that a pixel without weight leaves the sums as they are).  A chain of additions per thread:
-// the loads of PREFIX_BATCH pixels are issued together, ahead of their additions and stores
-// (3000 forests of the 0.8 A grid: 0.54 ms, one pixel at a time 1.66 ms).
+// Prefix sums of the listed forests for both roles: one thread per forest and field, in pixel
+// order (so that a pixel without weight leaves the sums as they are).  A chain of additions per
+// thread: the loads of PREFIX_BATCH pixels are issued together, ahead of their additions and
+// stores (3000 forests of the 0.8 A grid: 0.54 ms, one pixel at a time 1.66 ms).
 constexpr int PREFIX_BATCH = 8;
-__global__ __launch_bounds__(256) void dmat_prefix_kernel(DmatForests F, int64_t num_forests,
-                                                          bool roles_differ,
+__global__ __launch_bounds__(256) void dmat_prefix_kernel(DmatForests F, DmatListed T,
                                                           DmatPrefix *__restrict__ pa,
                                                           DmatPrefix *__restrict__ pb) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int field = (int)(k & 15);
-    const int64_t f = k >> 4;
-    if (f >= num_forests) return;
-    const bool second = field >= 8;
-    if (second && !roles_differ) return;
-    const int c = field & 7;
+    const int64_t at = pb ? k >> 4 : k >> 3;
+    if (at >= T.count) return;
+    const bool second = pb && (k & 8);
+    const int64_t f = T.forest[at];
+    const int c = (int)(k & 7);
     const int64_t o = F.off[f];
     const int n = (int)(F.off[f + 1] - o);
-    const double *__restrict__ zf = (second || !roles_differ ? F.zfb : F.zfa) + o;
+    const double *__restrict__ zf = (second ? F.zfb : F.zfa) + o;
     const double *__restrict__ w = F.w + o;
     const double *__restrict__ l = F.dll + o;
     const double *__restrict__ r = F.r + o;
     const double *__restrict__ d = F.d + o;
     const double *__restrict__ z = F.z + o;
-    double *out = (double *)((second || !roles_differ ? pb : pa) + (o + f)) + c;
+    double *out = (double *)((second ? pb : pa) + T.at[at]) + c;
     const double rc = n > 0 ? r[n / 2] : 0.0, dc = n > 0 ? d[n / 2] : 0.0;
     double acc = 0.0;
     out[0] = 0.0;
@@ -248,17 +248,18 @@ __global__ __launch_bounds__(256) void dmat_prefix_kernel(DmatForests F, int64_t
     }
 }
 
-// Index tables of r_comov and dist_m (BandTable) of every forest with rising values: one wave
-// per forest, a binary search per entry.
-__global__ __launch_bounds__(256) void dmat_table_kernel(DmatForests F, int64_t num_forests,
+// Index tables of r_comov and dist_m (BandTable) of the listed forests: one wave per forest, a
+// binary search per entry.
+__global__ __launch_bounds__(256) void dmat_table_kernel(DmatForests F, DmatListed T,
                                                          int32_t *__restrict__ tr,
                                                          int32_t *__restrict__ td) {
-    const int64_t f = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (f >= num_forests) return;
+    const int64_t at = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (at >= T.count) return;
     const int lane = threadIdx.x & 63;
+    const int64_t f = T.forest[at];
     const int64_t o = F.off[f];
     const int n = (int)(F.off[f + 1] - o);
-    if (n <= 0 || (F.mono[f] & 3) != 3) return;
+    const int64_t to = T.at[at];
     for (int axis = 0; axis < 2; ++axis) {
         const double *__restrict__ v = (axis ? F.d : F.r) + o;
         const double v0 = v[0], h = band_mean_step(v0, v[n - 1], n);
@@ -270,7 +271,7 @@ __global__ __launch_bounds__(256) void dmat_table_kernel(DmatForests F, int64_t 
                 if (v[lo + half] < x) { lo += half + 1; m -= half + 1; }
                 else m = half;
             }
-            (axis ? td : tr)[o + k] = lo;
+            (axis ? td : tr)[to + k] = lo;
         }
     }
 }
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(DMAT_BAND_PASS_BLOCK) void dmat_band_pass_kernel(
                 // the lane's pixels of this band of rows
                 const BandAxis A = band_trans_axis(d1, mul_t, q.sin_half, C.rtmax, C.ntm,
                                                    M.fast_t);
-                const BandTable B = load_table(W.table_d + q.ob, Bd, q.lb);
+                const BandTable B = load_table(W.table_d + q.at_b, Bd, q.lb);
                 auto v = [&](int p) { return Bd[p]; };
                 if (uc0 > u0) L.j_lo = max(T.j_lo, band_edge(A, B, v, uc0));
                 if (uc0 + rows < u0 + nu) L.j_hi = min(T.j_hi, band_edge(A, B, v, uc0 + rows));
@@ -374,7 +375,7 @@ __global__ __launch_bounds__(DMAT_BAND_PASS_BLOCK) void dmat_band_pass_kernel(
                     L.j_lo = T.j_lo;
                 }
             }
-            BandPassMem mem{Br, Bd, F.w + q.ob, F.z + q.ob, W.pre_b + (q.ob + q.b), acc, rng,
+            BandPassMem mem{Br, Bd, F.w + q.ob, F.z + q.ob, W.pre_b + q.at_b, acc, rng,
                             &s_special, stride, nu, uc0 * C.npm, u0, i, l1, &s_const, 0, -1, 0, 0};
             walk_lane<false, true, DmatAcc>(M, T, L, mem, active);
             mem.note();
@@ -638,11 +639,11 @@ __global__ __launch_bounds__(DMAT_BAND_FILL_BLOCK, 3) void dmat_band_fill_kernel
                         const int np_ = side ? q.la : q.lb;   // pixels of the partner
                         const double *__restrict__ Pr = F.r + op;
                         const double *__restrict__ Pd = F.d + op;
+                        const int64_t at = side ? q.at_a : q.at_b;   // of the partner
                         const double2 *__restrict__ pre =
-                            (const double2 *)(side ? W.pre_a + (q.oa + q.a)
-                                                   : W.pre_b + (q.ob + q.b));
-                        const BandTable Tr = load_table(W.table_r + op, Pr, np_);
-                        const BandTable Td = load_table(W.table_d + op, Pd, np_);
+                            (const double2 *)((side ? W.pre_a : W.pre_b) + at);
+                        const BandTable Tr = load_table(W.table_r + at, Pr, np_);
+                        const BandTable Td = load_table(W.table_d + at, Pd, np_);
                         const double inv_w = side ? q.inv_w1 : q.inv_w2;
                         const double inv_s = side ? (q.order1 ? q.inv_s1 : 0.0)
                                                   : (q.order2 ? q.inv_s2 : 0.0);
@@ -785,8 +786,8 @@ __global__ __launch_bounds__(256) void dmat_quasar_rows_kernel(XiConst M, DmatCo
     const double *__restrict__ D = F.d + oa;
     const double cos_half = P.cs[2 * s], sin_half = P.cs[2 * s + 1];
     const double rq = F.r[ob], dq = F.d[ob];
-    const BandTable Tr{W.table_r + oa, R[0], 1.0 / band_mean_step(R[0], R[n - 1], n), n};
-    const BandTable Td{W.table_d + oa, D[0], 1.0 / band_mean_step(D[0], D[n - 1], n), n};
+    const BandTable Tr{W.table_r + q.at_a, R[0], 1.0 / band_mean_step(R[0], R[n - 1], n), n};
+    const BandTable Td{W.table_d + q.at_a, D[0], 1.0 / band_mean_step(D[0], D[n - 1], n), n};
     auto r = [&](int p) { return R[p]; };
     auto d = [&](int p) { return D[p]; };
     const BandAxis Ap = band_signed_axis(rq, cos_half * C.npm / C.span_p, cos_half, C.rpmin,
@@ -868,11 +869,11 @@ __global__ __launch_bounds__(DMAT_BAND_FILL_BLOCK, 3) void dmat_quasar_fill_kern
                     const int n = (int)(F.off[q.a + 1] - oa);
                     const double *__restrict__ Pr = F.r + oa;
                     const double *__restrict__ Pd = F.d + oa;
-                    const DmatPrefix *__restrict__ rec = W.pre_a + (oa + q.a);
+                    const DmatPrefix *__restrict__ rec = W.pre_a + q.at_a;
                     const double2 *__restrict__ pre = (const double2 *)rec;
-                    const BandTable Tr{W.table_r + oa, Pr[0],
+                    const BandTable Tr{W.table_r + q.at_a, Pr[0],
                                        1.0 / band_mean_step(Pr[0], Pr[n - 1], n), n};
-                    const BandTable Td{W.table_d + oa, Pd[0],
+                    const BandTable Td{W.table_d + q.at_a, Pd[0],
                                        1.0 / band_mean_step(Pd[0], Pd[n - 1], n), n};
                     const double cos_half = P.cs[2 * s], sin_half = P.cs[2 * s + 1];
                     const double rq = F.r[ob], dq = F.d[ob], zq = F.z[ob];
@@ -1009,15 +1010,15 @@ size_t dmat_band_pass_lds(const DmatConst &C, int rows) {
            sizeof(double) * DMAT_BAND_SUMS * (size_t)C.npm * rows;
 }
 
-hipError_t launch_dmat_prefix(const DmatForests &F, int64_t num_forests, bool roles_differ,
-                              DmatPrefix *pa, DmatPrefix *pb, int32_t *table_r,
-                              int32_t *table_d, hipStream_t stream) {
-    if (num_forests <= 0) return hipSuccess;
-    const int64_t blocks = (16 * num_forests + 255) / 256;
-    hipLaunchKernelGGL(dmat_prefix_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, F,
-                       num_forests, roles_differ, pa, pb);
-    hipLaunchKernelGGL(dmat_table_kernel, dim3((unsigned)((num_forests + 3) / 4)), dim3(256), 0,
-                       stream, F, num_forests, table_r, table_d);
+hipError_t launch_dmat_prefix(const DmatForests &F, const DmatListed &T, DmatPrefix *pa,
+                              DmatPrefix *pb, int32_t *table_r, int32_t *table_d,
+                              hipStream_t stream) {
+    if (T.count <= 0) return hipSuccess;
+    const int64_t blocks = ((pb ? 16 : 8) * T.count + 255) / 256;
+    hipLaunchKernelGGL(dmat_prefix_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, F, T, pa,
+                       pb);
+    hipLaunchKernelGGL(dmat_table_kernel, dim3((unsigned)((T.count + 3) / 4)), dim3(256), 0,
+                       stream, F, T, table_r, table_d);
     return hipGetLastError();
 }
 

@@ -247,6 +247,7 @@ constexpr int DMAT_QUASAR_ITEM = 64;        // forest x quasar pairs (16 to a pa
 struct DmatBandSlot {
     int32_t a, b, t0, nt, u0, nu;
     int64_t t_row, u_row;
+    int64_t at_a, at_b;   // the forests' first entries in the prefix sums and index tables
 };
 
 struct DmatBandSlots {
@@ -260,9 +261,9 @@ struct DmatPrefix;   // dmat_band.h
 
 struct DmatBandWork {
     const DmatPrefix *__restrict__ pre_a;   // prefix sums with delta1's evolution factors
-    const DmatPrefix *__restrict__ pre_b;   // and with delta2's
-    const int32_t *__restrict__ table_r;    // index tables of r_comov and dist_m, forest f at
-    const int32_t *__restrict__ table_d;    // off[f]
+    const DmatPrefix *__restrict__ pre_b;   // and with delta2's (forest x quasar: none)
+    const int32_t *__restrict__ table_r;    // index tables of r_comov and dist_m
+    const int32_t *__restrict__ table_d;
     double *S;            // [t row][4][np]   S0, Sj, Si, Sij
     double *eta;          // [u row][4][npm]  eta5..eta8
     double *eff;          // [u row][5][npm]  effective-coordinate sums, pair-bin term
@@ -275,10 +276,18 @@ struct DmatBandWork {
     unsigned long long *stats;  // [DMAT_NSTATS]
 };
 
-// prefix sums and index tables (dmat_band.h) of every forest
-hipError_t launch_dmat_prefix(const DmatForests &F, int64_t num_forests, bool roles_differ,
-                              DmatPrefix *pa, DmatPrefix *pb, int32_t *table_r,
-                              int32_t *table_d, hipStream_t stream);
+// The forests that a call's pairs need, each with its first entry in the prefix sums and index
+// tables: L + 1 entries for a forest of L pixels.
+struct DmatListed {
+    const int32_t *__restrict__ forest;
+    const int64_t *__restrict__ at;
+    int64_t count;
+};
+// prefix sums and index tables (dmat_band.h) of the listed forests; pb: the sums with delta2's
+// evolution factors, nullptr to leave them out
+hipError_t launch_dmat_prefix(const DmatForests &F, const DmatListed &T, DmatPrefix *pa,
+                              DmatPrefix *pb, int32_t *table_r, int32_t *table_d,
+                              hipStream_t stream);
 hipError_t launch_dmat_band_pass(const XiConst &M, const DmatConst &C, const DmatForests &F,
                                  const DmatBandSlots &P, const DmatBandWork &W,
                                  const DmatOut &O, int band_rows, hipStream_t stream);

@@ -282,6 +282,16 @@ class Engine:
               "picca_dmat_last_report")
         return rep.as_dict()
 
+    def dmat_routes(self):
+        """Pairs of the last dmat() call by the kernels they took (picca_dmat_last_routes)."""
+        routes = np.zeros(len(_native.DMAT_ROUTES), dtype=np.int64)
+        check(self._lib.picca_dmat_last_routes(self._ctx, ptr(routes)), "picca_dmat_last_routes")
+        return dict(zip(_native.DMAT_ROUTES, (int(n) for n in routes)))
+
+    def set_dmat_workspace(self, batch_bytes=_native.DMAT_BATCH_BYTES, prefix_bytes=2 ** 63 - 1):
+        """Device memory that dmat() may take (picca_dmat_set_workspace)."""
+        check(self._lib.picca_dmat_set_workspace(self._ctx, int(batch_bytes), int(prefix_bytes)),
+              "picca_dmat_set_workspace")
 
     # -- subsampling covariance --------------------------------------------------
     def cov_subsample(self, xi, weights):
