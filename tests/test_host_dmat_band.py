@@ -58,3 +58,22 @@ def test_signed_r_par(grid, bins, lo, hi):
                                       bins + 1, lo)
             assert np.array_equal(np.maximum(keys, -1), ref)
             assert np.array_equal(edges, np.searchsorted(ref, np.arange(bins + 1)))
+
+
+def test_no_pair_of_an_auto_correlation_rounds_past_the_end():
+    """r_trans, and |r_par| from 0, below the range's end have a bin below the number of bins:
+    x <= pred(end) gives x / end <= 1 - 2^-53 after rounding, and (1 - 2^-53) n rounds to n minus
+    one spacing.  At the end the bin is n.  (A signed r_par counts from r_par_min: there the
+    difference to r_par_min may round to the whole range, and the pair is handed back.)"""
+    rng = np.random.default_rng(0)
+    ends = np.concatenate([2.0 ** np.arange(-2, 10), rng.uniform(0.1, 1000, 4000),
+                           np.nextafter(2.0 ** np.arange(-2, 10), 0)])
+    for n in (1, 2, 3, 7, 32, 33, 50, 63, 64, 65, 100, 127, 128, 4095, 8192, 100003):
+        below = np.nextafter(ends, 0)
+        assert np.all(np.floor(below / ends * n) == n - 1)
+        assert np.all(np.floor(ends / ends * n) == n)
+    for end in ends[:200]:
+        for kind in (H.BAND_TRANS, H.BAND_PAR):
+            v = np.array([np.nextafter(end, 0), end])   # own coordinate 0, scale 1
+            keys, _ = H.dmat_band(kind, v, 0.0, 1.0, end, 50, 1e-9, 0, 1)
+            assert list(keys) == [49, 50]
