@@ -963,18 +963,30 @@ struct DmatRun {
     picca::DmatConst C;
     picca::DmatForests F;
     picca::DmatOut O;
+    unsigned long long *stats;   // [DMAT_NSTATS]
     size_t pass_lds;        // of dmat_pass_kernel
     int64_t batches;
     int64_t routes[PICCA_DMAT_ROUTES];
-    // uploads of the general kernels, kept until the stream is done
+    int32_t *num_redo;      // on the device: pairs that the prefix sums hand back, cleared
+    // what the copies to the device read, kept until the stream is done
     std::vector<double> cs;
     std::vector<std::vector<int64_t>> pix_off;
+    std::vector<picca::DmatBandSlot> slots;
+    std::vector<double> slot_cs;
+    std::vector<picca::DmatListedForest> listed;
+    std::vector<int64_t> origin;   // index in the call's list of each pair of `slots`
 };
 
 // the redshift-evolution factors of delta1 and delta2 differ
 bool roles_differ(const picca_cf_params &p) {
     return p.redshift_evolution && p.alpha != p.alpha2;
 }
+
+// Waits for the stream when it goes out of scope.
+struct StreamDone {
+    hipStream_t stream;
+    ~StreamDone() { (void)hipStreamSynchronize(stream); }
+};
 
 struct DmatPairList {
     std::vector<int32_t> a, b;
@@ -1063,7 +1075,7 @@ int dmat_run_general(DmatRun &R, const DmatPairList &L) {
                           ctx->ws_cnt.ptr,
                           ctx->ws_pix.ptr,
                           (uint32_t *)ctx->ws_touched.ptr,
-                          ctx->dstats.ptr};
+                          R.stats};
         hipEvent_t *ev = nullptr;
         PICCA_HIP_CHECK(dmat_next_events(R, &ev));
         PICCA_HIP_CHECK(hipEventRecord(ev[0], ctx->stream));
@@ -1085,8 +1097,8 @@ bool power_of_two_times(int n, int base) {
     return (k & (k - 1)) == 0;
 }
 
-// The kernels for pairs without cuts (dmat_band_kernel.hip): takes the pairs they cover from
-// the list into `rest` what is left, and the pairs that they hand back.  Rule, per call: standard
+// The kernels for pairs without cuts (dmat_band_kernel.hip): takes the pairs they cover from the
+// list and puts what is left into `rest`.  Rule, per call: standard
 // binning without a pair-redshift cut, model bins that split the data bins in 2^k parts, and
 // either the auto-correlation from r_par_min == 0 (with LDS for a row of model bins) or the
 // signed r_par of forest x quasar pairs; per pair: no zerr or same-half-plate cut, the forests
@@ -1178,9 +1190,8 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
             s.nu = s.nt * kt;
         }
     });
-    std::vector<picca::DmatBandSlot> slots;
-    std::vector<double> cs;
-    std::vector<int64_t> origin;
+    std::vector<picca::DmatBandSlot> &slots = R.slots;
+    std::vector<double> &cs = R.slot_cs;
     for (int64_t k = 0; k < num_pairs; ++k) {
         if (kind[(size_t)k] == 1)
             rest.push(L.a[(size_t)k], L.b[(size_t)k], L.ang[(size_t)k], L.flags[(size_t)k]);
@@ -1188,7 +1199,7 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
         slots.push_back(all[(size_t)k]);
         cs.push_back(half[(size_t)(2 * k)]);
         cs.push_back(half[(size_t)(2 * k + 1)]);
-        origin.push_back(k);
+        R.origin.push_back(k);
     }
     const int64_t total = (int64_t)slots.size();
     if (total == 0) return PICCA_OK;
@@ -1200,14 +1211,12 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
         at[(size_t)s.a] = 0;
         if (!quasar) at[(size_t)s.b] = 0;
     }
-    std::vector<int32_t> listed;
-    std::vector<int64_t> listed_at;
+    std::vector<picca::DmatListedForest> &listed = R.listed;
     int64_t entries = 0;
     for (int64_t f = 0; f < ctx->num_forests; ++f) {
         if (at[(size_t)f] < 0) continue;
         at[(size_t)f] = entries;
-        listed.push_back((int32_t)f);
-        listed_at.push_back(entries);
+        listed.push_back(picca::DmatListedForest{f, entries});
         entries += ctx->h_offsets[(size_t)f + 1] - ctx->h_offsets[(size_t)f] + 1;
     }
     const bool differ = roles_differ(*R.params) && !quasar;
@@ -1260,12 +1269,11 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
         if (differ) next(ctx->db_pre_b, entries);
         next(ctx->db_table_r, entries);
         next(ctx->db_table_d, entries);
-        next(ctx->db_forest, (int64_t)listed.size());
-        next(ctx->db_at, (int64_t)listed.size());
+        next(ctx->db_listed, (int64_t)listed.size());
         next(ctx->db_cs, 2 * total);
         next(ctx->db_tile, (int64_t)tiles + 1);
         next(ctx->db_redo, total);
-        next(ctx->db_num, 4);
+        next(ctx->db_num, 2);
         next(ctx->db_slot, most.end);
         if (!quasar) {
             next(ctx->db_S, most.t_rows * 4 * C.np);
@@ -1287,14 +1295,11 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
     }
     PICCA_HIP_CHECK(fits);
     picca::DmatPrefix *pre_a = ctx->db_pre_a.ptr, *pre_b = differ ? ctx->db_pre_b.ptr : pre_a;
-    PICCA_HIP_CHECK(ctx->db_forest.upload(listed.data(), listed.size(), st));
-    PICCA_HIP_CHECK(ctx->db_at.upload(listed_at.data(), listed_at.size(), st));
+    PICCA_HIP_CHECK(ctx->db_listed.upload(listed.data(), listed.size(), st));
     PICCA_HIP_CHECK(ctx->db_cs.upload(cs.data(), cs.size(), st));
-    const picca::DmatListed T{ctx->db_forest.ptr, ctx->db_at.ptr, (int64_t)listed.size()};
+    const picca::DmatListed T{ctx->db_listed.ptr, (int64_t)listed.size()};
     PICCA_HIP_CHECK(picca::launch_dmat_prefix(R.F, T, pre_a, differ ? pre_b : nullptr,
                                               ctx->db_table_r.ptr, ctx->db_table_d.ptr, st));
-    // two 32-bit counters a word: items and queue, redo count
-    PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->db_num.ptr, 2, st));
     for (const Batch &b : plan) {
         const int64_t count = b.end - b.begin;
         PICCA_HIP_CHECK(ctx->db_slot.upload(slots.data() + b.begin, (size_t)count, st));
@@ -1305,7 +1310,7 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
                               ctx->db_S.ptr, ctx->db_eta.ptr, ctx->db_eff.ptr,
                               ctx->db_rng_t.ptr, ctx->db_rng_u.ptr, ctx->db_tile.ptr,
                               ctx->db_list.ptr, ctx->db_items.ptr, num, num + 1,
-                              ctx->db_redo.ptr, num + 2, ctx->dstats.ptr};
+                              ctx->db_redo.ptr, R.num_redo, R.stats};
         PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->db_tile.ptr,
                                                (tiles + 1) / 2, st));
         hipEvent_t *ev = nullptr;
@@ -1321,21 +1326,19 @@ int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
     }
     R.routes[PICCA_DMAT_ROUTE_SUMS] = total;
     R.routes[PICCA_DMAT_ROUTE_OUTSIDE] = num_pairs - total - rest.size();
-    int32_t num_redo = 0;
-    PICCA_HIP_CHECK(hipMemcpyAsync(&num_redo, ctx->db_num.ptr + 2, sizeof(num_redo),
-                                   hipMemcpyDeviceToHost, st));
-    PICCA_HIP_CHECK(hipStreamSynchronize(st));
-    R.routes[PICCA_DMAT_ROUTE_HANDED_BACK] = num_redo;
-    if (num_redo > 0) {
-        std::vector<int32_t> redo((size_t)num_redo);
-        PICCA_HIP_CHECK(hipMemcpyAsync(redo.data(), ctx->db_redo.ptr,
-                                       sizeof(int32_t) * redo.size(), hipMemcpyDeviceToHost, st));
-        PICCA_HIP_CHECK(hipStreamSynchronize(st));
-        std::sort(redo.begin(), redo.end());
-        for (int32_t r : redo) {
-            const size_t k = (size_t)origin[(size_t)r];
-            rest.push(L.a[k], L.b[k], L.ang[k], L.flags[k]);
-        }
+    return PICCA_OK;
+}
+
+// The pairs of the call's list L that the prefix sums handed back, in its order.
+int dmat_handed_back(DmatRun &R, const DmatPairList &L, int64_t count, DmatPairList &back) {
+    std::vector<int32_t> redo((size_t)count);
+    PICCA_HIP_CHECK(hipMemcpyAsync(redo.data(), R.ctx->db_redo.ptr, sizeof(int32_t) * redo.size(),
+                                   hipMemcpyDeviceToHost, R.ctx->stream));
+    PICCA_HIP_CHECK(hipStreamSynchronize(R.ctx->stream));
+    std::sort(redo.begin(), redo.end());
+    for (int32_t r : redo) {
+        const size_t k = (size_t)R.origin[(size_t)r];
+        back.push(L.a[k], L.b[k], L.ang[k], L.flags[k]);
     }
     return PICCA_OK;
 }
@@ -1425,44 +1428,39 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
     PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     const int64_t npix = ctx->num_pixels;
     const size_t pad = picca::PIXEL_PAD;
-    {   // redshift-evolution factors of each pixel (py/picca/cf.py:680-685)
-        std::vector<double> f((size_t)std::max<int64_t>(npix, 1), 1.0);
-        auto factors = [&](double alpha) {
-            const double zr = 1 + params->z_ref, e = alpha - 1;
-            parallel_for(npix, [&](int64_t lo, int64_t hi) {
-                for (int64_t k = lo; k < hi; ++k) f[k] = std::pow((1 + ctx->h_z[k]) / zr, e);
-            });
-        };
-        if (params->redshift_evolution) factors(params->alpha);
-        PICCA_HIP_CHECK(ctx->zfa.upload_padded(f.data(), (size_t)npix, pad, ctx->stream));
-        PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-        if (roles_differ(*params)) {
-            factors(params->alpha2);
-            PICCA_HIP_CHECK(ctx->zfb.upload_padded(f.data(), (size_t)npix, pad, ctx->stream));
-            PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-        }
+    // redshift-evolution factors of each pixel (py/picca/cf.py:680-685), for each role where they
+    // differ
+    std::vector<double> fa((size_t)std::max<int64_t>(npix, 1), 1.0), fb;
+    StreamDone done{ctx->stream};   // before the arrays go that copies to the device read
+    auto factors = [&](std::vector<double> &f, double alpha) {
+        const double zr = 1 + params->z_ref, e = alpha - 1;
+        parallel_for(npix, [&](int64_t lo, int64_t hi) {
+            for (int64_t k = lo; k < hi; ++k) f[k] = std::pow((1 + ctx->h_z[k]) / zr, e);
+        });
+    };
+    if (params->redshift_evolution) factors(fa, params->alpha);
+    PICCA_HIP_CHECK(ctx->zfa.upload_padded(fa.data(), (size_t)npix, pad, ctx->stream));
+    if (roles_differ(*params)) {
+        fb.resize(fa.size());
+        factors(fb, params->alpha2);
+        PICCA_HIP_CHECK(ctx->zfb.upload_padded(fb.data(), (size_t)npix, pad, ctx->stream));
     }
     const double *zfb = roles_differ(*params) ? ctx->zfb.ptr : ctx->zfa.ptr;
     // outputs, accumulated over all batches on the device
     const int64_t nb = C.nb, nm = C.nm;
-    PICCA_HIP_CHECK(ctx->o_wdm.reserve((size_t)nb));
-    PICCA_HIP_CHECK(ctx->o_dmat.reserve((size_t)(nb * nm)));
-    PICCA_HIP_CHECK(ctx->o_eff.reserve((size_t)(4 * nm)));
-    PICCA_HIP_CHECK(ctx->dstats.reserve(picca::DMAT_NSTATS));
-    PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->o_wdm.ptr, nb, ctx->stream));
-    PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->o_dmat.ptr, nb * nm,
-                                           ctx->stream));
-    PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->o_eff.ptr, 4 * nm,
-                                           ctx->stream));
-    PICCA_HIP_CHECK(picca::launch_zero_u64(ctx->dstats.ptr, picca::DMAT_NSTATS, ctx->stream));
+    MatrixBlock B;
+    PICCA_HIP_CHECK(make_matrix_block(ctx, nb, nm, B));
+    constexpr int REDO = picca::DMAT_NSTATS;   // the counter of pairs handed back
+    static_assert(REDO < MATRIX_COUNTERS, "counters of a distortion matrix");
 
     picca::DmatForests F{ctx->r.ptr,   ctx->d.ptr,     ctx->z.ptr,     ctx->w.ptr,   ctx->dll.ptr,
                          ctx->zfa.ptr, zfb,            ctx->off.ptr,   ctx->zq.ptr,  ctx->sum_w.ptr,
                          ctx->sw_dll.ptr, ctx->order.ptr, ctx->mono.ptr};
-    picca::DmatOut O{ctx->o_wdm.ptr, ctx->o_dmat.ptr, ctx->o_eff.ptr, ctx->o_eff.ptr + nm,
-                     ctx->o_eff.ptr + 2 * nm, ctx->o_eff.ptr + 3 * nm};
-    DmatRun R{ctx, params, C, F, O, pass_lds, 0, {}, {}, {}};
-    DmatPairList pairs, rest;
+    picca::DmatOut O{B.weights, B.matrix, B.eff, B.eff + nm, B.eff + 2 * nm, B.eff + 3 * nm};
+    DmatPairList pairs, rest, back;
+    DmatRun R{ctx, params, C, F, O, B.counters, pass_lds, 0, {}, (int32_t *)(B.counters + REDO),
+              {}, {}, {}, {}, {}, {}};
+    StreamDone done_run{ctx->stream};
     pairs.a.assign(pair_a, pair_a + num_pairs);
     pairs.b.assign(pair_b, pair_b + num_pairs);
     pairs.ang.assign(pair_ang, pair_ang + num_pairs);
@@ -1471,13 +1469,31 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
     if (status == PICCA_OK) status = dmat_run_general(R, rest);
     if (status != PICCA_OK) return status;
     R.routes[PICCA_DMAT_ROUTE_GENERAL] = rest.size();
+    // the results, taken at once unless a pair was handed back; what has a negative bin is refused
+    unsigned long long h_stats[MATRIX_COUNTERS];
+    auto fetch = [&]() -> hipError_t {
+        return fetch_matrix(
+            ctx, B,
+            [&](const unsigned long long *c) {
+                std::copy(c, c + MATRIX_COUNTERS, h_stats);
+                return c[REDO] == 0 && c[picca::DMAT_STAT_NEGATIVE] == 0;
+            },
+            weights_dmat, dmat, r_par_eff, r_trans_eff, z_eff, weight_eff);
+    };
+    PICCA_HIP_CHECK(fetch());
+    if (h_stats[REDO] > 0) {
+        const int64_t count = (int64_t)h_stats[REDO];
+        status = dmat_handed_back(R, pairs, count, back);
+        if (status != PICCA_OK) return status;
+        PICCA_HIP_CHECK(picca::launch_zero_u64(B.counters + REDO, 1, ctx->stream));
+        status = dmat_run_general(R, back);
+        if (status != PICCA_OK) return status;
+        R.routes[PICCA_DMAT_ROUTE_HANDED_BACK] = count;
+        R.routes[PICCA_DMAT_ROUTE_GENERAL] += count;
+        PICCA_HIP_CHECK(fetch());
+    }
     std::copy(R.routes, R.routes + PICCA_DMAT_ROUTES, ctx->dmat_routes);
     const int64_t batches = R.batches;
-
-    unsigned long long h_stats[picca::DMAT_NSTATS];
-    PICCA_HIP_CHECK(hipMemcpyAsync(h_stats, ctx->dstats.ptr, sizeof(h_stats),
-                                   hipMemcpyDeviceToHost, ctx->stream));
-    PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     ctx->dmat_report = picca_dmat_report{0.0, 0.0, batches,
                                          (int64_t)h_stats[picca::DMAT_STAT_MFMA] * 2048};
     for (int64_t k = 0; k < batches; ++k) {
@@ -1491,8 +1507,6 @@ int picca_dmat_run(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pa
     }
     if (h_stats[picca::DMAT_STAT_NEGATIVE] > 0)
         return fail(PICCA_E_INDEX, "a selected pair has a negative data bin index");
-    PICCA_HIP_CHECK(add_dmat_outputs(ctx, nb, nm, weights_dmat, dmat, r_par_eff, r_trans_eff,
-                                     z_eff, weight_eff));
     if (stats) {
         stats[0] = (int64_t)h_stats[picca::DMAT_STAT_IN_RANGE];
         stats[1] = (int64_t)h_stats[picca::DMAT_STAT_SELECTED];

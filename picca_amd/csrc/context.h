@@ -97,15 +97,18 @@ inline void parallel_for(int64_t n, F body, int64_t work = 0) {
     for (auto &th : pool) th.join();
 }
 
-// All of [0, n) pass ok(k).
+// All of [0, n) pass ok(k), a test of a few instructions: on several threads from 2^20 on (on
+// 3e5 values starting them took longer than the tests, 0.13 ms of a covariance).
 template <typename F>
 inline bool parallel_all(int64_t n, F ok) {
     std::atomic<bool> all{true};
-    parallel_for(n, [&](int64_t lo, int64_t hi) {
+    auto range = [&](int64_t lo, int64_t hi) {
         bool good = true;
         for (int64_t k = lo; k < hi; ++k) good = good && ok(k);
         if (!good) all.store(false, std::memory_order_relaxed);
-    });
+    };
+    if (n < ((int64_t)1 << 20)) range(0, n);
+    else parallel_for(n, range);
     return all.load();
 }
 
@@ -185,8 +188,9 @@ struct picca_ctx {
     DeviceBuffer<uint32_t> ws_U;
     DeviceBuffer<int32_t> ws_band, ws_rng, ws_cnt;
     DeviceBuffer<int64_t> ws_pix;
-    DeviceBuffer<unsigned long long> ws_touched, dstats;
-    DeviceBuffer<double> o_wdm, o_dmat, o_eff;
+    DeviceBuffer<unsigned long long> ws_touched;
+    DeviceBuffer<double> o_wdm, o_dmat;
+    DeviceBuffer<double> o_matrix;   // MatrixBlock of a distortion matrix
     // forest pairs without cuts: prefix sums of both roles (64 bytes a pixel of the call's
     // forests and role, 8 of index tables) and the workspace of a batch
     int64_t dmat_batch_bytes = PICCA_DMAT_BATCH_BYTES, dmat_prefix_bytes = INT64_MAX;
@@ -195,8 +199,8 @@ struct picca_ctx {
     DeviceBuffer<picca::DmatBandSlot> db_slot;
     DeviceBuffer<double> db_cs, db_S, db_eta, db_eff;
     DeviceBuffer<int4> db_rng_t, db_rng_u, db_items;
-    DeviceBuffer<int32_t> db_tile, db_list, db_redo, db_num, db_table_r, db_table_d, db_forest;
-    DeviceBuffer<int64_t> db_at;
+    DeviceBuffer<int32_t> db_tile, db_list, db_redo, db_num, db_table_r, db_table_d;
+    DeviceBuffer<picca::DmatListedForest> db_listed;
     void release_dmat_band() {
         db_pre_a.release();
         db_pre_b.release();
@@ -219,7 +223,6 @@ struct picca_ctx {
     MetalSlot metal[4];
     DeviceBuffer<int64_t> m_task_begin;
     DeviceBuffer<int32_t> m_task_pair;
-    DeviceBuffer<unsigned long long> m_stats;
 
     // subsampling covariance: rows, weights, per-bin means and weight sums, matrix
     DeviceBuffer<double> cv_xi, cv_w, cv_y, cv_s, cv_cov;
@@ -300,16 +303,65 @@ struct picca_ctx {
     DeviceBuffer<unsigned long long> queue, stats;
 };
 
-// Adds a distortion matrix's device outputs (o_wdm, o_dmat, o_eff) to the caller's.
-inline hipError_t add_dmat_outputs(picca_ctx *ctx, int64_t nb, int64_t nm, double *weights_dmat,
-                                   double *dmat, double *r_par_eff, double *r_trans_eff,
-                                   double *z_eff, double *weight_eff) {
-    hipError_t err = download_values<true>(ctx->ring, ctx->o_wdm.ptr, nb, ctx->stream,
-                                           weights_dmat);
-    double *const eff[4] = {r_par_eff, r_trans_eff, z_eff, weight_eff};
-    for (int k = 0; k < 4 && err == hipSuccess; ++k)
-        err = download_values<true>(ctx->ring, ctx->o_eff.ptr + k * nm, nm, ctx->stream, eff[k]);
+// A distortion matrix's results on the device, in one block that one copy fetches: counters, then
+// weights_dmat, the four effective sums and the matrix.
+constexpr int MATRIX_COUNTERS = 16;
+struct MatrixBlock {
+    unsigned long long *counters;
+    double *weights, *eff, *matrix;
+    int64_t nb, nm;
+    int64_t words() const { return MATRIX_COUNTERS + nb + 4 * nm + nb * nm; }
+};
+
+// The block in the context, cleared by the stream.
+inline hipError_t make_matrix_block(picca_ctx *ctx, int64_t nb, int64_t nm, MatrixBlock &B) {
+    B = MatrixBlock{nullptr, nullptr, nullptr, nullptr, nb, nm};
+    const hipError_t err = ctx->o_matrix.reserve((size_t)B.words());
     if (err != hipSuccess) return err;
-    return download_values<true>(ctx->ring, ctx->o_dmat.ptr, nb * nm, ctx->stream, dmat);
+    B.counters = (unsigned long long *)ctx->o_matrix.ptr;
+    B.weights = ctx->o_matrix.ptr + MATRIX_COUNTERS;
+    B.eff = B.weights + nb;
+    B.matrix = B.eff + 4 * nm;
+    return picca::launch_zero_u64(B.counters, B.words(), ctx->stream);
+}
+
+// Fetches the counters when the stream is done and, if accept(counters), adds the results to the
+// caller's arrays.  A matrix that fits a chunk of the ring is copied with its counters.
+template <class Accept>
+inline hipError_t fetch_matrix(picca_ctx *ctx, const MatrixBlock &B, const Accept &accept,
+                               double *weights_dmat, double *dmat, double *r_par_eff,
+                               double *r_trans_eff, double *z_eff, double *weight_eff) {
+    constexpr int64_t HEAD = 8 * MATRIX_COUNTERS;
+    struct Field {
+        double *to;
+        int64_t size;
+    };
+    const Field fields[6] = {{weights_dmat, 8 * B.nb}, {r_par_eff, 8 * B.nm},
+                             {r_trans_eff, 8 * B.nm},  {z_eff, 8 * B.nm},
+                             {weight_eff, 8 * B.nm},   {dmat, 8 * B.nb * B.nm}};
+    // bytes [lo, hi) of the results (behind the counters), whose first is at src
+    auto add = [&](const char *src, int64_t lo, int64_t hi) {
+        int64_t first = 0;
+        for (const Field &f : fields) {
+            const int64_t p = std::max(lo, first), q = std::min(hi, first + f.size);
+            const double *s = (const double *)(src + (p - lo));
+            double *o = f.to + (p - first) / 8;
+            for (int64_t k = 0; k < (q - p) / 8; ++k) o[k] += s[k];
+            first += f.size;
+        }
+    };
+    const int64_t bytes = 8 * B.words();
+    const bool whole = bytes <= picca_host::DownloadRing::BYTES;
+    hipError_t err = ctx->ring.fetch(B.counters, whole ? bytes : HEAD, ctx->stream);
+    if (err != hipSuccess) return err;
+    unsigned long long counters[MATRIX_COUNTERS];
+    std::memcpy(counters, ctx->ring.slot[0], HEAD);
+    if (!accept(counters)) return hipSuccess;
+    if (!whole)
+        return picca_host::download(ctx->ring, B.weights, bytes - HEAD, ctx->stream, add);
+    parallel_for((bytes - HEAD) / 8, [&](int64_t lo, int64_t hi) {
+        add(ctx->ring.slot[0] + HEAD + 8 * lo, 8 * lo, 8 * hi);
+    });
+    return hipSuccess;
 }
 

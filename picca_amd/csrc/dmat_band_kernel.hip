@@ -209,7 +209,7 @@ __global__ __launch_bounds__(256) void dmat_prefix_kernel(DmatForests F, DmatLis
     const int64_t at = pb ? k >> 4 : k >> 3;
     if (at >= T.count) return;
     const bool second = pb && (k & 8);
-    const int64_t f = T.forest[at];
+    const int64_t f = T.forest[at].forest;
     const int c = (int)(k & 7);
     const int64_t o = F.off[f];
     const int n = (int)(F.off[f + 1] - o);
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(256) void dmat_prefix_kernel(DmatForests F, DmatLis
     const double *__restrict__ r = F.r + o;
     const double *__restrict__ d = F.d + o;
     const double *__restrict__ z = F.z + o;
-    double *out = (double *)((second ? pb : pa) + T.at[at]) + c;
+    double *out = (double *)((second ? pb : pa) + T.forest[at].at) + c;
     const double rc = n > 0 ? r[n / 2] : 0.0, dc = n > 0 ? d[n / 2] : 0.0;
     double acc = 0.0;
     out[0] = 0.0;
@@ -256,10 +256,10 @@ __global__ __launch_bounds__(256) void dmat_table_kernel(DmatForests F, DmatList
     const int64_t at = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (at >= T.count) return;
     const int lane = threadIdx.x & 63;
-    const int64_t f = T.forest[at];
+    const int64_t f = T.forest[at].forest;
     const int64_t o = F.off[f];
     const int n = (int)(F.off[f + 1] - o);
-    const int64_t to = T.at[at];
+    const int64_t to = T.forest[at].at;
     for (int axis = 0; axis < 2; ++axis) {
         const double *__restrict__ v = (axis ? F.d : F.r) + o;
         const double v0 = v[0], h = band_mean_step(v0, v[n - 1], n);

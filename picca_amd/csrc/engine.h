@@ -272,15 +272,17 @@ struct DmatBandWork {
     int32_t *list;        // forest pairs of each tile
     int4 *items;          // tile, first list entry, entries
     int32_t *num_items, *queue;
-    int32_t *redo, *num_redo;   // pairs left to the general kernels
+    int32_t *redo, *num_redo;   // pairs handed back for the general kernels
     unsigned long long *stats;  // [DMAT_NSTATS]
 };
 
 // The forests that a call's pairs need, each with its first entry in the prefix sums and index
 // tables: L + 1 entries for a forest of L pixels.
+struct DmatListedForest {
+    int64_t forest, at;
+};
 struct DmatListed {
-    const int32_t *__restrict__ forest;
-    const int64_t *__restrict__ at;
+    const DmatListedForest *__restrict__ forest;
     int64_t count;
 };
 // prefix sums and index tables (dmat_band.h) of the listed forests; pb: the sums with delta2's

@@ -133,17 +133,9 @@ int picca_metal_pass(picca_ctx *ctx, const picca_cf_params *params, int32_t mode
     PICCA_HIP_CHECK(ctx->dflags.upload(flags.data(), (size_t)num_pairs, ctx->stream));
     PICCA_HIP_CHECK(ctx->m_task_begin.upload(task_begin.data(), (size_t)num_pairs, ctx->stream));
     PICCA_HIP_CHECK(ctx->m_task_pair.upload(task_pair.data(), (size_t)tasks, ctx->stream));
-    PICCA_HIP_CHECK(ctx->o_wdm.reserve((size_t)nb));
-    PICCA_HIP_CHECK(ctx->o_dmat.reserve((size_t)(nb * nm)));
-    PICCA_HIP_CHECK(ctx->o_eff.reserve((size_t)(4 * nm)));
-    PICCA_HIP_CHECK(ctx->m_stats.reserve(picca::METAL_NSTATS));
+    MatrixBlock B;
+    PICCA_HIP_CHECK(make_matrix_block(ctx, nb, nm, B));
     PICCA_HIP_CHECK(ctx->queue.reserve(1));
-    PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->o_wdm.ptr, nb, ctx->stream));
-    PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->o_dmat.ptr, nb * nm,
-                                           ctx->stream));
-    PICCA_HIP_CHECK(picca::launch_zero_u64((unsigned long long *)ctx->o_eff.ptr, 4 * nm,
-                                           ctx->stream));
-    PICCA_HIP_CHECK(picca::launch_zero_u64(ctx->m_stats.ptr, picca::METAL_NSTATS, ctx->stream));
     PICCA_HIP_CHECK(picca::launch_zero_u64(ctx->queue.ptr, 1, ctx->stream));
 
     const picca_ctx::MetalSlot &sa = ctx->metal[slot_a];
@@ -152,9 +144,8 @@ int picca_metal_pass(picca_ctx *ctx, const picca_cf_params *params, int32_t mode
     picca::MetalTable TB{sb.z.ptr, sb.r.ptr, sb.d.ptr, sb.w.ptr, sb.f.ptr, sb.rec.ptr};
     picca::MetalPairs P{ctx->dpa.ptr, ctx->dpb.ptr, ctx->dcs.ptr, ctx->dflags.ptr,
                         ctx->m_task_begin.ptr, num_pairs, tasks};
-    picca::MetalOut O{ctx->o_wdm.ptr, ctx->o_dmat.ptr, ctx->o_eff.ptr, ctx->o_eff.ptr + nm,
-                      ctx->o_eff.ptr + 2 * nm, ctx->o_eff.ptr + 3 * nm, ctx->queue.ptr,
-                      ctx->m_stats.ptr};
+    picca::MetalOut O{B.weights,      B.matrix,         B.eff,          B.eff + nm,
+                      B.eff + 2 * nm, B.eff + 3 * nm, ctx->queue.ptr, B.counters};
     const size_t static_lds = 1024;
     const bool lds_hist = (int64_t)(picca::metal_lds_bytes(C) + static_lds) <= ctx->lds_limit;
     const int64_t waves = std::max<int64_t>(1, tasks);
@@ -167,14 +158,17 @@ int picca_metal_pass(picca_ctx *ctx, const picca_cf_params *params, int32_t mode
                                         ctx->stream));
     PICCA_HIP_CHECK(hipEventRecord(ctx->ev_stop, ctx->stream));
 
+    static_assert(picca::METAL_NSTATS <= MATRIX_COUNTERS, "counters of a metal pass");
     unsigned long long h_stats[picca::METAL_NSTATS];
-    PICCA_HIP_CHECK(hipMemcpyAsync(h_stats, ctx->m_stats.ptr, sizeof(h_stats),
-                                   hipMemcpyDeviceToHost, ctx->stream));
-    PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+    PICCA_HIP_CHECK(fetch_matrix(
+        ctx, B,
+        [&](const unsigned long long *c) {
+            std::copy(c, c + picca::METAL_NSTATS, h_stats);
+            return true;
+        },
+        weights_dmat, dmat, r_par_eff, r_trans_eff, z_eff, weight_eff));
     float ms = 0.f;
     PICCA_HIP_CHECK(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
-    PICCA_HIP_CHECK(add_dmat_outputs(ctx, nb, nm, weights_dmat, dmat, r_par_eff, r_trans_eff,
-                                     z_eff, weight_eff));
     if (report) {
         report->data_pairs = (int64_t)h_stats[picca::METAL_STAT_DATA];
         report->model_pairs = (int64_t)h_stats[picca::METAL_STAT_MODEL];
