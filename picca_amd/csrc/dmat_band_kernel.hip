@@ -197,82 +197,106 @@ struct BandPassMem {
 
 }  // namespace
 
-// Prefix sums of the listed forests for both roles: one thread per forest and field, in pixel
-// order (so that a pixel without weight leaves the sums as they are).  A chain of additions per
-// thread: the loads of PREFIX_BATCH pixels are issued together, ahead of their additions and
-// stores (3000 forests of the 0.8 A grid: 0.54 ms, one pixel at a time 1.66 ms).
-constexpr int PREFIX_BATCH = 8;
-__global__ __launch_bounds__(256) void dmat_prefix_kernel(DmatForests F, DmatListed T,
-                                                          DmatPrefix *__restrict__ pa,
-                                                          DmatPrefix *__restrict__ pb) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t at = pb ? k >> 4 : k >> 3;
-    if (at >= T.count) return;
-    const bool second = pb && (k & 8);
-    const int64_t f = T.forest[at].forest;
-    const int c = (int)(k & 7);
+// Prefix sums of the listed forests for both roles: one wave per forest.  The sums are taken in
+// pixel order (so that a pixel without weight leaves them as they are), a lane per field, from
+// terms that all lanes make of 64 pixels at a time in LDS, the next 64 pixels already loading; the
+// rows leave as they lie in memory.  Bound by the chain of additions where the list is short and
+// by the stores where it is long: 100 forests of up to 1500 pixels, both roles, PREFIX_SHORT, 3000
+// forests PREFIX_LONG (a thread per forest and field that loads eight pixels ahead: 460 us and
+// 540 us).
+template <bool BOTH>
+__global__ __launch_bounds__(64) void dmat_prefix_kernel(DmatForests F, DmatListed T,
+                                                         DmatPrefix *__restrict__ pa,
+                                                         DmatPrefix *__restrict__ pb) {
+    constexpr int FIELDS = BOTH ? 16 : 8;
+    constexpr int ROW = FIELDS + 1;   // odd: the lanes' rows start in different banks
+    __shared__ double term[64 * ROW];
+    const int lane = threadIdx.x;
+    const int64_t f = T.forest[blockIdx.x].forest, at = T.forest[blockIdx.x].at;
     const int64_t o = F.off[f];
     const int n = (int)(F.off[f + 1] - o);
-    const double *__restrict__ zf = (second ? F.zfb : F.zfa) + o;
-    const double *__restrict__ w = F.w + o;
-    const double *__restrict__ l = F.dll + o;
-    const double *__restrict__ r = F.r + o;
-    const double *__restrict__ d = F.d + o;
-    const double *__restrict__ z = F.z + o;
-    double *out = (double *)((second ? pb : pa) + T.forest[at].at) + c;
-    const double rc = n > 0 ? r[n / 2] : 0.0, dc = n > 0 ? d[n / 2] : 0.0;
-    double acc = 0.0;
-    out[0] = 0.0;
-    // the other factor of the field's terms, and what is taken from it
-    const double *__restrict__ x = c == 1 ? l : c == 5 ? r : c == 6 ? d : c == 7 ? z : zf;
-    const double off = c == 5 ? rc : c == 6 ? dc : 0.0;
-    for (int q0 = 0; q0 < n; q0 += PREFIX_BATCH) {
-        double wq[PREFIX_BATCH], xq[PREFIX_BATCH], lq[PREFIX_BATCH];
+    const double rc = n > 0 ? F.r[o + n / 2] : 0.0, dc = n > 0 ? F.d[o + n / 2] : 0.0;
+    // field c of entry k of delta1's sums (c < 8) and of delta2's
+    auto out = [&](int c) { return (double *)((BOTH && c >= 8 ? pb : pa) + at) + (c & 7); };
+    if (lane < FIELDS) out(lane)[0] = 0.0;
+    double acc = 0.0;   // lane c < FIELDS: field c
+    double w = 0, l = 0, za = 0, zb = 0, r = 0, d = 0, z = 0;
+    auto load = [&](int q) {
+        if (q >= n) return;
+        w = F.w[o + q];
+        l = F.dll[o + q];
+        za = F.zfa[o + q];
+        if (BOTH) zb = F.zfb[o + q];
+        r = F.r[o + q];
+        d = F.d[o + q];
+        z = F.z[o + q];
+    };
+    load(lane);
+    for (int q0 = 0; q0 < n; q0 += 64) {
+        const int count = min(64, n - q0);
+        double *t = term + lane * ROW;
+        if (lane < count) {
+            const double common[8] = {w, w * l, 0, 0, w != 0 ? 1.0 : 0.0, w * (r - rc),
+                                      w * (d - dc), w * z};
 #pragma unroll
-        for (int k = 0; k < PREFIX_BATCH; ++k) {
-            const int q = min(q0 + k, n - 1);
-            wq[k] = w[q];
-            xq[k] = x[q];
-            lq[k] = l[q];
+            for (int c = 0; c < FIELDS; ++c) {
+                const double zw = w * (c < 8 ? za : zb);
+                t[c] = (c & 7) == 2 ? zw : (c & 7) == 3 ? zw * l : common[c & 7];
+            }
         }
+        __syncthreads();
+        load(q0 + 64 + lane);
+        if (lane < FIELDS) {
+            double *field = term + lane;
+            int k = 0;
+            for (; k + 8 <= count; k += 8) {
+                double v[8];
 #pragma unroll
-        for (int k = 0; k < PREFIX_BATCH; ++k) {
-            if (q0 + k >= n) break;
-            double v = wq[k] * (xq[k] - off);
-            if (c == 0) v = wq[k];
-            if (c == 3) v *= lq[k];
-            if (c == 4) v = wq[k] != 0 ? 1.0 : 0.0;
-            acc += v;
-            out[(int64_t)(q0 + k + 1) * 8] = acc;
+                for (int u = 0; u < 8; ++u) v[u] = field[(k + u) * ROW];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    acc += v[u];
+                    field[(k + u) * ROW] = acc;
+                }
+            }
+            for (; k < count; ++k) {
+                acc += field[k * ROW];
+                field[k * ROW] = acc;
+            }
         }
+        __syncthreads();
+        for (int k = lane; k < 8 * count; k += 64) {
+            const int64_t to = (int64_t)(q0 + 1 + (k >> 3)) * 8;
+            const double *row = term + (k >> 3) * ROW + (k & 7);
+            out(k & 7)[to] = row[0];
+            if (BOTH) out(8 + (k & 7))[to] = row[8];
+        }
+        __syncthreads();   // the terms are read
     }
 }
 
-// Index tables of r_comov and dist_m (BandTable) of the listed forests: one wave per forest, a
-// binary search per entry.
+// Index tables of r_comov (blockIdx.y 0) and dist_m (1) (BandTable) of the listed forests: one
+// workgroup per forest and coordinate, a binary search per entry: 10 us for 100 forests, 49 us for
+// 3000 (one wave for both coordinates: 68 us and 150 us).
 __global__ __launch_bounds__(256) void dmat_table_kernel(DmatForests F, DmatListed T,
                                                          int32_t *__restrict__ tr,
                                                          int32_t *__restrict__ td) {
-    const int64_t at = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (at >= T.count) return;
-    const int lane = threadIdx.x & 63;
-    const int64_t f = T.forest[at].forest;
+    const int64_t f = T.forest[blockIdx.x].forest;
     const int64_t o = F.off[f];
     const int n = (int)(F.off[f + 1] - o);
-    const int64_t to = T.forest[at].at;
-    for (int axis = 0; axis < 2; ++axis) {
-        const double *__restrict__ v = (axis ? F.d : F.r) + o;
-        const double v0 = v[0], h = band_mean_step(v0, v[n - 1], n);
-        for (int k = lane; k < n; k += 64) {
-            const double x = v0 + k * h;
-            int lo = 0;
-            for (int m = n; m > 0;) {
-                const int half = m >> 1;
-                if (v[lo + half] < x) { lo += half + 1; m -= half + 1; }
-                else m = half;
-            }
-            (axis ? td : tr)[to + k] = lo;
+    if (n <= 0) return;
+    const double *__restrict__ v = (blockIdx.y ? F.d : F.r) + o;
+    int32_t *__restrict__ first = (blockIdx.y ? td : tr) + T.forest[blockIdx.x].at;
+    const double v0 = v[0], h = band_mean_step(v0, v[n - 1], n);
+    for (int k = threadIdx.x; k < n; k += 256) {
+        const double x = v0 + k * h;
+        int lo = 0;
+        for (int m = n; m > 0;) {
+            const int half = m >> 1;
+            if (v[lo + half] < x) { lo += half + 1; m -= half + 1; }
+            else m = half;
         }
+        first[k] = lo;
     }
 }
 
@@ -485,7 +509,7 @@ __global__ __launch_bounds__(256) void dmat_band_count_kernel(DmatConst C, DmatB
 // One workgroup: list offsets of the tiles and their work items of at most item_pairs pairs.
 __global__ __launch_bounds__(1024) void dmat_band_scan_kernel(int tiles, int item_pairs,
                                                               DmatBandWork W) {
-    __shared__ int s_list[1024], s_item[1024];
+    __shared__ int s_list[16], s_item[16];   // of a wave
     const int tid = threadIdx.x;
     const int per = (tiles + 1023) / 1024;
     const int k0 = min(tiles, tid * per), k1 = min(tiles, k0 + per);
@@ -494,23 +518,31 @@ __global__ __launch_bounds__(1024) void dmat_band_scan_kernel(int tiles, int ite
         n += W.tile_count[k];
         m += (W.tile_count[k] + item_pairs - 1) / item_pairs;
     }
-    s_list[tid] = n;
-    s_item[tid] = m;
-    __syncthreads();
-    if (tid == 0) {
-        int a = 0, b = 0;
-        for (int k = 0; k < 1024; ++k) {
-            const int x = s_list[k], y = s_item[k];
-            s_list[k] = a;
-            s_item[k] = b;
+    // exclusive sums over the threads: inside each wave, then over the waves
+    int a = n, b = m;
+    const int lane = tid & 63, wave = tid >> 6;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int x = __shfl_up(a, d, 64), y = __shfl_up(b, d, 64);
+        if (lane >= d) {
             a += x;
             b += y;
         }
-        *W.num_items = b;
-        *W.queue = 0;
+    }
+    if (lane == 63) {
+        s_list[wave] = a;
+        s_item[wave] = b;
     }
     __syncthreads();
-    int first = s_list[tid], item = s_item[tid];
+    int before = 0, items_before = 0;
+    for (int k = 0; k < wave; ++k) {
+        before += s_list[k];
+        items_before += s_item[k];
+    }
+    if (tid == 1023) {
+        *W.num_items = items_before + b;
+        *W.queue = 0;
+    }
+    int first = before + a - n, item = items_before + b - m;
     for (int k = k0; k < k1; ++k) {
         const int count = W.tile_count[k];
         W.tile_count[k] = first;   // fill position of the list kernel
@@ -1014,11 +1046,13 @@ hipError_t launch_dmat_prefix(const DmatForests &F, const DmatListed &T, DmatPre
                               DmatPrefix *pb, int32_t *table_r, int32_t *table_d,
                               hipStream_t stream) {
     if (T.count <= 0) return hipSuccess;
-    const int64_t blocks = ((pb ? 16 : 8) * T.count + 255) / 256;
-    hipLaunchKernelGGL(dmat_prefix_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, F, T, pa,
-                       pb);
-    hipLaunchKernelGGL(dmat_table_kernel, dim3((unsigned)((T.count + 3) / 4)), dim3(256), 0,
-                       stream, F, T, table_r, table_d);
+    const dim3 forests((unsigned)T.count);
+    if (pb)
+        hipLaunchKernelGGL(dmat_prefix_kernel<true>, forests, dim3(64), 0, stream, F, T, pa, pb);
+    else
+        hipLaunchKernelGGL(dmat_prefix_kernel<false>, forests, dim3(64), 0, stream, F, T, pa, pb);
+    hipLaunchKernelGGL(dmat_table_kernel, dim3((unsigned)T.count, 2), dim3(256), 0, stream, F, T,
+                       table_r, table_d);
     return hipGetLastError();
 }
 
