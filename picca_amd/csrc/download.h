@@ -13,10 +13,11 @@
 #include <stdint.h>
 
 #include <algorithm>
-#include <atomic>
+#include <condition_variable>
 #include <cstdlib>
 #include <cstring>
-#include <system_error>
+#include <exception>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -106,10 +107,12 @@ hipError_t download(DownloadRing &ring, const void *from, int64_t bytes, hipStre
                                       hipMemcpyDeviceToHost, stream);
         return e == hipSuccess ? hipEventRecord(ring.copied[c % SLOTS], stream) : e;
     };
-    std::atomic<int64_t> ready{0};    // chunks copied
-    std::atomic<bool> failed{false};
-    std::vector<std::atomic<int>> taken((size_t)chunks);   // threads done with a chunk
-    for (auto &t : taken) t.store(0, std::memory_order_relaxed);
+    // chunks copied, pieces taken over all chunks; a thread takes its slice of a chunk once, and
+    // the next chunk is not ready before every slice of this one is taken
+    std::mutex lock;
+    std::condition_variable copied, took;
+    int64_t ready = 0, taken = 0;
+    bool settled = false, failed = false;   // settled: the number of workers is known
     const unsigned hw = std::thread::hardware_concurrency();
     int workers = (int)std::max<unsigned>(1, std::min<unsigned>(hw, 16));
     // slice w of chunk c, in whole 4 KiB pages
@@ -118,38 +121,54 @@ hipError_t download(DownloadRing &ring, const void *from, int64_t bytes, hipStre
         const int64_t step = ((n + workers - 1) / workers + 4095) & ~(int64_t)4095;
         const int64_t a = std::min(n, w * step), b = std::min(n, a + step);
         if (a < b) take((const char *)ring.slot[c % SLOTS] + a, lo + a, lo + b);
-        taken[(size_t)c].fetch_add(1, std::memory_order_release);
     };
     std::vector<std::thread> pool;
-    std::atomic<int> started{0};   // 0: the number of workers is not settled
     try {
+        pool.reserve((size_t)workers);
         for (int w = 1; w < workers; ++w)
             pool.emplace_back([&, w] {
-                while (started.load(std::memory_order_acquire) == 0) std::this_thread::yield();
                 for (int64_t c = 0; c < chunks; ++c) {
-                    while (ready.load(std::memory_order_acquire) <= c) {
-                        if (failed.load(std::memory_order_acquire)) return;
-                        std::this_thread::yield();
+                    {
+                        std::unique_lock<std::mutex> hold(lock);
+                        copied.wait(hold, [&] { return settled && (failed || ready > c); });
+                        if (failed) return;
                     }
                     work(c, w);
+                    std::lock_guard<std::mutex> hold(lock);
+                    if (++taken == (c + 1) * (workers - 1)) took.notify_one();
                 }
             });
-    } catch (const std::system_error &) {   // fewer threads
+    } catch (const std::exception &) {   // fewer threads
     }
-    workers = (int)pool.size() + 1;
-    started.store(1, std::memory_order_release);
+    {
+        std::lock_guard<std::mutex> hold(lock);
+        workers = (int)pool.size() + 1;
+        settled = true;
+    }
     for (int64_t c = 0; c < std::min<int64_t>(SLOTS, chunks) && err == hipSuccess; ++c)
         err = issue(c);
     for (int64_t c = 0; c < chunks && err == hipSuccess; ++c) {
         err = hipEventSynchronize(ring.copied[c % SLOTS]);
         if (err != hipSuccess) break;
-        ready.store(c + 1, std::memory_order_release);
+        {
+            std::lock_guard<std::mutex> hold(lock);
+            ready = c + 1;
+        }
+        copied.notify_all();
         work(c, 0);
-        while (taken[(size_t)c].load(std::memory_order_acquire) < workers)
-            std::this_thread::yield();
+        {
+            std::unique_lock<std::mutex> hold(lock);
+            took.wait(hold, [&] { return taken == (c + 1) * (workers - 1); });
+        }
         if (c + SLOTS < chunks) err = issue(c + SLOTS);
     }
-    if (err != hipSuccess) failed.store(true, std::memory_order_release);
+    if (err != hipSuccess) {
+        {
+            std::lock_guard<std::mutex> hold(lock);
+            failed = true;
+        }
+        copied.notify_all();
+    }
     for (auto &t : pool) t.join();
     if (err != hipSuccess) (void)hipStreamSynchronize(stream);   // no copy into the ring is left
     return err;
@@ -159,6 +178,14 @@ hipError_t download(DownloadRing &ring, const void *from, int64_t bytes, hipStre
 template <bool ADD>
 hipError_t download_values(DownloadRing &ring, const double *from, int64_t n, hipStream_t stream,
                            double *out) {
+    // of 8 to 16 MB the threads cost more than they save (12.5 MB: 1.24 ms with the ring, 0.95 ms
+    // without; 18 MB: 1.2 ms and 1.35 ms)
+    if (!ADD && n * 8 > DownloadRing::BYTES && n * 8 <= 2 * DownloadRing::BYTES) {
+        const hipError_t err =
+            hipMemcpyAsync(out, from, (size_t)n * 8, hipMemcpyDeviceToHost, stream);
+        const hipError_t done = hipStreamSynchronize(stream);
+        return err == hipSuccess ? done : err;
+    }
     return download(ring, from, n * 8, stream, [out](const char *src, int64_t lo, int64_t hi) {
         const double *s = (const double *)src;
         double *o = out + lo / 8;

@@ -1,6 +1,7 @@
 """Results of more than one chunk of the pinned download ring: a matrix of 13.5 MB added to what
 the caller's array holds, and the six interleaved results of 300 000 continuum fits."""
 import ctypes
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -8,7 +9,7 @@ import pytest
 import walk_cases as W
 from picca_amd import continuum
 from picca_amd._native import check
-from picca_amd.engine import as_f64, as_i32, get_engine, params_from_globals, ptr
+from picca_amd.engine import Engine, as_f64, as_i32, get_engine, params_from_globals, ptr
 from test_gpu_continuum_lengths import make_inputs
 from test_gpu_dmat_band import dmat_store, with_model
 
@@ -55,3 +56,41 @@ def test_many_continuum_fits():
            for x, m in ((few, 5), (many, copies))]
     for key in ("a", "b", "chi2", "ndata", "status"):
         assert np.array_equal(np.tile(res[0][key], copies // 5), res[1][key]), key
+
+
+def test_two_contexts_at_once():
+    """Two contexts on two host threads, each with downloads of several chunks."""
+    rng = np.random.default_rng(3)
+    inputs = [(rng.normal(size=(30, bins)), rng.uniform(0.5, 2, (30, bins)))
+              for bins in (1500, 1460)]
+    engines = [Engine(0), Engine(0)]
+    try:
+        alone = [eng.cov_subsample(*x)[0] for eng, x in zip(engines, inputs)]
+        assert all(c.nbytes > 2 ** 24 for c in alone)
+        with ThreadPoolExecutor(2) as pool:
+            together = [pool.submit(lambda e=eng, v=x: [e.cov_subsample(*v)[0]
+                                                        for _ in range(20)])
+                        for eng, x in zip(engines, inputs)]
+            for first, results in zip(alone, together):
+                assert all(np.array_equal(first, c) for c in results.result())
+    finally:
+        for eng in engines:
+            eng.close()
+
+
+def test_sizes_around_a_chunk():
+    """Results of one chunk, just below and just above, of two chunks and of more, one after
+    the other in one context, so that the ring grows; the matrix is symmetric by construction, so
+    that a piece in the wrong place shows."""
+    rng = np.random.default_rng(4)
+    eng = Engine(0)
+    try:
+        for bins in (3, 90, 91, 1023, 1024, 1025, 1448, 1449, 1774, 100):
+            xi, w = rng.normal(size=(20, bins)), rng.uniform(0.5, 2, (20, bins))
+            cov = eng.cov_subsample(xi, w)[0]
+            mean = (xi * w).sum(0) / w.sum(0)
+            x = w * (xi - mean)
+            ref = x.T @ x / np.outer(w.sum(0), w.sum(0))
+            np.testing.assert_allclose(cov, ref, rtol=1e-9, atol=1e-12 * np.abs(ref).max())
+    finally:
+        eng.close()
