@@ -457,9 +457,8 @@ typedef struct picca_wick_report {
  * wx + wx_offsets[f] is forest f's n x n weighted 1-D correlation
  * w_k w_l xi_1d(|log_lambda_k - log_lambda_l|) sqrt(v_k v_l) (py/picca/cf.py:1392-1398),
  * symmetric (its rows are read as its columns), needed for every forest of the pair list.
- * Device memory per call: per batch 16 bytes per segment (consecutive pixels of delta1 that one
- * pixel of delta2 pairs with in one bin) and up to 1 GiB of segment sums, more only where the
- * segments of one (pair, bin) need it.  Outputs (accumulated):
+ * Device memory per call: per batch 32 bytes per segment (consecutive pixels of delta1 that one
+ * pixel of delta2 pairs with in one bin) and up to 1 GiB of segment sums.  Outputs (accumulated):
  * weights_wick[nb], num_pairs_wick[nb], t1, t2, t3 [nb][nb].  report may be NULL.
  */
 int picca_wick_t123(picca_ctx *ctx, const picca_cf_params *params, int64_t num_pairs,

@@ -232,7 +232,7 @@ struct picca_ctx {
     DeviceBuffer<int64_t> wk_wxoff;
     DeviceBuffer<int32_t> wk_segcount, wk_segpos, wk_forests;
     DeviceBuffer<int4> wk_seg, wk_seg_raw;
-    DeviceBuffer<picca::WickTask> wk_task;
+    DeviceBuffer<picca::WickTask> wk_task, wk_rows;   // (pair, bin); the row kernel's parts
     DeviceBuffer<unsigned long long> wk_nb, wk_stats;
 
     // continuum fit: resident spectra (forest pixels) and per-forest results

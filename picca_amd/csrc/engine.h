@@ -447,8 +447,8 @@ struct WickPairs {
     int32_t count;
 };
 
-// One (pair, bin P): the pair's segments in the bin, all of the pair's segments, and the first
-// entry of its rows in rsum.
+// One (pair, bin P), or part of its segments: the segments, all of the pair's segments, and the
+// first entry of their rows in rsum.
 struct WickTask {
     int32_t pair, bin, start, count, pair_start, pair_count;
     int64_t rows;

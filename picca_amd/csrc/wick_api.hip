@@ -98,14 +98,14 @@ int picca_wick_t123(picca_ctx *ctx, const picca_cf_params *params, int64_t num_p
                      ctx->o_dmat.ptr + 2 * nb * nb, ctx->wk_stats.ptr};
 
     // batches of pairs: at most 2^20 (pair, bin) counts and 2^27 pixel pairs (the segments are
-    // fewer); inside a batch, runs of tasks whose segment sums fit 1 GiB
+    // fewer); inside a batch, runs of tasks, or of parts of them, whose segment sums fit 1 GiB
     const int64_t pixel_budget = (int64_t)1 << 27, count_budget = (int64_t)1 << 20;
     const int64_t rsum_budget = (int64_t)1 << 27;
     double total_ms = 0.0;
     int64_t batches = 0;
     std::vector<double> cs;
     std::vector<int32_t> seg_count, seg_pos;
-    std::vector<picca::WickTask> tasks;
+    std::vector<picca::WickTask> tasks, rows_of;
     auto add_time = [&]() -> int {
         PICCA_HIP_CHECK(hipEventRecord(ctx->ev_stop, ctx->stream));
         PICCA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
@@ -160,6 +160,8 @@ int picca_wick_t123(picca_ctx *ctx, const picca_cf_params *params, int64_t num_p
             const size_t first_task = tasks.size();
             for (int64_t p = 0; p < nb; ++p) {
                 const int32_t n = seg_count[(size_t)(k * nb + p)];
+                if (n < 0 || segs + n > INT32_MAX)   // a forest pair whose pixels hardly rise
+                    return fail(PICCA_E_VALUE, "more than 2^31 segments in one pair");
                 seg_pos[(size_t)(k * nb + p)] = (int32_t)segs;
                 if (n > 0)
                     tasks.push_back(picca::WickTask{(int32_t)k, (int32_t)p, (int32_t)segs, n,
@@ -171,23 +173,34 @@ int picca_wick_t123(picca_ctx *ctx, const picca_cf_params *params, int64_t num_p
         }
         ++batches;
         if (!tasks.empty()) {
-            // runs of tasks: rsum rows from 0 in each
+            // The row kernel's tasks: a (pair, bin) each, in parts where its segment sums exceed
+            // the budget, and runs of them whose sums fit it, from row 0 in each run.
+            rows_of.clear();
             std::vector<int64_t> run_begin{0};
             int64_t rows = 0, most = 0;
-            for (size_t t = 0; t < tasks.size(); ++t) {
-                const int32_t f = pair_a[p0 + tasks[t].pair];
-                const int64_t need = (int64_t)tasks[t].count * (off[f + 1] - off[f] + 1);
-                if (rows > 0 && rows + need > rsum_budget) {
-                    run_begin.push_back((int64_t)t);
-                    rows = 0;
+            for (const picca::WickTask &task : tasks) {
+                const int32_t f = pair_a[p0 + task.pair];
+                const int64_t row = off[f + 1] - off[f] + 1;
+                const int32_t part = (int32_t)std::min<int64_t>(
+                    task.count, std::max<int64_t>(1, rsum_budget / row));
+                for (int32_t first = 0; first < task.count; first += part) {
+                    picca::WickTask t = task;
+                    t.start += first;
+                    t.count = std::min(part, task.count - first);
+                    if (rows > 0 && rows + t.count * row > rsum_budget) {
+                        run_begin.push_back((int64_t)rows_of.size());
+                        rows = 0;
+                    }
+                    t.rows = rows;
+                    rows += t.count * row;
+                    most = std::max(most, rows);
+                    rows_of.push_back(t);
                 }
-                tasks[t].rows = rows;
-                rows += need;
-                most = std::max(most, rows);
             }
-            run_begin.push_back((int64_t)tasks.size());
+            run_begin.push_back((int64_t)rows_of.size());
             PICCA_HIP_CHECK(ctx->wk_segpos.upload(seg_pos.data(), (size_t)cells, ctx->stream));
             PICCA_HIP_CHECK(ctx->wk_task.upload(tasks.data(), tasks.size(), ctx->stream));
+            PICCA_HIP_CHECK(ctx->wk_rows.upload(rows_of.data(), rows_of.size(), ctx->stream));
             PICCA_HIP_CHECK(ctx->wk_seg_raw.reserve((size_t)segs));
             PICCA_HIP_CHECK(ctx->wk_seg.reserve((size_t)segs));
             PICCA_HIP_CHECK(ctx->wk_rsum.reserve((size_t)most));
@@ -201,7 +214,7 @@ int picca_wick_t123(picca_ctx *ctx, const picca_cf_params *params, int64_t num_p
             W.task = ctx->wk_task.ptr;
             PICCA_HIP_CHECK(picca::launch_wick_sort(W, (int64_t)tasks.size(), ctx->stream));
             for (size_t r = 0; r + 1 < run_begin.size(); ++r) {
-                W.task = ctx->wk_task.ptr + run_begin[r];
+                W.task = ctx->wk_rows.ptr + run_begin[r];
                 PICCA_HIP_CHECK(picca::launch_wick_rows(C, I, P, W, O,
                                                         run_begin[r + 1] - run_begin[r],
                                                         ctx->stream));

@@ -1,11 +1,13 @@
 """Wick terms from segments at their edges: pixels in no order (segments of one pixel, more of
-them in one bin than are sorted), one-pixel forests, one bin, a pair of a forest with itself.
-Against the FP64 oracle, bars of test_gpu_wick."""
+them in one bin than the 4096 that are sorted), one-pixel forests, one bin, a pair of a forest with
+itself.  Against the FP64 oracle, bars of test_gpu_wick.  And a (pair, bin) whose segment sums
+exceed the budget of 1 GiB, against the same pixels in rising order."""
 import numpy as np
 import pytest
+import torch
 
 from oracle import cf_oracle as O
-from picca_amd.engine import get_engine, params_from_globals
+from picca_amd.engine import Engine, get_engine, params_from_globals
 from picca_amd.store import ForestStore
 from test_gpu_wick import _G, assert_close
 
@@ -25,11 +27,27 @@ def forests(rng, lengths, shuffled):
                        np.arange(m))
 
 
+def most_segments(store, a, b, ang, bins, r_max):
+    """The most segments that any (pair, bin) has."""
+    most = 0
+    for x, y, angle in zip(a, b, ang):
+        r1, r2 = (store.r_comov[store.offsets[k]:store.offsets[k + 1]] for k in (x, y))
+        r_par = np.abs(r1[:, None] - r2[None]) * np.cos(angle / 2)
+        r_trans = (r1[:, None] + r2[None]) * np.sin(angle / 2)
+        key = (np.floor(r_trans / r_max * bins) + bins * np.floor(r_par / r_max * bins)).astype(int)
+        key[(r_par >= r_max) | (r_trans >= r_max)] = -1
+        first = np.diff(key, axis=0, prepend=-1) != 0   # along delta1's pixels
+        counts = np.bincount(key[first & (key >= 0)], minlength=1)
+        most = max(most, int(counts.max()))
+    return most
+
+
 @pytest.mark.parametrize("shuffled", [False, True])
-@pytest.mark.parametrize("lengths,bins,r_max", [((130, 140), 1, 300.0), ((1, 2, 100), 1, 300.0),
-                                                ((1, 2, 300), 7, 20.0),
-                                                ((255, 256, 257, 65), 7, 20.0)])
-def test_segments(lengths, shuffled, bins, r_max):
+@pytest.mark.parametrize("lengths,bins,r_max,unsorted",
+                         [((130, 140), 1, 300.0, False), ((1, 2, 100), 1, 300.0, False),
+                          ((1, 2, 300), 7, 20.0, False), ((255, 256, 257, 65), 7, 20.0, False),
+                          ((300, 250), 1, 20.0, True)])
+def test_segments(lengths, shuffled, bins, r_max, unsorted):
     rng = np.random.default_rng(len(lengths) + 10 * bins)
     store = forests(rng, lengths, shuffled)
     g = _G()
@@ -38,6 +56,8 @@ def test_segments(lengths, shuffled, bins, r_max):
     m = len(lengths)
     a, b = (x.ravel() for x in np.meshgrid(np.arange(m), np.arange(m), indexing="ij"))
     ang = rng.uniform(0.001, 0.01, len(a))
+    # (WICK_SORT of engine.h)
+    assert (most_segments(store, a, b, ang, bins, r_max) > 4096) == (shuffled and unsorted)
     off, mats = [0], []
     for k in range(m):
         n = lengths[k]
@@ -64,3 +84,49 @@ def test_segments(lengths, shuffled, bins, r_max):
     for k in range(3):
         assert_close(mine[2 + k], t[k].reshape(nb, nb), "t%d" % (k + 1))
     assert 0 < mine[5]["products"] <= n * (n - 1) // 2
+
+
+def test_segment_sums_in_parts():
+    """Two forests of 900 pixels in no order, half of the pixel pairs in the one bin: 2e5 segments
+    of 901 sums are 1.4 GiB, which the row kernel takes in parts.  The terms are sums over pixel
+    pairs, so that the order of the pixels only reorders FP64 sums (t2, t3 cancel: 1e-10 of the
+    sum of magnitudes)."""
+    rng = np.random.default_rng(11)
+    n = 900
+    r = [3800.0 + np.cumsum(rng.uniform(0.2, 1.0, n)) for _ in range(2)]
+    w, zev1, zev2 = rng.uniform(0.5, 2.0, (3, 2, n))
+    wx = [0.01 * (q + q.T) for q in rng.normal(size=(2, n, n))]
+    g = _G()
+    g.num_bins_r_par = g.num_bins_r_trans = 1
+    g.r_par_max, g.r_trans_max = 160.0, 300.0
+    ang, pair = np.array([0.002]), np.array([[0], [1]])
+    out = []
+    for shuffled in (False, True):
+        order = [rng.permutation(n) if shuffled else np.arange(n) for _ in range(2)]
+        flat = lambda x: np.concatenate([x[k][order[k]] for k in range(2)])
+        rr = flat(r)
+        store = ForestStore(np.array([0, n, 2 * n]), 2.0 + rr / 1e4, rr, rr, flat(w), 0 * rr,
+                            np.full(2, 3.0), np.array([0.01, 0.011]), np.full(2, 0.01),
+                            np.arange(2))
+        m = np.concatenate([wx[k][np.ix_(order[k], order[k])].ravel() for k in range(2)])
+        if shuffled:
+            segments = most_segments(store, *pair, ang, 1, 160.0)
+            assert segments * (n + 1) * 8 > 1.2 * 2 ** 30
+        eng = Engine(0)
+        try:
+            eng.set_forests(store)
+            free = torch.cuda.mem_get_info(0)[0]
+            out.append(eng.wick_t123(params_from_globals(g), *pair, ang, flat(zev1), flat(zev2),
+                                     np.array([0, n * n]), m))
+            held = free - torch.cuda.mem_get_info(0)[0]
+        finally:
+            eng.close()
+        assert held < (1 << 30) + 32 * n * n + (64 << 20), held
+    rising, mixed = out
+    assert np.array_equal(rising[1], mixed[1]) and rising[1][0] > n * n // 3
+    np.testing.assert_allclose(mixed[0], rising[0], rtol=1e-12)
+    np.testing.assert_allclose(mixed[2], rising[2], rtol=1e-12)
+    big = np.abs(wx[0]).sum() * np.abs(wx[1]).sum()
+    for k in (3, 4):
+        np.testing.assert_allclose(mixed[k], rising[k], rtol=0, atol=1e-10 * big)
+    assert mixed[5]["products"] == rising[5]["products"]
