@@ -50,3 +50,49 @@ def test_lengths(constant):
         # (a, b) are known to the square root of the stopping rule's 1e-12
         assert res["a"][k] == pytest.approx(a, rel=1e-5)
         assert abs(res["b"][k] - b) <= 1e-5 * abs(a)
+
+
+def test_order_0():
+    inputs, parts = make_inputs(6)
+    res = continuum.fit_arrays(inputs, order=0)
+    assert np.all(res["status"] == 0) and not res["b"].any()
+    for k, spec in enumerate(parts):
+        a, _, chi, _, _ = C.fit(spec, order=0)
+        assert res["ndata"][k] == (spec["ivar"] > 0).sum()
+        assert res["chi2"][k] == pytest.approx(chi, rel=1e-9)
+        assert res["a"][k] == pytest.approx(a, rel=1e-5)
+
+
+@pytest.mark.parametrize("constant", [False, True])
+def test_validity_of_every_wave(constant):
+    """The checks of the final continuum see each pixel, whichever wave holds it, masked ones too:
+    negative in the last or the first pixel alone (status 2), zero but for the last or the first
+    pixel (valid), zero everywhere (3)."""
+    inputs, parts = make_inputs(7)
+    specs, want, orders = [], [], []
+    for p in parts:
+        n = len(p["flux"])
+        if n < 63:
+            continue
+        for kind, status in (("negative_last", 2), ("negative_first", 2), ("last", 0),
+                             ("first", 0), ("none", 3)):
+            q = {k: p[k].copy() for k in ("flux", "ivar", "mean_cont", "x", "eta", "var_lss",
+                                          "fudge")}
+            pixel = n - 1 if "last" in kind else 0
+            if "negative" in kind:
+                q["mean_cont"][pixel] *= -1
+                q["ivar"][pixel] = 0.0
+            else:
+                keep = q["mean_cont"][pixel]
+                q["mean_cont"][:] = 0.0
+                q["flux"][pixel], q["ivar"][pixel] = 1.5 * keep, 10.0
+                if kind != "none":
+                    q["mean_cont"][pixel] = keep
+            specs.append(q)
+            want.append(status)
+            orders.append(1 if "negative" in kind else 0)
+    many = {k: np.concatenate([q[k] for q in specs]) for k in specs[0]}
+    many["offsets"] = np.concatenate([[0], np.cumsum([len(q["flux"]) for q in specs])])
+    res = continuum.fit_arrays(many, order=np.array(orders), use_constant_weight=constant)
+    assert list(res["status"]) == want
+    assert list(res["ndata"]) == [(q["ivar"] > 0).sum() for q in specs]
