@@ -354,8 +354,12 @@ int picca_xi_set_pairs(picca_ctx *ctx, int64_t num_pairs, const int32_t *pair_a,
 
 namespace {
 
-// Windows of r_par rows up to which the cross-correlation takes the specialised kernel: 16
-// windows of 50 rows hold 800 x 50 bins.
+// Windows of r_par rows up to which the cross-correlation takes the specialised kernel, a launch
+// each: enough for 800 x 50 bins, eight times those of a usual run.  The general kernel, which adds
+// its runs to the rows in HBM, takes over there without being the faster one (120 x 120 forests of
+// the 0.8 A grid, 100 x 50 bins in 2 windows 5.6 ms against 155 ms, 400 x 50 in 7 14 ms against 549
+// ms, 800 x 50 in 13 23 ms against 899 ms; 1600 x 50 general 781 ms): the limit bounds the launches
+// of one call.
 constexpr int XI_MAX_ROW_WINDOWS = 16;
 
 // picca_xi_execute's work with the output rows, the work-queue head and the counters in the

@@ -352,7 +352,8 @@ inline hipError_t fetch_matrix(picca_ctx *ctx, const MatrixBlock &B, const Accep
     };
     const int64_t bytes = 8 * B.words();
     const bool whole = bytes <= picca_host::DownloadRing::BYTES;
-    hipError_t err = ctx->ring.fetch(B.counters, whole ? bytes : HEAD, ctx->stream);
+    hipError_t err = ctx->ring.ensure(bytes);
+    if (err == hipSuccess) err = ctx->ring.fetch(B.counters, whole ? bytes : HEAD, ctx->stream);
     if (err != hipSuccess) return err;
     unsigned long long counters[MATRIX_COUNTERS];
     std::memcpy(counters, ctx->ring.slot[0], HEAD);

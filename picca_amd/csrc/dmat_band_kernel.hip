@@ -3,11 +3,10 @@
 // sums over the forests instead of pixel pair by pixel pair.
 //
 // It covers the standard auto-correlation binning (r_par_min == 0, |r_par|; forest x quasar
-// pairs below), forests whose
-// r_comov and dist_m rise strictly with steps above the rounding margins, model bins that
-// split the data bins in 2^k parts (so that a model bin lies in one data bin to the last bit)
-// and no pair-redshift, zerr or same-half-plate cut on the pair; the host sends the other pairs
-// to dmat_kernel.hip.  Every pair in range is then selected, the model bins U of a pair are all
+// pairs below), forests whose r_comov and dist_m rise strictly with steps above the rounding
+// margins and whose weights are level (xi_walk.h), model bins that split the data bins in 2^k
+// parts (so that a model bin lies in one data bin to the last bit) and no pair-redshift, zerr or
+// same-half-plate cut on the pair; the host sends the other pairs to dmat_kernel.hip.  Every pair in range is then selected, the model bins U of a pair are all
 // that it reaches, and the pair-bin term of (A, M) is the pair's sum of w1 w2 zf in M.
 //
 // dmat_band_pass_kernel  one workgroup per forest pair, a lane per pixel of delta1: the run walk
@@ -35,9 +34,12 @@
 // every 16 pixels.  On those pairs (2500 forests, 50 x 50 data and 100 x 50 model bins) the
 // call takes 88 ms against 350 ms, the fill 61 ms against 264 ms, the pass 15 ms against 83 ms.
 //
-// A pair whose bins do not follow the runs (an r_trans or r_par that rounds up to the range's
-// end, which the reference writes into the next row or past the end) is left to
-// dmat_kernel.hip: the pass puts it in the redo list and adds nothing.
+// In range means binned here: for r_trans, and for |r_par| from 0, x < end gives x / end <=
+// 1 - 2^-53 after rounding, which times n stays below n.  Only a signed r_par can round to the end
+// of its range (its distance from r_par_min may); such a quasar's pair, and one with a pixel at
+// r_par_min exactly, which xcf counts apart, goes into the redo list for dmat_kernel.hip and adds
+// nothing.  The pass does the same with a run outside the rows that the host bounded, which the
+// bounds leave no pair.
 #include <hip/hip_runtime.h>
 #include <limits.h>
 #include <stdint.h>
@@ -800,7 +802,7 @@ __global__ __launch_bounds__(DMAT_BAND_FILL_BLOCK, 3) void dmat_band_fill_kernel
 // edges, the matrix-core panel holds 16 pairs (K = the pairs), and the tile of a data row and
 // its own model rows adds the pair-bin term, weights_dmat and the effective sums.  With a pair
 // per workgroup and one quasar pixel a tile, the general pass and fill leave 15 of 16 lanes and
-// rows of K idle: 3000 forests, 50k kept pairs, 100 x 50 bins take 2.4 ms here, 36 ms (fill) and
+// rows of K idle: 3000 forests, 145k kept pairs, 100 x 50 bins take 2.4 ms here, 36 ms (fill) and
 // 11 ms (pass) there.  Bound by the chain of table, probe and prefix loads of an edge.
 
 // Rows that each pair reaches (as non-empty pixel ranges for the tile lists), and the pairs

@@ -517,7 +517,9 @@ struct ContOut {
 };
 
 // Pixels of a forest that one lane of the fit holds in registers: a forest takes 1, 2, 4 or 8
-// waves, or the kernel that reads its pixels at every evaluation.
+// waves, or the kernel that reads its pixels at every evaluation.  Also where two waves are half
+// empty it pays: 6000 forests of 641 to 900 pixels (the 0.8 A grid) take 0.146 ms against 0.305 ms
+// with their pixels read at every evaluation, of 500 to 640 pixels 0.095 ms against 0.226 ms.
 constexpr int CONT_PIXELS_PER_LANE = 10;
 constexpr int CONT_CLASSES = 5;
 

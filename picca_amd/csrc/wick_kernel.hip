@@ -26,8 +26,8 @@
 // A step per two segments replaces one per pixel pair and segment (7 pixels a segment on the
 // 0.8 A grid), and the prefix sums of every row of Wx1, which took 7.0 ms of the kernels' 22 ms
 // on 24 pairs (2.6e7 values of Wx) where the segments' sums take 0.49 ms and the rows 2.2 ms
-// (11.1 ms before); the pixel pairs are walked by 240 waves (twice 0.3 ms, 3.6 ms for one workgroup
-// per pair).
+// (11.1 ms before); the pixel pairs are walked by a thread per pixel of delta2 (twice 0.3 ms on
+// those pairs, 3.6 ms for one workgroup per pair).
 // FP64 throughout; bins by truncation after divide-then-multiply, as the reference.
 #include <hip/hip_runtime.h>
 
