@@ -326,7 +326,7 @@ inline hipError_t make_matrix_block(picca_ctx *ctx, int64_t nb, int64_t nm, Matr
 }
 
 // Fetches the counters when the stream is done and, if accept(counters), adds the results to the
-// caller's arrays.  A matrix that fits a chunk of the ring is copied with its counters.
+// caller's arrays.  A matrix of up to 1 MB is copied with its counters.
 template <class Accept>
 inline hipError_t fetch_matrix(picca_ctx *ctx, const MatrixBlock &B, const Accept &accept,
                                double *weights_dmat, double *dmat, double *r_par_eff,
@@ -351,18 +351,16 @@ inline hipError_t fetch_matrix(picca_ctx *ctx, const MatrixBlock &B, const Accep
         }
     };
     const int64_t bytes = 8 * B.words();
-    const bool whole = bytes <= picca_host::DownloadRing::BYTES;
+    const bool whole = bytes <= picca_host::DownloadRing::SMALL;
     hipError_t err = ctx->ring.ensure(bytes);
     if (err == hipSuccess) err = ctx->ring.fetch(B.counters, whole ? bytes : HEAD, ctx->stream);
     if (err != hipSuccess) return err;
     unsigned long long counters[MATRIX_COUNTERS];
-    std::memcpy(counters, ctx->ring.slot[0], HEAD);
+    std::memcpy(counters, ctx->ring.memory, HEAD);
     if (!accept(counters)) return hipSuccess;
     if (!whole)
         return picca_host::download(ctx->ring, B.weights, bytes - HEAD, ctx->stream, add);
-    parallel_for((bytes - HEAD) / 8, [&](int64_t lo, int64_t hi) {
-        add(ctx->ring.slot[0] + HEAD + 8 * lo, 8 * lo, 8 * hi);
-    });
+    add(ctx->ring.memory + HEAD, 0, bytes - HEAD);
     return hipSuccess;
 }
 

@@ -23,38 +23,43 @@
 
 namespace picca_host {
 
-// The pinned memory of one context, freed with it: one slot of the largest result so far (a power
-// of two from 64 KB), from 8 MB on two slots of 8 MB.  (Two of 8 MB for any result took the first
-// download of an engine, of 0.1 to 4 MB, from 0.4-0.8 ms to 0.8-1.9 ms.)
+// The pinned memory of one context, freed with it: one block of the largest result so far (a power
+// of two from 64 KB) up to 1 MB, two chunks of 1 MB for results up to 16 MB, which the calling
+// thread moves on, two of 8 MB beyond, on several threads (12.5 MB: 0.73 ms, with threads 0.83 to
+// 1.24 ms; 18 MB: 1.1 ms with threads, 1.38 ms as one pageable copy).  The first reading of fresh
+// pinned pages takes the host 0.4 ms a MB, as much as a small result's whole call.
 struct DownloadRing {
     static constexpr int SLOTS = 2;
-    static constexpr int64_t BYTES = (int64_t)8 << 20;
-    char *slot[SLOTS] = {nullptr, nullptr};
+    static constexpr int64_t SMALL = (int64_t)1 << 20, LARGE = (int64_t)8 << 20;   // a chunk
+    static constexpr int64_t ONE_THREAD = 2 * LARGE;   // results that take no other threads
+    char *memory = nullptr;
     hipEvent_t copied[SLOTS] = {nullptr, nullptr};
-    int64_t room = 0;   // bytes at slot[0]
+    int64_t room = 0;   // bytes of memory
     bool pinned = false;
     ~DownloadRing() { release(); }
+    // bytes of one chunk of a result that takes several
+    static int64_t chunk(int64_t bytes) { return bytes <= ONE_THREAD ? SMALL : LARGE; }
     void release() {
         for (int k = 0; k < SLOTS; ++k) {
             if (copied[k]) (void)hipEventDestroy(copied[k]);
             copied[k] = nullptr;
         }
-        release_slots();
+        release_memory();
     }
-    void release_slots() {
-        if (slot[0] && pinned)
-            (void)hipHostFree(slot[0]);
+    void release_memory() {
+        if (memory && pinned)
+            (void)hipHostFree(memory);
         else
-            std::free(slot[0]);
-        slot[0] = slot[1] = nullptr;
+            std::free(memory);
+        memory = nullptr;
         room = 0;
     }
-    // Room for a result of `bytes` bytes, in chunks of BYTES; no copy into the slots is under way.
+    // Room for a result of `bytes` bytes; no copy into the memory is under way.
     hipError_t ensure(int64_t bytes) {
         int64_t want = (int64_t)64 << 10;
-        while (want < bytes && want < BYTES) want <<= 1;
-        if (bytes > BYTES) {
-            want = SLOTS * BYTES;
+        while (want < bytes && want < SMALL) want <<= 1;
+        if (bytes > SMALL) {
+            want = SLOTS * chunk(bytes);
             for (int k = 0; k < SLOTS; ++k)
                 if (!copied[k]) {
                     const hipError_t err =
@@ -63,47 +68,47 @@ struct DownloadRing {
                 }
         }
         if (room >= want) return hipSuccess;
-        release_slots();
-        pinned = hipHostMalloc((void **)&slot[0], (size_t)want) == hipSuccess;
+        release_memory();
+        pinned = hipHostMalloc((void **)&memory, (size_t)want) == hipSuccess;
         if (!pinned) {   // no pinned memory left: pageable memory does as well, slower
             (void)hipGetLastError();
-            slot[0] = (char *)std::malloc((size_t)want);
-            if (!slot[0]) return hipErrorOutOfMemory;
+            memory = (char *)std::malloc((size_t)want);
+            if (!memory) return hipErrorOutOfMemory;
         }
         room = want;
-        if (want == SLOTS * BYTES) slot[1] = slot[0] + BYTES;
         return hipSuccess;
     }
-    // The first n <= BYTES bytes at `from`, at slot[0] when it returns.
+    // The first n <= SMALL bytes at `from`, in memory when it returns.
     hipError_t fetch(const void *from, int64_t n, hipStream_t stream) {
         hipError_t err = ensure(n);
         if (err == hipSuccess)
-            err = hipMemcpyAsync(slot[0], from, (size_t)n, hipMemcpyDeviceToHost, stream);
+            err = hipMemcpyAsync(memory, from, (size_t)n, hipMemcpyDeviceToHost, stream);
         const hipError_t done = hipStreamSynchronize(stream);
         return err == hipSuccess ? done : err;
     }
 };
 
 // Calls take(src, lo, hi) for pieces [lo, hi) that cover the first `bytes` bytes at the device
-// pointer `from`, src the host copy of byte lo; on several threads when there is more than a
-// chunk.  The copies follow the stream's work; every piece is taken when it returns.
+// pointer `from`, src the host copy of byte lo; on several threads beyond ONE_THREAD bytes.  The copies
+// follow the stream's work; every piece is taken when it returns.
 template <class Take>
 hipError_t download(DownloadRing &ring, const void *from, int64_t bytes, hipStream_t stream,
                     const Take &take) {
     if (bytes <= 0) return hipSuccess;
     constexpr int SLOTS = DownloadRing::SLOTS;
-    constexpr int64_t CHUNK = DownloadRing::BYTES;
-    if (bytes <= CHUNK) {
+    if (bytes <= DownloadRing::SMALL) {
         const hipError_t one = ring.fetch(from, bytes, stream);
-        if (one == hipSuccess) take((const char *)ring.slot[0], (int64_t)0, bytes);
+        if (one == hipSuccess) take((const char *)ring.memory, (int64_t)0, bytes);
         return one;
     }
+    const int64_t CHUNK = DownloadRing::chunk(bytes);
+    auto slot = [&](int64_t c) { return ring.memory + (c % SLOTS) * CHUNK; };
     hipError_t err = ring.ensure(bytes);
     if (err != hipSuccess) return err;
     const int64_t chunks = (bytes + CHUNK - 1) / CHUNK;
     auto issue = [&](int64_t c) {
         const int64_t lo = c * CHUNK, n = std::min(CHUNK, bytes - lo);
-        hipError_t e = hipMemcpyAsync(ring.slot[c % SLOTS], (const char *)from + lo, (size_t)n,
+        hipError_t e = hipMemcpyAsync(slot(c), (const char *)from + lo, (size_t)n,
                                       hipMemcpyDeviceToHost, stream);
         return e == hipSuccess ? hipEventRecord(ring.copied[c % SLOTS], stream) : e;
     };
@@ -114,13 +119,14 @@ hipError_t download(DownloadRing &ring, const void *from, int64_t bytes, hipStre
     int64_t ready = 0, taken = 0;
     bool settled = false, failed = false;   // settled: the number of workers is known
     const unsigned hw = std::thread::hardware_concurrency();
-    int workers = (int)std::max<unsigned>(1, std::min<unsigned>(hw, 16));
+    int workers = bytes <= DownloadRing::ONE_THREAD
+                      ? 1 : (int)std::max<unsigned>(1, std::min<unsigned>(hw, 16));
     // slice w of chunk c, in whole 4 KiB pages
     auto work = [&](int64_t c, int w) {
         const int64_t lo = c * CHUNK, n = std::min(CHUNK, bytes - lo);
         const int64_t step = ((n + workers - 1) / workers + 4095) & ~(int64_t)4095;
         const int64_t a = std::min(n, w * step), b = std::min(n, a + step);
-        if (a < b) take((const char *)ring.slot[c % SLOTS] + a, lo + a, lo + b);
+        if (a < b) take((const char *)slot(c) + a, lo + a, lo + b);
     };
     std::vector<std::thread> pool;
     try {
@@ -178,14 +184,6 @@ hipError_t download(DownloadRing &ring, const void *from, int64_t bytes, hipStre
 template <bool ADD>
 hipError_t download_values(DownloadRing &ring, const double *from, int64_t n, hipStream_t stream,
                            double *out) {
-    // of 8 to 16 MB the threads cost more than they save (12.5 MB: 1.24 ms with the ring, 0.95 ms
-    // without; 18 MB: 1.2 ms and 1.35 ms)
-    if (!ADD && n * 8 > DownloadRing::BYTES && n * 8 <= 2 * DownloadRing::BYTES) {
-        const hipError_t err =
-            hipMemcpyAsync(out, from, (size_t)n * 8, hipMemcpyDeviceToHost, stream);
-        const hipError_t done = hipStreamSynchronize(stream);
-        return err == hipSuccess ? done : err;
-    }
     return download(ring, from, n * 8, stream, [out](const char *src, int64_t lo, int64_t hi) {
         const double *s = (const double *)src;
         double *o = out + lo / 8;

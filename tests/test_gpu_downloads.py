@@ -16,10 +16,11 @@ from test_gpu_dmat_band import dmat_store, with_model
 pytestmark = pytest.mark.gpu
 
 
-def test_matrix_is_added():
+@pytest.mark.parametrize("n_par", [46, 56])
+def test_matrix_is_added(n_par):
     case = with_model(W.random_case(3), 2, 1)
     g, p = case.g, case.pairs
-    g.num_bins_r_par, g.num_bins_r_trans = 46, 20
+    g.num_bins_r_par, g.num_bins_r_trans = n_par, 20
     with_model(case, 2, 1)
     store = dmat_store(case.store, 0, (1,))
     eng = get_engine(0)
@@ -30,7 +31,7 @@ def test_matrix_is_added():
     nb = g.num_bins_r_par * g.num_bins_r_trans
     nm = g.num_model_bins_r_par * g.num_model_bins_r_trans
     shapes = [nb, nb * nm, nm, nm, nm, nm]
-    assert 8 * nb * nm > 1.5 * 2 ** 23
+    assert (8 * nb * nm > 2 ** 24) == (n_par > 46) and 8 * nb * nm > 1.5 * 2 ** 23
     rng = np.random.default_rng(1)
     start = [rng.integers(1, 9, n).astype(float) for n in shapes]
     out = [x.copy() for x in start]
@@ -79,13 +80,12 @@ def test_two_contexts_at_once():
 
 
 def test_sizes_around_a_chunk():
-    """Results of one chunk, just below and just above, of two chunks and of more, one after
-    the other in one context, so that the ring grows; the matrix is symmetric by construction, so
-    that a piece in the wrong place shows."""
+    """Results around the smallest block (64 KB), one and two chunks of 1 MB, and 16 MB, where the
+    chunks grow and other threads take part, one after the other in one context."""
     rng = np.random.default_rng(4)
     eng = Engine(0)
     try:
-        for bins in (3, 90, 91, 1023, 1024, 1025, 1448, 1449, 1774, 100):
+        for bins in (3, 90, 91, 362, 363, 512, 513, 1448, 1449, 1774, 100):
             xi, w = rng.normal(size=(20, bins)), rng.uniform(0.5, 2, (20, bins))
             cov = eng.cov_subsample(xi, w)[0]
             mean = (xi * w).sum(0) / w.sum(0)
