@@ -80,10 +80,10 @@ def cpu_cores():
         return os.cpu_count() or 1
 
 
-def measured_traffic(workload, scale, kernel="xi_kernel"):
+def measured_traffic(workload, scale, kernel="xi_kernel", instance=None):
     """HBM bytes of one step of the pair kernel (all its launches), measured with FETCH_SIZE +
     WRITE_SIZE (each scaled by the same counters on a plain copy), as recorded beside the
-    profiles."""
+    profiles; 0 when the record is of another kernel instance than ``instance``."""
     path = os.path.join(ROOT, "profiles", "%s_hbm_traffic.json" % kernel)
     try:
         with open(path) as f:
@@ -91,7 +91,9 @@ def measured_traffic(workload, scale, kernel="xi_kernel"):
     except (OSError, ValueError):
         return 0.0
     entry = table.get("%s@%g" % (workload, scale))
-    return float(entry["traffic_bytes"]) if entry else 0.0
+    if not entry or (instance and entry["kernel"].replace(" ", "") != instance.replace(" ", "")):
+        return 0.0
+    return float(entry["traffic_bytes"])
 
 
 def copy_probe(eng, mib):
@@ -267,8 +269,6 @@ def bench_xi(args):
     upload_s = time.time() - t2
     log("device %s: upload %.1f s" % (info["name"], upload_s))
 
-    if args.traffic_bytes < 0:
-        args.traffic_bytes = measured_traffic(args.workload, args.scale)
     if args.copy_probe > 0:
         copy_probe(eng, args.copy_probe)
 
@@ -289,14 +289,17 @@ def bench_xi(args):
     # the operations the kernel itself executes: it walks only the pixel pairs left after
     # the r_par / r_trans window pruning
     executed = FLOPS_EVALUATED * rep["visited_pairs"] + FLOPS_ACCEPTED_EXTRA * rep["accepted_pairs"]
+    # the run-walk instance runs whenever any task took the walk
+    kernel = ("picca::xi_kernel<0,false,false,false,true,%s>"
+              % ("true" if rep["walk_tasks"] > 0 else "false"))
+    if args.traffic_bytes < 0:
+        args.traffic_bytes = measured_traffic(args.workload, args.scale, instance=kernel)
     roofline = {"bound": "valu", "achieved": achieved, "peak": FP64_VALU_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": achieved / FP64_VALU_PEAK_TFLOPS,
                 "traffic": args.traffic_bytes if args.traffic_bytes > 0 else None,
                 "flops_per_launch": flops,
                 "executed_tflops": executed / (kernel_ms / 1e3) / 1e12,
-                # the run-walk instance runs whenever any task took the walk
-                "kernel": "picca::xi_kernel<0,false,false,false,true,%s>"
-                          % ("true" if rep["walk_tasks"] > 0 else "false"),
+                "kernel": kernel,
                 "kernel_ms": kernel_ms,
                 "hbm_gbs_at_traffic": (args.traffic_bytes / (kernel_ms / 1e3) / 1e9
                                        if args.traffic_bytes > 0 else None)}

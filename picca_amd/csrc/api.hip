@@ -318,9 +318,9 @@ int picca_xi_set_pairs(picca_ctx *ctx, int64_t num_pairs, const int32_t *pair_a,
     });
     // groups: <= XI_GROUP_PAIRS consecutive pairs of one row, half as many when the list holds
     // fewer than 16 full groups per CU: the waves of a workgroup wait for each other at a
-    // group's end, and the last groups leave CUs idle.  125k pairs with the half-plate cut: 23.6
-    // ms against 25.7 ms, signed r_par 32.8 / 34.0, log grid 4.29 / 4.28; 16 a group there 4.71,
-    // and 32 on 2.7M pairs 345.4 ms against 342.4 ms.
+    // group's end, and the last groups leave CUs idle.  125k pairs with the half-plate cut: 20.4
+    // ms against 22.0 ms, signed r_par 29.3 / 30.5, log grid 4.11 / 4.12 (16 a group 4.71 against
+    // 4.29); 32 on 2.7M pairs 345.4 ms against 342.4 ms.
     const int64_t full = (int64_t)16 * picca::XI_GROUP_PAIRS * ctx->num_cus;
     const int64_t per_group = num_pairs < full ? picca::XI_GROUP_PAIRS / 2 : picca::XI_GROUP_PAIRS;
     ctx->h_group_begin.clear();
@@ -1102,16 +1102,15 @@ bool power_of_two_times(int n, int base) {
 }
 
 // The kernels for pairs without cuts (dmat_band_kernel.hip): takes the pairs they cover from the
-// list and puts what is left into `rest`.  Rule, per call: standard
-// binning without a pair-redshift cut, model bins that split the data bins in 2^k parts, and
-// either the auto-correlation from r_par_min == 0 (with LDS for a row of model bins) or the
-// signed r_par of forest x quasar pairs; per pair: no zerr or same-half-plate cut, the forests
-// (of a quasar's pair: the first) with no negative r_trans, a proper fit normalisation and strictly rising r_comov and
-// dist_m whose steps lie above the rounding margins in both coordinates (the run walk's
-// condition; 1e4 margins, so that the index tables' 1e-3 of a step covers the rounding too) and
-// level weights (level_values), and
-// a projected delta2, or with signed r_par a one-pixel delta2 that is not projected and xcf's
-// count pass.
+// list and puts what is left into `rest`.  Rule, per call: standard binning without a
+// pair-redshift cut, model bins that split the data bins in 2^k parts, and either the
+// auto-correlation from r_par_min == 0 (with LDS for a row of model bins) or the signed r_par of
+// forest x quasar pairs; per pair: no zerr or same-half-plate cut, no negative r_trans, the forests
+// (of a quasar's pair: the first) with a proper fit normalisation, level weights (level_values) and
+// strictly rising r_comov and dist_m whose steps lie above the rounding margins in both
+// coordinates (the run walk's condition; 1e4 margins, so that the index tables' 1e-3 of a step
+// covers the rounding too), and a projected delta2, or with signed r_par a one-pixel delta2 that is
+// not projected and xcf's count pass.
 int dmat_run_band(DmatRun &R, const DmatPairList &L, DmatPairList &rest) {
     picca_ctx *ctx = R.ctx;
     const picca::DmatConst &C = R.C;

@@ -3,10 +3,10 @@
 // A copy into the caller's pageable pages runs at 18 GB/s, one thread filling fresh memory for
 // it at 4 to 5 GB/s; a copy into pinned memory runs at 57 GB/s, and the host threads move (or
 // add) a chunk on while the next is copied.  A 5000 x 5000 matrix (forest x quasar distortion,
-// 3000 forests) takes the call from 64 ms to 21 ms, a 2500 x 2500 one (covariance of 1196
-// samples, whose inputs are now scanned by all threads) from 8.3 ms to 4.3 ms, the six results
-// of 20 000 continuum fits in one copy from 0.76 ms to 0.71 ms.  Chunks of 4 MB: 4.8 ms for the
-// covariance.
+// 3000 forests) takes the call from 64 ms to 19 ms, a 2500 x 2500 one (covariance of 1196
+// samples, whose inputs are now scanned by all threads) from 8.2 ms to 4.4 ms, the six results
+// of 20 000 continuum fits in one copy from 0.76 ms to 0.69 ms.  Chunks of 4 MB instead of 8: 4.8 ms
+// against 4.3 ms for the covariance.
 #pragma once
 
 #include <hip/hip_runtime.h>

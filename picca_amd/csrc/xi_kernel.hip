@@ -35,12 +35,12 @@
 //   * the cross-correlation's (signed r_par) histogram, 100 x 50 bins in the usual run, does
 //     not fit in LDS: the host runs one launch per window of r_par rows, each pruned to the
 //     window's r_par limits, so that a pair's runs are split over the launches and not
-//     walked twice.  400 x 400 forests of the 0.8 A grid (6.2e10 evaluated pixel pairs): 34 ms,
-//     against 1103 ms for the general loop with its runs added straight to the HBM rows;
+//     walked twice.  400 x 400 forests of the 0.8 A grid (6.2e10 evaluated pixel pairs): 31 ms,
+//     against 1090 ms for the general loop with its runs added straight to the HBM rows;
 //   * cuts: a lane walks the window of delta2 inside the pair-redshift cut, the runs of r_par
 //     row 0 of a pair of one half plate are dropped, and the tasks the walk cannot take (a
 //     zerr cut, z not rising along delta2) take the pair loop.  500 forests of that grid with
-//     the half-plate cut: 25.9 ms, against 61.2 ms for the general loop, which evaluates every
+//     the half-plate cut: 22 ms, against 62 ms for the general loop, which evaluates every
 //     pair with the reference's arithmetic.
 //
 // Arithmetic: r_par, r_trans and the bin index follow the reference's FP64 operations

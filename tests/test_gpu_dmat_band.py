@@ -176,7 +176,8 @@ def check_quasars(case, kp, kt, seed=0, orders=(0, 1), sums=None):
     return check_quasar_pairs(case, new, args, kp, kt, sums)
 
 
-def check_quasar_pairs(case, new, args, kp, kt, sums=None):
+def check_quasar_pairs(case, new, args, kp, kt, sums=None, copies=1):
+    """copies: times that the pair list repeats, each of which adds the same to the result."""
     g = case.g
     g.x_correlation = True
     with_model(case, kp, kt)
@@ -188,14 +189,14 @@ def check_quasar_pairs(case, new, args, kp, kt, sums=None):
     nb = g.num_bins_r_par * g.num_bins_r_trans
     ref = [np.zeros(nb), np.zeros(nb * nm)] + [np.zeros(nm) for _ in range(4)]
     stats = np.zeros(4, dtype=np.int64)
-    for x, y, angle in zip(*args[:3]):
+    for x, y, angle in zip(*(v[:len(v) // copies] for v in args[:3])):
         i, j = (slice(new.offsets[k], new.offsets[k + 1]) for k in (x, y))
         O.xdmat_forest(params, new.log_lambda[i], new.r_comov[i], new.dist_m[i], new.z[i],
                        new.weights[i], new.r_comov[j], new.dist_m[j], new.z[j], new.weights[j],
                        [angle], ref, new.order[x], stats)
     ref[1] = ref[1].reshape(nb, nm)
-    assert list(mine[6]) == list(stats) and stats[0] > 0
-    assert_outputs_close(mine[:6], ref)
+    assert list(mine[6]) == list(copies * stats) and stats[0] > 0
+    assert_outputs_close(mine[:6], [copies * x for x in ref])
     assert_routes(eng, len(args[0]), sums, None)
     return eng.dmat_routes()
 
@@ -207,11 +208,12 @@ def test_quasars_on_exact_bin_edges(kp, kt, angle):
     check_quasars(lattice_case(angle), kp, kt, sums=taken)
 
 
-@pytest.mark.parametrize("limit", ["r_par_min", "r_par_max"])
-def test_quasar_pairs_handed_back(limit):
+@pytest.mark.parametrize("limit,copies", [("r_par_min", 1), ("r_par_max", 1),
+                                          ("r_par_max", 300)])
+def test_quasar_pairs_handed_back(limit, copies):
     """A pixel at r_par == r_par_min, which xcf's count pass leaves out, and one just below
     r_par_max whose distance from r_par_min rounds to the whole range: its pair goes back to the
-    general kernels, the others stay."""
+    general kernels, the others stay; also with the whole list several times over."""
     angle = 0.02
     case = W.random_case(3)
     g = case.g
@@ -232,8 +234,9 @@ def test_quasar_pairs_handed_back(limit):
         if found:
             break
     assert found
-    routes = check_quasar_pairs(case, new, args, 2, 1)
-    assert 0 < routes["handed_back"] < routes["sums"]
+    routes = check_quasar_pairs(case, new, tuple(np.tile(x, copies) for x in args), 2, 1,
+                                copies=copies)
+    assert copies <= routes["handed_back"] < routes["sums"]
 
 
 @pytest.mark.parametrize("angle", [0.004, 0.03])

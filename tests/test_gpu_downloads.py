@@ -1,5 +1,6 @@
-"""Results of more than one chunk of the pinned download ring: a matrix of 13.5 MB added to what
-the caller's array holds, and the six interleaved results of 300 000 continuum fits."""
+"""Results of more than one chunk of the pinned download ring: matrices of 13.5 MB (one thread) and
+20 MB (several) added to what the caller's array holds, the six interleaved results of 300 000
+continuum fits, sizes around a chunk, and two contexts' downloads at once."""
 import ctypes
 from concurrent.futures import ThreadPoolExecutor
 
