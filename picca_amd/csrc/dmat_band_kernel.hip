@@ -75,7 +75,7 @@ __device__ __forceinline__ void lds_add(double *p, double v) {
 
 struct BandPair {
     int a, b, la, lb;
-    int64_t oa, ob, at_a, at_b;
+    int64_t oa, ob;
     double cos_half, sin_half;
     double inv_w1, inv_w2, inv_s1, inv_s2;
     bool order1, order2;
@@ -89,8 +89,6 @@ __device__ BandPair load_band_pair(const DmatForests &F, const DmatBandSlots &P,
     q.la = (int)(uniform_i64(F.off[q.a + 1]) - q.oa);
     q.ob = uniform_i64(F.off[q.b]);
     q.lb = (int)(uniform_i64(F.off[q.b + 1]) - q.ob);
-    q.at_a = uniform_i64(P.slot[s].at_a);
-    q.at_b = uniform_i64(P.slot[s].at_b);
     q.cos_half = uniform_f64(P.cs[2 * s]);
     q.sin_half = uniform_f64(P.cs[2 * s + 1]);
     q.inv_w1 = 1.0 / uniform_f64(F.sum_w[q.a]);
@@ -326,6 +324,7 @@ __global__ __launch_bounds__(DMAT_BAND_PASS_BLOCK) void dmat_band_pass_kernel(
     const int u0 = uniform_int(P.slot[s].u0), nu = uniform_int(P.slot[s].nu);
     const int t0 = uniform_int(P.slot[s].t0), nt = uniform_int(P.slot[s].nt);
     const int64_t urow = uniform_i64(P.slot[s].u_row), trow = uniform_i64(P.slot[s].t_row);
+    const int64_t at_b = uniform_i64(P.slot[s].at_b);
     const int kp = C.npm / C.np, kt = C.ntm / C.nt;
     int32_t *rng = (int32_t *)smem;                       // [nu][4]
     double *acc = (double *)(smem + ((16 * (size_t)C.ntm + 15) & ~(size_t)15));
@@ -392,7 +391,7 @@ __global__ __launch_bounds__(DMAT_BAND_PASS_BLOCK) void dmat_band_pass_kernel(
                 // the lane's pixels of this band of rows
                 const BandAxis A = band_trans_axis(d1, mul_t, q.sin_half, C.rtmax, C.ntm,
                                                    M.fast_t);
-                const BandTable B = load_table(W.table_d + q.at_b, Bd, q.lb);
+                const BandTable B = load_table(W.table_d + at_b, Bd, q.lb);
                 auto v = [&](int p) { return Bd[p]; };
                 if (uc0 > u0) L.j_lo = max(T.j_lo, band_edge(A, B, v, uc0));
                 if (uc0 + rows < u0 + nu) L.j_hi = min(T.j_hi, band_edge(A, B, v, uc0 + rows));
@@ -401,7 +400,7 @@ __global__ __launch_bounds__(DMAT_BAND_PASS_BLOCK) void dmat_band_pass_kernel(
                     L.j_lo = T.j_lo;
                 }
             }
-            BandPassMem mem{Br, Bd, F.w + q.ob, F.z + q.ob, W.pre_b + q.at_b, acc, rng,
+            BandPassMem mem{Br, Bd, F.w + q.ob, F.z + q.ob, W.pre_b + at_b, acc, rng,
                             &s_special, stride, nu, uc0 * C.npm, u0, i, l1, &s_const, 0, -1, 0, 0};
             walk_lane<false, true, DmatAcc>(M, T, L, mem, active);
             mem.note();
@@ -673,7 +672,8 @@ __global__ __launch_bounds__(DMAT_BAND_FILL_BLOCK, 3) void dmat_band_fill_kernel
                         const int np_ = side ? q.la : q.lb;   // pixels of the partner
                         const double *__restrict__ Pr = F.r + op;
                         const double *__restrict__ Pd = F.d + op;
-                        const int64_t at = side ? q.at_a : q.at_b;   // of the partner
+                        const int64_t at = uniform_i64(side ? P.slot[s].at_a   // of the partner
+                                                            : P.slot[s].at_b);
                         const double2 *__restrict__ pre =
                             (const double2 *)((side ? W.pre_a : W.pre_b) + at);
                         const BandTable Tr = load_table(W.table_r + at, Pr, np_);
