@@ -440,8 +440,9 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
 
     int j_lo = 0, j_hi = lb;
     bool pruned = false;
+    int flags_b = 0;
     if (MODE == MODE_STANDARD && (C.flags & XI_PRUNE) && cos_half > 0 &&
-        (uniform_int(F.mono[b]) & 3) == 3) {
+        ((flags_b = uniform_int(F.mono[b])) & 3) == 3) {
         pruned = true;
         const double r_min = wave_min(active ? r1 : INFINITY);
         const double r_max = wave_max(active ? r1 : -INFINITY);
@@ -481,8 +482,7 @@ __device__ void xi_task(const XiConst &C, const XiConst &C_lds, const ForestView
         const double z_hi = CUTS && (C.flags & XI_HAS_ZMAX) ? C.zmax : INFINITY;
         if (CUTS || XCORR) {
             const int need = FOREST_LEVEL_W | FOREST_LEVEL_DW | (z_cut ? FOREST_RISES_Z : 0);
-            walk_cuts = !zerr_on && !(XCORR && shp) &&
-                        (uniform_int(F.mono[b]) & need) == need;
+            walk_cuts = !zerr_on && !(XCORR && shp) && (flags_b & need) == need;
         }
         if (WALK && (C.flags & XI_WALK) && pruned && walk_cuts) {
             // Run walk (xi_walk.h) for the tasks walk_task admits; otherwise the pair loop
